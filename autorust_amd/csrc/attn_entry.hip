@@ -94,7 +94,7 @@ __device__ __forceinline__ AttnParams dense_params(const void *q, const void *k,
 }  // namespace
 
 namespace {
-__device__ __forceinline__ void flash_f32_entry(float *lds, const float *Q, const float *K, const float *V, float *O,
+__device__ __forceinline__ void flash_f32_entry(unsigned char *lds, const float *Q, const float *K, const float *V, float *O,
                                                 const float *M, const int *L, int N, int head_dim, int causal, int has_mask,
                                                 int hq, int hkv)
 {
@@ -112,11 +112,11 @@ __device__ __forceinline__ void flash_f32_entry(float *lds, const float *Q, cons
     p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
     const int wg = linear_wg();
     if (head_dim == 64) {
-        if (causal) flash_f32_body<64, 4, true>(p, lds, wg);
-        else flash_f32_body<64, 4, false>(p, lds, wg);
+        if (causal) flash_f32_body<64, 4, 1, true>(p, lds, wg);
+        else flash_f32_body<64, 4, 1, false>(p, lds, wg);
     } else if (head_dim == 128) {
-        if (causal) flash_f32_body<128, 4, true>(p, lds, wg);
-        else flash_f32_body<128, 4, false>(p, lds, wg);
+        if (causal) flash_f32_body<128, 4, 1, true>(p, lds, wg);
+        else flash_f32_body<128, 4, 1, false>(p, lds, wg);
     }
 }
 }  // namespace
@@ -126,7 +126,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_f32(const float *Q, c
                                                                 const float *M, int N, int head_dim, int causal,
                                                                 int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[flash_f32_lds_floats<128>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<128, 4, 1>()];
     flash_f32_entry(lds, Q, K, V, O, M, nullptr, N, head_dim, causal, has_mask, hq, hkv);
 }
 
@@ -134,7 +134,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_f32_lens(const float 
                                                                      const float *M, const int *L, int N, int head_dim,
                                                                      int causal, int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[flash_f32_lds_floats<128>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<128, 4, 1>()];
     flash_f32_entry(lds, Q, K, V, O, M, L, N, head_dim, causal, has_mask, hq, hkv);
 }
 
@@ -142,7 +142,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_fwd(const float *Q, cons
                                                              float *LSE, const float *M, int N, int head_dim, int causal,
                                                              int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[flash_f32_lds_floats<128>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<128, 4, 1>()];
     FlashF32Params p = {};
     p.q = Q; p.k = K; p.v = V; p.o = O; p.lse = LSE;
     p.mask = has_mask ? M : nullptr;
@@ -156,11 +156,11 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_fwd(const float *Q, cons
     p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
     const int wg = linear_wg();
     if (head_dim == 64) {
-        if (causal) flash_f32_body<64, 4, true>(p, lds, wg);
-        else flash_f32_body<64, 4, false>(p, lds, wg);
+        if (causal) flash_f32_body<64, 4, 1, true>(p, lds, wg);
+        else flash_f32_body<64, 4, 1, false>(p, lds, wg);
     } else if (head_dim == 128) {
-        if (causal) flash_f32_body<128, 4, true>(p, lds, wg);
-        else flash_f32_body<128, 4, false>(p, lds, wg);
+        if (causal) flash_f32_body<128, 4, 1, true>(p, lds, wg);
+        else flash_f32_body<128, 4, 1, false>(p, lds, wg);
     }
 }
 
@@ -170,7 +170,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_fwd(const float *Q, cons
 // only (the reference's own head size); any other returns without writing.  LSE may be null.
 namespace {
 __device__ __forceinline__ void flash_f32_short(const float *Q, const float *K, const float *V, float *O, float *LSE,
-                                                const float *M, int N, int causal, int has_mask, int hq, int hkv, float *lds)
+                                                const float *M, int N, int causal, int has_mask, int hq, int hkv, unsigned char *lds)
 {
     FlashF32Params p = {};
     p.q = Q; p.k = K; p.v = V; p.o = O; p.lse = LSE;
@@ -184,8 +184,8 @@ __device__ __forceinline__ void flash_f32_short(const float *Q, const float *K, 
     dense(p.os, hq, N, 64);
     p.scale = 0.125f;
     const int wg = linear_wg();
-    if (causal) flash_f32_body<64, 4, true, true>(p, lds, wg);
-    else flash_f32_body<64, 4, false, true>(p, lds, wg);
+    if (causal) flash_f32_body<64, 1, 4, true>(p, lds, wg);
+    else flash_f32_body<64, 1, 4, false>(p, lds, wg);
 }
 }  // namespace
 
@@ -194,7 +194,7 @@ extern "C" __global__ void __launch_bounds__(256, 2) ar_flash_f32_short(const fl
                                                                          const float *M, int N, int head_dim, int causal,
                                                                          int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[flash_f32_lds_floats<64, 4, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<64, 1, 4>()];
     if (head_dim != 64) return;
     flash_f32_short(Q, K, V, O, nullptr, M, N, causal, has_mask, hq, hkv, lds);
 }
@@ -203,7 +203,7 @@ extern "C" __global__ void __launch_bounds__(256, 2) ar_fl_fwd_short(const float
                                                                       float *LSE, const float *M, int N, int head_dim,
                                                                       int causal, int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[flash_f32_lds_floats<64, 4, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<64, 1, 4>()];
     if (head_dim != 64) return;
     flash_f32_short(Q, K, V, O, LSE, M, N, causal, has_mask, hq, hkv, lds);
 }

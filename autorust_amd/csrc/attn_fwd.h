@@ -125,6 +125,25 @@ __device__ __forceinline__ float xhalf_sum(float x)
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+typedef __attribute__((address_space(3))) void *lds_ptr_t;
+
+// s_waitcnt vmcnt(n) only (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
+template <int N>
+__device__ __forceinline__ void wait_vmem_le()
+{
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// f(integral_constant<int, A>) ... f(integral_constant<int, B - 1>), unrolled at compile time
+template <int A, int B, typename F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    if constexpr (A < B) {
+        f(std::integral_constant<int, A>{});
+        static_for<A + 1, B>(f);
+    }
+}
+
 // Four keys of one channel: the transposing LDS read described above.
 __device__ __forceinline__ uint2 lds_read_tr16(const unsigned char *p)
 {

@@ -52,25 +52,6 @@
 
 namespace arhip {
 
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
-
-// s_waitcnt vmcnt(n) only (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
-template <int N>
-__device__ __forceinline__ void wait_vmem_le()
-{
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-// f(integral_constant<int, A>) ... f(integral_constant<int, B - 1>), unrolled at compile time
-template <int A, int B, typename F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    if constexpr (A < B) {
-        f(std::integral_constant<int, A>{});
-        static_for<A + 1, B>(f);
-    }
-}
-
 // The 4-wave form keeps K and V in rings of their own (two and three tiles) so that two workgroups fit a compute
 // unit at D = 128; with 8-bit operands at D = 64 four whole stages fit twice as well (48 KB each), and with them the
 // four-tiles-per-trip loop and one more tile of latency cover: int8 B4 H32 N = 2048 / 8192 -7 / -5 %, causal -4 / -5 %,

@@ -11,6 +11,7 @@
 #include "flash_f32.h"
 
 #include <algorithm>
+#include <cmath>
 
 
 using namespace arhip;
@@ -113,6 +114,28 @@ static int pick_waves(arhip_device *dev, int64_t heads, int64_t N, int64_t D, bo
     return nw;
 }
 
+// Tiling of the fp32 forward: 8 or 4 waves of 32 queries that share their key tiles (81, 41: 256 and 128 queries per workgroup),
+// or 4 waves on the same 32 queries with the key tiles dealt out between them (14).  The one whose busiest compute unit is done
+// first, in units of what a workgroup of 8 waves takes for all its tiles: 4 waves alone on a CU need 0.57 of it (one wave per SIMD
+// hides less), 14 splits every tile itself instead of sharing and needs 0.2 (head size 64) or 0.29 for its eighth.  A causal
+// grid runs longest workgroup first: the longest one, or its even share where there are enough to balance; the constants on
+// top are what that leaves unbalanced, more the smaller the share of a workgroup.  us, 81 / 41 / 14: B2 H16 N2048 D64
+// 159 / 170 / 250, D128 299 / 339 / 598, causal 227 / 187 / 350; B4 H32 N2048 D128 causal 674 / 788 / 1432; B3 H16 N2048 D64
+// (a third round of 4-wave workgroups instead of a second of 8) 267 / 249 / 363; B8 H12 N197 D64 20.4 / 16.5 / 20.3;
+// B2 H12 N500 D64 36 / 25 / 21; B1 H12 N197 D64 19 / 15 / 9; B1 H4 N4096 D128 causal 411 / 283 / 166.
+static int f32_form(int64_t heads, int64_t N, int64_t D, bool causal, int cus)
+{
+    auto cost = [&](int64_t rows, double unit, double unbalanced) {
+        const int64_t nq = (N + rows - 1) / rows;
+        const double per_cu = (double)(heads * nq) / cus;
+        if (!causal) return unit * std::ceil(per_cu);
+        return unit * std::max(1.0, per_cu * (double)(nq + 1) / (double)(2 * nq)) + unbalanced;
+    };
+    const double c81 = cost(256, 1.0, 0.0), c41 = cost(128, 0.57, 0.1), c14 = cost(32, D == 64 ? 0.2 : 0.29, 0.3);
+    if (c14 < c41 && c14 < c81) return 14;
+    return c81 < c41 ? 81 : 41;
+}
+
 static void dense_strides(long s[3], int64_t H, int64_t N, int64_t D)
 {
     s[0] = (long)(H * N * D);
@@ -178,29 +201,30 @@ extern "C" int arhip_flash_fwd_lse(arhip_device *dev, const void *q, const void 
             fp.ks[i] = (long)kv_strides[i];
             fp.os[i] = (long)o_strides[i];
         }
-        // 128 queries per workgroup of 4 waves when that still fills the chip, else 32 queries whose key
-        // tiles are dealt out between the waves of the workgroup: 4 waves, or 2 when that lets every
-        // workgroup be resident at once (8 waves per CU) and 4 would need a second round
-        const bool splitk = B * Hq * ((N + 127) / 128) < 2 * (int64_t)dev->cus;
-        const int bq = splitk ? 32 : 128;
+        const int form = f32_form(B * Hq, N, D, causal != 0, dev->cus);
+        const int qw = form / 10, kw = form % 10;
+        const int bq = qw * 32;
         fp.nq = (int)((N + bq - 1) / bq);
         fp.scale = scale;
         const int64_t wgs = fp.nq * B * Hq;
         fp.total = (int)wgs;
         fp.lpt_heads = causal ? (int)(B * Hq) : 0;  // causal: longest query tile first over all heads
-        const bool two = splitk && D == 64 && wgs > 2 * (int64_t)dev->cus && wgs <= 4 * (int64_t)dev->cus;
         if (int rc = t.begin()) return rc;
-        const dim3 grid((unsigned)wgs), block(two ? 128 : 256);
-#define F32_LAUNCH(DD, NWW, SK)                                                                         \
+        const dim3 grid((unsigned)wgs), block(qw * kw * 64);
+#define F32_LAUNCH(DD, QW, KW)                                                                         \
     do {                                                                                              \
-        if (causal) hipLaunchKernelGGL((flash_f32_kernel<DD, NWW, true, SK>), grid, block, 0, dev->stream, fp);  \
-        else hipLaunchKernelGGL((flash_f32_kernel<DD, NWW, false, SK>), grid, block, 0, dev->stream, fp); \
+        if (causal) hipLaunchKernelGGL((flash_f32_kernel<DD, QW, KW, true>), grid, block, 0, dev->stream, fp);  \
+        else hipLaunchKernelGGL((flash_f32_kernel<DD, QW, KW, false>), grid, block, 0, dev->stream, fp); \
     } while (0)
-        if (D == 64) {
-            if (two) F32_LAUNCH(64, 2, true); else if (splitk) F32_LAUNCH(64, 4, true); else F32_LAUNCH(64, 4, false);
-        } else {
-            if (splitk) F32_LAUNCH(128, 4, true); else F32_LAUNCH(128, 4, false);
-        }
+#define F32_FORMS(DD)                                                                                 \
+    do {                                                                                              \
+        if (form == 81) F32_LAUNCH(DD, 8, 1);                                                         \
+        else if (form == 41) F32_LAUNCH(DD, 4, 1);                                                    \
+        else F32_LAUNCH(DD, 1, 4);                                                                    \
+    } while (0)
+        if (D == 64) F32_FORMS(64);
+        else F32_FORMS(128);
+#undef F32_FORMS
 #undef F32_LAUNCH
         arhip_note_selected(ARHIP_K_FLASH_F32);
         return t.end();

@@ -6,25 +6,35 @@
 // exponential is v_exp_f32 (base 2, 1 ulp) on logits scaled by scale * log2(e), where the reference
 // calls expf on logits scaled by scale: the same function to a few ulp.
 //
-// The two contractions run on the fp32 matrix instruction v_mfma_f32_32x32x2_f32 (fp32 in,
-// fp32 accumulate) with the same decomposition as the bf16 kernel: a wave owns 32 queries and
-// computes S^T = K . Q^T, so each lane owns one query (column lane%32) and 16 of a block's 32
+// The two contractions run on the bf16 matrix instruction with every fp32 operand taken as the exact sum of three
+// bf16 values (f32_split.h), with the decomposition of the bf16 kernel: a wave owns 32 queries and
+// computes S^T = K . Q^T, so each lane owns one query (column lane%32) and 16 of a tile's 32
 // keys; O^T = V^T . P^T keeps one query per lane, and the online-softmax state is per lane.
-//   A[32 x 2] . B[2 x 32]: lane holds A[lane%32][lane/32] and B[lane/32][lane%32]
 //   result C[32 x 32]: lane holds column lane%32, rows 8*(r/4) + 4*(lane/32) + r%4
-// The order of the channels inside Q.K^T is free as long as Q and K agree, so MFMA step s of
-// lane half h multiplies channel h*D/2 + s: every lane reads its K row as D/2 consecutive
-// floats.  For P.V the step (g, t) multiplies key 8g + 4h + t, which is exactly the key the
-// S^T result left in register 4g + t of that lane.
+// P is split in registers, in the order the S^T result left it there; Q is split once, K and V while they are staged.
+//
+// Bound: the matrix pipe, at a clock that its power draw sets.  Against the same kernel on v_mfma_f32_32x32x2_f32 (which
+// never runs beside a vector instruction): B2 H16 N2048 D128 639 -> 299 us (107 -> 230 TFLOP/s of attention, 1380 TFLOP/s of
+// bf16 products; a loop of nothing but such products on random data holds 1740 ... 1840), D64 290 -> 159 us, causal D128 352 ->
+// 187 us, B8 H6 N789 D64 87 -> 55 us, B8 H12 N197 D64 23.3 -> 16.5 us, B1 H12 N197 D64 9.9 -> 9.0 us.  Relative error (2-norm,
+// against float64) on the same inputs: 9.1e-7 -> 7.7e-7, 8.7e-7 -> 7.4e-7, 4.5e-7 -> 3.8e-7, 3.9e-7 -> 4.9e-7, 3.3e-7 -> 3.0e-7,
+// 3.1e-7 -> 2.4e-7.
+// Tried on B2 H16 N2048 (D64 / D128): the same loop with the phases one after the other, as the compiler schedules them
+// 184 / 402 us; interleaved by hand but with the compiler free to sink vector work past the matrix instructions 178 / 331 us;
+// values pinned where they are computed 168 / 336 us; tiles through registers instead of straight to LDS 168 / 325 us; a row
+// sum above 16 moving the exponent reference to the maximum instead of 2 above it 175 / 321 us (the move stalls the other waves
+// at the barrier).
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <type_traits>
 
+#include "f32_split.h"
+
 namespace arhip {
 
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef f32x16 f32x16_t;
 
 constexpr int F32_BK = 32;  // keys per tile
 
@@ -41,39 +51,34 @@ struct FlashF32Params {
     float scale;
 };
 
-// LDS floats flash_f32_body needs: one padded K tile and one V tile (one pair per wave with SPLITK)
-template <int D, int NW = 1, bool SPLITK = false>
-constexpr int flash_f32_lds_floats()
+// LDS bytes flash_f32_body needs: per key group three K tiles, two V tiles and the tile pair in flight from memory, or the merge of the key groups' partial results (which reuses them)
+template <int D, int QW, int KW>
+constexpr int flash_f32_lds_bytes()
 {
-    return (SPLITK ? NW : 1) * (F32_BK * (D + 4) + F32_BK * D);
+    constexpr int tiles = (QW == 1) ? 0 : KW * (5 * SplitTile<D>::BYTES + 2 * 32 * D * 4);
+    constexpr int merge = (KW == 1) ? 0 : QW * KW * (32 * (D + 4) + 64) * 4;
+    return tiles > merge ? tiles : merge;
 }
 
-// The kernel body.  lds: flash_f32_lds_floats<D, NW, SPLITK>() floats of workgroup memory, 16-byte
+// The kernel body.  lds: flash_f32_lds_bytes<D, QW, KW>() bytes of workgroup memory, 16-byte
 // aligned; wg_linear: this workgroup's index in [0, nq * B * Hq).
 //
-// SPLITK (few, short heads: the launch would otherwise leave most SIMDs idle behind one wave's
-// chain of matrix instructions): the NW waves of a workgroup share the same 32 queries and deal
-// the key tiles out between them (wave w takes tiles w, w + NW, ...), each staging its own tiles
-// in its own LDS slab with no workgroup barrier; at the end the partial (m, l, O) of the waves are
-// merged through LDS: m = max m_w, l = sum l_w e^(m_w - m), O = sum O_w e^(m_w - m).
-template <int D, int NW, bool CAUSAL, bool SPLITK = false>
-__device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *lds, int wg_linear)
+// A workgroup is QW x KW waves: QW blocks of 32 queries, and KW groups of waves among which the key tiles are dealt
+// out (group g takes tiles g, g + KW, ...); the partial (m, l, O) of the groups are merged through LDS at the
+// end: m = max m_g, l = sum l_g e^(m_g - m), O = sum O_g e^(m_g - m).  The waves of a group share their K and V
+// tiles: each splits its share of a tile into the three bf16 parts and writes them to LDS.  With QW = 1 there is nothing to
+// share, and a wave loads and splits its own operands without LDS or barriers.
+template <int D, int QW, int KW, bool CAUSAL>
+__device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned char *lds, int wg_linear)
 {
-    constexpr int T = SPLITK ? 64 : NW * 64;      // threads staging one tile
-    constexpr int BQ = SPLITK ? 32 : NW * 32;
-    constexpr int HALF = D / 2;          // channels per lane half
-    constexpr int KROW = D + 4;          // padded K row (floats): conflict-free 128-bit row reads
-    constexpr int DB = D / 32;
-    constexpr int CHUNKS = F32_BK * D / 4;             // float4 chunks per K (or V) tile
-    constexpr int PER_THREAD = (CHUNKS + T - 1) / T;
-    static_assert(CHUNKS % T == 0, "tile staging must divide evenly");
+    constexpr int T = QW * 64;           // threads staging one tile
+    constexpr int BQ = QW * 32;
+    constexpr int DB = D / 32, KSTEPS = D / 16;
+    using Tile = SplitTile<D>;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // a scalar: tile indices and K/V tile addresses stay scalar
-    constexpr int SLAB = F32_BK * KROW + F32_BK * D;
-    float *ks = lds + (SPLITK ? wave * SLAB : 0);  // [F32_BK][KROW]
-    float *vs = ks + F32_BK * KROW;                // [F32_BK][D]
-    const int stid = SPLITK ? lane : tid;          // index among the threads staging a tile
+    const int qw = wave % QW, kg = wave / QW;
     const int i32 = lane & 31, h = lane >> 5;
     // causal: the longest query tiles first over the whole grid, so that no head's long tiles are left for the end
     // (these kernels are bound by the matrix pipe at any grid size: every workgroup may stream its own K/V)
@@ -91,7 +96,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *l
     const int b = bh / p.Hq, head = bh - b * p.Hq;
     const int N = p.N;
     const int qblk = qt * BQ;
-    const int wq0 = qblk + (SPLITK ? 0 : wave * 32);
+    const int wq0 = qblk + qw * 32;
     const int q_row = wq0 + i32;
 
     int kvl = N;
@@ -102,23 +107,21 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *l
     int kend = kvl;
     if (CAUSAL) kend = min(kend, min(N, qblk + BQ));
     const int ntiles = (kend + F32_BK - 1) / F32_BK;
-    const int my_tiles = CAUSAL ? min(ntiles, (wq0 + 31) / F32_BK + 1) : ntiles;
+    // tiles this wave computes on: under the causal mask none past its last query, and none for queries past the end
+    const int my_tiles = wq0 >= N ? 0 : CAUSAL ? min(ntiles, (wq0 + 31) / F32_BK + 1) : ntiles;
 
     const int kvh = head / (p.Hq / p.Hkv);
     const size_t kv_off = (size_t)b * p.ks[0] + (size_t)kvh * p.ks[1];
     const size_t k_rs = (size_t)p.ks[2];
-    const char *kp = (const char *)(p.k + kv_off);
-    const char *vp = (const char *)(p.v + kv_off);
+    const float *kp = p.k + kv_off;
+    const float *vp = p.v + kv_off;
 
-    // Q: this lane's half of its query row (rows past N read row N-1; never stored)
-    float qr[HALF];
+    // Q: this lane's part of its query row as matrix operands (rows past N read row N-1; never stored)
+    split8 qr[KSTEPS];
     {
-        const float *qp = p.q + (size_t)b * p.qs[0] + (size_t)head * p.qs[1] + (size_t)min(q_row, N - 1) * p.qs[2] + h * HALF;
+        const float *qp = p.q + (size_t)b * p.qs[0] + (size_t)head * p.qs[1] + (size_t)min(q_row, N - 1) * p.qs[2] + h * 8;
 #pragma unroll
-        for (int s = 0; s < HALF; s += 4) {
-            const float4 x = *(const float4 *)(qp + s);
-            qr[s] = x.x; qr[s + 1] = x.y; qr[s + 2] = x.z; qr[s + 3] = x.w;
-        }
+        for (int s = 0; s < KSTEPS; ++s) qr[s] = split_8(*(const float4 *)(qp + 16 * s), *(const float4 *)(qp + 16 * s + 4));
     }
 
     f32x16_t oacc[DB];
@@ -128,59 +131,14 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *l
         for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
     // The softmax runs on base-2 exponentials: logits are scaled by scale * log2(e) and the running
     // maximum is kept in those units (one multiply-add and one v_exp_f32 per logit).
-    constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
+    constexpr float LN2 = 0.69314718055994530942f;
     const float c2 = p.scale * LOG2E;
     float m_run = -1e30f, l_run = 0.f;
 
-    // The global loads of a tile are issued one tile ahead of its use, into registers, so that
-    // their latency is spent under the matrix instructions of the tile before.  Thread t stages
-    // rows t / (D/4) + j * RPJ, 16 bytes at column 4 * (t % (D/4)): a per-thread byte offset on top
-    // of a scalar address per (tile, j).
-    constexpr int RPJ = T / (D / 4);
-    const int row0 = stid / (D / 4), col0 = (stid % (D / 4)) * 4;
-    const size_t voff = ((size_t)row0 * k_rs + col0) * sizeof(float);
-    float4 kx[PER_THREAD], vx[PER_THREAD];
-    auto fetch = [&](int tile) __attribute__((always_inline)) {
-        const size_t t0 = (size_t)tile * F32_BK * k_rs * sizeof(float);
-        if (tile * F32_BK + F32_BK <= kend) {
-#pragma unroll
-            for (int j = 0; j < PER_THREAD; ++j) {
-                const size_t so = t0 + (size_t)j * RPJ * k_rs * sizeof(float);
-                kx[j] = *(const float4 *)(kp + so + voff);
-                vx[j] = *(const float4 *)(vp + so + voff);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < PER_THREAD; ++j) {
-                const size_t so = t0 + (size_t)j * RPJ * k_rs * sizeof(float);
-                kx[j] = vx[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (tile * F32_BK + row0 + j * RPJ < kend) {
-                    kx[j] = *(const float4 *)(kp + so + voff);
-                    vx[j] = *(const float4 *)(vp + so + voff);
-                }
-            }
-        }
-    };
-
-    // one key tile; GENERIC: additive mask, keys past the end or hidden by the causal mask, or a
-    // negative scale (the plain path takes the maximum before scaling)
-    auto tile_body = [&](auto generic, int k0) __attribute__((always_inline)) {
+    // logits of one key tile -> probabilities, as the matrix operands of the second product; GENERIC: additive mask,
+    // keys past the end or hidden by the causal mask, or a negative scale (the plain path takes the maximum before scaling)
+    auto softmax = [&](auto generic, int k0, const f32x16_t &s, split8 (&pb)[2]) __attribute__((always_inline)) {
         constexpr bool GENERIC = decltype(generic)::value;
-        // ---- S^T = K . Q^T ----
-        f32x16_t s;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = 0.f;
-        const float *krow = &ks[i32 * KROW + h * HALF];
-#pragma unroll
-        for (int st = 0; st < HALF; st += 4) {
-            const float4 kq = *(const float4 *)(krow + st);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.x, qr[st + 0], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.y, qr[st + 1], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.z, qr[st + 2], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.w, qr[st + 3], s, 0, 0, 0);
-        }
-
-        // ---- scale, masks, online softmax ----
         float x[16];
         float m_new;
         if constexpr (GENERIC) {
@@ -190,20 +148,18 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *l
                 const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
                 float xv = s[r] * c2;
                 if (p.mask != nullptr && key < N && q_row < N) xv = fmaf(p.mask[(size_t)q_row * N + key], LOG2E, xv);
-                if (key >= kend || (CAUSAL && key > q_row)) xv = -1e30f;
+                if (key >= kend || (CAUSAL && key > q_row)) xv = -__builtin_inff();
                 x[r] = xv;
                 mx = fmaxf(mx, xv);
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            m_new = fmaxf(m_run, mx);
+            m_new = fmaxf(m_run, xhalf_max(mx));
 #pragma unroll
             for (int r = 0; r < 16; ++r) x[r] = __builtin_amdgcn_exp2f(x[r] - m_new);
         } else {
             float mx = fmaxf(s[0], s[1]);
 #pragma unroll
             for (int r = 2; r < 16; ++r) mx = fmaxf(mx, s[r]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            m_new = fmaxf(m_run, mx * c2);   // c2 >= 0 here: the largest logit is the largest product
+            m_new = fmaxf(m_run, xhalf_max(mx) * c2);   // c2 >= 0 here: the largest logit is the largest product
 #pragma unroll
             for (int r = 0; r < 16; ++r) x[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c2, -m_new));
         }
@@ -219,45 +175,328 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *l
 #pragma unroll
                 for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
         }
-
-        // ---- O^T += V^T . P^T : step (g, t) uses key 8g + 4h + t ----
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float *vrow = &vs[(8 * (r >> 2) + 4 * h + (r & 3)) * D + i32];
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-                oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[db * 32], x[r], oacc[db], 0, 0, 0);
-        }
+        pb[0] = split_8(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]);
+        pb[1] = split_8(x[8], x[9], x[10], x[11], x[12], x[13], x[14], x[15]);
+    };
+    const bool always_generic = p.mask != nullptr || !(c2 >= 0.f);
+    auto is_generic = [&](int k0) __attribute__((always_inline)) {
+        return always_generic || k0 + F32_BK > kend || (CAUSAL && k0 + F32_BK - 1 > wq0);
     };
 
-    const bool always_generic = p.mask != nullptr || !(c2 >= 0.f);
-    constexpr int STEP = SPLITK ? NW : 1;
-    const int first = SPLITK ? wave : 0;
-    if (first < ntiles) fetch(first);
-    for (int it = first; it < ntiles; it += STEP) {
-        const int k0 = it * F32_BK;
-        if (!SPLITK) __syncthreads();  // the previous tile has been consumed
+    if constexpr (QW > 1) {
+        // ---- the pipelined tile loop ----
+        // A wave issues in order, and while a matrix instruction runs the wave may issue vector instructions; so the two
+        // streams are interleaved by hand, one tile ahead (n counts the tiles of this wave's key group):
+        //   R1(n)  S(n+1) = K(n+1) . Q^T   (MFMA)  |  P(n) split into its three parts                     (VALU)
+        //   R2(n)  O^T += V(n)^T . P(n)^T  (MFMA)  |  this thread's share of K(n+3) and V(n+1) split and written to LDS,
+        //                                             P(n+1) = exp2(S(n+1) c2 - m) and its row sum        (VALU)
+        // then the check of P(n+1), one barrier, and the next tile.  K(n+3) and V(n+1) were requested from memory one
+        // tile earlier.  With three K tiles and two V tiles in LDS every fragment is read ahead of the matrix
+        // instruction that uses it, the first of a region in the region before.
+        constexpr int PER_THREAD = 2 * Tile::ITEMS / T;  // items of 8 channels a thread stages per tile, half of them K's
+        static_assert(2 * Tile::ITEMS % T == 0 && (Tile::ITEMS % T == 0 || T == 2 * Tile::ITEMS), "tile staging must divide evenly");
+        const int stid = tid - kg * T;
+        unsigned char *k_ring = lds + kg * 5 * Tile::BYTES, *v_ring = k_ring + 3 * Tile::BYTES;
+        const int tiles = (ntiles - kg + KW - 1) / KW;          // of this key group
+        const int mine = max(0, (my_tiles - kg + KW - 1) / KW);  // of them, those this wave computes on
+        const int rounds = (ntiles + KW - 1) / KW;
+        // items of K (is_v = 0) or V
+        auto item_is_v = [&](int j) __attribute__((always_inline)) { return T > Tile::ITEMS ? qw >= QW / 2 : j >= PER_THREAD / 2; };
+        // A tile pair on its way from memory goes straight to LDS (global_load_lds, 16 bytes per lane, no registers), into an area
+        // of its own per wave, where the thread that requested an item reads it back to split it: no barrier, and a whole
+        // tile of matrix instructions to arrive in.  (Inline assembly: the compiler would make every LDS read wait for every
+        // transfer in flight.)
+        const uint32_t raw_at = (uint32_t)(uintptr_t)(lds_ptr_t)(lds + KW * 5 * Tile::BYTES) + wave * PER_THREAD * 2048;
+        const unsigned char *raw = lds + KW * 5 * Tile::BYTES + wave * PER_THREAD * 2048 + lane * 16;
+        const char *src[PER_THREAD];  // the next request of every item
+        int put_at[PER_THREAD];       // its place in a split tile
+        auto item = [&](int j) __attribute__((always_inline)) { return stid + j * T - (item_is_v(j) ? Tile::ITEMS : 0); };
+        auto point = [&](int j, int n) __attribute__((always_inline)) {
+            // rows past the last visible key repeat it: their probabilities are zero, and so is what they add
+            const int row = min((n * KW + kg) * F32_BK + Tile::item_row(item(j)), kend - 1);
+            src[j] = (const char *)((item_is_v(j) ? vp : kp) + (size_t)row * k_rs + Tile::item_col(item(j)));
+        };
+        const size_t tile_step = (size_t)KW * F32_BK * k_rs * sizeof(float);
+        // moves the request of item j from tile n - 1 to tile n
+        auto next_tile = [&](int j, int n) __attribute__((always_inline)) {
+            if ((n * KW + kg) * F32_BK + F32_BK <= kend) src[j] += tile_step;
+            else point(j, n);
+        };
+        auto request = [&](int j) __attribute__((always_inline)) {
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, off"
+                         : : "s"(raw_at + j * 2048), "v"(src[j]) : "memory", "m0");
+            // (the instruction's offset counts for both addresses)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, off offset:16"
+                         : : "s"(raw_at + j * 2048 + 1024 - 16), "v"(src[j]) : "memory", "m0");
+        };
+        auto read_raw = [&](int j, float (&xi)[8]) __attribute__((always_inline)) {
+            const float4 a = *(const float4 *)(raw + j * 2048), b4 = *(const float4 *)(raw + j * 2048 + 1024);
+            xi[0] = a.x; xi[1] = a.y; xi[2] = a.z; xi[3] = a.w;
+            xi[4] = b4.x; xi[5] = b4.y; xi[6] = b4.z; xi[7] = b4.w;
+        };
+        const int r_addr[2] = {Tile::row_addr(i32, h, 0), Tile::row_addr(i32, h, 1)};
+        const int c_addr[2] = {Tile::col_addr(lane, 0), Tile::col_addr(lane, 1)};
+        SplitFrag fr;
+        // part P of the K fragment of step st / of the V^T fragment i = ks * DB + db
+        auto next_k = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
+            constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+            fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
+        };
+        auto next_v = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
+            constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+            const int o = (i % DB) * 2048 + (i / DB) * 1024;
+            fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
+        };
+
+        f32x16_t s;
+        float x[16], rs = 0.f;
+        split8 pb[2];
+        // P(n) from S(n) where the interleaved softmax does not do: masks, keys past the end, a negative scale, or a row sum
+        // that says that a probability has outgrown the reference by 2^4
+        auto exact_softmax = [&](int k0) __attribute__((always_inline)) {
+            float mx = -1e30f;
 #pragma unroll
-        for (int j = 0; j < PER_THREAD; ++j) {
-            *(float4 *)&ks[(row0 + j * RPJ) * KROW + col0] = kx[j];
-            *(float4 *)&vs[(row0 + j * RPJ) * D + col0] = vx[j];
+            for (int r = 0; r < 16; ++r) {
+                const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
+                float xv = s[r] * c2;
+                if (p.mask != nullptr && key < N && q_row < N) xv = fmaf(p.mask[(size_t)q_row * N + key], LOG2E, xv);
+                if (key >= kend || (CAUSAL && key > q_row)) xv = -__builtin_inff();
+                x[r] = xv;
+                mx = fmaxf(mx, xv);
+            }
+            mx = xhalf_max(mx);
+            if (__any(mx > m_run + 4.0f)) {
+                const float m_new = fmaxf(m_run, mx + 2.0f), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+                m_run = m_new;
+                l_run *= alpha;
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+            }
+            rs = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                x[r] = __builtin_amdgcn_exp2f(x[r] - m_run);
+                rs += x[r];
+            }
+        };
+        uint32_t tmp[4];
+        auto split_p = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, g = i / SPLIT_STEPS;
+            split_op<i % SPLIT_STEPS>(x + 8 * g, tmp, pb[g]);
+        };
+
+        // prologue: K(0), K(1), K(2) and V(0) to LDS, K(3) and V(1) requested, S(0), P(0)
+#pragma unroll
+        for (int j = 0; j < PER_THREAD; ++j) put_at[j] = Tile::item_addr(item(j));
+        if (tiles > 0) {
+            // (every load before the first split: one memory round trip, not four)
+            float4 first[PER_THREAD][3][2];
+#pragma unroll
+            for (int j = 0; j < PER_THREAD; ++j)
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    if (t == 0 || !item_is_v(j)) {
+                        point(j, t);
+                        first[j][t][0] = *(const float4 *)src[j];
+                        first[j][t][1] = *(const float4 *)(src[j] + 16);
+                    }
+#pragma unroll
+            for (int j = 0; j < PER_THREAD; ++j) {
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    if (t == 0 || !item_is_v(j))
+                        Tile::put(item_is_v(j) ? v_ring : k_ring + t * Tile::BYTES, put_at[j], split_8(first[j][t][0], first[j][t][1]));
+                point(j, item_is_v(j) ? 1 : 3);
+            }
+#pragma unroll
+            for (int j = 0; j < PER_THREAD; ++j) {
+                request(j);
+                next_tile(j, item_is_v(j) ? 2 : 4);
+            }
         }
-        if (it + STEP < ntiles) fetch(it + STEP);
-        if (!SPLITK) __syncthreads();
-        if (it >= my_tiles) continue;  // under the causal mask this wave is done (it still helps staging)
-        if (always_generic || k0 + F32_BK > kend || (CAUSAL && k0 + F32_BK - 1 > wq0))
-            tile_body(std::true_type{}, k0);
-        else
-            tile_body(std::false_type{}, k0);
+        __syncthreads();
+        if (mine > 0) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+            for (int st = 0; st < KSTEPS; ++st) s = mfma_split(Tile::get_row(k_ring, r_addr[st & 1] + (st >> 1) * 2048), qr[st], s);
+            exact_softmax(kg * F32_BK);
+            l_run += rs;
+            static_for<0, 3>([&](auto pi) __attribute__((always_inline)) {
+                next_k(std::integral_constant<int, 0>{}, pi, k_ring + Tile::BYTES, 0);
+            });
+        }
+        __syncthreads();  // K(0) has been read: its slot is the first to be written again
+        int k_cur = 1, k_wr = 0;  // ring slots of K(n+1) and K(n+3)
+        // where item j of K(n+3) / V(n+1) goes (past the last tile: a slot nobody reads again)
+        auto put_tile = [&](int j, int n) __attribute__((always_inline)) {
+            return item_is_v(j) ? v_ring + ((n + 1) & 1) * Tile::BYTES : k_ring + k_wr * Tile::BYTES;
+        };
+        auto advance = [&]() __attribute__((always_inline)) {
+            k_cur = k_cur == 2 ? 0 : k_cur + 1;
+            k_wr = k_wr == 2 ? 0 : k_wr + 1;
+        };
+        int n = 0;
+#pragma clang loop unroll(disable)
+        for (; n < mine - 1; ++n) {
+            const unsigned char *kt = k_ring + k_cur * Tile::BYTES, *vt = v_ring + (n & 1) * Tile::BYTES;
+            // ---- R1 ----
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = 0.f;
+            mfma_region<KSTEPS, 2 * SPLIT_STEPS>(
+                [&](auto fi, auto mi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    s = mfma_split_step<decltype(mi)::value>(fr.template get<(f & 1)>(), qr[f], s);
+                },
+                [&](auto fi, auto pi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    if constexpr (f < KSTEPS) next_k(fi, pi, kt, f);
+                    else next_v(fi, pi, vt, 0);
+                },
+                split_p);
+            // ---- R2 ----
+            const unsigned char *kn = k_ring + (k_cur == 2 ? 0 : k_cur + 1) * Tile::BYTES;
+            split8 sp;
+            float xi[8], sum[2];
+            // a staged item: its arrival and the read, the split, the write and the next request; then the probabilities, two at
+            // a time, and their sum
+            constexpr int ITEM = 3 + SPLIT_STEPS, CONV = ITEM * PER_THREAD, NS = CONV + 20;
+            auto r2_step = [&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (i < CONV) {
+                    constexpr int j = i / ITEM, t = i % ITEM;
+                    if constexpr (t == 0) {
+                        // in flight behind item j: the rest of this tile pair and what has been requested of the next
+                        wait_vmem_le<2 * (PER_THREAD - 1)>();
+                        read_raw(j, xi);
+                    } else if constexpr (t == ITEM - 1) {
+                        Tile::put(put_tile(j, n), put_at[j], sp);
+                        request(j);
+                    } else if constexpr (t >= 2) {
+                        split_op<t - 2>(xi, tmp, sp);
+                    }
+                } else {
+                    constexpr int t = i - CONV;
+                    if constexpr (t < 16) {
+                        constexpr int e = (t >> 1) * 2;
+                        if constexpr ((t & 1) == 0) {
+                            x[e] = fmaf(s[e], c2, -m_run);
+                            x[e + 1] = fmaf(s[e + 1], c2, -m_run);
+                        } else {
+                            x[e] = __builtin_amdgcn_exp2f(x[e]);
+                            x[e + 1] = __builtin_amdgcn_exp2f(x[e + 1]);
+                        }
+                        pin(x[e], x[e + 1]);
+                    } else {
+                        constexpr int g = t - 16;
+                        sum[g & 1] = (g < 2 ? 0.f : sum[g & 1]) + ((x[4 * g] + x[4 * g + 1]) + (x[4 * g + 2] + x[4 * g + 3]));
+                        asm volatile("" : "+v"(sum[g & 1]));
+                    }
+                }
+            };
+            mfma_region<2 * DB, NS>(
+                [&](auto fi, auto mi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    oacc[f % DB] = mfma_split_step<decltype(mi)::value>(fr.template get<(f & 1)>(), pb[f / DB], oacc[f % DB]);
+                },
+                [&](auto fi, auto pi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    if constexpr (f < 2 * DB) next_v(fi, pi, vt, f);
+                    else next_k(fi, pi, kn, 0);
+                },
+                r2_step);
+            rs = sum[0] + sum[1];
+#pragma unroll
+            for (int j = 0; j < PER_THREAD; ++j) next_tile(j, item_is_v(j) ? n + 3 : n + 5);
+            const int k0 = ((n + 1) * KW + kg) * F32_BK;
+            if (is_generic(k0) || __any(!(rs <= 16.0f))) exact_softmax(k0);
+            l_run += rs;
+            advance();
+            __syncthreads();
+        }
+        if (mine > 0) {
+            // the last tile of this wave: no S to look ahead for
+            static_for<0, 2 * SPLIT_STEPS>(split_p);
+            const unsigned char *vt = v_ring + (n & 1) * Tile::BYTES;
+#pragma unroll
+            for (int f = 0; f < 2 * DB; ++f) {
+                const int o = (f % DB) * 2048 + (f / DB) * 1024;
+                oacc[f % DB] = mfma_split(Tile::get_col(vt, c_addr[0] + o, c_addr[1] + o), pb[f / DB], oacc[f % DB]);
+            }
+        }
+        // under the causal mask a wave is done before others of its workgroup: it still stages tiles for them
+        for (; n < rounds - 1; ++n) {
+#pragma unroll
+            for (int j = 0; j < PER_THREAD; ++j) {
+                float xi[8];
+                wait_vmem_le<2 * (PER_THREAD - 1)>();
+                read_raw(j, xi);
+                Tile::put(put_tile(j, n), put_at[j], split_8(xi[0], xi[1], xi[2], xi[3], xi[4], xi[5], xi[6], xi[7]));
+                request(j);
+                next_tile(j, item_is_v(j) ? n + 3 : n + 5);
+            }
+            advance();
+            __syncthreads();
+        }
+        wait_vmem_le<0>();  // nothing is on its way to LDS any more
+    } else {
+        // One wave, its own tiles: the K operand of a lane is 8 consecutive channels of key row i32, the V^T operand 8 rows of
+        // channel i32; both come straight from memory (a row of V is 128 consecutive bytes over the lanes), one tile ahead.
+        float4 kx[2 * KSTEPS];
+        float vx[DB][16];
+        auto fetch_k = [&](int tile) __attribute__((always_inline)) {
+            const float *src = kp + (size_t)min(tile * F32_BK + i32, kend - 1) * k_rs + h * 8;
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                kx[2 * s] = *(const float4 *)(src + 16 * s);
+                kx[2 * s + 1] = *(const float4 *)(src + 16 * s + 4);
+            }
+        };
+        // (rows past the last visible key repeat it: their probabilities are zero, and so is what they add)
+        auto fetch_v = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float *src = vp + (size_t)min(tile * F32_BK + 8 * (r >> 2) + 4 * h + (r & 3), kend - 1) * k_rs + i32;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) vx[db][r] = src[32 * db];
+            }
+        };
+        if (kg < my_tiles) {
+            fetch_k(kg);
+            fetch_v(kg);
+        }
+        for (int it = kg; it < my_tiles; it += KW) {
+            const int k0 = it * F32_BK;
+            f32x16_t s;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+            for (int st = 0; st < KSTEPS; ++st) s = mfma_split(split_8(kx[2 * st], kx[2 * st + 1]), qr[st], s);
+            if (it + KW < my_tiles) fetch_k(it + KW);
+            split8 pb[2];
+            if (is_generic(k0)) softmax(std::true_type{}, k0, s, pb);
+            else softmax(std::false_type{}, k0, s, pb);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int db = 0; db < DB; ++db) {
+                    const float *v = &vx[db][8 * ks];
+                    oacc[db] = mfma_split(split_8(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]), pb[ks], oacc[db]);
+                }
+            if (it + KW < my_tiles) fetch_v(it + KW);
+        }
     }
 
-    const float l_tot = l_run + __shfl_xor(l_run, 32);
-    if constexpr (SPLITK) {
-        // ---- merge the waves' partial results ----
-        // slab of wave w, reused: O_w as [32 queries][D + 4], then m_w[32], l_w[32]
-        constexpr int OROW = D + 4;
-        static_assert(32 * OROW + 64 <= SLAB, "merge buffers fit the staging slab");
-        float *ow = lds + wave * SLAB;
+    const float l_tot = xhalf_sum(l_run);
+    if constexpr (KW > 1) {
+        // ---- merge the key groups' partial results ----
+        // slab of wave w: O_w as [32 queries][D + 4], then m_w[32], l_w[32]
+        constexpr int OROW = D + 4, SLAB = 32 * OROW + 64;
+        float *ml = (float *)lds;
+        if (QW > 1) __syncthreads();  // the tiles have been consumed
+        float *ow = ml + wave * SLAB;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -269,24 +508,25 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *l
             ow[32 * OROW + 32 + i32] = l_tot;
         }
         __syncthreads();
-        // thread t: query t % 32, channels [cg * CPT, cg * CPT + CPT)
-        constexpr int CPT = D / (NW * 2);
+        // thread t: query t % BQ, channels [cg * CPT, cg * CPT + CPT)
+        constexpr int CPT = D / (KW * 2);
         static_assert(CPT % 4 == 0, "whole float4s per thread");
-        const int q = tid & 31, cg = tid >> 5;
+        const int q = tid % BQ, cg = tid / BQ;
+        const float *mq = ml + (q >> 5) * SLAB + (q & 31) * OROW, *st = ml + (q >> 5) * SLAB + 32 * OROW + (q & 31);
         const int row = qblk + q;
         float m = -1e30f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) m = fmaxf(m, lds[w * SLAB + 32 * OROW + q]);
+        for (int g = 0; g < KW; ++g) m = fmaxf(m, st[g * QW * SLAB]);
         float l = 0.f, acc[CPT];
 #pragma unroll
         for (int c = 0; c < CPT; ++c) acc[c] = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const float f = __builtin_amdgcn_exp2f(lds[w * SLAB + 32 * OROW + q] - m);
-            l += lds[w * SLAB + 32 * OROW + 32 + q] * f;
+        for (int g = 0; g < KW; ++g) {
+            const float f = __builtin_amdgcn_exp2f(st[g * QW * SLAB] - m);
+            l += st[g * QW * SLAB + 32] * f;
 #pragma unroll
             for (int c = 0; c < CPT; c += 4) {
-                const float4 x = *(const float4 *)&lds[w * SLAB + q * OROW + cg * CPT + c];
+                const float4 x = *(const float4 *)&mq[g * QW * SLAB + cg * CPT + c];
                 acc[c] += x.x * f; acc[c + 1] += x.y * f; acc[c + 2] += x.z * f; acc[c + 3] += x.w * f;
             }
         }
@@ -316,12 +556,17 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, float *l
     }
 }
 
-// D = 64: two waves per SIMD (registers held to 256 per lane); D = 128 needs more than that
-template <int D, int NW, bool CAUSAL, bool SPLITK = false>
-__global__ void __launch_bounds__(NW * 64, (D == 64 ? 2 : 1)) flash_f32_kernel(const FlashF32Params p)
+template <int D, int QW, int KW>
+constexpr int flash_f32_waves_per_simd()
 {
-    __shared__ __attribute__((aligned(16))) float lds[flash_f32_lds_floats<D, NW, SPLITK>()];
-    flash_f32_body<D, NW, CAUSAL, SPLITK>(p, lds, (int)blockIdx.x);
+    return QW * KW == 8 ? 2 : (D == 64 ? 2 : (KW == 1 ? 2 : 1));
+}
+
+template <int D, int QW, int KW, bool CAUSAL>
+__global__ void __launch_bounds__(QW * KW * 64, (flash_f32_waves_per_simd<D, QW, KW>())) flash_f32_kernel(const FlashF32Params p)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<D, QW, KW>()];
+    flash_f32_body<D, QW, KW, CAUSAL>(p, lds, (int)blockIdx.x);
 }
 
 }  // namespace arhip

@@ -402,10 +402,11 @@ bool mid_variant(const std::shared_ptr<Device> &dev, int64_t b, int64_t h, int64
 
 }  // namespace
 
-// The fp32 kernels: 128 queries (keys) per workgroup when that still fills the chip, else 32
+// The fp32 kernels at head size 64: 128 queries (keys) per workgroup, or 32 whose tiles are dealt out between the waves where
+// 128 would leave half the chip idle (the rule of arhip_flash_bwd)
 static bool short_f32(const std::shared_ptr<Device> &dev, int64_t b, int64_t heads, int64_t n)
 {
-    return b * heads * ((n + 127) / 128) < 2 * (int64_t)dev->compute_units();
+    return b * heads * ((n + 127) / 128) < (int64_t)dev->compute_units() / 2;
 }
 
 std::vector<HostCall> attention_host_calls(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor *attn_mask,
@@ -431,7 +432,7 @@ std::vector<HostCall> attention_host_calls(const Tensor &q, const Tensor &k, con
     };
 
     if (kern == Kernel::FlashF32) {
-        // few, short heads: 32 queries per workgroup instead of 128 (the rule of arhip_flash_fwd)
+        // few, short heads: 32 queries per workgroup instead of 128
         if (d == 64 && short_f32(dev, b, h, n) && !key_lengths)
             calls.push_back(make_call(dev, "ar_flash_f32_short", {q, k, v, out, mslot}, {F, F, F, F, F},
                                       {(n + 31) / 32, b * h, 1}, {256, 1, 1}, vals));

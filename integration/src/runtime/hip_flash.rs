@@ -168,10 +168,10 @@ fn mid_variant(dev: &str, b: i64, h: i64, n: i64, d: i64, causal: bool, has_lens
     n <= 1024 || (n <= 2048 && causal && !has_lens)
 }
 
-/// The fp32 kernels take 128 queries (keys) per workgroup when that still fills the chip, else 32
-/// with the tiles of the other side dealt out between the waves (`*_short`, `head_dim` 64).
+/// The fp32 kernels take 128 queries (keys) per workgroup, or 32 with the tiles of the other side dealt out
+/// between the waves where 128 would leave half the chip idle (`*_short`, `head_dim` 64).
 fn short_f32(dev: &str, b: i64, heads: i64, n: i64, d: i64) -> bool {
-    d == 64 && b * heads * ((n + 127) / 128) < 2 * crate::runtime::ops_hip::compute_units(dev)
+    d == 64 && b * heads * ((n + 127) / 128) < crate::runtime::ops_hip::compute_units(dev) / 2
 }
 
 /// fp32 exact mode: `bufs = [q, k, v, o, mask-or-o]`, all f32 `[b, h, n, d]`; `lens`: int32 `[b]` key lengths.

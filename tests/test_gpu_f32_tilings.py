@@ -1,0 +1,31 @@
+"""The tilings of the fp32 forward at the edges of their tiles, against the float64 oracle on sampled heads: many heads, so that
+the launches take the tilings whose waves share their key tiles and not the one for few, short heads."""
+import numpy as np
+import pytest
+
+import oracle
+from autorust_amd import synth
+from autorust_amd.device import F32
+from gpu_util import run_flash
+
+pytestmark = pytest.mark.gpu
+
+# 256 heads: 128 queries per workgroup (last tile of one key, full tiles, waves without queries); 128 heads: 256 queries
+SHAPES = [(16, 16, 65, 64), (16, 16, 97, 64), (16, 16, 128, 64), (16, 16, 33, 128), (16, 16, 65, 128), (16, 16, 128, 128),
+          (8, 16, 257, 64), (8, 16, 289, 64), (8, 16, 384, 64), (8, 16, 257, 128), (8, 16, 320, 128)]
+
+
+@pytest.mark.parametrize("mode", ["plain", "causal", "causal+len", "len"])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_f32_forward_tilings(dev, shape, mode):
+    B, H, N, D = shape
+    # operands whose three bf16 parts all matter, over a few binary orders of magnitude
+    q, k, v = (synth.normal(900 + i, (B, H, N, D)) for i in range(3))
+    v *= np.exp2(np.arange(B, dtype=np.float32) - 8)[:, None, None, None]
+    causal = "causal" in mode
+    lens = ((np.arange(B) * 37 + 1) % (N + 1)).astype(np.int32) if "len" in mode else None
+    got = run_flash(dev, q, k, v, F32, kv_len=lens, causal=causal)
+    for b, h in ((0, 0), (B // 2, 3), (B - 1, H - 1)):
+        want = oracle.sdpa_f64(q[b:b + 1, h:h + 1], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], causal=causal,
+                               kv_len=None if lens is None else lens[b:b + 1]) if lens is None or lens[b] > 0 else np.zeros((1, 1, N, D))
+        assert np.abs(got[b, h] - want[0, 0]).max() <= 3e-6 * max(np.abs(v[b, h]).max(), 1e-30), (b, h)
