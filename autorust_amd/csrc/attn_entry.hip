@@ -239,16 +239,16 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dq(const float *Q, c
                                                                 const float *M, float *dQ, int N, int head_dim, int causal,
                                                                 int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[bwd_lds_floats<128>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dq_lds_bytes<128, false>()];
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dq = dQ;
     const int wg = linear_wg();
     if (head_dim == 64) {
-        if (causal) bwd_dq_body<64, 4, true>(p, lds, wg);
-        else bwd_dq_body<64, 4, false>(p, lds, wg);
+        if (causal) bwd_dq_body<64, true, false>(p, lds, wg);
+        else bwd_dq_body<64, false, false>(p, lds, wg);
     } else if (head_dim == 128) {
-        if (causal) bwd_dq_body<128, 4, true>(p, lds, wg);
-        else bwd_dq_body<128, 4, false>(p, lds, wg);
+        if (causal) bwd_dq_body<128, true, false>(p, lds, wg);
+        else bwd_dq_body<128, false, false>(p, lds, wg);
     }
 }
 
@@ -257,16 +257,16 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv(const float *Q, 
                                                                  const float *M, float *dK, float *dV, int N, int head_dim,
                                                                  int causal, int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[bwd_lds_floats<128>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dkv_lds_bytes<128, false>()];
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dk = dK; p.dv = dV;
     const int wg = linear_wg();
     if (head_dim == 64) {
-        if (causal) bwd_dkv_body<64, 4, true>(p, lds, wg);
-        else bwd_dkv_body<64, 4, false>(p, lds, wg);
+        if (causal) bwd_dkv_body<64, true, false>(p, lds, wg);
+        else bwd_dkv_body<64, false, false>(p, lds, wg);
     } else if (head_dim == 128) {
-        if (causal) bwd_dkv_body<128, 4, true>(p, lds, wg);
-        else bwd_dkv_body<128, 4, false>(p, lds, wg);
+        if (causal) bwd_dkv_body<128, true, false>(p, lds, wg);
+        else bwd_dkv_body<128, false, false>(p, lds, wg);
     }
 }
 
@@ -274,18 +274,18 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv(const float *Q, 
 // The same for short shapes: 32 queries (dQ) / 32 keys (dK, dV) per workgroup, grid [ceil(N/32), B*hq, 1] /
 // [ceil(N/32), B*hkv, 1], the tiles of the other side dealt out between the four waves.  head_dim 64 only.
 #if ARHIP_PART(1)
-extern "C" __global__ void __launch_bounds__(256, 2) ar_fl_bwd_dq_short(const float *Q, const float *K, const float *V,
+extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dq_short(const float *Q, const float *K, const float *V,
                                                                          const float *dO, const float *LSE, const float *D,
                                                                          const float *M, float *dQ, int N, int head_dim,
                                                                          int causal, int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[bwd_lds_floats<64, 4, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dq_lds_bytes<64, true>()];
     if (head_dim != 64) return;
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dq = dQ;
     const int wg = linear_wg();
-    if (causal) bwd_dq_body<64, 4, true, true>(p, lds, wg);
-    else bwd_dq_body<64, 4, false, true>(p, lds, wg);
+    if (causal) bwd_dq_body<64, true, true>(p, lds, wg);
+    else bwd_dq_body<64, false, true>(p, lds, wg);
 }
 
 extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv_short(const float *Q, const float *K, const float *V,
@@ -293,13 +293,13 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv_short(const floa
                                                                        const float *M, float *dK, float *dV, int N,
                                                                        int head_dim, int causal, int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) float lds[bwd_lds_floats<64, 4, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dkv_lds_bytes<64, true>()];
     if (head_dim != 64) return;
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dk = dK; p.dv = dV;
     const int wg = linear_wg();
-    if (causal) bwd_dkv_body<64, 4, true, true>(p, lds, wg);
-    else bwd_dkv_body<64, 4, false, true>(p, lds, wg);
+    if (causal) bwd_dkv_body<64, true, true>(p, lds, wg);
+    else bwd_dkv_body<64, false, true>(p, lds, wg);
 }
 
 #endif

@@ -539,9 +539,10 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     p.scale = scale;
     if (int rc = t.begin()) return rc;
     const long rows = (long)(B * Hq * N);
-    // 4 waves per workgroup: 128 queries / keys when that still fills the chip, else the same 32
-    // queries / keys with the tiles of the other side dealt out between the waves
-    const bool split = B * Hkv * ((N + 127) / 128) < 2 * (int64_t)dev->cus;
+    // 4 waves per workgroup: 128 queries / keys that share their tiles, or (head size 64, so few workgroups that half the chip would
+    // idle behind them) the same 32 queries / keys with the tiles of the other side dealt out between the waves.  128 against 32
+    // rows per workgroup: B1 H12 N197 40 / 26 us, B4 H8 N512 (128 workgroups: the line) 73 / 77, B8 H12 N197 46 / 70
+    const bool split = D == 64 && B * Hkv * ((N + 127) / 128) < dev->cus / 2;
     const int rows_wg = split ? 32 : 128;
     const int nt = (int)((N + rows_wg - 1) / rows_wg);
     const dim3 block(256), grid_prep((unsigned)((rows + 3) / 4)), grid_q((unsigned)(nt * B * Hq)),
@@ -556,15 +557,15 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     do {                                                                                                \
         hipLaunchKernelGGL((bwd_prep_kernel<DD>), grid_prep, dim3(256), 0, dev->stream, o, dout, delta, rows); \
         if (causal) {                                                                                   \
-            hipLaunchKernelGGL((bwd_dq_kernel<DD, 4, true, SP>), grid_q, block, 0, dev->stream, p);     \
-            hipLaunchKernelGGL((bwd_dkv_kernel<DD, 4, true, SP>), grid_kv, block, 0, dev->stream, p);   \
+            hipLaunchKernelGGL((bwd_dq_kernel<DD, true, SP>), grid_q, block, 0, dev->stream, p);     \
+            hipLaunchKernelGGL((bwd_dkv_kernel<DD, true, SP>), grid_kv, block, 0, dev->stream, p);   \
         } else {                                                                                        \
-            hipLaunchKernelGGL((bwd_dq_kernel<DD, 4, false, SP>), grid_q, block, 0, dev->stream, p);    \
-            hipLaunchKernelGGL((bwd_dkv_kernel<DD, 4, false, SP>), grid_kv, block, 0, dev->stream, p);  \
+            hipLaunchKernelGGL((bwd_dq_kernel<DD, false, SP>), grid_q, block, 0, dev->stream, p);    \
+            hipLaunchKernelGGL((bwd_dkv_kernel<DD, false, SP>), grid_kv, block, 0, dev->stream, p);  \
         }                                                                                               \
     } while (0)
     if (D == 64) { if (split) BWD_LAUNCH(64, true); else BWD_LAUNCH(64, false); }
-    else { if (split) BWD_LAUNCH(128, true); else BWD_LAUNCH(128, false); }
+    else BWD_LAUNCH(128, false);
 #undef BWD_LAUNCH
     arhip_note_selected(ARHIP_K_FLASH_BWD);
     return t.end();

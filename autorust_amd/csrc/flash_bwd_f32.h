@@ -9,14 +9,21 @@
 // Keys past the diagonal (causal) or past kv_len contribute p = 0.  head_dim and scale are parameters
 // here (the reference hard-codes 64 and 0.125).
 //
-// All contractions run on v_mfma_f32_32x32x2_f32 (fp32 in, fp32 accumulate) with the decomposition of
-// the forward kernel (flash_f32.h): one row of the "resident" operand per lane.
+// All contractions run on the bf16 matrix instruction with every fp32 operand as the exact sum of three bf16 values
+// (f32_split.h), with the decomposition of the forward kernel (flash_f32.h): one row of the "resident" operand per lane.
 //   dQ kernel   a wave owns 32 queries (lane = query): S^T = K Q^T and dP^T = V dO^T leave, per lane,
 //               16 keys of one query, so lse_i and D_i are per-lane scalars and dS^T is already the B
 //               operand of dQ^T += K^T dS^T.  K and V tiles of 32 keys are staged in LDS.
 //   dK/dV kernel  a wave owns 32 keys (lane = key): S = Q K^T and dP = dO V^T leave, per lane, 16
 //               queries of one key; P and dS are the B operands of dV^T += dO^T P and dK^T += Q^T dS.
 //               Q and dO tiles of 32 queries (with their lse and D) are staged in LDS.
+// A staged tile is split once and read twice, by rows for the first products and by columns (transposing reads) for the second.
+// The factor `scale` of dS is applied to the sums at the end.
+//
+// Bound: the matrix pipe (seven products of 2 N^2 D per head for the five of the mathematics: S and dP are formed in both
+// kernels).  Against the same kernels on v_mfma_f32_32x32x2_f32, whole backward: B2 H16 N2048 D128 2026 -> 1131 us, causal
+// 1119 -> 610 us, D64 992 -> 579 us, B8 H6 N789 D64 causal 201 -> 120 us, B8 H12 N197 D64 78 -> 46 us, B1 H12 N197 D64 30 -> 26 us;
+// relative error of dQ (2-norm, against float64) 1.07e-6 -> 9.4e-7 at N = 2048, 4.8e-7 -> 4.7e-7 at N = 197.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -37,8 +44,6 @@ struct FlashBwdParams {
     float scale;
 };
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
 constexpr float BWD_LSE_FLOOR = -5e29f;  // lse at or below: the row saw no key (cuda_flash_train.rs:206)
 constexpr float BWD_LOG2E = 1.44269504088896340736f;
 
@@ -58,37 +63,98 @@ __device__ __forceinline__ void bwd_prep_body(const float *o, const float *dout,
     if (lane == 0) delta[row] = s;
 }
 
-// LDS floats of the dQ and dK/dV bodies: two padded 32-row tiles and 64 row statistics (one such slab
-// per wave with SPLIT)
-template <int D, int NW = 1, bool SPLIT = false>
-constexpr int bwd_lds_floats()
+// One thread's share of a pair of 32-row tiles (A and B, e.g. K and V) between memory and LDS: items of 8 channels, the first
+// half of them A's.  Rows past `last` repeat it (whatever they hold is multiplied by P = dS = 0).
+template <int D, int T>
+struct PairStage {
+    using Tile = SplitTile<D>;
+    static constexpr int ITEMS = 2 * Tile::ITEMS / T;  // per thread
+    static constexpr int STEPS = (SPLIT_STEPS + 1) * ITEMS;  // of split_step
+    static_assert(Tile::ITEMS % T == 0, "tile staging must divide evenly");
+    float x[ITEMS][8];
+    split8 sp;
+    uint32_t tmp[4];
+
+    static constexpr bool is_b(int j) { return j >= ITEMS / 2; }
+    static __device__ __forceinline__ int item(int j, int t) { return t + (j - (is_b(j) ? ITEMS / 2 : 0)) * T; }
+    __device__ __forceinline__ void fetch(const float *a, const float *b, int t, int row0, int last)
+    {
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const int it = item(j, t);
+            const float *src = (is_b(j) ? b : a) + (size_t)min(row0 + Tile::item_row(it), last) * D + Tile::item_col(it);
+            const float4 u = *(const float4 *)src, v = *(const float4 *)(src + 4);
+            x[j][0] = u.x; x[j][1] = u.y; x[j][2] = u.z; x[j][3] = u.w;
+            x[j][4] = v.x; x[j][5] = v.y; x[j][6] = v.z; x[j][7] = v.w;
+        }
+    }
+    template <int I>
+    __device__ __forceinline__ void split_step(unsigned char *ta, unsigned char *tb, int t)
+    {
+        constexpr int j = I / (SPLIT_STEPS + 1), k = I % (SPLIT_STEPS + 1);
+        if constexpr (k < SPLIT_STEPS) split_op<k>(x[j], tmp, sp);
+        else Tile::put(is_b(j) ? tb : ta, Tile::item_addr(item(j, t)), sp);
+    }
+    __device__ __forceinline__ void put(unsigned char *ta, unsigned char *tb, int t)
+    {
+        static_for<0, STEPS>([&](auto ic) __attribute__((always_inline)) { split_step<decltype(ic)::value>(ta, tb, t); });
+    }
+};
+
+// LDS bytes of the bodies below.  Pipelined (128 queries / keys per workgroup): rings of tiles; SPLIT (32 per workgroup): a tile
+// pair per wave, or the partial sums of the waves, which reuse it
+template <int D, bool SPLIT>
+constexpr int bwd_dq_lds_bytes()
 {
-    return (SPLIT ? NW : 1) * (2 * F32_BK * (D + 4) + 64);
+    constexpr int merge = 4 * 32 * (D + 4) * 4, slabs = 4 * 2 * SplitTile<D>::BYTES;
+    return SPLIT ? (slabs > merge ? slabs : merge) : 5 * SplitTile<D>::BYTES;
+}
+template <int D, bool SPLIT>
+constexpr int bwd_dkv_lds_bytes()
+{
+    constexpr int merge = 4 * 2 * 32 * (D + 4) * 4, slabs = 4 * (2 * SplitTile<D>::BYTES + 256);
+    return SPLIT ? (slabs > merge ? slabs : merge) : 6 * SplitTile<D>::BYTES + 3 * 256;
 }
 
-// dQ.  lds: bwd_lds_floats<D, NW, SPLIT>() floats.  Workgroup wg_linear in [0, nt * B * Hq): 32 NW queries
-// of one head.  SPLIT (few, short heads: one wave per workgroup would leave each SIMD a long chain of
-// matrix instructions and most of the chip idle): the NW waves share the same 32 queries and deal the
-// key tiles out between them (wave w takes tiles w, w + NW, ...), each staging its tiles in its own
-// LDS slab with no workgroup barrier; the partial dQ of the waves are added through LDS in wave order.
-template <int D, int NW, bool CAUSAL, bool SPLIT = false>
-__device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, float *lds, int wg_linear)
+// 16 values per lane of a product of the first kind: c += A rows . B, A a tile in LDS
+template <int D>
+__device__ __forceinline__ f32x16 mul_rows(const unsigned char *tile, const int (&r_addr)[2], const split8 (&b)[D / 16])
 {
-    constexpr int T = SPLIT ? 64 : NW * 64;   // threads staging one tile
-    constexpr int BQ = SPLIT ? 32 : NW * 32;
-    constexpr int HALF = D / 2;
-    constexpr int ROW = D + 4;  // padded row: conflict-free 128-bit row reads
-    constexpr int DB = D / 32;
-    constexpr int CHUNKS = F32_BK * D / 4;
-    constexpr int PER_THREAD = CHUNKS / T;
-    static_assert(CHUNKS % T == 0, "tile staging must divide evenly");
+    f32x16 c;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c[r] = 0.f;
+#pragma unroll
+    for (int st = 0; st < D / 16; ++st) c = mfma_split(SplitTile<D>::get_row(tile, r_addr[st & 1] + (st >> 1) * 2048), b[st], c);
+    return c;
+}
+// acc += A columns . B
+template <int D>
+__device__ __forceinline__ void mul_cols(const unsigned char *tile, const int (&c_addr)[2], const split8 (&b)[2], f32x16 (&acc)[D / 32])
+{
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db) {
+            const int o = db * 2048 + ks * 1024;
+            acc[db] = mfma_split(SplitTile<D>::get_col(tile, c_addr[0] + o, c_addr[1] + o), b[ks], acc[db]);
+        }
+}
 
-    constexpr int SLAB = 2 * F32_BK * ROW + 64;
+// dQ.  lds: bwd_dq_lds_bytes<D, SPLIT>() bytes.  Workgroup wg_linear in [0, nt * B * Hq), four waves: 128 queries
+// of one head.  SPLIT (few, short heads: one wave per workgroup would leave each SIMD a long chain of
+// matrix instructions and most of the chip idle): the waves share the same 32 queries and deal the
+// key tiles out between them (wave w takes tiles w, w + 4, ...), each staging its tiles in its own
+// LDS slab with no workgroup barrier; the partial dQ of the waves are added through LDS in wave order.
+template <int D, bool CAUSAL, bool SPLIT>
+__device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned char *lds, int wg_linear)
+{
+    constexpr int NW = 4;
+    constexpr int BQ = SPLIT ? 32 : NW * 32;
+    constexpr int DB = D / 32, KSTEPS = D / 16;
+    using Tile = SplitTile<D>;
+
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    float *ks = lds + (SPLIT ? wave * SLAB : 0);
-    float *vs = ks + F32_BK * ROW;
-    const int stid = SPLIT ? lane : tid;      // index among the threads staging a tile
     const int i32 = lane & 31, h = lane >> 5;
     // every XCD (consecutive workgroups go to different ones) gets a contiguous range of heads
     const int wg_x = (p.total_q > 0 && (p.total_q & 7) == 0) ? (wg_linear & 7) * (p.total_q >> 3) + (wg_linear >> 3) : wg_linear;
@@ -113,115 +179,201 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, float *lds,
     int kend = kvl;
     if (CAUSAL) kend = min(kend, min(N, qblk + BQ));
     const int ntiles = (kend + F32_BK - 1) / F32_BK;
-    const int my_tiles = CAUSAL ? min(ntiles, (wq0 + 31) / F32_BK + 1) : ntiles;
+    const int my_tiles = wq0 >= N ? 0 : CAUSAL ? min(ntiles, (wq0 + 31) / F32_BK + 1) : ntiles;
     const int kvh = head / (p.Hq / p.Hkv);
     const float *kp = p.k + ((size_t)b * p.Hkv + kvh) * (size_t)N * D;
     const float *vp = p.v + ((size_t)b * p.Hkv + kvh) * (size_t)N * D;
-    const size_t qoff = ((size_t)bh * N + rr) * D + h * HALF;
+    const size_t qoff = ((size_t)bh * N + rr) * D + h * 8;
 
-    float qr[HALF], dor[HALF];
+    split8 qr[KSTEPS], dor[KSTEPS];
 #pragma unroll
-    for (int s = 0; s < HALF; s += 4) {
-        const float4 x = *(const float4 *)(p.q + qoff + s);
-        const float4 y = *(const float4 *)(p.dout + qoff + s);
-        qr[s] = x.x; qr[s + 1] = x.y; qr[s + 2] = x.z; qr[s + 3] = x.w;
-        dor[s] = y.x; dor[s + 1] = y.y; dor[s + 2] = y.z; dor[s + 3] = y.w;
+    for (int s = 0; s < KSTEPS; ++s) {
+        qr[s] = split_8(*(const float4 *)(p.q + qoff + 16 * s), *(const float4 *)(p.q + qoff + 16 * s + 4));
+        dor[s] = split_8(*(const float4 *)(p.dout + qoff + 16 * s), *(const float4 *)(p.dout + qoff + 16 * s + 4));
     }
     const float lse = p.lse[(size_t)bh * N + rr];
     const float di = p.delta[(size_t)bh * N + rr];
-    const bool row_live = lse > BWD_LSE_FLOOR;
-    // P = exp(x - lse) as v_exp_f32 (base 2) of x * log2(e) - lse * log2(e)
-    const float c2 = p.scale * BWD_LOG2E, lse2 = lse * BWD_LOG2E;
+    // P = exp(x - lse) as v_exp_f32 (base 2) of x * log2(e) - lse * log2(e); a row that saw no key has P = 0
+    const float c2 = p.scale * BWD_LOG2E, lse2 = lse > BWD_LSE_FLOOR ? lse * BWD_LOG2E : __builtin_inff();
 
     f32x16_t acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+    const int r_addr[2] = {Tile::row_addr(i32, h, 0), Tile::row_addr(i32, h, 1)};
+    const int c_addr[2] = {Tile::col_addr(lane, 0), Tile::col_addr(lane, 1)};
 
-    float4 kx[PER_THREAD], vx[PER_THREAD];
-    auto fetch = [&](int tile) __attribute__((always_inline)) {
-        if (tile * F32_BK + F32_BK <= kend) {  // a full tile: no row tests, no zero fill
+    // S^T = K Q^T and dP^T = V dO^T: lane = query, register r = key 8 (r / 4) + 4 h + r % 4
+    f32x16_t s, dp;
+    float ds[16], t4[4];  // dS / scale; scratch of ds_step
+    split8 db_[2];
+    // what the logits are multiplied by in the exponent: c2, or 1 where the mask has been added (add_mask)
+    const float cx = p.mask != nullptr ? 1.f : c2;
+    auto add_mask = [&](int k0) __attribute__((always_inline)) {
+        if (p.mask == nullptr) return;
 #pragma unroll
-            for (int j = 0; j < PER_THREAD; ++j) {
-                const int c = stid + j * T;
-                const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-                const size_t off = (size_t)(tile * F32_BK + row) * D + col;
-                kx[j] = *(const float4 *)(kp + off);
-                vx[j] = *(const float4 *)(vp + off);
-            }
-            return;
+        for (int r = 0; r < 16; ++r) {
+            const int key = min(k0 + 8 * (r >> 2) + 4 * h + (r & 3), N - 1);
+            s[r] = fmaf(p.mask[(size_t)rr * N + key], BWD_LOG2E, s[r] * c2);
         }
+    };
+    auto make_ds = [&](int r) __attribute__((always_inline)) {
+        ds[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cx, -lse2)) * (dp[r] - di);
+    };
+    // the same in steps 0 .. 23: exponents and exponentials two at a time, then the differences and the products four at a time
+    auto ds_step = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (i < 16) {
+            constexpr int e = (i >> 1) * 2;
 #pragma unroll
-        for (int j = 0; j < PER_THREAD; ++j) {
-            const int c = stid + j * T;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            const int gr = tile * F32_BK + row;
-            kx[j] = vx[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (gr < kend) {
-                kx[j] = *(const float4 *)(kp + (size_t)gr * D + col);
-                vx[j] = *(const float4 *)(vp + (size_t)gr * D + col);
+            for (int r = e; r < e + 2; ++r) ds[r] = (i & 1) ? __builtin_amdgcn_exp2f(ds[r]) : fmaf(s[r], cx, -lse2);
+            pin(ds[e], ds[e + 1]);
+        } else {
+            constexpr int e = ((i - 16) >> 1) * 4;
+#pragma unroll
+            for (int r = e; r < e + 4; ++r) {
+                float &v = (i & 1) ? ds[r] : t4[r - e];
+                v = (i & 1) ? ds[r] * t4[r - e] : dp[r] - di;
+                asm volatile("" : "+v"(v));
             }
         }
     };
-    constexpr int STEP = SPLIT ? NW : 1;
-    const int first = SPLIT ? wave : 0;
-    if (first < ntiles) fetch(first);
-    for (int it = first; it < ntiles; it += STEP) {
-        const int k0 = it * F32_BK;
-        if (!SPLIT) __syncthreads();
-#pragma unroll
-        for (int j = 0; j < PER_THREAD; ++j) {
-            const int c = stid + j * T;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            *(float4 *)&ks[row * ROW + col] = kx[j];
-            *(float4 *)&vs[row * ROW + col] = vx[j];
-        }
-        if (it + STEP < ntiles) fetch(it + STEP);
-        if (!SPLIT) __syncthreads();
-        if (it >= my_tiles) continue;
-
-        // S^T = K Q^T and dP^T = V dO^T: lane = query, register r = key 8 (r / 4) + 4 h + r % 4
-        f32x16_t s, dp;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-        const float *krow = &ks[i32 * ROW + h * HALF];
-        const float *vrow = &vs[i32 * ROW + h * HALF];
-#pragma unroll
-        for (int st = 0; st < HALF; st += 4) {
-            const float4 a = *(const float4 *)(krow + st);
-            const float4 c = *(const float4 *)(vrow + st);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, qr[st + 0], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.x, dor[st + 0], dp, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, qr[st + 1], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.y, dor[st + 1], dp, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, qr[st + 2], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.z, dor[st + 2], dp, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, qr[st + 3], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.w, dor[st + 3], dp, 0, 0, 0);
-        }
-        float ds[16];
+    // keys past the end or above the diagonal have P = 0
+    auto drop_dead = [&](int k0) __attribute__((always_inline)) {
+        if (!(k0 + F32_BK > kend || (CAUSAL && k0 + F32_BK - 1 > wq0))) return;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            float xv = fmaf(s[r], c2, -lse2);
-            if (p.mask != nullptr && key < N) xv = fmaf(p.mask[(size_t)rr * N + key], BWD_LOG2E, xv);
-            const bool dead = key >= kend || (CAUSAL && key > q_row) || !row_live;
-            const float pr = dead ? 0.f : __builtin_amdgcn_exp2f(xv);
-            ds[r] = pr * (dp[r] - di) * p.scale;
+            if (key >= kend || (CAUSAL && key > q_row)) ds[r] = 0.f;
         }
-        // dQ^T += K^T dS^T: step (g, t) multiplies key 8 g + 4 h + t
+    };
+    uint32_t tmp[4];
+    auto split_ds = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, g = i / SPLIT_STEPS;
+        split_op<i % SPLIT_STEPS>(ds + 8 * g, tmp, db_[g]);
+    };
+
+    if constexpr (SPLIT) {
+        PairStage<D, 64> stage;
+        unsigned char *kt = lds + wave * 2 * Tile::BYTES, *vt = kt + Tile::BYTES;
+        if (wave < ntiles) stage.fetch(kp, vp, lane, wave * F32_BK, kend - 1);
+        for (int it = wave; it < ntiles; it += NW) {
+            const int k0 = it * F32_BK;
+            stage.put(kt, vt, lane);
+            if (it + NW < ntiles) stage.fetch(kp, vp, lane, k0 + NW * F32_BK, kend - 1);
+            s = mul_rows<D>(kt, r_addr, qr);
+            dp = mul_rows<D>(vt, r_addr, dor);
+            add_mask(k0);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float *kcol = &ks[(8 * (r >> 2) + 4 * h + (r & 3)) * ROW + i32];
+            for (int r = 0; r < 16; ++r) make_ds(r);
+            drop_dead(k0);
+            static_for<0, 2 * SPLIT_STEPS>(split_ds);
+            mul_cols<D>(kt, c_addr, db_, acc);
+        }
+    } else {
+        // The pipelined tile loop (flash_f32.h), one tile ahead:
+        //   R1(n)  S(n+1), dP(n+1)   (MFMA)  |  dS(n) split into its three parts; this thread's share of K(n+2), V(n+2) split
+        //                                       and written to LDS                                  (VALU)
+        //   R2(n)  dQ += K(n)^T dS(n) (MFMA)  |  dS(n+1) from S(n+1), dP(n+1)                        (VALU)
+        // then a barrier.  K is read in two iterations (three tiles in LDS), V in one (two).
+        PairStage<D, NW * 64> stage;
+        unsigned char *k_ring = lds, *v_ring = lds + 3 * Tile::BYTES;
+        if (ntiles > 0) {
+            PairStage<D, NW * 64> first;
+            first.fetch(kp, vp, tid, 0, kend - 1);
+            stage.fetch(kp, vp, tid, F32_BK, kend - 1);
+            first.put(k_ring, v_ring, tid);
+            stage.put(k_ring + Tile::BYTES, v_ring + Tile::BYTES, tid);
+            stage.fetch(kp, vp, tid, 2 * F32_BK, kend - 1);
+        }
+        __syncthreads();
+        if (my_tiles > 0) {
+            s = mul_rows<D>(k_ring, r_addr, qr);
+            dp = mul_rows<D>(v_ring, r_addr, dor);
+            add_mask(0);
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
-                acc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(kcol[db * 32], ds[r], acc[db], 0, 0, 0);
+            for (int r = 0; r < 16; ++r) make_ds(r);
+            drop_dead(0);
+        }
+        __syncthreads();  // V(0) has been read: its slot is written next
+        int k_cur = 0;  // ring slot of K(n)
+        auto slot = [](int k) __attribute__((always_inline)) { return k >= 3 ? k - 3 : k; };
+        SplitFrag fr;
+        int n = 0;
+#pragma clang loop unroll(disable)
+        for (; n < my_tiles - 1; ++n) {
+            const unsigned char *kt = k_ring + k_cur * Tile::BYTES, *kt1 = k_ring + slot(k_cur + 1) * Tile::BYTES,
+                                *vt1 = v_ring + ((n + 1) & 1) * Tile::BYTES;
+            unsigned char *kt2 = k_ring + slot(k_cur + 2) * Tile::BYTES, *vt2 = v_ring + (n & 1) * Tile::BYTES;
+            auto load_row = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
+                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
+            };
+            auto load_col = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
+                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                const int o = (i % DB) * 2048 + (i / DB) * 1024;
+                fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
+            };
+            // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
+            static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, kt1, 0); });
+            static_for<0, 4>(split_ds);
+            ARHIP_FENCE();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+            mfma_region<2 * KSTEPS, 2 * SPLIT_STEPS - 4 + PairStage<D, NW * 64>::STEPS>(
+                [&](auto fi, auto mi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, m = decltype(mi)::value;
+                    if constexpr (f < KSTEPS) s = mfma_split_step<m>(fr.template get<(f & 1)>(), qr[f], s);
+                    else dp = mfma_split_step<m>(fr.template get<(f & 1)>(), dor[f - KSTEPS], dp);
+                },
+                [&](auto fi, auto pi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    if constexpr (f < KSTEPS) load_row(fi, pi, kt1, f);
+                    else if constexpr (f < 2 * KSTEPS) load_row(fi, pi, vt1, f - KSTEPS);
+                    else load_col(fi, pi, kt, 0);
+                },
+                [&](auto ic) __attribute__((always_inline)) {
+                    constexpr int i = decltype(ic)::value;
+                    if constexpr (i < 2 * SPLIT_STEPS - 4) split_ds(std::integral_constant<int, i + 4>{});
+                    else stage.template split_step<i - (2 * SPLIT_STEPS - 4)>(kt2, vt2, tid);
+                });
+            if (n + 3 < ntiles) stage.fetch(kp, vp, tid, (n + 3) * F32_BK, kend - 1);
+            add_mask((n + 1) * F32_BK);
+            // ---- R2 ----
+            mfma_region<2 * DB, 24>(
+                [&](auto fi, auto mi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    acc[f % DB] = mfma_split_step<decltype(mi)::value>(fr.template get<(f & 1)>(), db_[f / DB], acc[f % DB]);
+                },
+                [&](auto fi, auto pi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    if constexpr (f < 2 * DB) load_col(fi, pi, kt, f);
+                },
+                ds_step);
+            drop_dead((n + 1) * F32_BK);
+            k_cur = slot(k_cur + 1);
+            __syncthreads();
+        }
+        if (my_tiles > 0) {
+            static_for<0, 2 * SPLIT_STEPS>(split_ds);
+            mul_cols<D>(k_ring + k_cur * Tile::BYTES, c_addr, db_, acc);
+        }
+        // under the causal mask a wave is done before others of its workgroup: it still stages tiles for them
+        for (; n < ntiles - 1; ++n) {
+            stage.put(k_ring + slot(k_cur + 2) * Tile::BYTES, v_ring + (n & 1) * Tile::BYTES, tid);
+            if (n + 3 < ntiles) stage.fetch(kp, vp, tid, (n + 3) * F32_BK, kend - 1);
+            k_cur = slot(k_cur + 1);
+            __syncthreads();
         }
     }
+
     if constexpr (SPLIT) {
-        // the waves' partial sums, each as [32 queries][ROW] in its own slab (its tiles are consumed)
-        float *ow = lds + wave * SLAB;
+        // the waves' partial sums, each as [32 queries][ROW]
+        constexpr int ROW = D + 4, SLAB = 32 * ROW;
+        float *part = (float *)lds;
+        __syncthreads();  // every wave's tiles are consumed
+        float *ow = part + wave * SLAB;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -237,13 +389,13 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, float *lds,
             float *op = p.dq + ((size_t)bh * N + qblk + q) * D + cg * CPT;
 #pragma unroll
             for (int c = 0; c < CPT; c += 4) {
-                float4 sum = *(const float4 *)&lds[q * ROW + cg * CPT + c];
+                float4 sum = *(const float4 *)&part[q * ROW + cg * CPT + c];
 #pragma unroll
                 for (int w = 1; w < NW; ++w) {
-                    const float4 x = *(const float4 *)&lds[w * SLAB + q * ROW + cg * CPT + c];
+                    const float4 x = *(const float4 *)&part[w * SLAB + q * ROW + cg * CPT + c];
                     sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
                 }
-                *(float4 *)(op + c) = sum;
+                *(float4 *)(op + c) = make_float4(sum.x * p.scale, sum.y * p.scale, sum.z * p.scale, sum.w * p.scale);
             }
         }
         return;
@@ -254,32 +406,24 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, float *lds,
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
-                *(float4 *)(op + db * 32 + 8 * g + 4 * h) =
-                    make_float4(acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]);
+                *(float4 *)(op + db * 32 + 8 * g + 4 * h) = make_float4(acc[db][4 * g] * p.scale, acc[db][4 * g + 1] * p.scale,
+                                                                        acc[db][4 * g + 2] * p.scale, acc[db][4 * g + 3] * p.scale);
     }
 }
 
-// dK and dV.  Workgroup wg_linear in [0, nt * B * Hkv): 32 NW keys of one K/V head.  SPLIT: the NW waves
+// dK and dV.  Workgroup wg_linear in [0, nt * B * Hkv), four waves: 128 keys of one K/V head.  SPLIT: the waves
 // share the same 32 keys and deal the (head of the group, query tile) steps out between them, each in
 // its own LDS slab; the partial dK and dV of the waves are added through LDS in wave order.
-template <int D, int NW, bool CAUSAL, bool SPLIT = false>
-__device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, float *lds, int wg_linear)
+template <int D, bool CAUSAL, bool SPLIT>
+__device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned char *lds, int wg_linear)
 {
-    constexpr int T = SPLIT ? 64 : NW * 64;   // threads staging one tile
+    constexpr int NW = 4;
     constexpr int BKW = SPLIT ? 32 : NW * 32;  // keys per workgroup
-    constexpr int HALF = D / 2;
-    constexpr int ROW = D + 4;
-    constexpr int DB = D / 32;
-    constexpr int CHUNKS = F32_BK * D / 4;
-    constexpr int PER_THREAD = CHUNKS / T;
-    static_assert(CHUNKS % T == 0, "tile staging must divide evenly");
+    constexpr int DB = D / 32, KSTEPS = D / 16;
+    using Tile = SplitTile<D>;
 
-    constexpr int SLAB = 2 * F32_BK * ROW + 64;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    float *qs = lds + (SPLIT ? wave * SLAB : 0);
-    float *dos = qs + F32_BK * ROW;
-    float *stat = qs + 2 * F32_BK * ROW;  // lse[32], D[32] of the staged queries
     const int stid = SPLIT ? lane : tid;      // index among the threads staging a tile
     const int i32 = lane & 31, h = lane >> 5;
     const int wg_x = (p.total_kv > 0 && (p.total_kv & 7) == 0) ? (wg_linear & 7) * (p.total_kv >> 3) + (wg_linear >> 3) : wg_linear;
@@ -304,15 +448,13 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, float *lds
     const bool key_live = key < kvl;
     const float c2 = p.scale * BWD_LOG2E;
 
-    float kr[HALF], vr[HALF];
+    split8 kr[KSTEPS], vr[KSTEPS];
     {
-        const size_t off = ((size_t)kv_bh * N + jj) * D + h * HALF;
+        const size_t off = ((size_t)kv_bh * N + jj) * D + h * 8;
 #pragma unroll
-        for (int s = 0; s < HALF; s += 4) {
-            const float4 x = *(const float4 *)(p.k + off + s);
-            const float4 y = *(const float4 *)(p.v + off + s);
-            kr[s] = x.x; kr[s + 1] = x.y; kr[s + 2] = x.z; kr[s + 3] = x.w;
-            vr[s] = y.x; vr[s + 1] = y.y; vr[s + 2] = y.z; vr[s + 3] = y.w;
+        for (int s = 0; s < KSTEPS; ++s) {
+            kr[s] = split_8(*(const float4 *)(p.k + off + 16 * s), *(const float4 *)(p.k + off + 16 * s + 4));
+            vr[s] = split_8(*(const float4 *)(p.v + off + 16 * s), *(const float4 *)(p.v + off + 16 * s + 4));
         }
     }
     f32x16_t dk[DB], dv[DB];
@@ -320,138 +462,269 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, float *lds
     for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.f;
+    const int r_addr[2] = {Tile::row_addr(i32, h, 0), Tile::row_addr(i32, h, 1)};
+    const int c_addr[2] = {Tile::col_addr(lane, 0), Tile::col_addr(lane, 1)};
 
     // queries before the workgroup's first key see none of its keys under the causal mask
     const int qt0 = CAUSAL ? kblk / F32_BK : 0;
-    const int qtiles = (N + F32_BK - 1) / F32_BK;
-    const int steps = group * (qtiles - qt0);  // (head of the group, query tile) pairs, head-major
+    const int qtiles = (N + F32_BK - 1) / F32_BK, per_head = qtiles - qt0;
+    // (head of the group, query tile) pairs, head-major; a workgroup whose keys are all past the key length has none
+    const int steps = kblk < kvl ? group * per_head : 0;
+    // the last query tile first, so that under the causal mask the tiles a wave has no part in come at the end of a head
+    auto step_head = [&](int st) __attribute__((always_inline)) { return (size_t)b * p.Hq + (size_t)kvh * group + st / per_head; };
+    auto step_q0 = [&](int st) __attribute__((always_inline)) { return (qtiles - 1 - st % per_head) * F32_BK; };
 
-    f32x4_t qx[PER_THREAD], dx[PER_THREAD];
+    PairStage<D, SPLIT ? 64 : NW * 64> stage;
     float st_l = 0.f, st_d = 0.f;
-    auto fetch = [&](int step) __attribute__((always_inline)) {
-        const int g = step / (qtiles - qt0);
-        const int q0 = (qt0 + step - g * (qtiles - qt0)) * F32_BK;
-        const size_t bh = (size_t)b * p.Hq + (size_t)kvh * group + g;
-        // Rows past the last query repeat it: whatever they hold is multiplied by P = dS = 0 (finite values, not
-        // zeros, are all that takes).  One path without a branch, and native vectors (typed loads and stores): both
-        // keep the staged tile in registers at D = 128.
-#pragma unroll
-        for (int j = 0; j < PER_THREAD; ++j) {
-            const int c = stid + j * T;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            const size_t off = (bh * N + min(q0 + row, N - 1)) * D + col;
-            qx[j] = *(const f32x4_t *)(p.q + off);
-            dx[j] = *(const f32x4_t *)(p.dout + off);
-        }
+    auto fetch_tiles = [&](decltype(stage) &to, int st) __attribute__((always_inline)) {
+        const size_t off = step_head(st) * N * D;
+        to.fetch(p.q + off, p.dout + off, stid, step_q0(st), N - 1);
+    };
+    // base-2 units: P = 2^(x log2(e) - lse log2(e)); rows that saw no key (and rows past the end) have P = 0
+    auto fetch_stats = [&](int st) __attribute__((always_inline)) {
         if (stid < F32_BK) {
-            const int gr = q0 + stid;
-            st_l = gr < N ? p.lse[bh * N + gr] : -1e30f;
+            const int gr = step_q0(st) + stid;
+            const size_t bh = step_head(st);
+            const float lse = gr < N ? p.lse[bh * N + gr] : -1e30f;
+            st_l = lse > BWD_LSE_FLOOR ? lse * BWD_LOG2E : __builtin_inff();
             st_d = gr < N ? p.delta[bh * N + gr] : 0.f;
         }
     };
-    constexpr int STEP = SPLIT ? NW : 1;
-    const int first = SPLIT ? wave : 0;
-    if (first < steps) fetch(first);
-    // the staged tile of the previous step goes to LDS, the next one is requested
-    auto stage = [&](int step) __attribute__((always_inline)) {
-        if (!SPLIT) __syncthreads();
-#pragma unroll
-        for (int j = 0; j < PER_THREAD; ++j) {
-            const int c = stid + j * T;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            *(f32x4_t *)&qs[row * ROW + col] = qx[j];
-            *(f32x4_t *)&dos[row * ROW + col] = dx[j];
-        }
+    auto put_stats = [&](float *stat) __attribute__((always_inline)) {
         if (stid < F32_BK) {
-            stat[stid] = st_l * BWD_LOG2E;   // base-2 units: P = 2^(x log2(e) - lse log2(e))
+            stat[stid] = st_l;
             stat[32 + stid] = st_d;
         }
-        if (step + STEP < steps) fetch(step + STEP);
-        if (!SPLIT) __syncthreads();
     };
-    auto compute = [&](int step) __attribute__((always_inline)) {
-        const int g = step / (qtiles - qt0);
-        const int q0 = (qt0 + step - g * (qtiles - qt0)) * F32_BK;
 
-        // S = Q K^T and dP = dO V^T: lane = key, register r = query 8 (r / 4) + 4 h + r % 4 of the tile
-        f32x16_t s, dp;
+    // S = Q K^T and dP = dO V^T: lane = key, register r = query 8 (r / 4) + 4 h + r % 4 of the tile
+    f32x16_t s, dp;
+    float pr[16], ds[16];  // P and dS / scale
+    float4 st4[4];         // lse, then D, of the lane's 16 queries
+    split8 pb[2], db_[2];
+    auto read_stats = [&](const float *stat) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-        const float *qrow = &qs[i32 * ROW + h * HALF];
-        const float *drow = &dos[i32 * ROW + h * HALF];
-#pragma unroll
-        for (int st = 0; st < HALF; st += 4) {
-            const float4 a = *(const float4 *)(qrow + st);
-            const float4 c = *(const float4 *)(drow + st);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, kr[st + 0], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.x, vr[st + 0], dp, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, kr[st + 1], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.y, vr[st + 1], dp, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, kr[st + 2], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.z, vr[st + 2], dp, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, kr[st + 3], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(c.w, vr[st + 3], dp, 0, 0, 0);
-        }
-        float pr[16], ds[16];
-        const int kq = key - q0 - 4 * h;  // causal: query 8 gq + 4 h + t of the tile sees this lane's key iff kq <= 8 gq + t
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-            const float4 l4 = *(const float4 *)&stat[8 * gq + 4 * h];
-            const float4 d4 = *(const float4 *)&stat[32 + 8 * gq + 4 * h];
-            const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dvv[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int r = 4 * gq + t;
-                const int qi = q0 + 8 * gq + 4 * h + t;
-                float xv = fmaf(s[r], c2, -lv[t]);
-                if (p.mask != nullptr && qi < N) xv = fmaf(p.mask[(size_t)qi * N + jj], BWD_LOG2E, xv);
-                const bool dead = qi >= N || !key_live || (CAUSAL && kq > 8 * gq + t) || !(lv[t] > BWD_LSE_FLOOR);
-                pr[r] = dead ? 0.f : __builtin_amdgcn_exp2f(xv);
-                ds[r] = pr[r] * (dp[r] - dvv[t]) * p.scale;
-            }
-        }
-        // dV^T += dO^T P and dK^T += Q^T dS: step (g, t) multiplies query 8 g + 4 h + t of the tile
+        for (int g = 0; g < 4; ++g) st4[g] = *(const float4 *)&stat[8 * g + 4 * h];
+    };
+    auto stat_of = [&](int r) __attribute__((always_inline)) {
+        const float4 &v = st4[r >> 2];
+        return (r & 3) == 0 ? v.x : (r & 3) == 1 ? v.y : (r & 3) == 2 ? v.z : v.w;
+    };
+    // what the logits are multiplied by in the exponent: c2, or 1 where the mask has been added (add_mask)
+    const float cx = p.mask != nullptr ? 1.f : c2;
+    auto add_mask = [&](int q0) __attribute__((always_inline)) {
+        if (p.mask == nullptr) return;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int qi = 8 * (r >> 2) + 4 * h + (r & 3);
-            const float *dcol = &dos[qi * ROW + i32];
-            const float *qcol = &qs[qi * ROW + i32];
-#pragma unroll
-            for (int db = 0; db < DB; ++db) {
-                dv[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(dcol[db * 32], pr[r], dv[db], 0, 0, 0);
-                dk[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(qcol[db * 32], ds[r], dk[db], 0, 0, 0);
-            }
+            const int qi = min(q0 + 8 * (r >> 2) + 4 * h + (r & 3), N - 1);
+            s[r] = fmaf(p.mask[(size_t)qi * N + jj], BWD_LOG2E, s[r] * c2);
         }
     };
-    if constexpr (CAUSAL && !SPLIT) {
-        // Every query of the first `wave` tiles of a head precedes this wave's keys: those tiles are staged (all
-        // waves pass the same barriers) and not computed.  Two plain loops instead of a branch around the matrix
-        // work, which costs the register allocator the accumulators twice.
-        const int tiles = qtiles - qt0, nskip = min(wave, tiles);
-        for (int g = 0; g < group; ++g) {
-            for (int t = 0; t < nskip; ++t) stage(g * tiles + t);
-            for (int t = nskip; t < tiles; ++t) {
-                stage(g * tiles + t);
-                compute(g * tiles + t);
+    auto make_p = [&](int r) __attribute__((always_inline)) { pr[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cx, -stat_of(r))); };
+    auto make_ds = [&](int r) __attribute__((always_inline)) { ds[r] = pr[r] * (dp[r] - stat_of(r)); };
+    // keys past the key length or below the diagonal have P = 0
+    auto drop_dead = [&](int q0) __attribute__((always_inline)) {
+        if (!(wk0 + 31 >= kvl || (CAUSAL && wk0 + 31 > q0))) return;
+        const int kq = key - q0 - 4 * h;  // causal: query 8 gq + 4 h + t of the tile sees this lane's key iff kq <= 8 gq + t
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            if (!key_live || (CAUSAL && kq > 8 * (r >> 2) + (r & 3))) pr[r] = ds[r] = 0.f;
+    };
+    auto make_all = [&](int q0, const float *stat) __attribute__((always_inline)) {
+        add_mask(q0);
+        read_stats(stat);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) make_p(r);
+        read_stats(stat + 32);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) make_ds(r);
+        drop_dead(q0);
+    };
+    uint32_t tmp[4];
+    auto split_p = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, g = i / SPLIT_STEPS;
+        split_op<i % SPLIT_STEPS>(pr + 8 * g, tmp, pb[g]);
+    };
+    auto split_ds = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, g = i / SPLIT_STEPS;
+        split_op<i % SPLIT_STEPS>(ds + 8 * g, tmp, db_[g]);
+    };
+
+    if constexpr (SPLIT) {
+        unsigned char *qs = lds + wave * (2 * Tile::BYTES + 256), *dos = qs + Tile::BYTES;
+        float *stat = (float *)(qs + 2 * Tile::BYTES);
+        if (wave < steps) {
+            fetch_tiles(stage, wave);
+            fetch_stats(wave);
+        }
+        for (int st = wave; st < steps; st += NW) {
+            stage.put(qs, dos, lane);
+            put_stats(stat);
+            if (st + NW < steps) {
+                fetch_tiles(stage, st + NW);
+                fetch_stats(st + NW);
             }
+            s = mul_rows<D>(qs, r_addr, kr);
+            dp = mul_rows<D>(dos, r_addr, vr);
+            make_all(step_q0(st), stat);
+            static_for<0, 2 * SPLIT_STEPS>(split_p);
+            mul_cols<D>(dos, c_addr, pb, dv);
+            static_for<0, 2 * SPLIT_STEPS>(split_ds);
+            mul_cols<D>(qs, c_addr, db_, dk);
         }
     } else {
-        // (SPLIT: the tiles start at the workgroup's first key, so none lies wholly before its keys)
-        for (int step = first; step < steps; step += STEP) {
-            stage(step);
-            compute(step);
+        // The pipelined loop (flash_f32.h), one step ahead:
+        //   R1(n)  S(n+1), dP(n+1)                            (MFMA)  |  P(n) and dS(n) split into their three parts   (VALU)
+        //   R2(n)  dV += dO(n)^T P(n), dK += Q(n)^T dS(n)      (MFMA)  |  P(n+1), dS(n+1); this thread's share of Q(n+2), dO(n+2)
+        //                                                                split and written to LDS                     (VALU)
+        // then a barrier.  Both tiles are read in two iterations: rings of three.
+        unsigned char *q_ring = lds, *o_ring = lds + 3 * Tile::BYTES;
+        float *stats = (float *)(lds + 6 * Tile::BYTES);
+        // steps this wave computes on (heads sharing the K/V head: all but those at the very end)
+        const int mine = wk0 >= kvl ? 0 : CAUSAL ? max(0, steps - wave) : steps;
+        if (steps > 0) {
+            decltype(stage) first;
+            fetch_tiles(first, 0);
+            fetch_stats(0);
+            if (steps > 1) fetch_tiles(stage, 1);
+            first.put(q_ring, o_ring, tid);
+            put_stats(stats);
+            if (steps > 1) {
+                stage.put(q_ring + Tile::BYTES, o_ring + Tile::BYTES, tid);
+                fetch_stats(1);
+                put_stats(stats + 64);
+            }
+            if (steps > 2) {
+                fetch_tiles(stage, 2);
+                fetch_stats(2);
+            }
+        }
+        __syncthreads();
+        if (mine > 0) {
+            s = mul_rows<D>(q_ring, r_addr, kr);
+            dp = mul_rows<D>(o_ring, r_addr, vr);
+            make_all(step_q0(0), stats);
+        }
+        int cur = 0;  // ring slot of step n
+        auto slot = [](int k) __attribute__((always_inline)) { return k >= 3 ? k - 3 : k; };
+        SplitFrag fr;
+        int n = 0;
+#pragma clang loop unroll(disable)
+        for (; n < mine - 1; ++n) {
+            const int s1 = slot(cur + 1), s2 = slot(cur + 2);
+            const unsigned char *qt = q_ring + cur * Tile::BYTES, *ot = o_ring + cur * Tile::BYTES;
+            const unsigned char *qt1 = q_ring + s1 * Tile::BYTES, *ot1 = o_ring + s1 * Tile::BYTES;
+            unsigned char *qt2 = q_ring + s2 * Tile::BYTES, *ot2 = o_ring + s2 * Tile::BYTES;
+            auto load_row = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
+                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
+            };
+            auto load_col = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
+                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                const int o = (i % DB) * 2048 + (i / DB) * 1024;
+                fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
+            };
+            // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
+            static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, qt1, 0); });
+            static_for<0, 4>(split_p);
+            ARHIP_FENCE();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+            mfma_region<2 * KSTEPS, 4 * SPLIT_STEPS - 4>(
+                [&](auto fi, auto mi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, m = decltype(mi)::value;
+                    if constexpr (f < KSTEPS) s = mfma_split_step<m>(fr.template get<(f & 1)>(), kr[f], s);
+                    else dp = mfma_split_step<m>(fr.template get<(f & 1)>(), vr[f - KSTEPS], dp);
+                },
+                [&](auto fi, auto pi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    if constexpr (f < KSTEPS) load_row(fi, pi, qt1, f);
+                    else if constexpr (f < 2 * KSTEPS) load_row(fi, pi, ot1, f - KSTEPS);
+                    else load_col(fi, pi, ot, 0);
+                },
+                [&](auto ic) __attribute__((always_inline)) {
+                    constexpr int i = decltype(ic)::value;
+                    if constexpr (i < 2 * SPLIT_STEPS - 4) split_p(std::integral_constant<int, i + 4>{});
+                    else split_ds(std::integral_constant<int, i - (2 * SPLIT_STEPS - 4)>{});
+                });
+            add_mask(step_q0(n + 1));
+            read_stats(stats + s1 * 64);
+            // ---- R2 ----
+            constexpr int CONV = decltype(stage)::STEPS;
+            mfma_region<4 * DB, 24 + CONV>(
+                [&](auto fi, auto mi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, m = decltype(mi)::value, g = f % (2 * DB);
+                    if constexpr (f < 2 * DB) dv[g % DB] = mfma_split_step<m>(fr.template get<(f & 1)>(), pb[g / DB], dv[g % DB]);
+                    else dk[g % DB] = mfma_split_step<m>(fr.template get<(f & 1)>(), db_[g / DB], dk[g % DB]);
+                },
+                [&](auto fi, auto pi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    if constexpr (f < 2 * DB) load_col(fi, pi, ot, f);
+                    else if constexpr (f < 4 * DB) load_col(fi, pi, qt, f - 2 * DB);
+                },
+                [&](auto ic) __attribute__((always_inline)) {
+                    constexpr int i = decltype(ic)::value;
+                    if constexpr (i < 16) {
+                        constexpr int e = (i >> 1) * 2;
+#pragma unroll
+                        for (int r = e; r < e + 2; ++r) pr[r] = (i & 1) ? __builtin_amdgcn_exp2f(pr[r]) : fmaf(s[r], cx, -stat_of(r));
+                        pin(pr[e], pr[e + 1]);
+                        if constexpr (i == 15) read_stats(stats + s1 * 64 + 32);
+                    } else if constexpr (i < 24) {
+                        constexpr int e = ((i - 16) >> 1) * 4;
+#pragma unroll
+                        for (int r = e; r < e + 4; ++r) {
+                            ds[r] = (i & 1) ? pr[r] * ds[r] : dp[r] - stat_of(r);
+                            asm volatile("" : "+v"(ds[r]));
+                        }
+                    } else {
+                        stage.template split_step<i - 24>(qt2, ot2, tid);
+                    }
+                });
+            if (n + 2 < steps) put_stats(stats + s2 * 64);
+            if (n + 3 < steps) {
+                fetch_tiles(stage, n + 3);
+                fetch_stats(n + 3);
+            }
+            drop_dead(step_q0(n + 1));
+            cur = s1;
+            __syncthreads();
+        }
+        if (mine > 0) {
+            static_for<0, 2 * SPLIT_STEPS>(split_p);
+            mul_cols<D>(o_ring + cur * Tile::BYTES, c_addr, pb, dv);
+            static_for<0, 2 * SPLIT_STEPS>(split_ds);
+            mul_cols<D>(q_ring + cur * Tile::BYTES, c_addr, db_, dk);
+        }
+        // a wave that is done before others of its workgroup still stages tiles for them
+        for (; n < steps - 1; ++n) {
+            const int s2 = slot(cur + 2);
+            if (n + 2 < steps) {
+                stage.put(q_ring + s2 * Tile::BYTES, o_ring + s2 * Tile::BYTES, tid);
+                put_stats(stats + s2 * 64);
+            }
+            if (n + 3 < steps) {
+                fetch_tiles(stage, n + 3);
+                fetch_stats(n + 3);
+            }
+            cur = slot(cur + 1);
+            __syncthreads();
         }
     }
+
     if constexpr (SPLIT) {
-        // the waves' partial sums: dK as [32 keys][ROW] in the first tile of the slab, dV in the second
-        float *ow = lds + wave * SLAB;
+        // the waves' partial sums: dK, then dV, each as [32 keys][ROW]
+        constexpr int ROW = D + 4, SLAB = 2 * 32 * ROW;
+        float *part = (float *)lds;
+        __syncthreads();  // every wave's tiles are consumed
+        float *ow = part + wave * SLAB;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int d = db * 32 + 8 * g + 4 * h;
                 *(float4 *)&ow[i32 * ROW + d] = make_float4(dk[db][4 * g], dk[db][4 * g + 1], dk[db][4 * g + 2], dk[db][4 * g + 3]);
-                *(float4 *)&ow[(F32_BK + i32) * ROW + d] = make_float4(dv[db][4 * g], dv[db][4 * g + 1], dv[db][4 * g + 2], dv[db][4 * g + 3]);
+                *(float4 *)&ow[(32 + i32) * ROW + d] = make_float4(dv[db][4 * g], dv[db][4 * g + 1], dv[db][4 * g + 2], dv[db][4 * g + 3]);
             }
         __syncthreads();
         // thread t: key t % 32, channels [cg * CPT, cg * CPT + CPT) of dK and of dV
@@ -463,15 +736,16 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, float *lds
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
                 float *op = (half ? p.dv : p.dk) + orow;
+                const float f = half ? 1.f : p.scale;
 #pragma unroll
                 for (int c = 0; c < CPT; c += 4) {
-                    float4 sum = *(const float4 *)&lds[(half * F32_BK + kq) * ROW + cg * CPT + c];
+                    float4 sum = *(const float4 *)&part[(half * 32 + kq) * ROW + cg * CPT + c];
 #pragma unroll
                     for (int w = 1; w < NW; ++w) {
-                        const float4 x = *(const float4 *)&lds[w * SLAB + (half * F32_BK + kq) * ROW + cg * CPT + c];
+                        const float4 x = *(const float4 *)&part[w * SLAB + (half * 32 + kq) * ROW + cg * CPT + c];
                         sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
                     }
-                    *(float4 *)(op + c) = sum;
+                    *(float4 *)(op + c) = make_float4(sum.x * f, sum.y * f, sum.z * f, sum.w * f);
                 }
             }
         }
@@ -485,7 +759,8 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, float *lds
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int d = db * 32 + 8 * g + 4 * h;
-                *(float4 *)(okp + d) = make_float4(dk[db][4 * g], dk[db][4 * g + 1], dk[db][4 * g + 2], dk[db][4 * g + 3]);
+                *(float4 *)(okp + d) = make_float4(dk[db][4 * g] * p.scale, dk[db][4 * g + 1] * p.scale, dk[db][4 * g + 2] * p.scale,
+                                                   dk[db][4 * g + 3] * p.scale);
                 *(float4 *)(ovp + d) = make_float4(dv[db][4 * g], dv[db][4 * g + 1], dv[db][4 * g + 2], dv[db][4 * g + 3]);
             }
     }
@@ -497,20 +772,19 @@ __global__ void __launch_bounds__(256) bwd_prep_kernel(const float *o, const flo
     bwd_prep_body<D>(o, dout, delta, rows, (long)blockIdx.x * 4);
 }
 
-// D = 64: registers held to 256 per lane so that a SIMD holds two waves (the split dK/dV variant would
-// spill at that limit and keeps one)
-template <int D, int NW, bool CAUSAL, bool SPLIT>
-__global__ void __launch_bounds__(NW * 64, (D == 64 ? 2 : 1)) bwd_dq_kernel(const FlashBwdParams p)
+// D = 64: registers held to 256 per lane so that a SIMD holds two waves; D = 128 needs more than that
+template <int D, bool CAUSAL, bool SPLIT>
+__global__ void __launch_bounds__(256, (D == 64 ? 2 : 1)) bwd_dq_kernel(const FlashBwdParams p)
 {
-    __shared__ __attribute__((aligned(16))) float lds[bwd_lds_floats<D, NW, SPLIT>()];
-    bwd_dq_body<D, NW, CAUSAL, SPLIT>(p, lds, (int)blockIdx.x);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dq_lds_bytes<D, SPLIT>()];
+    bwd_dq_body<D, CAUSAL, SPLIT>(p, lds, (int)blockIdx.x);
 }
 
-template <int D, int NW, bool CAUSAL, bool SPLIT>
-__global__ void __launch_bounds__(NW * 64, (D == 64 && !SPLIT ? 2 : 1)) bwd_dkv_kernel(const FlashBwdParams p)
+template <int D, bool CAUSAL, bool SPLIT>
+__global__ void __launch_bounds__(256, 1) bwd_dkv_kernel(const FlashBwdParams p)
 {
-    __shared__ __attribute__((aligned(16))) float lds[bwd_lds_floats<D, NW, SPLIT>()];
-    bwd_dkv_body<D, NW, CAUSAL, SPLIT>(p, lds, (int)blockIdx.x);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dkv_lds_bytes<D, SPLIT>()];
+    bwd_dkv_body<D, CAUSAL, SPLIT>(p, lds, (int)blockIdx.x);
 }
 
 }  // namespace arhip

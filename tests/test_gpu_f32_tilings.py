@@ -1,5 +1,5 @@
-"""The tilings of the fp32 forward at the edges of their tiles, against the float64 oracle on sampled heads: many heads, so that
-the launches take the tilings whose waves share their key tiles and not the one for few, short heads."""
+"""The tilings of the fp32 kernels at the edges of their tiles, against the float64 oracle on sampled heads: many heads, so that
+the launches take the tilings whose waves share their key (query) tiles and not the one for few, short heads."""
 import numpy as np
 import pytest
 
@@ -7,6 +7,7 @@ import oracle
 from autorust_amd import synth
 from autorust_amd.device import F32
 from gpu_util import run_flash
+from test_gpu_bwd import run_fwd_bwd
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +30,24 @@ def test_f32_forward_tilings(dev, shape, mode):
         want = oracle.sdpa_f64(q[b:b + 1, h:h + 1], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], causal=causal,
                                kv_len=None if lens is None else lens[b:b + 1]) if lens is None or lens[b] > 0 else np.zeros((1, 1, N, D))
         assert np.abs(got[b, h] - want[0, 0]).max() <= 3e-6 * max(np.abs(v[b, h]).max(), 1e-30), (b, h)
+
+
+@pytest.mark.parametrize("mode", ["plain", "causal", "causal+len", "mask"])
+@pytest.mark.parametrize("shape", [(16, 16, 16, 1, 64), (16, 8, 8, 33, 64), (8, 32, 16, 97, 64), (16, 8, 8, 129, 64), (16, 8, 8, 32, 128),
+                                   (8, 16, 8, 65, 128), (8, 8, 8, 257, 128)], ids=str)
+def test_f32_backward_tilings(dev, shape, mode):
+    B, Hq, Hkv, N, D = shape
+    q, do = (synth.normal(920 + i, (B, Hq, N, D)) for i in range(2))
+    k, v = (synth.normal(930 + i, (B, Hkv, N, D)) for i in range(2))
+    causal = "causal" in mode
+    lens = (1 + (np.arange(B) * 37) % N).astype(np.int32) if "len" in mode else None
+    mask = synth.normal(940, (N, N)) if mode == "mask" else None
+    got = run_fwd_bwd(dev, q, k, v, do, mask=mask, kv_len=lens, causal=causal)
+    g = Hq // Hkv
+    for b, h in ((0, 0), (B - 1, Hkv - 1)):
+        hs = slice(h * g, (h + 1) * g)
+        want = oracle.attention_backward_f64(q[b:b + 1, hs], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], do[b:b + 1, hs], mask=mask,
+                                             kv_len=None if lens is None else lens[b:b + 1], causal=causal)
+        for name, x, w in zip(("o", "lse", "dq", "dk", "dv"), got, want):
+            x = x[b:b + 1, hs] if name in ("o", "lse", "dq") else x[b:b + 1, h:h + 1]
+            assert np.abs(x - w).max() <= 1e-5 * max(1.0, np.abs(w).max()), (name, b, h)
