@@ -6,7 +6,9 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <map>
 #include <string>
+#include <string_view>
 #include <unordered_map>
 #include <vector>
 
@@ -16,7 +18,11 @@
 struct arhip_module_entry {
     std::vector<hipModule_t> mods;
     std::vector<std::vector<char>> images;  // private copies, alive as long as the modules are loaded
-    std::unordered_map<std::string, hipFunction_t> fns;
+    struct kernel {
+        hipFunction_t fn;
+        const void *entry;  // what a launch of this name must look like (device.hip), or null
+    };
+    std::map<std::string, kernel, std::less<>> fns;  // (found by std::string_view)
 };
 
 struct arhip_device {

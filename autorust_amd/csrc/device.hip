@@ -496,12 +496,16 @@ const named_entry NAMED[] = {
     {"ar_fl_bwd_dkv_short", 9, 6, 256, 32, true, false, false, 0, true},
 };
 
-int check_named_entry(const char *name, const unsigned grid[3], const unsigned block[3], int nbufs, const int64_t *vals,
-                      int nvals)
+const named_entry *find_named_entry(const char *name)
 {
-    const named_entry *e = nullptr;
     for (const named_entry &c : NAMED)
-        if (std::strcmp(c.name, name) == 0) e = &c;
+        if (std::strcmp(c.name, name) == 0) return &c;
+    return nullptr;
+}
+
+int check_named_entry(const named_entry *e, const char *name, const unsigned grid[3], const unsigned block[3], int nbufs,
+                      const int64_t *vals, int nvals)
+{
     if (!e) return ARHIP_OK;
     ARHIP_REQUIRE(nbufs == e->nbufs && nvals == e->nvals, "arhip_launch: %s takes %d buffers and %d scalars, got %d and %d", name,
                   e->nbufs, e->nvals, nbufs, nvals);
@@ -552,8 +556,9 @@ extern "C" int arhip_launch(arhip_device *dev, void *module, const char *name,
     ARHIP_REQUIRE(nbufs >= 0 && nvals >= 0 && nbufs + nvals <= 64, "arhip_launch: too many arguments");
     ARHIP_REQUIRE(nvals == 0 || (vals && val_bits), "arhip_launch: scalar values without widths");
     arhip_module_entry *m = (arhip_module_entry *)module;
+    // the function and its entry in NAMED, looked up once per name (without making a std::string of it afterwards)
     hipFunction_t fn;
-    auto it = m->fns.find(name);
+    auto it = m->fns.find(std::string_view(name));
     if (it == m->fns.end()) {
         hipError_t err = hipErrorNotFound;
         for (hipModule_t mod : m->mods) {
@@ -564,9 +569,9 @@ extern "C" int arhip_launch(arhip_device *dev, void *module, const char *name,
         if (err != hipSuccess) {
             return arhip_fail(ARHIP_EHIP, "arhip_launch: no kernel named %s in the module: %s", name, hipGetErrorString(err));
         }
-        m->fns[name] = fn;
+        it = m->fns.emplace(name, arhip_module_entry::kernel{fn, find_named_entry(name)}).first;
     } else {
-        fn = it->second;
+        fn = it->second.fn;
     }
     // A zero-sized grid is a no-op (the reference clamps negatives to 0, session.rs:241-251).
     if (grid[0] == 0 || grid[1] == 0 || grid[2] == 0) {
@@ -575,7 +580,7 @@ extern "C" int arhip_launch(arhip_device *dev, void *module, const char *name,
     }
     ARHIP_REQUIRE(block[0] * block[1] * block[2] >= 1 && block[0] * block[1] * block[2] <= 1024,
                   "arhip_launch: block of %u threads", block[0] * block[1] * block[2]);
-    if (int rc = check_named_entry(name, grid, block, nbufs, vals, nvals)) return rc;
+    if (int rc = check_named_entry((const named_entry *)it->second.entry, name, grid, block, nbufs, vals, nvals)) return rc;
     void *ptrs[64];
     int32_t v32[64];
     int64_t v64[64];

@@ -89,7 +89,7 @@ private:
 
 // Path of the code object with the named attention kernels (autorust_amd/attn_kernels.hsaco):
 // $AUTORUST_HIP_KERNELS, else the file next to this library.
-std::string attention_kernels_src();
+const std::string &attention_kernels_src();
 
 struct Storage {  // OpaqueT: base pointer + size, views share it (buffer.rs:32-39)
     std::shared_ptr<Device> dev;
@@ -151,7 +151,7 @@ struct HostCall {              // session.rs:210-256, field for field
     int64_t global[3];         // launch grid
     std::optional<std::array<int64_t, 3>> local;       // launch block
     std::vector<int64_t> vals; // scalar arguments
-    void exec() const;         // run_host_kernel(..., wait = true), session.rs:230-255
+    void exec() const;         // run_host_kernel on the device's stream (session.rs:230-255, which waits for every launch)
 };
 
 class Session {                // session.rs:44-193 (the part the path touches)
