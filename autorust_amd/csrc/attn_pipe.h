@@ -56,10 +56,11 @@ namespace arhip {
 // unit at D = 128; with 8-bit operands at D = 64 four whole stages fit twice as well (48 KB each), and with them the
 // four-tiles-per-trip loop and one more tile of latency cover: int8 B4 H32 N = 2048 / 8192 -7 / -5 %, causal -4 / -5 %,
 // per-key scales -7 / -5 %, B8 H6 N789 -4 %, same bits (bf16 at D = 64 gains nothing and loses 6 % on short causal shapes).
-template <int D, int MODE, int NW>
+// With an additive mask every form keeps rings: four whole stages would leave no room for the mask's blocks.
+template <int D, int MODE, int NW, bool HAS_MASK = false>
 constexpr bool attn_pipe_rings()
 {
-    return NW == 4 && !(D == 64 && MODE != MODE_BF16);
+    return HAS_MASK || (NW == 4 && !(D == 64 && MODE != MODE_BF16));
 }
 
 // LDS bytes attn_pipe_body needs: [piece][64 rows][64 B] K and V tiles, four stages of both, or a
@@ -68,12 +69,13 @@ constexpr bool attn_pipe_rings()
 // derived factors.
 // QFUSE (Q is quantised in the prologue): with scales over blocks of 128 queries, 256 bytes for the exchange of the
 // waves' maxima.
-template <int D, int MODE, int NW = 8, bool PER_KEY = false, bool QFUSE = false>
+// HAS_MASK: per wave, two blocks of 32 queries x 32 keys of the additive mask.
+template <int D, int MODE, int NW = 8, bool PER_KEY = false, bool QFUSE = false, bool HAS_MASK = false>
 constexpr int attn_pipe_lds_bytes()
 {
-    constexpr bool R = attn_pipe_rings<D, MODE, NW>();
+    constexpr bool R = attn_pipe_rings<D, MODE, NW, HAS_MASK>();
     return 4096 * ((R ? 2 : 4) * (D * ((MODE != MODE_BF16) ? 1 : 2) / 64) + (R ? 3 : 4) * (D * 2 / 64)) +
-           (PER_KEY ? 1024 + NW * 1024 : 0) + ((QFUSE && !PER_KEY) ? 256 : 0);
+           (PER_KEY ? 1024 + NW * 1024 : 0) + ((QFUSE && !PER_KEY) ? 256 : 0) + (HAS_MASK ? NW * 8192 : 0);
 }
 
 // workgroup index -> (batch * heads + head, query tile of 256), as in attn_fwd_kernel
@@ -100,7 +102,9 @@ __device__ __forceinline__ void pipe_work_item(const AttnParams &p, int wg, int 
 // that of quantising first; p.sq_out / p.q8_out, where not null, receive the scales and the codes.  Two forms: with K
 // scales over whole tiles, p.q holds bf16 values and a scale covers a block of 128 queries; with PER_KEY, p.q holds
 // f32 values and every query has its own scale (the reference's convention, src/runtime/cuda_flash_sage.rs:201-223).
-template <int D, bool CAUSAL, int MODE, bool OUT_F32, bool BIAS, int NW = 8, bool PER_KEY = false, bool QFUSE = false>
+// HAS_MASK (bf16): p.mask, f32 [N, N], is added to the scaled logits.  See mask_block below.
+template <int D, bool CAUSAL, int MODE, bool OUT_F32, bool BIAS, int NW = 8, bool PER_KEY = false, bool QFUSE = false,
+          bool HAS_MASK = false>
 __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned char *lds, int wg_linear)
 {
     static_assert(!QFUSE || MODE != MODE_BF16, "the fused Q quantiser produces 8-bit operands");
@@ -110,7 +114,8 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     static_assert(!BIAS || MODE == MODE_I8, "biased accumulators are an int8 device");
     static_assert(!PER_KEY || BIAS || MODE == MODE_FP8, "per-key scales: int8 (on the biased accumulators) and FP8");
     static_assert(NW == 8 || NW == 4, "8 waves (one workgroup per CU) or 4 (two)");
-    constexpr bool RINGS = attn_pipe_rings<D, MODE, NW>();  // K and V in rings of their own, two and three tiles deep
+    static_assert(!HAS_MASK || MODE == MODE_BF16, "additive masks: bf16 only");
+    constexpr bool RINGS = attn_pipe_rings<D, MODE, NW, HAS_MASK>();  // K and V in rings of their own, two and three tiles deep
     constexpr int BQ = NW * 32;
     constexpr int QK_BYTES = (MODE != MODE_BF16) ? 1 : 2;
     constexpr int KP = D * QK_BYTES / 64;  // 64-byte pieces per K row
@@ -120,7 +125,8 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     constexpr int STAGE = K_TILE + V_TILE;
     constexpr int NSTAGE = 4;
     constexpr int AHEAD = RINGS ? 2 : 3;          // a tile is requested this many iterations before the one that computes on it
-    constexpr int LDS_BYTES = attn_pipe_lds_bytes<D, MODE, NW>();  // the tiles (PER_KEY: the scale areas follow)
+    // the tiles (PER_KEY: the scale areas follow; HAS_MASK: the mask's blocks)
+    constexpr int LDS_BYTES = attn_pipe_lds_bytes<D, MODE, NW, false, false, HAS_MASK>() - (HAS_MASK ? NW * 8192 : 0);
     constexpr int SK_RAW = LDS_BYTES;          // PER_KEY: [4][64] raw scales of the tiles in flight
     constexpr int SK_OWN = LDS_BYTES + 1024;   // PER_KEY: [wave][2][2][64] factors of the current and the next tile
     constexpr int QF_RED = LDS_BYTES;          // QFUSE: [wave] largest |q| of the wave's 32 queries
@@ -244,6 +250,38 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
                              : "memory", "m0");
             }
         }
+    };
+
+    // HAS_MASK.  A lane needs 16 mask values of its query's row per block, four keys at a time; read from memory in that
+    // order an instruction touches 32 rows for 32 bytes each and the L1's line rate bounds the kernel.  So a wave
+    // moves its 32 x 32 block like K and V, whole 128-byte row pieces straight to LDS, into a place of its own (no
+    // other wave reads it: no barrier), two blocks deep.  Chunk c of row r lies at chunk position c ^ (r % 8): eight
+    // consecutive rows, which is what eight lanes of a read want of one chunk, cover all banks.
+    i32x4 m_rsrc = k_rsrc;
+    uint32_t m_off = 0;
+    if constexpr (HAS_MASK) {
+        const int rows = max(0, min(32, N - wq0));  // (rows past the last query read as zero)
+        m_rsrc = make_rsrc(p.mask + (size_t)min(wq0, N - 1) * N, (uint32_t)rows * (uint32_t)N * 4);
+        m_off = (uint32_t)(lane >> 3) * (uint32_t)N * 4 + (uint32_t)((lane & 7) ^ (lane >> 3)) * 16;
+    }
+    auto mask_block = [&](int j) __attribute__((always_inline)) {
+        if constexpr (HAS_MASK) {
+            if (j * 32 >= kend) return;
+            const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr_t)lds + LDS_BYTES + wave * 8192 + (j & 1) * 4096;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const uint32_t off = m_off + (uint32_t)(x * 8) * (uint32_t)N * 4 + (uint32_t)j * 128;
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                             : : "s"(dst + x * 1024), "v"(off), "s"(m_rsrc) : "memory", "m0");
+            }
+        }
+    };
+    // this lane's mask values of group G (keys 8 G + 4 h .. + 3 of the block) lie at chunk 2 G + h of row i32
+    const int m_row = LDS_BYTES + wave * 8192 + i32 * 128;
+    float mkv[8];  // those of the half block the softmax list works on next
+    auto load_mask = [&](int slot, int G, float *d) __attribute__((always_inline)) {
+        const float4 v = *(const float4 *)(lds + m_row + slot * 4096 + (((2 * G + h) ^ (i32 & 7)) * 16));
+        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
     };
 
     uint4 qreg[KSTEPS];  // Q operand (loaded in the prologue below)
@@ -476,8 +514,9 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     // which is still in LDS (block blk of stage st).
     // (RINGS: K of the block is gone from LDS by now; its logits are still in their registers, s_blk, as
     // the matrix instructions left them, i.e. with the bias in the int8 case.)
+    // (HAS_MASK: the block's mask values may have left LDS too and are read from memory again; kb0 is its first key.)
     auto fix_reference = [&](auto masked, const unsigned char *st, int blk, const acc_t &s_blk, float c, int rel, uint4 (&pb)[2],
-                             float &rs, const float *kp) __attribute__((always_inline)) {
+                             float &rs, const float *kp, int kb0) __attribute__((always_inline)) {
         constexpr bool M = decltype(masked)::value;
         acc_t s;
         if constexpr (RINGS) {
@@ -515,6 +554,10 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             x[r] = (PER_KEY ? y[r] : (float)s[r]) * c;
+            if constexpr (HAS_MASK) {
+                const int key = min(kb0 + 8 * (r >> 2) + 4 * h + (r & 3), N - 1);
+                x[r] = __builtin_fmaf(p.mask[(size_t)min(q_row, N - 1) * N + key], LOG2E, x[r]);
+            }
             if (M && 8 * (r >> 2) + (r & 3) > rel) x[r] = NEG_SENTINEL;
         }
         float mx = max3(x[0], x[1], x[2]);
@@ -522,7 +565,7 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         for (int r = 3; r < 15; r += 2) mx = max3(mx, x[r], x[r + 1]);
         mx = xhalf_max(fmaxf(mx, x[15]));
         move_reference(mx);
-        if constexpr (M) {
+        if constexpr (M || HAS_MASK) {
             // masked keys contribute exactly 0 whatever the reference is
             float half[2];
 #pragma unroll
@@ -531,7 +574,7 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
                     const int rr = ks * 8 + r;
-                    e[r] = (8 * (rr >> 2) + (rr & 3) > rel) ? 0.f : __builtin_amdgcn_exp2f(x[rr] - m_run);
+                    e[r] = (M && 8 * (rr >> 2) + (rr & 3) > rel) ? 0.f : __builtin_amdgcn_exp2f(x[rr] - m_run);
                 }
                 half[ks] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
                 pb[ks].x = pack_bf16x2(e[0], e[1]);
@@ -555,14 +598,18 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     // PER_KEY: 8 x fma(s, ck, -12582912 ck) first, then 4 LDS reads that refill kc / kn for the NEXT half block
     // (the second half of this block, or the first half of the next one, whose factors start at kpn), so that
     // they have the rest of the list to arrive; kp are this block's factors.
+    // HAS_MASK: 8 x fma(mask, log2 e, -m) first, then fma(s, c, that); behind the exponentials 2 LDS reads refill mkv for
+    // the next half block.
     constexpr int SM_CVT = (MODE == MODE_I8 && !BIAS) ? 8 : 0;
     constexpr int SM_KEY = PER_KEY ? (BIAS ? 12 : 10) : 0;
-    constexpr int SM_PRE = SM_CVT + SM_KEY;
-    constexpr int SM_HALF = SM_PRE + 8 + 8 + 7 + 4;
+    constexpr int SM_PRE = SM_CVT + SM_KEY + (HAS_MASK ? 8 : 0);
+    constexpr int SM_MK = HAS_MASK ? 2 : 0;
+    constexpr int SM_HALF = SM_PRE + 8 + 8 + SM_MK + 7 + 4;
     constexpr int SM_OPS = 2 * SM_HALF;
     float sm_t[8], sm_x[8], sm_a[6], sm_half[2];
-    auto sm_op = [&](auto masked, auto ic, const acc_t &s, float c, int rel, uint4 (&pn)[2], const float *kp, const float *kpn)
-                     __attribute__((always_inline)) {
+    // (slot: where the block's mask values are, HAS_MASK)
+    auto sm_op = [&](auto masked, auto ic, const acc_t &s, float c, int rel, uint4 (&pn)[2], const float *kp, const float *kpn,
+                     int slot) __attribute__((always_inline)) {
         constexpr bool M = decltype(masked)::value;
         constexpr int i = decltype(ic)::value;
         constexpr int ks = i / SM_HALF, k = i % SM_HALF;
@@ -573,21 +620,27 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
             else sm_t[k] = (float)s[ks * 8 + k] * kc[k];
         } else if constexpr (PER_KEY && k < SM_KEY) {
             load_factors(ks == 0 ? kp : kpn, ks == 0 ? 2 : 0, k - 8);
+        } else if constexpr (k < SM_PRE) {
+            sm_t[k] = __builtin_fmaf(mkv[k], LOG2E, -m_run);
         } else if constexpr (k < SM_PRE + 8) {
             constexpr int r = k - SM_PRE;
-            sm_t[r] = __builtin_fmaf((SM_CVT || PER_KEY) ? sm_t[r] : as_logit(s, ks * 8 + r), c, -m_bias);
+            if constexpr (HAS_MASK) sm_t[r] = __builtin_fmaf(s[ks * 8 + r], c, sm_t[r]);
+            else sm_t[r] = __builtin_fmaf((SM_CVT || PER_KEY) ? sm_t[r] : as_logit(s, ks * 8 + r), c, -m_bias);
             // a masked key: exp2 of the sentinel is exactly 0
             if (M && 8 * ((ks * 8 + r) >> 2) + (r & 3) > rel) sm_t[r] = NEG_SENTINEL;
         } else if constexpr (k < SM_PRE + 16) {
             constexpr int r = k - SM_PRE - 8;
             sm_x[r] = __builtin_amdgcn_exp2f(sm_t[r]);
-        } else if constexpr (k < SM_PRE + 23) {
-            constexpr int a = k - SM_PRE - 16;  // ((x0+x1)+(x2+x3)) + ((x4+x5)+(x6+x7))
+        } else if constexpr (k < SM_PRE + 16 + SM_MK) {
+            constexpr int part = k - SM_PRE - 16;
+            load_mask(ks == 0 ? slot : slot ^ 1, (ks == 0 ? 2 : 0) + part, mkv + 4 * part);
+        } else if constexpr (k < SM_PRE + 23 + SM_MK) {
+            constexpr int a = k - SM_PRE - 16 - SM_MK;  // ((x0+x1)+(x2+x3)) + ((x4+x5)+(x6+x7))
             if constexpr (a < 4) sm_a[a] = sm_x[2 * a] + sm_x[2 * a + 1];
             else if constexpr (a < 6) sm_a[a] = sm_a[2 * (a - 4)] + sm_a[2 * (a - 4) + 1];
             else sm_half[ks] = sm_a[4] + sm_a[5];
         } else {
-            constexpr int j = k - SM_PRE - 23;
+            constexpr int j = k - SM_PRE - 23 - SM_MK;
             const uint32_t w = pack_bf16x2(sm_x[2 * j], sm_x[2 * j + 1]);
             if constexpr (j == 0) pn[ks].x = w;
             else if constexpr (j == 1) pn[ks].y = w;
@@ -618,7 +671,9 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
                           const unsigned char *sc, int cb,
                           const unsigned char *sv, int vb, const unsigned char *sk, int kb, float c_cur, float c_next,
                           int rel_cur, int rel_next, auto chi, auto vhi, auto khi, const float *kp0, const float *kp1,
-                          const float *kp2) __attribute__((always_inline)) {
+                          const float *kp2, int kb0, auto &&mid) __attribute__((always_inline)) {
+        // kb0: first key of block j; mid: what is requested from memory in the middle of R1 (HAS_MASK)
+        const int slot = (kb0 >> 5) & 1;
         // kp0 / kp1 / kp2: the key factors of blocks j, j+1, j+2 (PER_KEY)
         const int *ka = decltype(khi)::value ? k_addr_hi : k_addr;
         const int *va = decltype(vhi)::value ? v_addr_hi : v_addr;
@@ -631,7 +686,8 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
             qk_step(si, s_new, kf[pv], kf[st], qreg[pv], qreg[st]);
             ARHIP_FENCE();
             constexpr int lo = SM_SPLIT + st * (SM_OPS - SM_SPLIT) / KSTEPS, hi = SM_SPLIT + (st + 1) * (SM_OPS - SM_SPLIT) / KSTEPS;
-            static_for<lo, hi>([&](auto ic) __attribute__((always_inline)) { sm_op(mc, ic, s_old, c_cur, rel_cur, p_cur, kp0, kp1); });
+            static_for<lo, hi>([&](auto ic) __attribute__((always_inline)) { sm_op(mc, ic, s_old, c_cur, rel_cur, p_cur, kp0, kp1, slot); });
+            if constexpr (HAS_MASK && st == KSTEPS / 2 - 1) mid();
             // refill behind the MFMA that read the fragment (FP8: behind the odd step, both halves)
             if constexpr (MODE == MODE_FP8) {
                 if constexpr (st % 2 == 1) {
@@ -645,7 +701,7 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         });
         rs = sm_half[0] + sm_half[1];
         if (__builtin_expect(__any(!(rs <= 16.0f * LAZY_LIMIT)), 0))
-            fix_reference(mc, sc + (decltype(chi)::value ? HI_BASE : 0), cb, s_old, c_cur, rel_cur, p_cur, rs, kp0);
+            fix_reference(mc, sc + (decltype(chi)::value ? HI_BASE : 0), cb, s_old, c_cur, rel_cur, p_cur, rs, kp0, kb0);
         l_run += rs;
         set_bias(c_next);  // the reference is final for block j+1 from here to the end of its softmax
         ARHIP_FENCE();
@@ -659,7 +715,7 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
             ARHIP_FENCE();
             if constexpr (g >= 2) {
                 constexpr int lo = (g - 2) * SM_SPLIT / R2_SLOTS, hi = (g - 1) * SM_SPLIT / R2_SLOTS;
-                static_for<lo, hi>([&](auto ic) __attribute__((always_inline)) { sm_op(mn, ic, s_new, c_next, rel_next, p_nxt, kp1, kp2); });
+                static_for<lo, hi>([&](auto ic) __attribute__((always_inline)) { sm_op(mn, ic, s_new, c_next, rel_next, p_nxt, kp1, kp2, slot ^ 1); });
             }
             if constexpr (ks == 1) {
 #pragma unroll
@@ -680,6 +736,8 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     // the tile it runs.
     const int nfull = CAUSAL ? min(kend / BK, wq0 / BK) : kend / BK;
     static_for<0, AHEAD>([&](auto ti) __attribute__((always_inline)) { issue_tile(decltype(ti)::value); });
+    mask_block(0);
+    mask_block(1);
     // Q operand, resident in registers.  Everything in flight is awaited here once, Q included, so
     // that no wait for a global load is left inside the loops.
     // QFUSE: the 16 values (bf16: 2 x 16 bytes, f32: 4 x 16 bytes) behind each 16-byte piece of the operand
@@ -834,10 +892,27 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         if constexpr (PER_KEY) {
             static_for<0, SM_KEY - 8>([&](auto pi) __attribute__((always_inline)) { load_factors(f0, 0, decltype(pi)::value); });
         }
+        if constexpr (HAS_MASK) {
+            // the reference of the first block, while its mask values are at hand
+            float x[16];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) load_mask(0, g, x + 4 * g);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                x[r] = __builtin_fmaf(x[r], LOG2E, s_a[r] * c0);
+                if (8 * (r >> 2) + (r & 3) > lim4h) x[r] = NEG_SENTINEL;
+            }
+            float mx = max3(x[0], x[1], x[2]);
+#pragma unroll
+            for (int r = 3; r < 15; r += 2) mx = max3(mx, x[r], x[r + 1]);
+            move_reference(xhalf_max(fmaxf(mx, x[15])));
+            load_mask(0, 0, mkv);
+            load_mask(0, 1, mkv + 4);
+        }
         if (nfull > 0)
-            static_for<0, SM_SPLIT>([&](auto ic) __attribute__((always_inline)) { sm_op(PLAIN, ic, s_a, c0, 0, p_a, f0, f1); });
+            static_for<0, SM_SPLIT>([&](auto ic) __attribute__((always_inline)) { sm_op(PLAIN, ic, s_a, c0, 0, p_a, f0, f1, 0); });
         else
-            static_for<0, SM_SPLIT>([&](auto ic) __attribute__((always_inline)) { sm_op(MASKED, ic, s_a, c0, lim4h, p_a, f0, f1); });
+            static_for<0, SM_SPLIT>([&](auto ic) __attribute__((always_inline)) { sm_op(MASKED, ic, s_a, c0, lim4h, p_a, f0, f1, 0); });
     }
 
     // one tile: its two blocks; m0 / m1 / m2 say whether the first block, the second block and the
@@ -854,7 +929,7 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         const std::integral_constant<bool, nxt_hi> hn;
         // tile it + 3 goes to the stage tile it - 1 vacated at the last barrier (RINGS: K(it + 2) to where
         // K(it) was, read for the last time before that barrier, V(it + 2) to where V(it - 1) was)
-        issue_tile(it + AHEAD);
+        if constexpr (!HAS_MASK) issue_tile(it + AHEAD);
         advance_sk_group(it);
         convert_sk(it + 1);  // visible since the barrier that ended the last iteration
         const float *f00 = key_factors(it, 0), *f01 = key_factors(it, 1), *f10 = key_factors(it + 1, 0), *f11 = key_factors(it + 1, 1);
@@ -862,8 +937,27 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         const float c_cur = c_carry, c_nxt = tile_c(it + 1, it);
         c_carry = c_nxt;
         const int rel0 = lim4h - it * BK;
-        pipe_block(m0, m1, s_a, s_b, p_a, p_b, k_cur, 0, v_cur, 1, k_nxt, 0, c_cur, c_cur, rel0, rel0 - 32, hc, hc, hn, f00, f01, f10);
-        pipe_block(m1, m2, s_b, s_a, p_b, p_a, k_cur, 1, v_nxt, 0, k_nxt, 1, c_cur, c_nxt, rel0 - 32, rel0 - 64, hc, hn, hn, f01, f10, f11);
+        // HAS_MASK: block j's mask values were read for the last time early in R1(j), and block j + 1's are first read late in
+        // it; in between its request for block j + 1 has to have landed and block j + 2 takes the place of block j.  The K / V
+        // tile is requested behind the first of the two, so that each waits for nothing younger than itself.
+        const bool more = it + AHEAD < ntiles;
+        pipe_block(m0, m1, s_a, s_b, p_a, p_b, k_cur, 0, v_cur, 1, k_nxt, 0, c_cur, c_cur, rel0, rel0 - 32, hc, hc, hn, f00, f01, f10, it * BK,
+                   [&]() __attribute__((always_inline)) {
+                       wait_vmem_le<0>();
+                       mask_block(2 * it + 2);
+                       issue_tile(it + AHEAD);
+                   });
+        pipe_block(m1, m2, s_b, s_a, p_b, p_a, k_cur, 1, v_nxt, 0, k_nxt, 1, c_cur, c_nxt, rel0 - 32, rel0 - 64, hc, hn, hn, f01, f10, f11,
+                   it * BK + 32, [&]() __attribute__((always_inline)) {
+                       if (more) wait_vmem_le<XPW>();
+                       else wait_vmem_le<0>();
+                       mask_block(2 * it + 3);
+                   });
+        if constexpr (HAS_MASK) {
+            wait_vmem_le<4>();  // tile it + 2 has landed, the block behind it may be in flight
+            __syncthreads();
+            return;
+        }
         wait_vmem_le<RINGS ? 0 : XPW_MIN>();  // tile it + 2 has landed (tile it + 3 may still be in flight)
         __syncthreads();
     };
@@ -956,17 +1050,17 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
 }
 
 // int8 uses the biased accumulators (see s_init); bf16 and FP8 the plain ones.
-template <int D, bool CAUSAL, int MODE, bool OUT_F32, int NW = 8, bool PER_KEY = false, bool QFUSE = false>
+template <int D, bool CAUSAL, int MODE, bool OUT_F32, int NW = 8, bool PER_KEY = false, bool QFUSE = false, bool HAS_MASK = false>
 __device__ __forceinline__ void attn_pipe_body(const AttnParams &p, unsigned char *lds, int wg_linear)
 {
-    attn_pipe_impl<D, CAUSAL, MODE, OUT_F32, (MODE == MODE_I8 && ARHIP_PIPE_INT_BIAS), NW, PER_KEY, QFUSE>(p, lds, wg_linear);
+    attn_pipe_impl<D, CAUSAL, MODE, OUT_F32, (MODE == MODE_I8 && ARHIP_PIPE_INT_BIAS), NW, PER_KEY, QFUSE, HAS_MASK>(p, lds, wg_linear);
 }
 
-template <int D, bool CAUSAL, int MODE, bool OUT_F32, int NW = 8, bool PER_KEY = false, bool QFUSE = false>
+template <int D, bool CAUSAL, int MODE, bool OUT_F32, int NW = 8, bool PER_KEY = false, bool QFUSE = false, bool HAS_MASK = false>
 __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) attn_pipe_kernel(const AttnParams p)
 {
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[attn_pipe_lds_bytes<D, MODE, NW, PER_KEY, QFUSE>()];
-    attn_pipe_body<D, CAUSAL, MODE, OUT_F32, NW, PER_KEY, QFUSE>(p, lds, (int)blockIdx.x);
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[attn_pipe_lds_bytes<D, MODE, NW, PER_KEY, QFUSE, HAS_MASK>()];
+    attn_pipe_body<D, CAUSAL, MODE, OUT_F32, NW, PER_KEY, QFUSE, HAS_MASK>(p, lds, (int)blockIdx.x);
 }
 
 }  // namespace arhip

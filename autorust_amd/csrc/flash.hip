@@ -86,6 +86,14 @@ static bool pipe_wants_4_waves(arhip_device *dev, int64_t heads, int64_t N, int6
     return N <= 1024 || (N <= 2048 && causal && !has_len);
 }
 
+// The same for launches with an additive mask, whose blocks need LDS of their own: at D = 128 one workgroup per compute
+// unit in either form, so 8 waves as soon as 4 would not all run at once.
+static bool mask_wants_4_waves(arhip_device *dev, int64_t heads, int64_t N, int64_t D)
+{
+    if (dev->attn_waves == 8 || dev->attn_waves == 40) return D == 64 || dev->attn_waves == 40;
+    return D == 64 || heads * ((N + 127) / 128) <= dev->cus;
+}
+
 // The pipelined kernel addresses K and V through 32-bit buffer offsets (rows of one head, plus the
 // tiles it requests past the end).
 static bool pipe_addressable(int64_t N, int64_t kv_token_stride, int64_t elem_bytes)
@@ -93,25 +101,16 @@ static bool pipe_addressable(int64_t N, int64_t kv_token_stride, int64_t elem_by
     return (N + 5 * 64) * kv_token_stride * elem_bytes < ((int64_t)1 << 31);
 }
 
-// Which kernel.  Launches without an additive mask, per-key scales or the logits export take the
-// software-pipelined kernel (returned as 8; whether it runs with 8 or 4 waves per workgroup is
-// pipe_wants_4_waves' choice): with its 4-wave form it is the fastest kernel down to the shortest sequences
-// (bf16, against the kernels that used to serve them: B8 H12 N197 D64 7.8 -> 7.0 us, B4 H16 N256 D128 11.8 ->
-// 9.0 us, B32 H12 N64 D64 9.1 -> 5.6 us, B8 H12 N400 D64 27.8 -> 12.9 us).  The others take the general
-// kernel with 4 waves of 32 queries, or 1 at D = 64 when that still leaves compute units idle.
-static int pick_waves(arhip_device *dev, int64_t heads, int64_t N, int64_t D, bool special)
+// Which kernel.  The software-pipelined kernel (with 8 or 4 waves per workgroup, pipe_wants_4_waves' choice) wherever it has a
+// form: with its 4-wave form it is the fastest kernel down to the shortest sequences (bf16, against the kernels that used to
+// serve them: B8 H12 N197 D64 7.8 -> 7.0 us, B4 H16 N256 D128 11.8 -> 9.0 us, B32 H12 N64 D64 9.1 -> 5.6 us, B8 H12 N400 D64
+// 27.8 -> 12.9 us).  special: 8-bit launches with an additive mask, K scales over a number of keys that is no power of two or
+// the logits export take the general kernel with 4 waves of 32 queries, as do K/V too large for 32-bit offsets.
+// (ARHIP_ATTN_WAVES, read once when the device is opened, is a tuning aid; results do not depend on it.  4: the general
+// kernel; 8, 40: the pipelined kernel with 8 / 4 waves.)
+static bool use_pipe(arhip_device *dev, bool special, int64_t N, int64_t kv_token_stride)
 {
-    const int64_t cus = dev->cus, wg128 = heads * ((N + 127) / 128);
-    int nw;
-    if (!special) nw = 8;
-    else if (D == 64 && wg128 < 2 * cus) nw = 1;
-    else nw = 4;
-    // ARHIP_ATTN_WAVES (read once when the device is opened) is a tuning aid; results do not depend on it
-    // (1, 4: the general kernel with that many waves; 8, 40: the pipelined kernel with 8 / 4 waves)
-    const int w = dev->attn_waves;
-    if ((w == 1 || w == 4 || w == 8) && !special && (w != 1 || D == 64)) nw = w;
-    if (w == 40 && !special) nw = 8;
-    return nw;
+    return !special && dev->attn_waves != 4 && pipe_addressable(N, kv_token_stride, 2);
 }
 
 // Tiling of the fp32 forward: 8 or 4 waves of 32 queries that share their key tiles (81, 41: 256 and 128 queries per workgroup),
@@ -243,19 +242,18 @@ extern "C" int arhip_flash_fwd_lse(arhip_device *dev, const void *q, const void 
     p.bq = p.bk = 1;
     p.scale = scale;
     const bool c = causal != 0, hm = mask != nullptr;
-    int nw = pick_waves(dev, B * Hq, N, D, hm);
-    if (nw == 8 && !pipe_addressable(N, kv_strides[2], 2)) nw = 4;
-    const bool pipe = nw == 8;  // the software-pipelined kernel; how many waves it runs with is its own choice
-    if (pipe && pipe_wants_4_waves(dev, B * Hq, N, D, causal != 0, kv_len != nullptr)) nw = 4;
+    const bool pipe = use_pipe(dev, false, N, kv_strides[2]);
+    const bool w4 = hm ? mask_wants_4_waves(dev, B * Hq, N, D) : pipe_wants_4_waves(dev, B * Hq, N, D, c, kv_len != nullptr);
+    const int nw = pipe && !w4 ? 8 : 4;
     p.nq = (int)((N + nw * 32 - 1) / (nw * 32));
     p.total = (int)(p.nq * B * Hq);
     p.lpt = p.total <= 16 * dev->cus;  // few workgroups per CU: balance them globally
     if (int rc = t.begin()) return rc;
     if (pipe) {
-        launch_pipe_bf16(dev->stream, p, (int)D, c, nw);
+        if (hm) launch_pipe_bf16_mask(dev->stream, p, (int)D, c, nw);
+        else launch_pipe_bf16(dev->stream, p, (int)D, c, nw);
     } else if (D == 64) {
-        if (nw == 1) launch_attn<64, 1, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
-        else launch_attn<64, 4, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
+        launch_attn<64, 4, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
     } else {
         launch_attn<128, 4, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
     }
@@ -330,12 +328,9 @@ static int sage_fwd_impl(arhip_device *dev, const int8_t *q8, const int8_t *k8,
     while (((int64_t)1 << key_shift) < bk) ++key_shift;
     const bool pipe_keys = per_key && ((int64_t)1 << key_shift) == bk;
     p.bk_key_shift = pipe_keys ? key_shift : -1;
-    int nw = pick_waves(dev, B * Hq, N, D, hm || (per_key && !pipe_keys) || dbg);
-    if (nw == 1) nw = 4;
-    if (nw == 8 && !pipe_addressable(N, std::max<int64_t>(D, v_strides ? v_strides[2] : D), 2)) nw = 4;
-    const bool pipe = nw == 8 && (!per_key || pipe_keys) && !dbg;
+    const bool pipe = use_pipe(dev, hm || (per_key && !pipe_keys) || dbg, N, std::max<int64_t>(D, v_strides ? v_strides[2] : D));
     const bool pipe4 = pipe && pipe_wants_4_waves(dev, B * Hq, N, D, causal != 0, kv_len != nullptr);
-    if (pipe4) nw = 4;
+    const int nw = pipe && !pipe4 ? 8 : 4;
     p.nq = (int)((N + nw * 32 - 1) / (nw * 32));
     p.total = (int)(p.nq * B * Hq);
     p.lpt = p.total <= 16 * dev->cus;

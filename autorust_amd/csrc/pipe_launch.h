@@ -11,6 +11,7 @@
 namespace arhip {
 
 void launch_pipe_bf16(hipStream_t stream, const AttnParams &p, int D, bool causal, int nw);
+void launch_pipe_bf16_mask(hipStream_t stream, const AttnParams &p, int D, bool causal, int nw);  // p.mask; D = 64: nw = 4
 void launch_pipe_i8(hipStream_t stream, const AttnParams &p, int D, bool causal, int nw);       // K scales over whole tiles
 void launch_pipe_i8_keys(hipStream_t stream, const AttnParams &p, int D, bool causal, int nw);  // K scales per key
 void launch_pipe_i8_qf(hipStream_t stream, const AttnParams &p, int D, bool causal, int nw);    // bf16 queries, quantised in the prologue
