@@ -8,7 +8,7 @@
 #include "attn_fwd.h"
 #include "pipe_launch.h"
 #include "flash_bwd_f32.h"
-#include "flash_f32.h"
+#include "f32_launch.h"
 
 #include <algorithm>
 #include <cmath>
@@ -221,7 +221,8 @@ extern "C" int arhip_flash_fwd_lse(arhip_device *dev, const void *q, const void 
         else if (form == 41) F32_LAUNCH(DD, 4, 1);                                                    \
         else F32_LAUNCH(DD, 1, 4);                                                                    \
     } while (0)
-        if (D == 64) F32_FORMS(64);
+        if (mask != nullptr) launch_f32_mask(dev->stream, fp, (int)D, causal != 0, form);
+        else if (D == 64) F32_FORMS(64);
         else F32_FORMS(128);
 #undef F32_FORMS
 #undef F32_LAUNCH

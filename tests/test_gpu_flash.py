@@ -263,12 +263,14 @@ def test_token_major_layout_long_sequences(dev, causal):
     assert np.abs(got[:, :, rows] - truth).max() <= 2e-2
 
 
+@pytest.mark.parametrize("dtype,tol", [(BF16, 2e-2), (F32, 1e-5)])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("B,Hq,Hkv,N", [(1, 2, 1, 1), (1, 1, 1, 33), (2, 2, 2, 64), (1, 3, 3, 95), (2, 4, 2, 129), (1, 2, 2, 258), (1, 2, 1, 771),
                                         (4, 24, 12, 515)])
-def test_bf16_additive_mask_on_tile_edges(dev, D, B, Hq, Hkv, N):
+def test_additive_mask_on_tile_edges(dev, dtype, tol, D, B, Hq, Hkv, N):
     """Mask rows of every alignment, last rows and last keys of the mask, -inf entries and rows, finite values in place of -inf,
-    rows whose maximum moves by hundreds from tile to tile; with 4 and with 8 waves (the last shape); against float64."""
+    rows whose maximum moves by hundreds from tile to tile, in every tiling (the last shapes: many workgroups); against
+    float64.  (f32: rows with logits in the thousands, whose steps are near 1e-3, only have to be finite.)"""
     q, k, v = (synth.normal(s, (B, H, N, D)) for s, H in ((941, Hq), (942, Hkv), (943, Hkv)))
     mask = (synth.normal(944, (N, N)) * np.float32(3.0)).astype(np.float32)
     mask[N - 1, N - 1] = 9.0
@@ -280,11 +282,13 @@ def test_bf16_additive_mask_on_tile_edges(dev, D, B, Hq, Hkv, N):
     if N > 40:
         mask[40, :] = -np.inf
     kv_len = np.array([max(1, N - 37 * (b % 2)) for b in range(B)], np.int32)
-    qb, kb, vb = (oracle.bf16_round(t) for t in (q, k, v))
+    qb, kb, vb = (oracle.bf16_round(t) if dtype == BF16 else t for t in (q, k, v))
+    rows = [i for i in range(N) if dtype == BF16 or i % 13 != 5 and i % 11 != 3]  # (f32: see above)
     for causal in (False, True):
         for lens in (None, kv_len):
-            got = run_flash(dev, q, k, v, BF16, mask=mask, kv_len=lens, causal=causal)
+            got = run_flash(dev, q, k, v, dtype, mask=mask, kv_len=lens, causal=causal)
             truth = oracle.sdpa_f64(qb, kb, vb, mask=mask, kv_len=lens, causal=causal)
             truth = np.where(np.isfinite(truth), truth, 0.0)   # a row without a visible key is zero here
-            bad = np.abs(got - truth) / np.maximum(np.abs(truth), 1.0)
-            assert bad.max() <= 2e-2, (causal, lens is not None, np.unravel_index(bad.argmax(), bad.shape), float(bad.max()))
+            assert np.isfinite(got).all()
+            bad = (np.abs(got - truth) / np.maximum(np.abs(truth), 1.0))[:, :, rows]
+            assert bad.max() <= tol, (causal, lens is not None, np.unravel_index(bad.argmax(), bad.shape), float(bad.max()))
