@@ -541,28 +541,27 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     const bool split = D == 64 && B * Hkv * ((N + 127) / 128) < dev->cus / 2;
     const int rows_wg = split ? 32 : 128;
     const int nt = (int)((N + rows_wg - 1) / rows_wg);
-    const dim3 block(256), grid_prep((unsigned)((rows + 3) / 4)), grid_q((unsigned)(nt * B * Hq)),
-        grid_kv((unsigned)(nt * B * Hkv));
     p.nt = nt;
     // causal: longest tile first over all heads, so that no head's long tiles are left for the end
     p.total_q = (int)(nt * B * Hq);
     p.total_kv = (int)(nt * B * Hkv);
     p.lpt_q = causal ? (int)(B * Hq) : 0;
     p.lpt_kv = causal ? (int)(B * Hkv) : 0;
-#define BWD_LAUNCH(DD, SP)                                                                              \
-    do {                                                                                                \
-        hipLaunchKernelGGL((bwd_prep_kernel<DD>), grid_prep, dim3(256), 0, dev->stream, o, dout, delta, rows); \
-        if (causal) {                                                                                   \
-            hipLaunchKernelGGL((bwd_dq_kernel<DD, true, SP>), grid_q, block, 0, dev->stream, p);     \
-            hipLaunchKernelGGL((bwd_dkv_kernel<DD, true, SP>), grid_kv, block, 0, dev->stream, p);   \
-        } else {                                                                                        \
-            hipLaunchKernelGGL((bwd_dq_kernel<DD, false, SP>), grid_q, block, 0, dev->stream, p);    \
-            hipLaunchKernelGGL((bwd_dkv_kernel<DD, false, SP>), grid_kv, block, 0, dev->stream, p);  \
-        }                                                                                               \
-    } while (0)
-    if (D == 64) { if (split) BWD_LAUNCH(64, true); else BWD_LAUNCH(64, false); }
-    else BWD_LAUNCH(128, false);
-#undef BWD_LAUNCH
+    const dim3 block(256);
+    auto go = [&](auto d, auto c) {
+        constexpr int DD = decltype(d)::value;
+        constexpr bool C = decltype(c)::value;
+        constexpr int PR = bwd_prep_rows<DD>();
+        hipLaunchKernelGGL((bwd_prep_kernel<DD>), dim3((unsigned)((rows + PR - 1) / PR)), block, 0, dev->stream, o, dout, delta, rows);
+        if (DD == 128 || split) {
+            hipLaunchKernelGGL((bwd_kernel<DD, C, DD == 64>), dim3((unsigned)(p.total_kv + p.total_q)), block, 0, dev->stream, p);
+        } else {
+            hipLaunchKernelGGL((bwd_dq_kernel<C>), dim3((unsigned)p.total_q), block, 0, dev->stream, p);
+            hipLaunchKernelGGL((bwd_dkv_kernel<C>), dim3((unsigned)p.total_kv), block, 0, dev->stream, p);
+        }
+    };
+    auto by_mask = [&](auto d) { causal ? go(d, std::true_type{}) : go(d, std::false_type{}); };
+    D == 64 ? by_mask(std::integral_constant<int, 64>{}) : by_mask(std::integral_constant<int, 128>{});
     arhip_note_selected(ARHIP_K_FLASH_BWD);
     return t.end();
 }

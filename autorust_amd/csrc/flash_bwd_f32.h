@@ -47,20 +47,27 @@ struct FlashBwdParams {
 constexpr float BWD_LSE_FLOOR = -5e29f;  // lse at or below: the row saw no key (cuda_flash_train.rs:206)
 constexpr float BWD_LOG2E = 1.44269504088896340736f;
 
-// D[bh, i] = O[i] . dO[i]; one wave per row group: lane l of a wave sums channels l, l + 64, ...
-// in increasing order, then the 64 partial sums are added by a fixed butterfly.
+// D[bh, i] = O[i] . dO[i], by D / 4 lanes of a wave, 16 bytes of the row each; their partial sums are added by a fixed
+// butterfly.  Rows row0, row0 + 1, ... by lane group of the workgroup (D = 64: 16 rows, D = 128: 8; a wave per row, 4 bytes
+// per lane, took 3.3 instead of 2.1 us on B8 H12 N197 D64).
+template <int D>
+constexpr int bwd_prep_rows() { return 256 / (D / 4); }
+template <int D>
+__device__ __forceinline__ void bwd_prep_row(const float *o, const float *dout, float *delta, long rows, long row, bool store)
+{
+    const int g = threadIdx.x & (D / 4 - 1);
+    if (row >= rows) return;  // (whole lane groups)
+    const float4 a = *(const float4 *)(o + row * D + 4 * g), b = *(const float4 *)(dout + row * D + 4 * g);
+    float s = (a.x * b.x + a.y * b.y) + (a.z * b.z + a.w * b.w);
+#pragma unroll
+    for (int off = D / 8; off >= 1; off >>= 1) s += __shfl_xor(s, off);
+    if (store && g == 0) delta[row] = s;
+}
+// four rows per workgroup, the shape of the named entry's grid: the lane groups of a wave share a row
 template <int D>
 __device__ __forceinline__ void bwd_prep_body(const float *o, const float *dout, float *delta, long rows, long row0)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long row = row0 + wave;
-    if (row >= rows) return;
-    float s = 0.f;
-#pragma unroll
-    for (int c = lane; c < D; c += 64) s += o[row * D + c] * dout[row * D + c];
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
-    if (lane == 0) delta[row] = s;
+    bwd_prep_row<D>(o, dout, delta, rows, row0 + (threadIdx.x >> 6), (threadIdx.x & 63) < D / 4);
 }
 
 // One thread's share of a pair of 32-row tiles (A and B, e.g. K and V) between memory and LDS: items of 8 channels, the first
@@ -769,22 +776,37 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
 template <int D>
 __global__ void __launch_bounds__(256) bwd_prep_kernel(const float *o, const float *dout, float *delta, long rows)
 {
-    bwd_prep_body<D>(o, dout, delta, rows, (long)blockIdx.x * 4);
+    bwd_prep_row<D>(o, dout, delta, rows, (long)blockIdx.x * bwd_prep_rows<D>() + threadIdx.x / (D / 4), true);
 }
 
-// D = 64: registers held to 256 per lane so that a SIMD holds two waves; D = 128 needs more than that
+// dK/dV and dQ in one grid: workgroups [0, total_kv) form dK/dV, which takes longer, the others dQ.  They have nothing to
+// do with each other, so where either grid alone leaves compute units idle (few or short heads, the end of any grid) the other's
+// workgroups run there; and it is a launch fewer.  Forward and backward, us: B1 H12 N197 D64 26 -> 24, B2 H16 N2048 D128 causal
+// 817 -> 800.
 template <int D, bool CAUSAL, bool SPLIT>
-__global__ void __launch_bounds__(256, (D == 64 ? 2 : 1)) bwd_dq_kernel(const FlashBwdParams p)
+__global__ void __launch_bounds__(256, 1) bwd_kernel(const FlashBwdParams p)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dq_lds_bytes<D, SPLIT>()];
-    bwd_dq_body<D, CAUSAL, SPLIT>(p, lds, (int)blockIdx.x);
+    constexpr int LQ = bwd_dq_lds_bytes<D, SPLIT>(), LKV = bwd_dkv_lds_bytes<D, SPLIT>();
+    __shared__ __attribute__((aligned(16))) unsigned char lds[LQ > LKV ? LQ : LKV];
+    const int wg = (int)blockIdx.x;
+    if (wg < p.total_kv) bwd_dkv_body<D, CAUSAL, SPLIT>(p, lds, wg);
+    else bwd_dq_body<D, CAUSAL, SPLIT>(p, lds, wg - p.total_kv);
 }
 
-template <int D, bool CAUSAL, bool SPLIT>
+// Head size 64, 128 rows per workgroup: dQ fits 256 registers, so that a SIMD holds two of its waves, and dK/dV does not.  In one
+// kernel either dQ would lose its second wave or dK/dV spill 73 registers (B8 H12 N197: 41 us together, 16 + 23 one after the other).
+template <bool CAUSAL>
+__global__ void __launch_bounds__(256, 2) bwd_dq_kernel(const FlashBwdParams p)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dq_lds_bytes<64, false>()];
+    bwd_dq_body<64, CAUSAL, false>(p, lds, (int)blockIdx.x);
+}
+
+template <bool CAUSAL>
 __global__ void __launch_bounds__(256, 1) bwd_dkv_kernel(const FlashBwdParams p)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dkv_lds_bytes<D, SPLIT>()];
-    bwd_dkv_body<D, CAUSAL, SPLIT>(p, lds, (int)blockIdx.x);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dkv_lds_bytes<64, false>()];
+    bwd_dkv_body<64, CAUSAL, false>(p, lds, (int)blockIdx.x);
 }
 
 }  // namespace arhip
