@@ -510,7 +510,7 @@ std::vector<HostCall> attention_host_calls(const Tensor &q, const Tensor &k, con
         vb = Tensor::empty(dev, {b, hk, n, d}, BF);
         const int64_t rows = b * hk * n, rpb = 256 / (d / 8), row_blocks = (rows + rpb - 1) / rpb, nv = rows * d;
         calls.push_back(make_call(dev, "ar_sage_quant_rows_cast_f32", {k, k8, sk, v, vb}, {F, I8, F, F, BF},
-                                  {row_blocks + std::min<int64_t>((nv + 255) / 256, 16384), 1, 1}, {256, 1, 1},
+                                  {row_blocks + std::min<int64_t>((nv / 8 + 255) / 256, 16384), 1, 1}, {256, 1, 1},
                                   {n, d, rows, nv, row_blocks}, {2, 3}));
     } else {
         quant(k, k8, sk, hk, bk, nkb, st.sage_smooth_k);

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 // Scratch of arhip_sage_quant_static, resident on the device: the partial channel sums of the K
 // mean.  Each GPU the library runs on holds its own copy until the process ends.
@@ -83,20 +84,38 @@ static int sage_quant_impl(arhip_device *dev, const void *x, const int64_t x_str
     arhip_call_timer t{dev, wait, secs};
     t.kernel = prof_kernel;
     if (int rc = t.begin()) return rc;
-    if (smooth) {
-        const int cpb = 256 / (int)(D / 8);  // chunks per workgroup
-        const dim3 pgrid((unsigned)((nchunk + cpb - 1) / cpb), (unsigned)(B * H));
-        if (dtype == ARHIP_F32)
-            hipLaunchKernelGGL(k_mean_partial_kernel<float>, pgrid, dim3(256), 0, dev->stream,
-                               (const float *)x, (float *)workspace, (int)N, (int)D, nchunk, lay);
-        else
-            hipLaunchKernelGGL(k_mean_partial_kernel<uint16_t>, pgrid, dim3(256), 0, dev->stream,
-                               (const uint16_t *)x, (float *)workspace, (int)N, (int)D, nchunk, lay);
-        hipLaunchKernelGGL(k_mean_final_kernel, dim3((unsigned)(B * H)), dim3((unsigned)D), 0, dev->stream,
+    const long rows = (long)(B * H * N);
+    // Fewer launches where a launch (2 to 5 us of its own) costs more than the repeated reads it saves: one where every
+    // workgroup's reading of its whole head stays below 32 MB over all of them (a few us of L2 bandwidth), two where a head's partial
+    // sums are no more than a workgroup's own 64 rows.
+    const bool one = smooth && block > 1 && nchunk * D <= SMOOTH_LDS_FLOATS && rows * D * (dtype == ARHIP_F32 ? 4 : 2) * nblk <= (32 << 20);
+    const bool two = smooth && block > 1 && !one && nchunk <= 32;
+    if (smooth && !one) {
+        // (two channels per thread while that leaves every SIMD less than two waves of it)
+        auto partial = [&](auto t, auto ch) {
+            using T = decltype(t);
+            constexpr int C = decltype(ch)::value;
+            const int cpb = 256 / (int)(D / C);  // chunks per workgroup
+            hipLaunchKernelGGL((k_mean_partial_kernel<T, C>), dim3((unsigned)((nchunk + cpb - 1) / cpb), (unsigned)(B * H)), dim3(256), 0,
+                               dev->stream, (const T *)x, (float *)workspace, (int)N, (int)D, nchunk, lay);
+        };
+        auto typ = [&](auto ch) { dtype == ARHIP_F32 ? partial(0.f, ch) : partial((uint16_t)0, ch); };
+        if (B * H * nchunk * (D / 2) <= 2 * 4 * 64 * (int64_t)dev->cus) typ(std::integral_constant<int, 2>{});
+        else typ(std::integral_constant<int, 8>{});
+        if (!two) hipLaunchKernelGGL(k_mean_final_kernel, dim3((unsigned)(B * H)), dim3((unsigned)D), 0, dev->stream,
                            (const float *)workspace, mean, (int)N, (int)D, nchunk);
     }
-    const long rows = (long)(B * H * N);
-    if (dtype == ARHIP_F32) {
+    if (one || two) {
+        auto go = [&](auto t, auto f8, auto single) {
+            using T = decltype(t);
+            hipLaunchKernelGGL((smooth_quant_blocks_kernel<T, decltype(f8)::value, decltype(single)::value>),
+                               dim3((unsigned)nblk, (unsigned)(B * H)), dim3(smooth_threads<decltype(single)::value>()), 0,
+                               dev->stream, (const T *)x, x8, scales, (const float *)workspace, mean, (int)N, (int)D, (int)block, nblk, nchunk, lay);
+        };
+        auto fmt = [&](auto t, auto single) { fp8 ? go(t, std::true_type{}, single) : go(t, std::false_type{}, single); };
+        auto typ = [&](auto single) { dtype == ARHIP_F32 ? fmt(0.f, single) : fmt((uint16_t)0, single); };
+        one ? typ(std::true_type{}) : typ(std::false_type{});
+    } else if (dtype == ARHIP_F32) {
         if (smooth) fp8 ? launch_quant<float, true, true>(dev, x, x8, scales, mean, N, D, block, nblk, rows, B * H, lay)
                         : launch_quant<float, true, false>(dev, x, x8, scales, mean, N, D, block, nblk, rows, B * H, lay);
         else fp8 ? launch_quant<float, false, true>(dev, x, x8, scales, nullptr, N, D, block, nblk, rows, B * H, lay)
@@ -176,7 +195,7 @@ extern "C" int arhip_sage_prep_kv_rows(arhip_device *dev, const float *k, int8_t
     const long rows = (long)(B * Hkv * N), nv = rows * (long)D;
     const int rpb = 256 / (int)(D / 8);
     const long row_blocks = (rows + rpb - 1) / rpb;
-    const long cast_blocks = std::min<long>((nv + 255) / 256, 16384);
+    const long cast_blocks = std::min<long>((nv / 8 + 255) / 256, 16384);
     ARHIP_REQUIRE(row_blocks + cast_blocks < ((long)1 << 31), "arhip_sage_prep_kv_rows: too many rows");
     arhip_call_timer t{dev, wait, secs};
     t.kernel = ARHIP_K_SAGE_QUANT;
@@ -194,7 +213,8 @@ extern "C" int arhip_cast_bf16(arhip_device *dev, const float *x, uint16_t *y, i
     arhip_call_timer t{dev, wait, secs};
     if (int rc = t.begin()) return rc;
     if (n > 0) {
-        size_t blocks = ((size_t)n + 255) / 256;
+        size_t blocks = ((size_t)n / 8 + 255) / 256;
+        if (blocks == 0) blocks = 1;
         if (blocks > 16384) blocks = 16384;
         hipLaunchKernelGGL(cast_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0, dev->stream, x, y, (size_t)n);
     }

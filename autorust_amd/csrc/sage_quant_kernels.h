@@ -46,54 +46,87 @@ __device__ __forceinline__ void ld8(const uint16_t *x, size_t e, float v[8])
     v[6] = __uint_as_float(a.w << 16); v[7] = __uint_as_float(a.w & 0xffff0000u);
 }
 
+// two adjacent channels
+__device__ __forceinline__ void ld2(const float *x, size_t e, float v[2])
+{
+    const float2 a = *(const float2 *)(x + e);
+    v[0] = a.x; v[1] = a.y;
+}
+__device__ __forceinline__ void ld2(const uint16_t *x, size_t e, float v[2])
+{
+    const uint32_t a = *(const uint32_t *)(x + e);
+    v[0] = __uint_as_float(a << 16); v[1] = __uint_as_float(a & 0xffff0000u);
+}
+
+// s[0..C) = x[j0] + x[j0 + 1] + ... + x[j1 - 1] of C (8 or 2) adjacent channels in token order; base: the channels of token 0.
+// U rows are in flight per thread (their loads are issued together) and added in token order: a short sequence has few
+// threads, and its time is the number of load round trips and of instructions of a wave that has its SIMD to itself.
+template <int U, int C, typename T>
+__device__ __forceinline__ void sum_rows(const T *x, size_t base, long st, int j0, int j1, float (&s)[C])
+{
+    auto ld = [&](int j, float *v) __attribute__((always_inline)) {
+        if constexpr (C == 8) ld8(x, base + (size_t)j * st, v);
+        else ld2(x, base + (size_t)j * st, v);
+    };
+#pragma unroll
+    for (int i = 0; i < C; ++i) s[i] = 0.f;
+    int j = j0;
+    for (; j + U <= j1; j += U) {
+        float v[U][C];
+#pragma unroll
+        for (int u = 0; u < U; ++u) ld(j + u, v[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < C; ++i) s[i] += v[u][i];
+    }
+    for (; j < j1; j += 8) {  // the last row stands in for those past the end and is not added
+        float v[8][C];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) ld(min(j + u, j1 - 1), v[u]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (j + u < j1) {
+#pragma unroll
+                for (int i = 0; i < C; ++i) s[i] += v[u][i];
+            }
+    }
+}
+
 // part[bh][c][d] = k[64c][d] + k[64c+1][d] + ... in token order.
-// One thread owns 8 adjacent channels of one 64-token chunk: D/8 threads read a whole row
-// (coalesced), 256/(D/8) chunks per workgroup.
-template <typename T>
+// One thread owns C adjacent channels of one 64-token chunk: D/C threads read a whole row
+// (coalesced), 256/(D/C) chunks per workgroup.  C = 8 for the memory's rate, 2 where the tensor is small and a
+// wave's own instructions are the time (B2 Hkv8 N2016 D64: 6.0 -> 4.5 us).
+template <typename T, int C = 8>
 __device__ __forceinline__ void k_mean_partial_body(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, const dim3 bid)
 {
-    const int gpr = D / 8;                       // 8-channel groups per row
+    const int gpr = D / C;                       // groups of C channels per row
     const int cpb = 256 / gpr;                   // chunks per workgroup
     const int c = bid.x * cpb + threadIdx.x / gpr;
     const int g = threadIdx.x % gpr, bh = bid.y;
     if (c >= nchunk) return;
     const int j0 = c * MEAN_CHUNK;
     const int j1 = min(N, j0 + MEAN_CHUNK);
-    const size_t base = lay.head(bh) + g * 8;
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    // eight rows in flight per thread (the loads of a group are issued together), added in token order
-    int j = j0;
-    for (; j + 8 <= j1; j += 8) {
-        float v[8][8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) ld8(x, base + (size_t)(j + u) * lay.st, v[u]);
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s[i] += v[u][i];
+    float s[C];
+    sum_rows<(C == 8 ? 16 : 32), C>(x, lay.head(bh) + g * C, lay.st, j0, j1, s);
+    float *o = part + ((size_t)bh * nchunk + c) * D + g * C;
+    if constexpr (C == 8) {
+        *(float4 *)o = make_float4(s[0], s[1], s[2], s[3]);
+        *(float4 *)(o + 4) = make_float4(s[4], s[5], s[6], s[7]);
+    } else {
+        *(float2 *)o = make_float2(s[0], s[1]);
     }
-    for (; j < j1; ++j) {
-        float v[8];
-        ld8(x, base + (size_t)j * lay.st, v);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s[i] += v[i];
-    }
-    float *o = part + ((size_t)bh * nchunk + c) * D + g * 8;
-    *(float4 *)o = make_float4(s[0], s[1], s[2], s[3]);
-    *(float4 *)(o + 4) = make_float4(s[4], s[5], s[6], s[7]);
 }
 
-template <typename T>
+template <typename T, int C>
 __global__ void __launch_bounds__(256) k_mean_partial_kernel(const T *x, float *part, int N, int D, int nchunk, const XLayout lay)
 {
-    k_mean_partial_body<T>(x, part, N, D, nchunk, lay, blockIdx);
+    k_mean_partial_body<T, C>(x, part, N, D, nchunk, lay, blockIdx);
 }
 
-// mean[bh][d] = (part[0] + part[1] + ...) / N in chunk order (loads batched, adds in order)
-__device__ __forceinline__ void k_mean_final_body(const float *part, float *mean, int N, int D, int nchunk, const dim3 bid)
+// (p[0] + p[D] + ...) / N: the mean of one channel from its nchunk partial sums, in chunk order (loads batched, adds in order)
+__device__ __forceinline__ float mean_of_chunks(const float *p, int N, int D, int nchunk)
 {
-    const int bh = bid.x, d = threadIdx.x;
-    const float *p = part + (size_t)bh * nchunk * D + d;
     float tot = 0.f;
     int c = 0;
     // few waves run this kernel (one per 64 channels of a head), so its time is the number of load round trips
@@ -112,7 +145,13 @@ __device__ __forceinline__ void k_mean_final_body(const float *part, float *mean
         for (int i = 0; i < 8; ++i) tot += v[i];
     }
     for (; c < nchunk; ++c) tot += p[(size_t)c * D];
-    mean[(size_t)bh * D + d] = tot / (float)N;
+    return tot / (float)N;
+}
+
+__device__ __forceinline__ void k_mean_final_body(const float *part, float *mean, int N, int D, int nchunk, const dim3 bid)
+{
+    const int bh = bid.x, d = threadIdx.x;
+    mean[(size_t)bh * D + d] = mean_of_chunks(part + (size_t)bh * nchunk * D + d, N, D, nchunk);
 }
 
 __global__ void k_mean_final_kernel(const float *part, float *mean, int N, int D, int nchunk)
@@ -155,15 +194,15 @@ __device__ __forceinline__ uint2 quantise8(const float (&v)[8], float inv)
     return make_uint2(w[0], w[1]);
 }
 
-// One workgroup per (block of `blk` tokens, head).  Blocks of up to 256*64 elements are kept
+// One workgroup of NT threads per (block of `blk` tokens, head).  Blocks of up to 256*64 elements are kept
 // in registers between the absmax pass and the quantising pass (one trip to memory); larger
-// ones are read twice.
-template <typename T, bool SMOOTH, bool FP8 = false>
-__device__ __forceinline__ void quant_blocks_body(const T *x, int8_t *x8, float *scales, const float *mean,
-                                                  int N, int D, int blk, int nblk, const XLayout lay, const dim3 bid)
+// ones are read twice.  mu: the mean of this head's channels (SMOOTH).
+template <typename T, bool SMOOTH, bool FP8 = false, int NT = 256>
+__device__ __forceinline__ void quant_block(const T *x, int8_t *x8, float *scales, const float *mu,
+                                            int N, int D, int blk, int nblk, const XLayout lay, const dim3 bid)
 {
-    constexpr int KEEP = 8;  // 8-element groups a thread can hold
-    __shared__ float red[4];  // one instance per kernel that inlines this body
+    constexpr int KEEP = 2048 / NT;  // 8-element groups a thread can hold
+    __shared__ float red[NT / 64];  // one instance per kernel that inlines this body
     const int bi = bid.x, bh = bid.y, tid = threadIdx.x;
     const int r0 = bi * blk;
     const int r1 = min(N, r0 + blk);
@@ -172,15 +211,14 @@ __device__ __forceinline__ void quant_blocks_body(const T *x, int8_t *x8, float 
     // element e of the block (row e / D, channel e % D) in the input
     auto xin = [&](int e) __attribute__((always_inline)) { return xbase + (size_t)(e / D) * lay.st + (e % D); };
     const int nelem = (r1 - r0) * D;  // multiple of 8
-    const float *mu = SMOOTH ? mean + (size_t)bh * D : nullptr;
-    const bool keep = nelem <= 256 * 8 * KEEP;
+    const bool keep = nelem <= NT * 8 * KEEP;
 
     float held[KEEP][8];
     float mx = 0.f;
     if (keep) {
 #pragma unroll
         for (int it = 0; it < KEEP; ++it) {
-            const int e = (it * 256 + tid) * 8;
+            const int e = (it * NT + tid) * 8;
             if (e < nelem) {
                 ld8(x, xin(e), held[it]);
                 const int d = e % D;
@@ -192,7 +230,7 @@ __device__ __forceinline__ void quant_blocks_body(const T *x, int8_t *x8, float 
             }
         }
     } else {
-        for (int e = tid * 8; e < nelem; e += 256 * 8) {
+        for (int e = tid * 8; e < nelem; e += NT * 8) {
             float v[8];
             ld8(x, xin(e), v);
             const int d = e % D;
@@ -208,7 +246,9 @@ __device__ __forceinline__ void quant_blocks_body(const T *x, int8_t *x8, float 
     for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    mx = red[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) mx = fmaxf(mx, red[w]);
 
     const float scale = (mx > 0.f) ? mx / QFormat<FP8>::QMAX : 1.f;
     const float inv = 1.f / scale;
@@ -218,11 +258,11 @@ __device__ __forceinline__ void quant_blocks_body(const T *x, int8_t *x8, float 
     if (keep) {
 #pragma unroll
         for (int it = 0; it < KEEP; ++it) {
-            const int e = (it * 256 + tid) * 8;
+            const int e = (it * NT + tid) * 8;
             if (e < nelem) *(uint2 *)(x8 + base + e) = quant8(held[it]);
         }
     } else {
-        for (int e = tid * 8; e < nelem; e += 256 * 8) {
+        for (int e = tid * 8; e < nelem; e += NT * 8) {
             float v[8];
             ld8(x, xin(e), v);
             const int d = e % D;
@@ -233,6 +273,47 @@ __device__ __forceinline__ void quant_blocks_body(const T *x, int8_t *x8, float 
             *(uint2 *)(x8 + base + e) = quant8(v);
         }
     }
+}
+
+template <typename T, bool SMOOTH, bool FP8 = false>
+__device__ __forceinline__ void quant_blocks_body(const T *x, int8_t *x8, float *scales, const float *mean,
+                                                  int N, int D, int blk, int nblk, const XLayout lay, const dim3 bid)
+{
+    quant_block<T, SMOOTH, FP8>(x, x8, scales, SMOOTH ? mean + (size_t)bid.y * D : nullptr, N, D, blk, nblk, lay, bid);
+}
+
+// The smoothing quantiser with fewer launches, for sequences where a launch costs more than the work it does: every
+// workgroup of a head forms the head's mean for itself, with the same sums in the same order, and the first one writes it.
+// ONE: from the rows (one launch instead of three; every workgroup reads the whole head, two channels per thread).
+// Otherwise from the partial sums of k_mean_partial_kernel (two launches instead of three).
+// nchunk * D <= SMOOTH_LDS_FLOATS with ONE.  Pre-pass, kernel times and the gaps between them: B2 Hkv3 N374 D128 12 -> 6.5 us (ONE),
+// B2 Hkv8 N2016 D64 15 -> 10 us (partial sums).
+constexpr int SMOOTH_LDS_FLOATS = 2048;
+template <bool ONE>
+constexpr int smooth_threads() { return ONE ? 1024 : 256; }
+template <typename T, bool FP8, bool ONE>
+__global__ void __launch_bounds__(smooth_threads<ONE>()) smooth_quant_blocks_kernel(const T *x, int8_t *x8, float *scales, const float *part,
+                                                                                  float *mean, int N, int D, int blk, int nblk, int nchunk,
+                                                                                  const XLayout lay)
+{
+    constexpr int NT = smooth_threads<ONE>();
+    __shared__ float sums[ONE ? SMOOTH_LDS_FLOATS : 1], mu[128];
+    const int bh = blockIdx.y, tid = threadIdx.x;
+    if constexpr (ONE) {
+        const int gpr = D / 2, g = tid % gpr;
+        for (int c = tid / gpr; c < nchunk; c += NT / gpr) {
+            float s[2];
+            sum_rows<32, 2>(x, lay.head(bh) + g * 2, lay.st, c * MEAN_CHUNK, min(N, (c + 1) * MEAN_CHUNK), s);
+            *(float2 *)&sums[c * D + g * 2] = make_float2(s[0], s[1]);
+        }
+        __syncthreads();
+    }
+    if (tid < D) {
+        mu[tid] = ONE ? mean_of_chunks(sums + tid, N, D, nchunk) : mean_of_chunks(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
+        if (blockIdx.x == 0) mean[(size_t)bh * D + tid] = mu[tid];
+    }
+    __syncthreads();
+    quant_block<T, true, FP8, NT>(x, x8, scales, mu, N, D, blk, nblk, lay, blockIdx);
 }
 
 template <typename T, bool SMOOTH, bool FP8 = false>
@@ -281,13 +362,35 @@ __global__ void __launch_bounds__(256) quant_rows_kernel(const T *x, int8_t *x8,
     quant_rows_body<T, SMOOTH, FP8>(x, x8, scales, mean, N, D, rows_total, lay, blockIdx);
 }
 
-__device__ __forceinline__ void cast_bf16_body(const float *x, uint16_t *y, size_t n, const dim3 bid)
+// y[0, n) = bf16(x[0, n)), round to nearest even, by `groups` workgroups of which this is number `group`; 8 values per
+// thread and step where both pointers are 16-byte aligned
+__device__ __forceinline__ void cast_rows_bf16(const float *x, uint16_t *y, size_t n, size_t group, size_t groups)
 {
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)bid.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const __bf16 b = (__bf16)x[i];  // round-to-nearest-even
+    const size_t i0 = group * blockDim.x + threadIdx.x, stride = groups * blockDim.x;
+    size_t done = 0;
+    if ((((uintptr_t)x | (uintptr_t)y) & 15u) == 0) {
+        for (size_t i = i0; i < n / 8; i += stride) {
+            float v[8];
+            ld8(x, i * 8, v);
+            uint32_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const __bf16 a = (__bf16)v[2 * j], b = (__bf16)v[2 * j + 1];
+                w[j] = (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+            }
+            *(uint4 *)(y + i * 8) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        done = n / 8 * 8;
+    }
+    for (size_t i = done + i0; i < n; i += stride) {
+        const __bf16 b = (__bf16)x[i];
         y[i] = __builtin_bit_cast(uint16_t, b);
     }
+}
+
+__device__ __forceinline__ void cast_bf16_body(const float *x, uint16_t *y, size_t n, const dim3 bid)
+{
+    cast_rows_bf16(x, y, n, bid.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(256) cast_bf16_kernel(const float *x, uint16_t *y, size_t n)
@@ -304,11 +407,7 @@ __device__ __forceinline__ void quant_rows_cast_body(const float *k, int8_t *k8,
     if ((int)bid.x < row_blocks) {
         quant_rows_body<float, false>(k, k8, scales, nullptr, N, D, rows_total, XLayout::dense(1, N, D), bid);
     } else {
-        const size_t stride = (size_t)(gridDim.x - row_blocks) * blockDim.x;
-        for (size_t i = (size_t)(bid.x - row_blocks) * blockDim.x + threadIdx.x; i < (size_t)nv; i += stride) {
-            const __bf16 b = (__bf16)v[i];  // round-to-nearest-even
-            vb[i] = __builtin_bit_cast(uint16_t, b);
-        }
+        cast_rows_bf16(v, vb, (size_t)nv, bid.x - row_blocks, gridDim.x - row_blocks);
     }
 }
 

@@ -317,3 +317,24 @@ def test_row_quantiser_inside_the_attention_kernel(dev, B, H, Hkv, N, D, bk, cau
     assert np.array_equal(got_sq, w_sq) and np.array_equal(got_q8, w_q8)
     assert w_sq[0, 0, zr] == 1.0
     assert np.array_equal(got, r["out"])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,N", [(1, 1, 1), (2, 3, 63), (1, 2, 65), (2, 3, 374), (1, 2, 1024), (1, 2, 1025), (3, 40, 700), (1, 2, 2048), (1, 2, 2049)])
+def test_smoothing_quantiser_by_sequence_length(dev, D, B, H, N):
+    """One, two or three launches, by the length of a sequence and the size of the tensor: codes, scales and means are the
+    oracle's bit for bit either way, for both input types, int8 and FP8."""
+    x = synth.normal(961, (B, H, N, D)) + np.float32(3.0) * synth.normal(962, (1, H, 1, D))
+    for dtype in (F32, BF16):
+        xv = oracle.bf16_round(x) if dtype == BF16 else x
+        mu = oracle.k_mean(xv)
+        for fp8 in (False, True):
+            want8, wants = (oracle.quant_blocks_fp8 if fp8 else oracle.quant_blocks)(xv, 64, sub=mu)
+            with Bufs(dev) as bufs:
+                dx = bufs.put(synth.to_bf16_bits(x) if dtype == BF16 else x)
+                x8, sc, mean = bufs.new(x.size), bufs.new(wants.size * 4), bufs.new(B * H * D * 4)
+                ws = bufs.new(dev.sage_quant_workspace(B, H, N, D))
+                (dev.sage_quant_fp8 if fp8 else dev.sage_quant)(dx, x8, sc, B, H, N, D, 64, dtype, mean=mean, workspace=ws, smooth=True)
+                assert np.array_equal(mean.copyout(np.float32, mu.shape), mu)
+                assert np.array_equal(sc.copyout(np.float32, wants.shape), wants)
+                assert np.array_equal(x8.copyout(want8.dtype, want8.shape), want8), (dtype, fp8)
