@@ -3,11 +3,21 @@ attention entry points.  Everything here calls libarhip.so; nothing computes on
 the host.
 """
 import ctypes
+import functools
 
 import numpy as np
 
 from . import _lib
 from ._lib import BF16, F32, check
+
+
+@functools.lru_cache(maxsize=None)
+def _default_scale(D):
+    """1 / sqrt(D) in float32 (numpy scalars take a microsecond)"""
+    return float(1.0 / np.sqrt(np.float32(D)))
+
+
+_Strides = ctypes.c_int64 * 3
 
 
 class Buffer:
@@ -156,7 +166,7 @@ class Device:
 
     def flash_fwd(self, q, k, v, o, B, Hq, Hkv, N, D, dtype, mask=None, kv_len=None, causal=False, scale=None,
                   wait=True):
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
+        scale = _default_scale(D) if scale is None else float(scale)
         s = ctypes.c_double()
         check(self.lib.arhip_flash_fwd(self.handle, self._ptr(q), self._ptr(k), self._ptr(v), self._ptr(o),
                                        self._ptr(mask), self._ptr(kv_len), B, Hq, Hkv, N, D, int(causal), dtype,
@@ -166,8 +176,8 @@ class Device:
     def flash_fwd_strided(self, q, k, v, o, q_strides, kv_strides, o_strides, B, Hq, Hkv, N, D, dtype, mask=None,
                           kv_len=None, causal=False, scale=None, wait=True):
         """Element strides {batch, head, token} per tensor; see include/arhip.h."""
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
-        arr = lambda t: (ctypes.c_int64 * 3)(*[int(x) for x in t])
+        scale = _default_scale(D) if scale is None else float(scale)
+        arr = lambda t: _Strides(*[int(x) for x in t])
         s = ctypes.c_double()
         check(self.lib.arhip_flash_fwd_strided(self.handle, self._ptr(q), self._ptr(k), self._ptr(v), self._ptr(o),
                                                arr(q_strides), arr(kv_strides), arr(o_strides), self._ptr(mask),
@@ -178,7 +188,7 @@ class Device:
     def flash_bwd(self, q, k, v, o, lse, dout, dq, dk, dv, delta, B, Hq, Hkv, N, D, mask=None, kv_len=None,
                   causal=False, scale=None, wait=True):
         """f32 dense [B,H,N,D]; o and lse from flash_fwd_lse of the same call; delta: B*Hq*N floats of scratch."""
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
+        scale = _default_scale(D) if scale is None else float(scale)
         s = ctypes.c_double()
         check(self.lib.arhip_flash_bwd(self.handle, self._ptr(q), self._ptr(k), self._ptr(v), self._ptr(o),
                                        self._ptr(lse), self._ptr(dout), self._ptr(dq), self._ptr(dk), self._ptr(dv),
@@ -189,12 +199,11 @@ class Device:
     def flash_fwd_lse(self, q, k, v, o, lse, B, Hq, Hkv, N, D, dtype, mask=None, kv_len=None, causal=False,
                       scale=None, wait=True):
         """Dense [B,H,N,D] tensors; also writes lse [B,Hq,N] (f32)."""
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
-        arr = lambda t: (ctypes.c_int64 * 3)(*[int(x) for x in t])
-        qs, ks = (Hq * N * D, N * D, D), (Hkv * N * D, N * D, D)
+        scale = _default_scale(D) if scale is None else float(scale)
+        qs, ks = _Strides(Hq * N * D, N * D, D), _Strides(Hkv * N * D, N * D, D)
         s = ctypes.c_double()
         check(self.lib.arhip_flash_fwd_lse(self.handle, self._ptr(q), self._ptr(k), self._ptr(v), self._ptr(o),
-                                           self._ptr(lse), arr(qs), arr(ks), arr(qs), self._ptr(mask),
+                                           self._ptr(lse), qs, ks, qs, self._ptr(mask),
                                            self._ptr(kv_len), B, Hq, Hkv, N, D, int(causal), dtype, scale,
                                            int(wait), ctypes.byref(s)))
         return s.value if wait else None
@@ -227,7 +236,7 @@ class Device:
 
     def sage_fwd_fp8(self, q8, k8, sq, sk, v, o, B, Hq, Hkv, N, D, bq, bk, out_dtype=F32, mask=None, kv_len=None,
                      causal=False, scale=None, wait=True):
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
+        scale = _default_scale(D) if scale is None else float(scale)
         s = ctypes.c_double()
         check(self.lib.arhip_sage_fwd_fp8(self.handle, self._ptr(q8), self._ptr(k8), self._ptr(sq), self._ptr(sk),
                                           self._ptr(v), self._ptr(o), self._ptr(mask), self._ptr(kv_len),
@@ -239,7 +248,7 @@ class Device:
                         causal=False, scale=None, wait=True, fp8=False):
         """sage_quant of Q (bf16, blocks of 128 queries) inside the attention kernel; sq_out / q8_out receive the
         scales and codes it derived.  fp8: E4M3 codes (k8 from sage_quant_fp8)."""
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
+        scale = _default_scale(D) if scale is None else float(scale)
         s = ctypes.c_double()
         fn = self.lib.arhip_sage_fwd_fp8_qfused if fp8 else self.lib.arhip_sage_fwd_qfused
         check(fn(self.handle, self._ptr(q), self._ptr(k8), self._ptr(sk), self._ptr(v), self._ptr(o),
@@ -258,7 +267,7 @@ class Device:
                              causal=False, scale=None, wait=True):
         """The reference's convention in one attention launch: f32 q quantised row by row inside the kernel, K scales
         per key (bk a power of two below 64)."""
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
+        scale = _default_scale(D) if scale is None else float(scale)
         s = ctypes.c_double()
         check(self.lib.arhip_sage_fwd_qfused_rows(self.handle, self._ptr(q), self._ptr(k8), self._ptr(sk), self._ptr(v),
                                                   self._ptr(o), self._ptr(sq_out), self._ptr(q8_out), self._ptr(kv_len),
@@ -280,7 +289,7 @@ class Device:
 
     def sage_fwd(self, q8, k8, sq, sk, v, o, B, Hq, Hkv, N, D, bq, bk, out_dtype=F32, mask=None, kv_len=None,
                  causal=False, scale=None, dbg_logits=None, dbg_sel=None, wait=True, v_strides=None, o_strides=None):
-        scale = float(1.0 / np.sqrt(np.float32(D))) if scale is None else float(scale)
+        scale = _default_scale(D) if scale is None else float(scale)
         sel = None
         if dbg_sel is not None:
             sel = (ctypes.c_int32 * 3)(*dbg_sel)
