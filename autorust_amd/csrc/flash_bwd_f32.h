@@ -192,14 +192,24 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
     const float *vp = p.v + ((size_t)b * p.Hkv + kvh) * (size_t)N * D;
     const size_t qoff = ((size_t)bh * N + rr) * D + h * 8;
 
+    // The first tiles are requested before the wave's own rows are waited for and split: one memory round trip, not two
+    // (few or short heads: a round trip is a tenth of the kernel).
+    PairStage<D, SPLIT ? 64 : NW * 64> first, stage;
+    if constexpr (SPLIT) {
+        if (wave < ntiles) stage.fetch(kp, vp, lane, wave * F32_BK, kend - 1);
+    } else if (ntiles > 0) {
+        first.fetch(kp, vp, tid, 0, kend - 1);
+        stage.fetch(kp, vp, tid, F32_BK, kend - 1);
+    }
+    const float lse = p.lse[(size_t)bh * N + rr];
+    const float di = p.delta[(size_t)bh * N + rr];
+    ARHIP_FENCE();
     split8 qr[KSTEPS], dor[KSTEPS];
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
         qr[s] = split_8(*(const float4 *)(p.q + qoff + 16 * s), *(const float4 *)(p.q + qoff + 16 * s + 4));
         dor[s] = split_8(*(const float4 *)(p.dout + qoff + 16 * s), *(const float4 *)(p.dout + qoff + 16 * s + 4));
     }
-    const float lse = p.lse[(size_t)bh * N + rr];
-    const float di = p.delta[(size_t)bh * N + rr];
     // P = exp(x - lse) as v_exp_f32 (base 2) of x * log2(e) - lse * log2(e); a row that saw no key has P = 0
     const float c2 = p.scale * BWD_LOG2E, lse2 = lse > BWD_LSE_FLOOR ? lse * BWD_LOG2E : __builtin_inff();
 
@@ -262,9 +272,7 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
     };
 
     if constexpr (SPLIT) {
-        PairStage<D, 64> stage;
         unsigned char *kt = lds + wave * 2 * Tile::BYTES, *vt = kt + Tile::BYTES;
-        if (wave < ntiles) stage.fetch(kp, vp, lane, wave * F32_BK, kend - 1);
         for (int it = wave; it < ntiles; it += NW) {
             const int k0 = it * F32_BK;
             stage.put(kt, vt, lane);
@@ -284,12 +292,8 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         //                                       and written to LDS                                  (VALU)
         //   R2(n)  dQ += K(n)^T dS(n) (MFMA)  |  dS(n+1) from S(n+1), dP(n+1)                        (VALU)
         // then a barrier.  K is read in two iterations (three tiles in LDS), V in one (two).
-        PairStage<D, NW * 64> stage;
         unsigned char *k_ring = lds, *v_ring = lds + 3 * Tile::BYTES;
         if (ntiles > 0) {
-            PairStage<D, NW * 64> first;
-            first.fetch(kp, vp, tid, 0, kend - 1);
-            stage.fetch(kp, vp, tid, F32_BK, kend - 1);
             first.put(k_ring, v_ring, tid);
             stage.put(k_ring + Tile::BYTES, v_ring + Tile::BYTES, tid);
             stage.fetch(kp, vp, tid, 2 * F32_BK, kend - 1);
@@ -455,15 +459,6 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
     const bool key_live = key < kvl;
     const float c2 = p.scale * BWD_LOG2E;
 
-    split8 kr[KSTEPS], vr[KSTEPS];
-    {
-        const size_t off = ((size_t)kv_bh * N + jj) * D + h * 8;
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            kr[s] = split_8(*(const float4 *)(p.k + off + 16 * s), *(const float4 *)(p.k + off + 16 * s + 4));
-            vr[s] = split_8(*(const float4 *)(p.v + off + 16 * s), *(const float4 *)(p.v + off + 16 * s + 4));
-        }
-    }
     f32x16_t dk[DB], dv[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -481,28 +476,49 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
     auto step_head = [&](int st) __attribute__((always_inline)) { return (size_t)b * p.Hq + (size_t)kvh * group + st / per_head; };
     auto step_q0 = [&](int st) __attribute__((always_inline)) { return (qtiles - 1 - st % per_head) * F32_BK; };
 
-    PairStage<D, SPLIT ? 64 : NW * 64> stage;
-    float st_l = 0.f, st_d = 0.f;
+    PairStage<D, SPLIT ? 64 : NW * 64> first, stage;
+    float st_l[2] = {0.f, 0.f}, st_d[2] = {0.f, 0.f};
     auto fetch_tiles = [&](decltype(stage) &to, int st) __attribute__((always_inline)) {
         const size_t off = step_head(st) * N * D;
         to.fetch(p.q + off, p.dout + off, stid, step_q0(st), N - 1);
     };
     // base-2 units: P = 2^(x log2(e) - lse log2(e)); rows that saw no key (and rows past the end) have P = 0
-    auto fetch_stats = [&](int st) __attribute__((always_inline)) {
+    auto fetch_stats = [&](int st, int to = 0) __attribute__((always_inline)) {
         if (stid < F32_BK) {
-            const int gr = step_q0(st) + stid;
-            const size_t bh = step_head(st);
-            const float lse = gr < N ? p.lse[bh * N + gr] : -1e30f;
-            st_l = lse > BWD_LSE_FLOOR ? lse * BWD_LOG2E : __builtin_inff();
-            st_d = gr < N ? p.delta[bh * N + gr] : 0.f;
+            const size_t at = step_head(st) * N + min(step_q0(st) + stid, N - 1);
+            st_l[to] = p.lse[at];
+            st_d[to] = p.delta[at];
         }
     };
-    auto put_stats = [&](float *stat) __attribute__((always_inline)) {
+    auto put_stats = [&](float *stat, int st, int from = 0) __attribute__((always_inline)) {
         if (stid < F32_BK) {
-            stat[stid] = st_l;
-            stat[32 + stid] = st_d;
+            const bool live = step_q0(st) + stid < N;
+            stat[stid] = live && st_l[from] > BWD_LSE_FLOOR ? st_l[from] * BWD_LOG2E : __builtin_inff();
+            stat[32 + stid] = live ? st_d[from] : 0.f;
         }
     };
+    // The first tiles are requested before the wave's own rows are waited for and split: one memory round trip, not three.
+    if constexpr (SPLIT) {
+        if (wave < steps) {
+            fetch_tiles(stage, wave);
+            fetch_stats(wave);
+        }
+    } else if (steps > 0) {
+        fetch_tiles(first, 0);
+        fetch_stats(0, 0);
+        fetch_tiles(stage, min(1, steps - 1));
+        fetch_stats(min(1, steps - 1), 1);
+    }
+    ARHIP_FENCE();
+    split8 kr[KSTEPS], vr[KSTEPS];
+    {
+        const size_t off = ((size_t)kv_bh * N + jj) * D + h * 8;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            kr[s] = split_8(*(const float4 *)(p.k + off + 16 * s), *(const float4 *)(p.k + off + 16 * s + 4));
+            vr[s] = split_8(*(const float4 *)(p.v + off + 16 * s), *(const float4 *)(p.v + off + 16 * s + 4));
+        }
+    }
 
     // S = Q K^T and dP = dO V^T: lane = key, register r = query 8 (r / 4) + 4 h + r % 4 of the tile
     f32x16_t s, dp;
@@ -560,13 +576,9 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
     if constexpr (SPLIT) {
         unsigned char *qs = lds + wave * (2 * Tile::BYTES + 256), *dos = qs + Tile::BYTES;
         float *stat = (float *)(qs + 2 * Tile::BYTES);
-        if (wave < steps) {
-            fetch_tiles(stage, wave);
-            fetch_stats(wave);
-        }
         for (int st = wave; st < steps; st += NW) {
             stage.put(qs, dos, lane);
-            put_stats(stat);
+            put_stats(stat, st);
             if (st + NW < steps) {
                 fetch_tiles(stage, st + NW);
                 fetch_stats(st + NW);
@@ -590,16 +602,11 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
         // steps this wave computes on (heads sharing the K/V head: all but those at the very end)
         const int mine = wk0 >= kvl ? 0 : CAUSAL ? max(0, steps - wave) : steps;
         if (steps > 0) {
-            decltype(stage) first;
-            fetch_tiles(first, 0);
-            fetch_stats(0);
-            if (steps > 1) fetch_tiles(stage, 1);
             first.put(q_ring, o_ring, tid);
-            put_stats(stats);
+            put_stats(stats, 0, 0);
             if (steps > 1) {
                 stage.put(q_ring + Tile::BYTES, o_ring + Tile::BYTES, tid);
-                fetch_stats(1);
-                put_stats(stats + 64);
+                put_stats(stats + 64, 1, 1);
             }
             if (steps > 2) {
                 fetch_tiles(stage, 2);
@@ -688,7 +695,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
                         stage.template split_step<i - 24>(qt2, ot2, tid);
                     }
                 });
-            if (n + 2 < steps) put_stats(stats + s2 * 64);
+            if (n + 2 < steps) put_stats(stats + s2 * 64, n + 2);
             if (n + 3 < steps) {
                 fetch_tiles(stage, n + 3);
                 fetch_stats(n + 3);
@@ -708,7 +715,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
             const int s2 = slot(cur + 2);
             if (n + 2 < steps) {
                 stage.put(q_ring + s2 * Tile::BYTES, o_ring + s2 * Tile::BYTES, tid);
-                put_stats(stats + s2 * 64);
+                put_stats(stats + s2 * 64, n + 2);
             }
             if (n + 3 < steps) {
                 fetch_tiles(stage, n + 3);

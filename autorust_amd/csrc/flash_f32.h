@@ -123,12 +123,27 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
     const float *vp = p.v + kv_off;
 
     // Q: this lane's part of its query row as matrix operands (rows past N read row N-1; never stored)
+    // Head size 128, one wave per SIMD: it is split once the first tiles have been requested, one memory round trip, not two,
+    // before the first product.
     split8 qr[KSTEPS];
+    float4 q_raw[2 * KSTEPS];
     {
         const float *qp = p.q + (size_t)b * p.qs[0] + (size_t)head * p.qs[1] + (size_t)min(q_row, N - 1) * p.qs[2] + h * 8;
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) qr[s] = split_8(*(const float4 *)(qp + 16 * s), *(const float4 *)(qp + 16 * s + 4));
+        for (int s = 0; s < KSTEPS; ++s) {
+            q_raw[2 * s] = *(const float4 *)(qp + 16 * s);
+            q_raw[2 * s + 1] = *(const float4 *)(qp + 16 * s + 4);
+        }
     }
+    // (B9 H6 N187 D128 causal 22.5 -> 20.1 us; where a second wave of the SIMD hides the trip it only costs registers:
+    // B1 H12 N197 D64 9.0 -> 9.3)
+    constexpr bool Q_LATE = D == 128 && QW == 1;
+    auto split_q = [&]() __attribute__((always_inline)) {
+        if (Q_LATE) ARHIP_FENCE();
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) qr[s] = split_8(q_raw[2 * s], q_raw[2 * s + 1]);
+    };
+    if (!Q_LATE) split_q();
 
     f32x16_t oacc[DB];
 #pragma unroll
@@ -329,6 +344,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                         first[j][t][0] = *(const float4 *)src[j];
                         first[j][t][1] = *(const float4 *)(src[j] + 16);
                     }
+            if (Q_LATE) split_q();
 #pragma unroll
             for (int j = 0; j < PER_THREAD; ++j) {
 #pragma unroll
@@ -509,6 +525,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
             fetch_k(kg);
             if constexpr (HAS_MASK) fetch_mask(kg * F32_BK);
             fetch_v(kg);
+            split_q();
         }
         for (int it = kg; it < my_tiles; it += KW) {
             const int k0 = it * F32_BK;
