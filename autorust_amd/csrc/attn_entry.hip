@@ -795,11 +795,11 @@ extern "C" __global__ void __launch_bounds__(256, 2) ar_flash_sage_fp8_mid_lens(
 #if ARHIP_PART(1)
 extern "C" __global__ void __launch_bounds__(256) ar_sage_kmean_partial_f32(const float *x, float *part, int N, int D, int nchunk)
 {
-    k_mean_partial_body<float>(x, part, N, D, nchunk, XLayout::dense(1, N, D), blockIdx);
+    k_mean_partial_any<float>(x, part, N, D, nchunk, XLayout::dense(1, N, D), blockIdx);
 }
 extern "C" __global__ void __launch_bounds__(256) ar_sage_kmean_partial_bf16(const uint16_t *x, float *part, int N, int D, int nchunk)
 {
-    k_mean_partial_body<uint16_t>(x, part, N, D, nchunk, XLayout::dense(1, N, D), blockIdx);
+    k_mean_partial_any<uint16_t>(x, part, N, D, nchunk, XLayout::dense(1, N, D), blockIdx);
 }
 extern "C" __global__ void ar_sage_kmean_final(const float *part, float *mean, int N, int D, int nchunk)
 {

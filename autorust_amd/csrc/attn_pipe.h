@@ -44,6 +44,7 @@
 #pragma once
 
 #include "attn_fwd.h"
+#include "lane_max.h"
 
 // 1: the int8 pipeline reads its int32 logit accumulators as biased floats (no conversions)
 #ifndef ARHIP_PIPE_INT_BIAS
@@ -798,8 +799,7 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         mx = xhalf_max(mx);  // the two lanes of a query
         float *red = (float *)(lds + QF_RED);
         if constexpr (!QROWS) {
-#pragma unroll
-            for (int o = 16; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+            mx = lane_group_max<32>(mx);
             if (lane == 0) red[wave] = mx;
             __syncthreads();
             // a block of 128 queries is four waves (a block past the last query holds copies of the last row and is
@@ -858,11 +858,8 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         // The exponent reference stays on a grid no finer than the unit in the last place of
         // 12582912 c for the largest c = sq sk scale log2(e) the workgroup can meet; every wave reduces
         // the same scales, so the grid is uniform over the workgroup.
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            mq = fmaxf(mq, __shfl_xor(mq, o));
-            mk = fmaxf(mk, __shfl_xor(mk, o));
-        }
+        mq = lane_group_max<64>(mq);
+        mk = lane_group_max<64>(mk);
         // 12582912 c_max < 2^(E+1): the sums stay below 2^(E+2) wherever the bias outweighs the
         // reference, so their unit in the last place is at most 2^(E-22); the grid is twice that.
         // (Scales that are not finite, or zero, give a grid of 1: the results are garbage or

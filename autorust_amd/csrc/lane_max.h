@@ -1,0 +1,39 @@
+// Maxima over groups of lanes without LDS: a __shfl_xor is an LDS round trip of some 100 cycles, and a reduction is a chain of
+// them; the vector ALU's own lane exchanges take a few cycles each.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace arhip {
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float x)
+{
+    const int u = __float_as_int(x);
+    return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(u, u, CTRL, 0xf, 0xf, false)));
+}
+
+// largest x of each aligned group of G lanes (8, 16, 32 or 64), in every lane of it
+template <int G>
+__device__ __forceinline__ float lane_group_max(float x)
+{
+    static_assert(G == 8 || G == 16 || G == 32 || G == 64, "group of lanes");
+    x = dpp_max<0xB1>(x);                    // quad_perm [1,0,3,2]: lane ^ 1
+    x = dpp_max<0x4E>(x);                    // quad_perm [2,3,0,1]: lane ^ 2
+    x = dpp_max<0x141>(x);                   // row_half_mirror: the other four of eight
+    if constexpr (G >= 16) x = dpp_max<0x140>(x);  // row_mirror: the other eight of sixteen
+    if constexpr (G >= 32) {
+        const uint32_t u = __float_as_uint(x);
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    if constexpr (G == 64) {
+        const uint32_t u = __float_as_uint(x);
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    return x;
+}
+
+}  // namespace arhip

@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lane_max.h"
+
 #pragma clang fp contract(off)
 
 namespace arhip {
@@ -93,28 +95,40 @@ __device__ __forceinline__ void sum_rows(const T *x, size_t base, long st, int j
     }
 }
 
-// part[bh][c][d] = k[64c][d] + k[64c+1][d] + ... in token order.
-// One thread owns C adjacent channels of one 64-token chunk: D/C threads read a whole row
-// (coalesced), 256/(D/C) chunks per workgroup.  C = 8 for the memory's rate, 2 where the tensor is small and a
-// wave's own instructions are the time (B2 Hkv8 N2016 D64: 6.0 -> 4.5 us).
-template <typename T, int C = 8>
-__device__ __forceinline__ void k_mean_partial_body(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, const dim3 bid)
+// part[bh][c][d] = k[64c][d] + k[64c+1][d] + ... in token order, for channels C g .. C g + C - 1
+template <typename T, int C>
+__device__ __forceinline__ void k_mean_chunk(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, int bh, int c, int g)
 {
-    const int gpr = D / C;                       // groups of C channels per row
-    const int cpb = 256 / gpr;                   // chunks per workgroup
-    const int c = bid.x * cpb + threadIdx.x / gpr;
-    const int g = threadIdx.x % gpr, bh = bid.y;
-    if (c >= nchunk) return;
-    const int j0 = c * MEAN_CHUNK;
-    const int j1 = min(N, j0 + MEAN_CHUNK);
     float s[C];
-    sum_rows<(C == 8 ? 16 : 32), C>(x, lay.head(bh) + g * C, lay.st, j0, j1, s);
+    sum_rows<(C == 8 ? 16 : 32), C>(x, lay.head(bh) + g * C, lay.st, c * MEAN_CHUNK, min(N, (c + 1) * MEAN_CHUNK), s);
     float *o = part + ((size_t)bh * nchunk + c) * D + g * C;
     if constexpr (C == 8) {
         *(float4 *)o = make_float4(s[0], s[1], s[2], s[3]);
         *(float4 *)(o + 4) = make_float4(s[4], s[5], s[6], s[7]);
     } else {
         *(float2 *)o = make_float2(s[0], s[1]);
+    }
+}
+
+// One thread owns C adjacent channels of one 64-token chunk: D/C threads read a whole row
+// (coalesced), 256/(D/C) chunks per workgroup.  C = 8 for the memory's rate, 2 where the tensor is small and a
+// wave's own instructions are the time (B2 Hkv8 N2016 D64: 6.0 -> 4.5 us).
+template <typename T, int C>
+__device__ __forceinline__ void k_mean_partial_body(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, const dim3 bid)
+{
+    const int gpr = D / C, c = bid.x * (256 / gpr) + threadIdx.x / gpr;
+    if (c < nchunk) k_mean_chunk<T, C>(x, part, N, D, nchunk, lay, bid.y, c, threadIdx.x % gpr);
+}
+
+// The grid of C = 8; a workgroup that has chunks for less than half of its threads deals them out two channels at a time.
+template <typename T>
+__device__ __forceinline__ void k_mean_partial_any(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, const dim3 bid)
+{
+    const int cpb = 256 / (D / 8), c0 = bid.x * cpb, n = min(cpb, nchunk - c0), gpr = D / 2;
+    if (2 * n > cpb) {
+        k_mean_partial_body<T, 8>(x, part, N, D, nchunk, lay, bid);
+    } else {
+        for (int i = threadIdx.x; i < n * gpr; i += 256) k_mean_chunk<T, 2>(x, part, N, D, nchunk, lay, bid.y, c0 + i / gpr, i % gpr);
     }
 }
 
@@ -242,8 +256,7 @@ __device__ __forceinline__ void quant_block(const T *x, int8_t *x8, float *scale
             }
         }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    mx = lane_group_max<64>(mx);
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
     mx = red[0];
@@ -346,7 +359,7 @@ __device__ __forceinline__ void quant_rows_body(const T *x, int8_t *x8, float *s
     float mx = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(v[i]));
-    for (int off = gpr >> 1; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    mx = gpr == 16 ? lane_group_max<16>(mx) : lane_group_max<8>(mx);
     const float scale = (mx > 0.f) ? mx / QFormat<FP8>::QMAX : 1.f;
     const float inv = 1.f / scale;
     if (live) {
