@@ -735,7 +735,9 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     // last partial one) run the same pipeline with the mask applied inside the softmax.  Every wave
     // passes one barrier per tile and requests its share of every tile's transfers, whichever form of
     // the tile it runs.
-    const int nfull = CAUSAL ? min(kend / BK, wq0 / BK) : kend / BK;
+    // A wave whose queries are all past the end computes nothing: its SIMD is left to the other workgroup's wave.
+    const bool idle = wq0 >= N;
+    const int nfull = idle ? 0 : CAUSAL ? min(kend / BK, wq0 / BK) : kend / BK;
     static_for<0, AHEAD>([&](auto ti) __attribute__((always_inline)) { issue_tile(decltype(ti)::value); });
     mask_block(0);
     mask_block(1);
@@ -980,7 +982,7 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     if (nplain < nfull) tile_iter(PLAIN, PLAIN, MASKED, nplain, any_stage);
     // under the causal mask a wave is done once the tiles start past its last query; it keeps
     // feeding the transfers and the barriers the other waves rely on
-    const int my_tiles = CAUSAL ? min(ntiles, (wq0 + 31) / BK + 1) : ntiles;
+    const int my_tiles = idle ? 0 : CAUSAL ? min(ntiles, (wq0 + 31) / BK + 1) : ntiles;
     // (two loops rather than a branch inside one: the accumulators would be copied at the join)
 #pragma clang loop unroll(disable)
     for (int it = nfull; it < my_tiles; ++it) tile_iter(MASKED, MASKED, MASKED, it, any_stage);
