@@ -729,6 +729,24 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
         });
     };
 
+    // The last block a wave works on: the rest of its softmax and O^T += V^T . P^T, with nothing to look ahead for.
+    auto last_block = [&](const acc_t &s_old, uint4 (&p_cur)[2], const unsigned char *sc, int cb, float c_cur, int rel_cur,
+                          const float *kp, int kb0) __attribute__((always_inline)) {
+        constexpr std::true_type M{};
+        ARHIP_FENCE();
+        static_for<SM_SPLIT, SM_OPS>([&](auto ic) __attribute__((always_inline)) { sm_op(M, ic, s_old, c_cur, rel_cur, p_cur, kp, kp, (kb0 >> 5) & 1); });
+        rs = sm_half[0] + sm_half[1];
+        if (__builtin_expect(__any(!(rs <= 16.0f * LAZY_LIMIT)), 0)) fix_reference(M, sc, cb, s_old, c_cur, rel_cur, p_cur, rs, kp, kb0);
+        l_run += rs;
+        ARHIP_FENCE();
+        static_for<0, DB * 2>([&](auto gi) __attribute__((always_inline)) {
+            constexpr int db = decltype(gi)::value / 2, ks = decltype(gi)::value % 2;
+            const uint4 a = make_uint4(vf[db][ks][0].x, vf[db][ks][0].y, vf[db][ks][1].x, vf[db][ks][1].y);
+            oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                               __builtin_bit_cast(bf16x8, p_cur[ks]), oacc[db], 0, 0, 0);
+        });
+    };
+
     // ---- prologue: tiles 0..2 on their way, tiles 0 and 1 visible ----
     // Tiles [0, nfull) have no masked key for this wave (all full tiles; under the causal mask those
     // before the wave's first query); the remaining ones (the one on the wave's causal diagonal, or the
@@ -963,8 +981,16 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     // RINGS: the first iteration requests K(2) into the place of K(0), which the lines above have just
     // read: every wave's reads must have returned first
     if constexpr (RINGS) __syncthreads();
-    // the last unmasked tile hands a masked block to the look-ahead: it is peeled off
-    const int nplain = (nfull < ntiles) ? max(nfull - 1, 0) : nfull;
+    // under the causal mask a wave is done once the tiles start past its last query; it keeps
+    // feeding the transfers and the barriers the other waves rely on
+    const int my_tiles = idle ? 0 : CAUSAL ? min(ntiles, (wq0 + 31) / BK + 1) : ntiles;
+    // A wave has one masked tile at most, its last (the one on its causal diagonal, or the one the keys end in): tiles
+    // [0, last) are unmasked.  At head size 64 the last one, masked or not, has a form of its own: nothing follows its last
+    // block, and a second block whose keys are all hidden from the wave is left out (N = 197: one block of eight; causal: half of
+    // the waves).  (At 128 the two ways out of it cost copies of the accumulators and 13 to 64 spilled registers.)
+    // The tile before a masked one hands a masked block to the look-ahead: it is peeled off.
+    constexpr bool OWN_LAST = D == 64;
+    const int last = my_tiles - 1, nplain = nfull < my_tiles ? max(nfull - 1, 0) : OWN_LAST ? max(last, 0) : nfull;
     // Four tiles per trip, so that the stage of a tile (it % 4) and with it every LDS offset and transfer
     // destination is a constant (int8: 15 vector and 23 scalar instructions fewer per tile, Sage B4 H32 S8192
     // 3.05 -> 2.96 ms; bf16, once no offset needs a register of its own: S8192 -1.8 %).
@@ -979,13 +1005,27 @@ __device__ __forceinline__ void attn_pipe_impl(const AttnParams &p, unsigned cha
     const std::integral_constant<int, -1> any_stage;
 #pragma clang loop unroll(disable)
     for (int it = nplain4; it < nplain; ++it) tile_iter(PLAIN, PLAIN, PLAIN, it, any_stage);
-    if (nplain < nfull) tile_iter(PLAIN, PLAIN, MASKED, nplain, any_stage);
-    // under the causal mask a wave is done once the tiles start past its last query; it keeps
-    // feeding the transfers and the barriers the other waves rely on
-    const int my_tiles = idle ? 0 : CAUSAL ? min(ntiles, (wq0 + 31) / BK + 1) : ntiles;
-    // (two loops rather than a branch inside one: the accumulators would be copied at the join)
+    if (nplain < (OWN_LAST ? last : nfull)) tile_iter(PLAIN, PLAIN, MASKED, nplain, any_stage);
+    if constexpr (!OWN_LAST) {
+        // (a loop rather than a branch: the accumulators would be copied at the join)
 #pragma clang loop unroll(disable)
-    for (int it = nfull; it < my_tiles; ++it) tile_iter(MASKED, MASKED, MASKED, it, any_stage);
+        for (int it = nfull; it < my_tiles; ++it) tile_iter(MASKED, MASKED, MASKED, it, any_stage);
+    } else if (last >= 0) {
+        const int it = last, rel0 = lim4h - it * BK;
+        const unsigned char *k_cur = lds + k_base(it), *k_nxt = lds + k_base(it + 1), *v_cur = lds + v_base(it);
+        const float *f0 = key_factors(it, 0), *f1 = key_factors(it, 1);
+        const std::false_type lo;
+        issue_tile(it + AHEAD);
+        if (min(kend - 1, CAUSAL ? wq0 + 31 : kend - 1) >= it * BK + 32) {
+            pipe_block(MASKED, MASKED, s_a, s_b, p_a, p_b, k_cur, 0, v_cur, 1, k_nxt, 0, c_carry, c_carry, rel0, rel0 - 32, lo, lo, lo,
+                       f0, f1, f1, it * BK, [&]() __attribute__((always_inline)) { wait_vmem_le<0>(); });
+            last_block(s_b, p_b, k_cur, 1, c_carry, rel0 - 32, f1, it * BK + 32);
+        } else {
+            last_block(s_a, p_a, k_cur, 0, c_carry, rel0, f0, it * BK);
+        }
+        wait_vmem_le<RINGS ? 0 : XPW_MIN>();
+        __syncthreads();
+    }
 #pragma clang loop unroll(disable)
     for (int it = max(nfull, my_tiles); it < ntiles; ++it) {
         issue_tile(it + AHEAD);
@@ -1056,7 +1096,7 @@ __device__ __forceinline__ void attn_pipe_body(const AttnParams &p, unsigned cha
 }
 
 template <int D, bool CAUSAL, int MODE, bool OUT_F32, int NW = 8, bool PER_KEY = false, bool QFUSE = false, bool HAS_MASK = false>
-__global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) attn_pipe_kernel(const AttnParams p)
+__global__ void __launch_bounds__(NW * 64, NW == 4 ? (D == 64 && !HAS_MASK && !PER_KEY ? 3 : 2) : 1) attn_pipe_kernel(const AttnParams p)
 {
     __shared__ __attribute__((aligned(1024))) unsigned char lds[attn_pipe_lds_bytes<D, MODE, NW, PER_KEY, QFUSE, HAS_MASK>()];
     attn_pipe_body<D, CAUSAL, MODE, OUT_F32, NW, PER_KEY, QFUSE, HAS_MASK>(p, lds, (int)blockIdx.x);

@@ -76,8 +76,8 @@ static void launch_attn(hipStream_t stream, const AttnParams &p, bool causal, bo
 // B2 H16 N = 1024 -22 %, N = 1024 -4 %; N = 2048 equal; N = 2048 causal with key lengths in [N/2, N]
 // (many equal workgroups) +3 %; N = 8192 +3 %, causal N = 32768 +4.5 %.
 // At D = 64 (B4 H32): N = 2048 -8 %, N = 8192 -2 %, causal N = 2048 -16 %, causal N = 8192 -4 %: always 4 waves.
-// (Three such workgroups per compute unit fit at D = 64, 154 registers and 40 KB of LDS each, and run no
-// faster than two.)
+// (D = 64 runs three workgroups per compute unit, 168 registers and 40 KB of LDS each: no faster than two on long
+// sequences, B16 H24 N140 10.2 -> 9.6 us.)
 static bool pipe_wants_4_waves(arhip_device *dev, int64_t heads, int64_t N, int64_t D, bool causal, bool has_len)
 {
     if (dev->attn_waves == 8 || dev->attn_waves == 40) return dev->attn_waves == 40;

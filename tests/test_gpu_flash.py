@@ -49,6 +49,20 @@ def test_f32_exact_matches_reference(dev, N, D):
     assert (np.abs(got - truth) / np.maximum(np.abs(truth), 1)).max() <= 1e-5
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [32, 33, 64, 65, 96, 97, 128, 129, 160, 193, 257])
+def test_last_tile_of_a_wave(dev, N, causal):
+    """The last key tile of a wave, full or not, one block of it or both, with waves that end a tile before their neighbours, with
+    key lengths on either side of a block's edge; few workgroups and many."""
+    for B, H in ((2, 3), (16, 20)):
+        q, k, v = (oracle.bf16_round(synth.normal(951 + i, (B, H, N, 64))) for i in range(3))
+        kv_len = np.array([max(1, N - 32 * (b % 2) - b % 3) for b in range(B)], np.int32)
+        got = run_flash(dev, q, k, v, BF16, kv_len=kv_len, causal=causal)
+        for b in (0, 1, B - 1):
+            want = oracle.sdpa_f64(q[b:b + 1], k[b:b + 1], v[b:b + 1], kv_len=kv_len[b:b + 1], causal=causal)
+            assert np.abs(got[b] - want[0]).max() <= 2e-2, b
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("case", MASK_CASES, ids=lambda c: c[0])
 def test_causal_mask_gqa(dev, case, D):
