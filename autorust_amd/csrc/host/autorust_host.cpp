@@ -201,6 +201,14 @@ int64_t Tensor::numel() const
     return n;
 }
 
+void *Tensor::ptr() const
+{
+    if (!st_) return nullptr;
+    st_->dev->sync();
+    st_->exposed = true;
+    return st_->ptr;
+}
+
 Tensor Tensor::empty(const std::shared_ptr<Device> &dev, const std::vector<int64_t> &shape, DType dtype)
 {
     Tensor t;
@@ -220,12 +228,12 @@ Tensor Tensor::from_slice(const std::shared_ptr<Device> &dev, const float *data,
     const int64_t n = t.numel();
     if (n == 0) return t;
     if (dtype == DType::Float32) {
-        dev->check(arhip_copyin(dev->handle(), t.ptr(), data, (size_t)n * 4));
+        dev->check(arhip_copyin(dev->handle(), t.ptr_on_stream(), data, (size_t)n * 4));
     } else {
         // cast on the device (round to nearest even, dtype/mod.rs:973-981) through an f32 staging buffer
         void *tmp = dev->alloc((size_t)n * 4);
         dev->check(arhip_copyin(dev->handle(), tmp, data, (size_t)n * 4));
-        dev->check(arhip_cast_bf16(dev->handle(), (const float *)tmp, (uint16_t *)t.ptr(), n, 1, nullptr));
+        dev->check(arhip_cast_bf16(dev->handle(), (const float *)tmp, (uint16_t *)t.ptr_on_stream(), n, 1, nullptr));
         dev->release(tmp, (size_t)n * 4);
     }
     return t;
@@ -234,7 +242,7 @@ Tensor Tensor::from_slice(const std::shared_ptr<Device> &dev, const float *data,
 Tensor Tensor::from_i32(const std::shared_ptr<Device> &dev, const int32_t *data, const std::vector<int64_t> &shape)
 {
     Tensor t = empty(dev, shape, DType::Int32);
-    if (t.numel() > 0) dev->check(arhip_copyin(dev->handle(), t.ptr(), data, (size_t)t.numel() * 4));
+    if (t.numel() > 0) dev->check(arhip_copyin(dev->handle(), t.ptr_on_stream(), data, (size_t)t.numel() * 4));
     return t;
 }
 
@@ -255,10 +263,10 @@ std::vector<float> Tensor::to_list() const
     if (n == 0) return out;
     auto &dev = st_->dev;
     if (dtype_ == DType::Float32) {
-        dev->check(arhip_copyout(dev->handle(), out.data(), ptr(), (size_t)n * 4));
+        dev->check(arhip_copyout(dev->handle(), out.data(), ptr_on_stream(), (size_t)n * 4));
     } else {
         std::vector<uint16_t> raw((size_t)n);
-        dev->check(arhip_copyout(dev->handle(), raw.data(), ptr(), (size_t)n * 2));
+        dev->check(arhip_copyout(dev->handle(), raw.data(), ptr_on_stream(), (size_t)n * 2));
         for (int64_t i = 0; i < n; ++i) {
             const uint32_t bits = (uint32_t)raw[(size_t)i] << 16;
             std::memcpy(&out[(size_t)i], &bits, 4);
@@ -338,11 +346,20 @@ void HostCall::exec() const
     if (dev->name() != device) throw std::runtime_error("TGERR: HostCall::exec: buffers live on " + dev->name() + ", not " + device);
     std::vector<void *> ptrs;
     ptrs.reserve(bufs.size());
-    for (const auto &b : bufs) ptrs.push_back(b.ptr());
-    // Not waited for: a launch goes to the device's stream, and so does everything that can look at what it writes
+    bool wait = false;
+    for (const auto &b : bufs) {
+        ptrs.push_back(b.ptr_on_stream());
+        if (b.defined() && b.device() != dev) {  // another handle: its stream may still write the buffer, and may write it again
+            b.device()->sync();
+            wait = true;
+        }
+        wait = wait || b.exposed();
+    }
+    // Not waited for otherwise: a launch goes to the device's stream, and so does everything that can look at what it writes
     // (to_list, copies, later launches, the reuse and the release of a buffer).  Waiting for each of them cost a ViT-B/16 layer
     // at batch 8 (a 7 us kernel) 17 us a call, and the two launches of a quantised layer 30.
     dev->run_host_kernel(src, name, signature, ptrs, global, local, vals, false);
+    if (wait) dev->sync();
 }
 
 std::optional<Tensor> fused_attention(const Tensor &q, const Tensor &k, const Tensor &v, Session &sess, const Settings &st)

@@ -61,6 +61,8 @@ public:
     ~Device();
     Device(const Device &) = delete;
     arhip_device *handle() const { return dev_; }
+    void sync() const { check(arhip_sync(dev_)); }               // until everything submitted through this handle has run
+    void *stream() const { return arhip_stream(dev_); }          // hipStream_t that all of it goes to
     std::string name() const { return ordinal_ == 0 ? "HIP" : "HIP:" + std::to_string(ordinal_); }
     int compute_units() const;
     void *alloc(size_t bytes);   // reuses a cached block of the same size (<= 32 kept per size)
@@ -95,6 +97,7 @@ struct Storage {  // OpaqueT: base pointer + size, views share it (buffer.rs:32-
     std::shared_ptr<Device> dev;
     void *ptr = nullptr;
     size_t bytes = 0;
+    bool exposed = false;  // the address has been handed out (Tensor::ptr): launches on it are waited for
     ~Storage();
 };
 
@@ -114,7 +117,12 @@ public:
     const std::vector<int64_t> &shape() const { return shape_; }
     DType dtype() const { return dtype_; }
     int64_t numel() const;
-    void *ptr() const { return st_ ? st_->ptr : nullptr; }
+    // The buffer's address, for any use: what has been submitted on the device is waited for, and so is every later launch
+    // on this buffer (HostCall::exec), so that whoever holds the address reads and writes it between calls on any stream.
+    void *ptr() const;
+    // The address for work on the device's own stream (Device::stream), or ordered behind it by the caller: nothing is waited for.
+    void *ptr_on_stream() const { return st_ ? st_->ptr : nullptr; }
+    bool exposed() const { return st_ && st_->exposed; }
     const std::shared_ptr<Device> &device() const { return st_->dev; }
     bool defined() const { return (bool)st_; }
 
@@ -151,7 +159,10 @@ struct HostCall {              // session.rs:210-256, field for field
     int64_t global[3];         // launch grid
     std::optional<std::array<int64_t, 3>> local;       // launch block
     std::vector<int64_t> vals; // scalar arguments
-    void exec() const;         // run_host_kernel on the device's stream (session.rs:230-255, which waits for every launch)
+    // run_host_kernel on the stream of the first buffer's device (session.rs:230-255, which waits for every launch).  Submits
+    // without waiting where everything that can see the buffers goes to that stream: not if an address has been handed out
+    // (Tensor::ptr) or a buffer belongs to another handle, whose stream is waited for before, and the launch itself after.
+    void exec() const;
 };
 
 class Session {                // session.rs:44-193 (the part the path touches)

@@ -261,7 +261,28 @@ int arh_run_host_kernel(void *d, const char *src, const char *name, void **bufs,
         return 0;
     }, -1);
 }
-void *arh_tensor_ptr(void *t) { return ((Tensor *)t)->ptr(); }
+// The address of a tensor's buffer.  arh_tensor_ptr: for any use, on any stream or by host copies; waits for what has been
+// submitted on the tensor's device, and from then on every launch on this buffer returns with it done (NULL on error).
+// arh_tensor_ptr_on: for work on the stream of device `d` (arh_device_stream); waits only if the tensor is another handle's.
+void *arh_tensor_ptr(void *t)
+{
+    return guard([&]() -> void * { return ((Tensor *)t)->ptr(); }, nullptr);
+}
+void *arh_tensor_ptr_on(void *t, void *d)
+{
+    return guard([&]() -> void * {
+        const Tensor &x = *(Tensor *)t;
+        return x.defined() && x.device() != *(std::shared_ptr<Device> *)d ? x.ptr() : x.ptr_on_stream();
+    }, nullptr);
+}
+int arh_device_sync(void *d)
+{
+    return guard([&]() -> int {
+        (*(std::shared_ptr<Device> *)d)->sync();
+        return 0;
+    }, -1);
+}
+void *arh_device_stream(void *d) { return (*(std::shared_ptr<Device> *)d)->stream(); }
 
 uint64_t arh_selections(int kernel) { return selections((Kernel)kernel); }
 

@@ -71,6 +71,11 @@ def host():
         h.arh_tensor_from_i32.argtypes = [vp, ctypes.c_void_p, i64p, ci]
         h.arh_tensor_ptr.restype = vp
         h.arh_tensor_ptr.argtypes = [vp]
+        h.arh_tensor_ptr_on.restype = vp
+        h.arh_tensor_ptr_on.argtypes = [vp, vp]
+        h.arh_device_sync.argtypes = [vp]
+        h.arh_device_stream.restype = vp
+        h.arh_device_stream.argtypes = [vp]
         h.arh_run_host_kernel.argtypes = [vp, ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(vp), ci, i64p, ci, i64p, i64p, ci,
                                           ctypes.POINTER(ctypes.c_double)]
         h.arh_tensor_free.argtypes = [vp]
@@ -130,10 +135,20 @@ class HipDevice:
     def raw_allocs(self):
         return int(host().arh_device_raw_allocs(self.h))
 
+    @property
+    def stream(self):
+        """The hipStream_t (as an integer) that every launch and copy of this handle goes to."""
+        return host().arh_device_stream(self.h)
+
+    def sync(self):
+        """Waits until everything submitted through this handle has run."""
+        if host().arh_device_sync(self.h) != 0:
+            raise _err()
+
     def run_host_kernel(self, src, name, bufs, vals, global_, local, wait=True):
         """`Compiled::run_host_kernel` (src/runtime/device.rs:383-402) on Tensor buffers and 32-bit
         scalars; returns the elapsed device seconds, or None for a launch that did not wait."""
-        ptrs = (ctypes.c_void_p * max(len(bufs), 1))(*[host().arh_tensor_ptr(b.h) for b in bufs])
+        ptrs = (ctypes.c_void_p * max(len(bufs), 1))(*[host().arh_tensor_ptr_on(b.h, self.h) for b in bufs])
         secs = ctypes.c_double(-1.0)
         if host().arh_run_host_kernel(self.h, src.encode(), name.encode(), ptrs, len(bufs), _i64(list(vals)), len(vals),
                                       _i64(list(global_)), _i64(list(local)), int(wait), ctypes.byref(secs)) != 0:
