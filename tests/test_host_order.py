@@ -1,6 +1,6 @@
 """What the C++ host layer waits for (csrc/host/): a launch is submitted without waiting only while everything that can see its
 buffers goes to the same stream.  CPU tests: the host layer on a stand-in for libarhip that logs launches and waits.  GPU tests:
-results read through the address on a stream of the reader's own, and buffers shared between two handles."""
+results read through the address on another stream, and buffers shared between two handles."""
 import ctypes
 import os
 import subprocess
@@ -116,28 +116,30 @@ def _arrays(b=2, h=4, n=300, d=64):
 
 
 @pytest.mark.gpu
-def test_an_address_is_good_on_any_stream():
-    """A tensor's memory read by torch on a stream of its own, after the call that made it and after every replay into it."""
-    import torch
-    dev, sess = host.HipDevice(0), Session()
-    q, k, v = (Tensor.from_slice(dev, x, x.shape) for x in _arrays())
+def test_an_address_is_good_on_any_stream(dev):
+    """A tensor's memory read and cleared through its address on the stream of another handle, after the call that made it and
+    after every replay into it."""
+    from autorust_amd._lib import check
+    hdev, sess = host.HipDevice(0), Session()
+    q, k, v = (Tensor.from_slice(hdev, x, x.shape) for x in _arrays())
+    want = q.flash_attention_with(k, v, None, 0.0, False, sess).to_list()
     sess.begin_capture()
     out = q.flash_attention_with(k, v, None, 0.0, False, sess)
     sess.end_capture()
+    address = host.host().arh_tensor_ptr(out.h)
+    got = np.empty_like(want)
 
-    class View:
-        __cuda_array_interface__ = {"data": (host.host().arh_tensor_ptr(out.h), False), "shape": out.shape, "typestr": "<f4",
-                                    "strides": None, "version": 2}
+    def read():
+        check(dev.lib.arhip_copyout(dev.handle, got.ctypes.data, address, got.nbytes))
+        return got
 
-    view = torch.as_tensor(View(), device="cuda")
-    want = out.to_list()
-    with torch.cuda.stream(torch.cuda.Stream()):
-        assert np.array_equal(view.cpu().numpy(), want)
-        for _ in range(3):
-            view.zero_()
-            torch.cuda.current_stream().synchronize()
-            sess.replay()
-            assert np.array_equal(view.cpu().numpy(), want)
+    assert np.array_equal(read(), want)
+    for _ in range(3):
+        check(dev.lib.arhip_fill_zero(dev.handle, address, got.nbytes))
+        dev.sync()
+        assert not read().any()
+        sess.replay()
+        assert np.array_equal(read(), want)
 
 
 @pytest.mark.gpu
