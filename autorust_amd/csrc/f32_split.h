@@ -1,5 +1,8 @@
 // fp32 contractions on the bf16 matrix instruction, at fp32 precision.
 //
+// (The method: G. Henry, P. T. P. Tang and A. Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for
+// higher-precision computations", IEEE ARITH 2019.)
+//
 // An fp32 value is the exact sum of three bf16 values: x = hi + mid + lo with hi = bf16(x), mid = bf16(x - hi),
 // lo = x - hi - mid (24 significant bits = 3 x 8; both differences are exact, and the last one fits bf16).  A
 // product a b is then the sum of nine bf16 products, each exact in the fp32 accumulator of
@@ -14,6 +17,13 @@
 // eight fp32 steps: measured on N(0,1) operands, against the exact sum and in units of 2^-24 of the sum of
 // magnitudes, root mean square 0.19 per instruction (16 products) against 0.40 per v_mfma_f32_32x32x2_f32 (2 products).
 // Subnormal operands are multiplied as such.
+//
+// The three parts exist where hi does not round to infinity (|x| < 3.3962e38) and lo needs no bit below the smallest bf16
+// (|x| > 2^-110, or 0).  Beyond the upper end lo (and for an infinity mid) is NaN, and so is every sum that the value enters.  Below
+// the lower end up to 2^-134 of the value is lost, which counts where the other operand is huge or the sum itself that small.  A
+// workgroup whose own rows (Q; dO; K, V in dK/dV) are out of range (beyond_split), or with results that are not finite or that small
+// (ResultRange), therefore forms its results again with v_mfma_f32_32x32x2_f32, which multiplies operands as they are.  Looking
+// at every staged value instead cost 1 % (forward) to 4 % (backward) of the time.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -64,6 +74,84 @@ __device__ __forceinline__ split8 split_8(float x0, float x1, float x2, float x3
 __device__ __forceinline__ split8 split_8(const float4 &a, const float4 &b)
 {
     return split_8(a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w);
+}
+
+// Whether rows that a wave (or four of them) holds have a nonzero value up to 2^-110, or one from 2^100 on; a scalar.  A bf16
+// code c, sign dropped and one subtracted (2 c - 1 in 16 bits), puts zero above everything else, so that a running minimum finds
+// the smallest nonzero value.  Called where the wave waits for memory anyway.
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+template <int STEPS>
+__device__ __forceinline__ bool beyond_split(const split8 *rows)
+{
+    u16x2 least = {0xffff, 0xffff}, most = {0, 0};
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+        const uint32_t hi[4] = {rows[i].hi.x, rows[i].hi.y, rows[i].hi.z, rows[i].hi.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2, hi[j]) * (uint16_t)2 - (uint16_t)1);
+            most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, hi[j] & 0x7fff7fffu));
+        }
+    }
+    return __any(min(least.x, least.y) <= 2 * ((127 - 110) << 7) - 1 || max(most.x, most.y) >= (127 + 100) << 7);
+}
+
+// The range of results: 0 * x is NaN where x is not finite, and the bits of |x| less one put zero above everything else.
+struct ResultRange {
+    float mark = 0.f;
+    uint32_t least = 0xffffffffu;
+    __device__ __forceinline__ void take(const f32x16 &x)
+    {
+        float m[4] = {mark, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            m[r & 3] = fmaf(x[r], 0.f, m[r & 3]);
+            least = min(least, (__float_as_uint(x[r]) << 1) - 1u);
+        }
+        mark = (m[0] + m[1]) + (m[2] + m[3]);
+    }
+    __device__ __forceinline__ void take(const float4 &x) { take(x.x); take(x.y); take(x.z); take(x.w); }
+    __device__ __forceinline__ void take(float x)
+    {
+        mark = fmaf(x, 0.f, mark);
+        least = min(least, (__float_as_uint(x) << 1) - 1u);
+    }
+    // not finite, or nonzero and below 2^EXP
+    template <int EXP>
+    __device__ __forceinline__ bool beyond() const { return mark != 0.f || least < ((uint32_t)(127 + EXP) << 24); }
+};
+
+// Whether any wave of the workgroup has something to say; flags: a word per wave, written before and read behind a barrier
+__device__ __forceinline__ void flag_write(uint32_t *flags, int wave, bool mine)
+{
+    const bool any = __any(mine);
+    if ((threadIdx.x & 63) == 0) flags[wave] = any;
+}
+template <int WAVES>
+__device__ __forceinline__ bool flag_read(const uint32_t *flags)
+{
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) any |= flags[w];
+    return __builtin_amdgcn_readfirstlane(any) != 0;
+}
+
+// For the code behind a flag: the lane and a row number that the compiler works out there, instead of keeping what depends on them in
+// registers all through the tile loop.
+__device__ __forceinline__ int fresh_lane() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+__device__ __forceinline__ int fresh(int scalar)
+{
+    asm volatile("" : "+s"(scalar));
+    return scalar;
+}
+
+// c += a . b over 8 channels on the fp32 instruction; lane: row (column) lane % 32, channels 4 (lane / 32) + 0 .. 3
+__device__ __forceinline__ f32x16 mfma_plain(const float4 &a, const float4 &b, f32x16 c)
+{
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, c, 0, 0, 0);
 }
 
 // step 0 .. 5 of c += a . b over 16 channels (32 x 32 result), smallest products first

@@ -46,6 +46,9 @@ struct FlashBwdParams {
 
 constexpr float BWD_LSE_FLOOR = -5e29f;  // lse at or below: the row saw no key (cuda_flash_train.rs:206)
 constexpr float BWD_LOG2E = 1.44269504088896340736f;
+// Gradients below 2^-80 are formed on the fp32 instruction: dS = P (dP - D) is split as well, and has lost no bit that counts in
+// sums above that.
+constexpr int BWD_TINY = -80;
 
 // D[bh, i] = O[i] . dO[i], by D / 4 lanes of a wave, 16 bytes of the row each; their partial sums are added by a fixed
 // butterfly.  Rows row0, row0 + 1, ... by lane group of the workgroup (D = 64: 16 rows, D = 128: 8; a wave per row, 4 bytes
@@ -114,13 +117,13 @@ template <int D, bool SPLIT>
 constexpr int bwd_dq_lds_bytes()
 {
     constexpr int merge = 4 * 32 * (D + 4) * 4, slabs = 4 * 2 * SplitTile<D>::BYTES;
-    return SPLIT ? (slabs > merge ? slabs : merge) : 5 * SplitTile<D>::BYTES;
+    return (SPLIT ? (slabs > merge ? slabs : merge) : 5 * SplitTile<D>::BYTES) + 16;  // and a flag per wave
 }
 template <int D, bool SPLIT>
 constexpr int bwd_dkv_lds_bytes()
 {
     constexpr int merge = 4 * 2 * 32 * (D + 4) * 4, slabs = 4 * (2 * SplitTile<D>::BYTES + 256);
-    return SPLIT ? (slabs > merge ? slabs : merge) : 6 * SplitTile<D>::BYTES + 3 * 256;
+    return (SPLIT ? (slabs > merge ? slabs : merge) : 6 * SplitTile<D>::BYTES + 3 * 256) + 16;  // and a flag per wave
 }
 
 // 16 values per lane of a product of the first kind: c += A rows . B, A a tile in LDS
@@ -144,6 +147,131 @@ __device__ __forceinline__ void mul_cols(const unsigned char *tile, const int (&
         for (int db = 0; db < D / 32; ++db) {
             const int o = db * 2048 + ks * 1024;
             acc[db] = mfma_split(SplitTile<D>::get_col(tile, c_addr[0] + o, c_addr[1] + o), b[ks], acc[db]);
+        }
+}
+
+// dQ of 32 queries, and dK / dV of 32 keys, by one wave on v_mfma_f32_32x32x2_f32, which takes infinities and values at either
+// end of the range as they are: for the workgroups whose operands are not the sum of three bf16 values (f32_split.h).  Operands
+// straight from memory.
+template <int D, bool CAUSAL>
+__device__ __forceinline__ void bwd_dq_plain(const FlashBwdParams &p, const float *kp, const float *vp, int bh, int wq0, int kend)
+{
+    constexpr int DB = D / 32;
+    const int lane = fresh_lane(), i32 = lane & 31, h = lane >> 5;
+    const int N = p.N, q_row = wq0 + i32, rr = min(q_row, N - 1);
+    if (wq0 >= N) return;
+    const size_t qoff = ((size_t)bh * N + rr) * D + 4 * h;
+    float4 q[D / 8], o[D / 8];
+#pragma unroll
+    for (int c = 0; c < D / 8; ++c) {
+        q[c] = *(const float4 *)(p.q + qoff + 8 * c);
+        o[c] = *(const float4 *)(p.dout + qoff + 8 * c);
+    }
+    const float lse = p.lse[(size_t)bh * N + rr], di = p.delta[(size_t)bh * N + rr];
+    const bool live = lse > BWD_LSE_FLOOR;
+    const float c2 = p.scale * BWD_LOG2E, lse2 = lse * BWD_LOG2E;
+    f32x16_t acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+    const int all = (kend + F32_BK - 1) / F32_BK, tiles = CAUSAL ? min(all, wq0 / F32_BK + 1) : all;
+#pragma clang loop unroll(disable)
+    for (int it = 0; it < tiles; ++it) {
+        const int k0 = it * F32_BK;
+        const size_t off = (size_t)min(k0 + i32, kend - 1) * D + 4 * h;
+        f32x16_t s, dp;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < D / 8; ++c) {
+            s = mfma_plain(*(const float4 *)(kp + off + 8 * c), q[c], s);
+            dp = mfma_plain(*(const float4 *)(vp + off + 8 * c), o[c], dp);
+        }
+        // step r multiplies key 8 (r / 4) + 4 h + r % 4
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3), kk = min(key, kend - 1);
+            float x = fmaf(s[r], c2, -lse2);
+            if (p.mask != nullptr) x = fmaf(p.mask[(size_t)rr * N + kk], BWD_LOG2E, x);
+            const bool dead = key >= kend || (CAUSAL && key > q_row) || !live;
+            const float ds = dead ? 0.f : __builtin_amdgcn_exp2f(x) * (dp[r] - di) * p.scale;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+                acc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(key < kend ? kp[(size_t)kk * D + 32 * db + i32] : 0.f, ds, acc[db], 0, 0, 0);
+        }
+    }
+    if (q_row >= N) return;
+    float *op = p.dq + ((size_t)bh * N + q_row) * D;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *(float4 *)(op + db * 32 + 8 * g + 4 * h) = make_float4(acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]);
+}
+
+template <int D, bool CAUSAL>
+__device__ __forceinline__ void bwd_dkv_plain(const FlashBwdParams &p, int b, int kvh, int wk0, int kvl)
+{
+    constexpr int DB = D / 32;
+    const int lane = fresh_lane(), i32 = lane & 31, h = lane >> 5;
+    const int N = p.N, key = wk0 + i32, jj = min(key, N - 1), group = p.Hq / p.Hkv;
+    if (wk0 >= N) return;
+    const size_t koff = (((size_t)b * p.Hkv + kvh) * N + jj) * D + 4 * h;
+    float4 k[D / 8], v[D / 8];
+#pragma unroll
+    for (int c = 0; c < D / 8; ++c) {
+        k[c] = *(const float4 *)(p.k + koff + 8 * c);
+        v[c] = *(const float4 *)(p.v + koff + 8 * c);
+    }
+    const float c2 = p.scale * BWD_LOG2E;
+    f32x16_t dk[DB], dv[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.f;
+    const int qt0 = CAUSAL ? wk0 / F32_BK : 0, per_head = (N + F32_BK - 1) / F32_BK - qt0;
+    const int steps = wk0 < kvl ? group * per_head : 0;
+#pragma clang loop unroll(disable)
+    for (int st = 0; st < steps; ++st) {
+        const size_t row0 = ((size_t)b * p.Hq + (size_t)kvh * group + st / per_head) * N;  // of the head
+        const int q0 = (qt0 + st % per_head) * F32_BK;
+        const size_t off = (row0 + min(q0 + i32, N - 1)) * D + 4 * h;
+        f32x16_t s, dp;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < D / 8; ++c) {
+            s = mfma_plain(*(const float4 *)(p.q + off + 8 * c), k[c], s);
+            dp = mfma_plain(*(const float4 *)(p.dout + off + 8 * c), v[c], dp);
+        }
+        // step r multiplies query 8 (r / 4) + 4 h + r % 4 of the tile
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int qi = q0 + 8 * (r >> 2) + 4 * h + (r & 3), qq = min(qi, N - 1);
+            const float lse = p.lse[row0 + qq];
+            float x = fmaf(s[r], c2, -lse * BWD_LOG2E);
+            if (p.mask != nullptr) x = fmaf(p.mask[(size_t)qq * N + jj], BWD_LOG2E, x);
+            const bool dead = qi >= N || key >= kvl || (CAUSAL && key > qi) || !(lse > BWD_LSE_FLOOR);
+            const float pr = dead ? 0.f : __builtin_amdgcn_exp2f(x);
+            const float ds = dead ? 0.f : pr * (dp[r] - p.delta[row0 + qq]) * p.scale;
+            const size_t at = (row0 + qq) * D + i32;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                dv[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(qi < N ? p.dout[at + 32 * db] : 0.f, pr, dv[db], 0, 0, 0);
+                dk[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(qi < N ? p.q[at + 32 * db] : 0.f, ds, dk[db], 0, 0, 0);
+            }
+        }
+    }
+    if (key >= N) return;
+    const size_t out = (((size_t)b * p.Hkv + kvh) * N + key) * D;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int d = db * 32 + 8 * g + 4 * h;
+            *(float4 *)(p.dk + out + d) = make_float4(dk[db][4 * g], dk[db][4 * g + 1], dk[db][4 * g + 2], dk[db][4 * g + 3]);
+            *(float4 *)(p.dv + out + d) = make_float4(dv[db][4 * g], dv[db][4 * g + 1], dv[db][4 * g + 2], dv[db][4 * g + 3]);
         }
 }
 
@@ -210,6 +338,7 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         qr[s] = split_8(*(const float4 *)(p.q + qoff + 16 * s), *(const float4 *)(p.q + qoff + 16 * s + 4));
         dor[s] = split_8(*(const float4 *)(p.dout + qoff + 16 * s), *(const float4 *)(p.dout + qoff + 16 * s + 4));
     }
+    const bool beyond = beyond_split<KSTEPS>(qr) || beyond_split<KSTEPS>(dor);
     // P = exp(x - lse) as v_exp_f32 (base 2) of x * log2(e) - lse * log2(e); a row that saw no key has P = 0
     const float c2 = p.scale * BWD_LOG2E, lse2 = lse > BWD_LSE_FLOOR ? lse * BWD_LOG2E : __builtin_inff();
 
@@ -379,6 +508,8 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         }
     }
 
+    uint32_t *flags = (uint32_t *)(lds + bwd_dq_lds_bytes<D, SPLIT>() - 16);
+    ResultRange results;
     if constexpr (SPLIT) {
         // the waves' partial sums, each as [32 queries][ROW]
         constexpr int ROW = D + 4, SLAB = 32 * ROW;
@@ -396,18 +527,29 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         constexpr int CPT = D / (NW * 2);
         static_assert(CPT % 4 == 0, "whole float4s per thread");
         const int q = tid & 31, cg = tid >> 5;
+        float4 sum[CPT / 4];
+#pragma unroll
+        for (int c = 0; c < CPT / 4; ++c) {
+            sum[c] = *(const float4 *)&part[q * ROW + cg * CPT + 4 * c];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) {
+                const float4 x = *(const float4 *)&part[w * SLAB + q * ROW + cg * CPT + 4 * c];
+                sum[c].x += x.x; sum[c].y += x.y; sum[c].z += x.z; sum[c].w += x.w;
+            }
+            results.take(sum[c]);
+        }
+        // operands that are not the sum of three bf16 values
+        flag_write(flags, wave, results.beyond<BWD_TINY>() || beyond);
+        __syncthreads();
+        if (__builtin_expect(flag_read<NW>(flags), 0)) {
+            if (wave == 0) bwd_dq_plain<D, CAUSAL>(p, kp, vp, bh, fresh(wq0), kend);
+            return;
+        }
         if (qblk + q < N) {
             float *op = p.dq + ((size_t)bh * N + qblk + q) * D + cg * CPT;
 #pragma unroll
-            for (int c = 0; c < CPT; c += 4) {
-                float4 sum = *(const float4 *)&part[q * ROW + cg * CPT + c];
-#pragma unroll
-                for (int w = 1; w < NW; ++w) {
-                    const float4 x = *(const float4 *)&part[w * SLAB + q * ROW + cg * CPT + c];
-                    sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
-                }
-                *(float4 *)(op + c) = make_float4(sum.x * p.scale, sum.y * p.scale, sum.z * p.scale, sum.w * p.scale);
-            }
+            for (int c = 0; c < CPT / 4; ++c)
+                *(float4 *)(op + 4 * c) = make_float4(sum[c].x * p.scale, sum[c].y * p.scale, sum[c].z * p.scale, sum[c].w * p.scale);
         }
         return;
     }
@@ -419,6 +561,15 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
             for (int g = 0; g < 4; ++g)
                 *(float4 *)(op + db * 32 + 8 * g + 4 * h) = make_float4(acc[db][4 * g] * p.scale, acc[db][4 * g + 1] * p.scale,
                                                                         acc[db][4 * g + 2] * p.scale, acc[db][4 * g + 3] * p.scale);
+    }
+    // operands that are not the sum of three bf16 values: the results are formed again, by the lanes that stored them
+#pragma unroll
+    for (int db = 0; db < DB; ++db) results.take(acc[db]);
+    flag_write(flags, wave, results.beyond<BWD_TINY>() || beyond);
+    __syncthreads();
+    if (__builtin_expect(flag_read<NW>(flags), 0)) {
+        wait_vmem_le<0>();
+        bwd_dq_plain<D, CAUSAL>(p, kp, vp, bh, fresh(wq0), kend);
     }
 }
 
@@ -519,6 +670,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
             vr[s] = split_8(*(const float4 *)(p.v + off + 16 * s), *(const float4 *)(p.v + off + 16 * s + 4));
         }
     }
+    const bool beyond = beyond_split<KSTEPS>(kr) || beyond_split<KSTEPS>(vr);
 
     // S = Q K^T and dP = dO V^T: lane = key, register r = query 8 (r / 4) + 4 h + r % 4 of the tile
     f32x16_t s, dp;
@@ -726,6 +878,8 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
         }
     }
 
+    uint32_t *flags = (uint32_t *)(lds + bwd_dkv_lds_bytes<D, SPLIT>() - 16);
+    ResultRange results;
     if constexpr (SPLIT) {
         // the waves' partial sums: dK, then dV, each as [32 keys][ROW]
         constexpr int ROW = D + 4, SLAB = 2 * 32 * ROW;
@@ -745,6 +899,27 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
         constexpr int CPT = D / (NW * 2);
         static_assert(CPT % 4 == 0, "whole float4s per thread");
         const int kq = tid & 31, cg = tid >> 5;
+        float4 sum[2][CPT / 4];
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int c = 0; c < CPT / 4; ++c) {
+                float4 &y = sum[half][c];
+                y = *(const float4 *)&part[(half * 32 + kq) * ROW + cg * CPT + 4 * c];
+#pragma unroll
+                for (int w = 1; w < NW; ++w) {
+                    const float4 x = *(const float4 *)&part[w * SLAB + (half * 32 + kq) * ROW + cg * CPT + 4 * c];
+                    y.x += x.x; y.y += x.y; y.z += x.z; y.w += x.w;
+                }
+                results.take(y);
+            }
+        // operands that are not the sum of three bf16 values
+        flag_write(flags, wave, results.beyond<BWD_TINY>() || beyond);
+        __syncthreads();
+        if (__builtin_expect(flag_read<NW>(flags), 0)) {
+            if (wave == 0) bwd_dkv_plain<D, CAUSAL>(p, b, kvh, fresh(wk0), kvl);
+            return;
+        }
         if (kblk + kq < N) {
             const size_t orow = ((size_t)kv_bh * N + kblk + kq) * D + cg * CPT;
 #pragma unroll
@@ -752,14 +927,9 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
                 float *op = (half ? p.dv : p.dk) + orow;
                 const float f = half ? 1.f : p.scale;
 #pragma unroll
-                for (int c = 0; c < CPT; c += 4) {
-                    float4 sum = *(const float4 *)&part[(half * 32 + kq) * ROW + cg * CPT + c];
-#pragma unroll
-                    for (int w = 1; w < NW; ++w) {
-                        const float4 x = *(const float4 *)&part[w * SLAB + (half * 32 + kq) * ROW + cg * CPT + c];
-                        sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
-                    }
-                    *(float4 *)(op + c) = make_float4(sum.x * f, sum.y * f, sum.z * f, sum.w * f);
+                for (int c = 0; c < CPT / 4; ++c) {
+                    const float4 &y = sum[half][c];
+                    *(float4 *)(op + 4 * c) = make_float4(y.x * f, y.y * f, y.z * f, y.w * f);
                 }
             }
         }
@@ -777,6 +947,18 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
                                                    dk[db][4 * g + 3] * p.scale);
                 *(float4 *)(ovp + d) = make_float4(dv[db][4 * g], dv[db][4 * g + 1], dv[db][4 * g + 2], dv[db][4 * g + 3]);
             }
+    }
+    // operands that are not the sum of three bf16 values: the results are formed again, by the lanes that stored them
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        results.take(dk[db]);
+        results.take(dv[db]);
+    }
+    flag_write(flags, wave, results.beyond<BWD_TINY>() || beyond);
+    __syncthreads();
+    if (__builtin_expect(flag_read<NW>(flags), 0)) {
+        wait_vmem_le<0>();
+        bwd_dkv_plain<D, CAUSAL>(p, b, kvh, fresh(wk0), kvl);
     }
 }
 

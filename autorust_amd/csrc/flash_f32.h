@@ -1,4 +1,4 @@
-// fp32 exact-mode FlashAttention forward: no reduced precision anywhere.
+// fp32 exact-mode FlashAttention forward: the accuracy and the range of fp32 arithmetic.
 //
 // Semantics of the reference's scalar kernel (src/runtime/cuda_flash.rs:53-141): fp32 products
 // and sums, fp32 exponentials, finite sentinel -1e30 for masked keys, acc * (l > 0 ? 1/l : 0) at
@@ -57,7 +57,84 @@ constexpr int flash_f32_lds_bytes()
 {
     constexpr int tiles = (QW == 1) ? 0 : KW * (5 * SplitTile<D>::BYTES + 2 * 32 * D * 4);
     constexpr int merge = (KW == 1) ? 0 : QW * KW * (32 * (D + 4) + 64) * 4;
-    return tiles > merge ? tiles : merge;
+    return (tiles > merge ? tiles : merge) + 32;  // and a flag per wave
+}
+
+// 32 queries by one wave on v_mfma_f32_32x32x2_f32, which takes infinities and values at either end of the range as they are:
+// for the workgroups whose operands are not the sum of three bf16 values (f32_split.h).  Operands straight from memory; the
+// softmax keeps the exact running maximum.  Keys past the end count as zero rows, whatever is in memory.
+template <int D, bool CAUSAL>
+__device__ __forceinline__ void flash_f32_plain(const FlashF32Params &p, const float *kp, const float *vp, int b, int head, int bh,
+                                                int wq0, int kend)
+{
+    constexpr int DB = D / 32;
+    const int lane = fresh_lane(), i32 = lane & 31, h = lane >> 5;
+    const int N = p.N, q_row = wq0 + i32;
+    const size_t k_rs = (size_t)p.ks[2];
+    const float c2 = p.scale * LOG2E;
+    float4 q[D / 8];
+    const float *qp = p.q + (size_t)b * p.qs[0] + (size_t)head * p.qs[1] + (size_t)min(q_row, N - 1) * p.qs[2] + 4 * h;
+#pragma unroll
+    for (int c = 0; c < D / 8; ++c) q[c] = *(const float4 *)(qp + 8 * c);
+    const float *m_row = p.mask != nullptr ? p.mask + (size_t)min(q_row, N - 1) * N : nullptr;
+    f32x16_t oacc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
+    float m_run = -1e30f, l_run = 0.f;
+    const int tiles = wq0 >= N ? 0 : CAUSAL ? min((kend + F32_BK - 1) / F32_BK, wq0 / F32_BK + 1) : (kend + F32_BK - 1) / F32_BK;
+#pragma clang loop unroll(disable)
+    for (int it = 0; it < tiles; ++it) {
+        const int k0 = it * F32_BK;
+        const float *krow = kp + (size_t)min(k0 + i32, kend - 1) * k_rs + 4 * h;
+        f32x16_t s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < D / 8; ++c) s = mfma_plain(*(const float4 *)(krow + 8 * c), q[c], s);
+        float x[16], mx = -1e30f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
+            x[r] = s[r] * c2;
+            if (m_row != nullptr) x[r] = fmaf(m_row[min(key, N - 1)], LOG2E, x[r]);
+            if (key >= kend || (CAUSAL && key > q_row)) x[r] = -__builtin_inff();
+            mx = fmaxf(mx, x[r]);
+        }
+        const float m_new = fmaxf(m_run, xhalf_max(mx)), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        float rs = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            x[r] = __builtin_amdgcn_exp2f(x[r] - m_new);
+            rs += x[r];
+        }
+        l_run = l_run * alpha + rs;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+        // step r multiplies key 8 (r / 4) + 4 h + r % 4, the one whose probability the lane holds in register r
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
+            const float *vrow = vp + (size_t)min(key, kend - 1) * k_rs + i32;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+                oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(key < kend ? vrow[32 * db] : 0.f, x[r], oacc[db], 0, 0, 0);
+        }
+    }
+    const float l = xhalf_sum(l_run), inv = l > 0.f ? 1.f / l : 0.f;
+    if (q_row >= N) return;
+    if (p.lse != nullptr && h == 0) p.lse[(size_t)bh * N + q_row] = l > 0.f ? m_run * 0.69314718055994530942f + logf(l) : -1e30f;
+    float *op = p.o + (size_t)b * p.os[0] + (size_t)head * p.os[1] + (size_t)q_row * p.os[2];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *(float4 *)(op + db * 32 + 8 * g + 4 * h) = make_float4(oacc[db][4 * g] * inv, oacc[db][4 * g + 1] * inv,
+                                                                    oacc[db][4 * g + 2] * inv, oacc[db][4 * g + 3] * inv);
 }
 
 // The kernel body.  lds: flash_f32_lds_bytes<D, QW, KW>() bytes of workgroup memory, 16-byte
@@ -125,6 +202,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
     // Q: this lane's part of its query row as matrix operands (rows past N read row N-1; never stored)
     // Head size 128, one wave per SIMD: it is split once the first tiles have been requested, one memory round trip, not two,
     // before the first product.
+    bool q_beyond = false;  // a query of this wave is out of the range that can be split
     split8 qr[KSTEPS];
     float4 q_raw[2 * KSTEPS];
     {
@@ -345,6 +423,8 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                         first[j][t][1] = *(const float4 *)(src[j] + 16);
                     }
             if (Q_LATE) split_q();
+            ARHIP_FENCE();
+            q_beyond = beyond_split<KSTEPS>(qr);
 #pragma unroll
             for (int j = 0; j < PER_THREAD; ++j) {
 #pragma unroll
@@ -526,6 +606,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
             if constexpr (HAS_MASK) fetch_mask(kg * F32_BK);
             fetch_v(kg);
             split_q();
+            q_beyond = beyond_split<KSTEPS>(qr);
         }
         for (int it = kg; it < my_tiles; it += KW) {
             const int k0 = it * F32_BK;
@@ -552,6 +633,8 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
     }
 
     const float l_tot = xhalf_sum(l_run);
+    uint32_t *flags = (uint32_t *)(lds + flash_f32_lds_bytes<D, QW, KW>() - 32);
+    ResultRange o_range;
     if constexpr (KW > 1) {
         // ---- merge the key groups' partial results ----
         // slab of wave w: O_w as [32 queries][D + 4], then m_w[32], l_w[32]
@@ -592,6 +675,16 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 acc[c] += x.x * f; acc[c + 1] += x.y * f; acc[c + 2] += x.z * f; acc[c + 3] += x.w * f;
             }
         }
+        // operands that are not the sum of three bf16 values
+        o_range.take(l);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) o_range.take(acc[c]);
+        flag_write(flags, wave, o_range.beyond<-100>() || q_beyond);
+        __syncthreads();
+        if (__builtin_expect(flag_read<QW * KW>(flags), 0)) {
+            if (kg == 0) flash_f32_plain<D, CAUSAL>(p, kp, vp, b, head, bh, fresh(wq0), kend);
+            return;
+        }
         const float inv = (l > 0.f) ? 1.f / l : 0.f;
         if (row < N) {
             if (p.lse != nullptr && cg == 0) p.lse[(size_t)bh * N + row] = (l > 0.f) ? m * LN2 + logf(l) : -1e30f;
@@ -615,6 +708,16 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 *(float4 *)(op + d) = make_float4(oacc[db][4 * g] * inv, oacc[db][4 * g + 1] * inv,
                                                   oacc[db][4 * g + 2] * inv, oacc[db][4 * g + 3] * inv);
             }
+    }
+    // operands that are not the sum of three bf16 values: the results are formed again, by the lanes that stored them
+    o_range.take(l_tot);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o_range.take(oacc[db]);
+    flag_write(flags, wave, o_range.beyond<-100>() || q_beyond);
+    __syncthreads();
+    if (__builtin_expect(flag_read<QW * KW>(flags), 0)) {
+        wait_vmem_le<0>();
+        flash_f32_plain<D, CAUSAL>(p, kp, vp, b, head, bh, fresh(wq0), kend);
     }
 }
 
