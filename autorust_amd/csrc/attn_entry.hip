@@ -112,8 +112,8 @@ __device__ __forceinline__ void flash_f32_entry(unsigned char *lds, const float 
     p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
     const int wg = linear_wg();
     if (head_dim == 64) {
-        if (causal) flash_f32_body<64, 4, 1, true>(p, lds, wg);
-        else flash_f32_body<64, 4, 1, false>(p, lds, wg);
+        if (causal) flash_f32_body<64, 4, 1, true, false, true>(p, lds, wg);
+        else flash_f32_body<64, 4, 1, false, false, true>(p, lds, wg);
     } else if (head_dim == 128) {
         if (causal) flash_f32_body<128, 4, 1, true>(p, lds, wg);
         else flash_f32_body<128, 4, 1, false>(p, lds, wg);
@@ -156,8 +156,8 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_fwd(const float *Q, cons
     p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
     const int wg = linear_wg();
     if (head_dim == 64) {
-        if (causal) flash_f32_body<64, 4, 1, true>(p, lds, wg);
-        else flash_f32_body<64, 4, 1, false>(p, lds, wg);
+        if (causal) flash_f32_body<64, 4, 1, true, false, true>(p, lds, wg);
+        else flash_f32_body<64, 4, 1, false, false, true>(p, lds, wg);
     } else if (head_dim == 128) {
         if (causal) flash_f32_body<128, 4, 1, true>(p, lds, wg);
         else flash_f32_body<128, 4, 1, false>(p, lds, wg);

@@ -6,6 +6,6 @@
 
 namespace arhip {
 
-void launch_f32_mask(hipStream_t stream, const FlashF32Params &p, int D, bool causal, int form);
+void launch_f32_mask(hipStream_t stream, const FlashF32Params &p, int D, bool causal, int form, bool tile_sums);
 
 }  // namespace arhip

@@ -13,9 +13,10 @@
 //
 // Six bf16 instructions contract 16 channels in 6 x 8 passes where v_mfma_f32_32x32x2_f32 takes 8 x 16, and they
 // run beside the vector ALU, which the fp32 instruction does not: a matrix pipe of 2.7 times the fp32 rate that
-// hides the softmax.  The bf16 instruction sums its 16 products and the accumulator with fewer roundings than
-// eight fp32 steps: measured on N(0,1) operands, against the exact sum and in units of 2^-24 of the sum of
-// magnitudes, root mean square 0.19 per instruction (16 products) against 0.40 per v_mfma_f32_32x32x2_f32 (2 products).
+// hides the softmax.  Rounding, measured against the exact sum: a sum of 16 products from zero on N(0,1) operands is off by 0.19
+// (root mean square, in units of 2^-24 of the sum of magnitudes) per bf16 instruction, 2 products by 0.40 per fp32 one; but where
+// the accumulator is much larger than the products, by 0.41 units in its last place per bf16 instruction and 0.29 per fp32 one.
+// A long sum over 32-row tiles is rounded 12 times a tile here and 16 times there: variances of 2.0 and 1.3.
 // Subnormal operands are multiplied as such.
 //
 // The three parts exist where hi does not round to infinity (|x| < 3.3962e38) and lo needs no bit below the smallest bf16
@@ -38,6 +39,10 @@ namespace arhip {
 // 8 consecutive elements of an operand row as the three parts of the matrix operand of one lane
 struct split8 {
     uint4 hi, mid, lo;
+};
+
+struct split4 {  // the same of 4 elements
+    uint2 hi, mid, lo;
 };
 
 // First (hi) or second (mid, lo) step of splitting a pair; a and b are left with the residuals.  The empty assembly keeps
@@ -196,6 +201,12 @@ struct SplitTile {
         *(uint4 *)(tile + PART + addr) = s.mid;
         *(uint4 *)(tile + 2 * PART + addr) = s.lo;
     }
+    static __device__ __forceinline__ void put(unsigned char *tile, int addr, const split4 &s)
+    {
+        *(uint2 *)(tile + addr) = s.hi;
+        *(uint2 *)(tile + PART + addr) = s.mid;
+        *(uint2 *)(tile + 2 * PART + addr) = s.lo;
+    }
     // operand rows: lane = row i32, channels 16 st + 8 h .. + 7.  addr = row_addr(lane, st & 1) + (st / 2) * 2048
     static __device__ __forceinline__ int row_addr(int i32, int h, int odd)
     {
@@ -268,18 +279,18 @@ __device__ __forceinline__ void mfma_region(Mul &&mul, Load &&load, Step &&step)
     });
 }
 
-// Splitting 8 values into an operand, one operation of four pairs at a time: the four instructions of a step are
+// Splitting 8 values into an operand (or 4, where registers are short), one operation of four pairs at a time: the four instructions of a step are
 // independent of each other and of everything since the matrix instruction before last, so a wave that has its SIMD to
 // itself issues them without waiting (a step that runs one pair from conversion to residual costs it twice the time:
 // measured, cycles per matrix instruction with six dependent / independent vector instructions behind it: 60 / 40, with
 // four 44 / 36, with two waves per SIMD 36 / 34).  x is left with the residuals; t is scratch.
 constexpr int SPLIT_STEPS = 11;
-template <int OP>
-__device__ __forceinline__ void split_op(float *x, uint32_t *t, split8 &s)
+template <int OP, typename S>
+__device__ __forceinline__ void split_op(float *x, uint32_t *t, S &s)
 {
     uint32_t *part = (uint32_t *)(OP < 5 ? &s.hi : OP < 10 ? &s.mid : &s.lo);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < (int)sizeof(s.hi) / 4; ++i) {
         constexpr int k = OP % 5;
         if constexpr (k == 0) {
             part[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);

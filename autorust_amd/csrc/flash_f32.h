@@ -151,7 +151,10 @@ __device__ __forceinline__ void flash_f32_plain(const FlashF32Params &p, const f
 // split of P, in the same region.  (Waiting for them there also waits for the K / V tiles requested before, which the
 // next instructions want anyway.)  Without it p.mask is still honoured, every tile taking exact_softmax with 16 scattered
 // loads: B2 H12 N1024 D64 118 us, 45 us without a mask.
-template <int D, int QW, int KW, bool CAUSAL, bool HAS_MASK = false>
+//
+// TILE_SUMS (QW > 1): the products of a key tile are summed from zero and then added to O, which is rounded once per tile instead
+// of with each of its 12 matrix instructions.
+template <int D, int QW, int KW, bool CAUSAL, bool HAS_MASK = false, bool TILE_SUMS = false>
 __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned char *lds, int wg_linear)
 {
     constexpr int T = QW * 64;           // threads staging one tile
@@ -310,7 +313,8 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
         //   R2(n)  O^T += V(n)^T . P(n)^T  (MFMA)  |  this thread's share of K(n+3) and V(n+1) split and written to LDS,
         //                                             P(n+1) = exp2(S(n+1) c2 - m) and its row sum        (VALU)
         // then the check of P(n+1), one barrier, and the next tile.  K(n+3) and V(n+1) were requested from memory one
-        // tile earlier.  With three K tiles and two V tiles in LDS every fragment is read ahead of the matrix
+        // tile earlier.  (With TILE_SUMS a part of the staging is done in R1: R2 adds the products of one 32-channel block to O
+        // while it multiplies the next.)  With three K tiles and two V tiles in LDS every fragment is read ahead of the matrix
         // instruction that uses it, the first of a region in the region before.
         constexpr int PER_THREAD = 2 * Tile::ITEMS / T;  // items of 8 channels a thread stages per tile, half of them K's
         static_assert(2 * Tile::ITEMS % T == 0 && (Tile::ITEMS % T == 0 || T == 2 * Tile::ITEMS), "tile staging must divide evenly");
@@ -348,26 +352,45 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, off offset:16"
                          : : "s"(raw_at + j * 2048 + 1024 - 16), "v"(src[j]) : "memory", "m0");
         };
-        auto read_raw = [&](int j, float (&xi)[8]) __attribute__((always_inline)) {
-            const float4 a = *(const float4 *)(raw + j * 2048), b4 = *(const float4 *)(raw + j * 2048 + 1024);
-            xi[0] = a.x; xi[1] = a.y; xi[2] = a.z; xi[3] = a.w;
-            xi[4] = b4.x; xi[5] = b4.y; xi[6] = b4.z; xi[7] = b4.w;
+        // 8 values of item j, or 4 from 4 half on
+        auto read_raw = [&](int j, int half, float *xi, auto values) __attribute__((always_inline)) {
+#pragma unroll
+            for (int v = 0; v < decltype(values)::value / 4; ++v) {
+                const float4 a = *(const float4 *)(raw + j * 2048 + (half + v) * 1024);
+                xi[4 * v] = a.x; xi[4 * v + 1] = a.y; xi[4 * v + 2] = a.z; xi[4 * v + 3] = a.w;
+            }
         };
         const int r_addr[2] = {Tile::row_addr(i32, h, 0), Tile::row_addr(i32, h, 1)};
         const int c_addr[2] = {Tile::col_addr(lane, 0), Tile::col_addr(lane, 1)};
         SplitFrag fr;
-        // part P of the K fragment of step st / of the V^T fragment i = ks * DB + db
+        // part P of the K fragment of step st / of the V^T fragment i = 2 db + ks
         auto next_k = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
             constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
             fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
         };
         auto next_v = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
             constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
-            const int o = (i % DB) * 2048 + (i / DB) * 1024;
+            const int o = (i >> 1) * 2048 + (i & 1) * 1024;
             fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
         };
 
-        f32x16_t s;
+        // c: products of the block being multiplied and of the one before, not yet in O.  Two waves per SIMD with 128 channels
+        // have registers for one: it is added before the next block begins, while the SIMD's other wave multiplies.
+        constexpr int NC = D == 128 && QW == 8 ? 1 : 2;
+        f32x16_t s, c[NC];
+        const f32x16_t zero = {};
+        c[NC - 1] = zero;
+        auto add_block = [&](auto db, auto part) __attribute__((always_inline)) {  // part 0 .. 3: four values
+            constexpr int d = decltype(db)::value, e = 4 * decltype(part)::value;
+#pragma unroll
+            for (int r = e; r < e + 4; ++r) {
+                oacc[d][r] += c[d % NC][r];
+                asm volatile("" : "+v"(oacc[d][r]));
+            }
+        };
+        // staged items of R1; the others are left to R2, unless it has no registers for them
+        constexpr int STAGE1 = !TILE_SUMS ? 0 : NC == 1 ? PER_THREAD : PER_THREAD / 2;
+        using last_db = std::integral_constant<int, DB - 1>;
         float x[16], rs = 0.f;
         split8 pb[2];
         // P(n) from S(n) where the interleaved softmax does not do: masks, keys past the end, a negative scale, or a row sum
@@ -389,6 +412,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 const float m_new = fmaxf(m_run, mx + 2.0f), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
                 m_run = m_new;
                 l_run *= alpha;
+                if (TILE_SUMS && NC == 2) c[NC - 1] *= alpha;
 #pragma unroll
                 for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -474,7 +498,31 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 if (k1 + F32_BK <= N) fetch_mask(k1);
                 ARHIP_FENCE();
             }
-            mfma_region<KSTEPS, 2 * SPLIT_STEPS + (HAS_MASK ? 8 : 0)>(
+            // A staged item: its arrival and the read, the split, the write and the next request.  (Where registers are short it goes
+            // through them in halves.)
+            constexpr int HALVES = TILE_SUMS && NC == 1 ? 2 : 1, ITEM = 3 + SPLIT_STEPS;
+            // ... and values that fit none are read back in R1, which waits for every transfer in flight: the next ones are
+            // requested behind it
+            constexpr bool LATE = HALVES == 2;
+            std::conditional_t<HALVES == 2, split4, split8> sp;
+            float xi[8 / HALVES], sum[2];
+            auto stage_step = [&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value, j = i / ITEM / HALVES, half = i / ITEM % HALVES, t = i % ITEM;
+                if constexpr (t == 0) {
+                    // in flight behind item j: the rest of this tile pair and what has been requested of the next
+                    if constexpr (half == 0) wait_vmem_le<2 * (PER_THREAD - 1 - (LATE ? j : 0))>();
+                    read_raw(j, half, xi, std::integral_constant<int, 8 / HALVES>{});
+                } else if constexpr (t == ITEM - 1) {
+                    Tile::put(put_tile(j, n), put_at[j] + 8 * half, sp);
+                    if constexpr (half == HALVES - 1 && !LATE) request(j);
+                } else if constexpr (t >= 2) {
+                    split_op<t - 2>(xi, tmp, sp);
+                }
+            };
+            // staged items of R1 (the others: R2), then the rest of the last tile's products, the split of P and the mask
+            constexpr int C1 = STAGE1 * ITEM * HALVES, PEND = C1 + (TILE_SUMS && NC == 2 ? 4 : 0), SP = PEND + 2 * SPLIT_STEPS, MK = SP + (HAS_MASK ? 8 : 0);
+            constexpr int C2 = PER_THREAD * ITEM * HALVES - C1;
+            mfma_region<KSTEPS, MK + (LATE ? PER_THREAD : 0)>(
                 [&](auto fi, auto mi) __attribute__((always_inline)) {
                     constexpr int f = decltype(fi)::value;
                     s = mfma_split_step<decltype(mi)::value>(fr.template get<(f & 1)>(), qr[f], s);
@@ -486,10 +534,16 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 },
                 [&](auto ic) __attribute__((always_inline)) {
                     constexpr int i = decltype(ic)::value;
-                    if constexpr (i < 2 * SPLIT_STEPS) {
-                        split_p(ic);
+                    if constexpr (i < C1) {
+                        stage_step(ic);
+                    } else if constexpr (i < PEND) {
+                        add_block(last_db{}, std::integral_constant<int, i - C1>{});
+                    } else if constexpr (i < SP) {
+                        split_p(std::integral_constant<int, i - PEND>{});
+                    } else if constexpr (i >= MK) {
+                        request(i - MK);
                     } else {
-                        constexpr int e = 2 * (i - 2 * SPLIT_STEPS);
+                        constexpr int e = 2 * (i - SP);
                         mv[e] = fmaf(mv[e], LOG2E, -m_run);
                         mv[e + 1] = fmaf(mv[e + 1], LOG2E, -m_run);
                         pin(mv[e], mv[e + 1]);
@@ -497,28 +551,30 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 });
             // ---- R2 ----
             const unsigned char *kn = k_ring + (k_cur == 2 ? 0 : k_cur + 1) * Tile::BYTES;
-            split8 sp;
-            float xi[8], sum[2];
-            // a staged item: its arrival and the read, the split, the write and the next request; then the probabilities, two at
-            // a time, and their sum
-            constexpr int ITEM = 3 + SPLIT_STEPS, CONV = ITEM * PER_THREAD, NS = CONV + 20;
-            auto r2_step = [&](auto ic) __attribute__((always_inline)) {
-                constexpr int i = decltype(ic)::value;
-                if constexpr (i < CONV) {
-                    constexpr int j = i / ITEM, t = i % ITEM;
-                    if constexpr (t == 0) {
-                        // in flight behind item j: the rest of this tile pair and what has been requested of the next
-                        wait_vmem_le<2 * (PER_THREAD - 1)>();
-                        read_raw(j, xi);
-                    } else if constexpr (t == ITEM - 1) {
-                        Tile::put(put_tile(j, n), put_at[j], sp);
-                        request(j);
-                    } else if constexpr (t >= 2) {
-                        split_op<t - 2>(xi, tmp, sp);
+            mfma_region<2 * DB, C2 + 20>(
+                [&](auto fi, auto mi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, m = decltype(mi)::value, db = f >> 1, ks = f & 1;
+                    if constexpr (!TILE_SUMS) {
+                        oacc[db] = mfma_split_step<m>(fr.template get<(f & 1)>(), pb[ks], oacc[db]);
+                    } else {
+                        if constexpr (NC == 1 && db > 0 && ks == 0 && m == 0)
+                            static_for<0, 4>([&](auto part) __attribute__((always_inline)) { add_block(std::integral_constant<int, db - 1>{}, part); });
+                        c[db % NC] = mfma_split_step<m>(fr.template get<(f & 1)>(), pb[ks], ks == 0 && m == 0 ? zero : c[db % NC]);
+                        if constexpr (NC == 2 && db > 0 && ks == 0 && m >= 2)
+                            add_block(std::integral_constant<int, db - 1>{}, std::integral_constant<int, m - 2>{});
                     }
-                } else {
-                    constexpr int t = i - CONV;
-                    if constexpr (t < 16) {
+                },
+                [&](auto fi, auto pi) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value;
+                    if constexpr (f < 2 * DB) next_v(fi, pi, vt, f);
+                    else next_k(fi, pi, kn, 0);
+                },
+                // the probabilities, two at a time, and their sum
+                [&](auto ic) __attribute__((always_inline)) {
+                    constexpr int t = decltype(ic)::value - C2;
+                    if constexpr (t < 0) {
+                        stage_step(std::integral_constant<int, t + C2 + C1>{});
+                    } else if constexpr (t < 16) {
                         constexpr int e = (t >> 1) * 2;
                         if constexpr ((t & 1) == 0) {
                             x[e] = fmaf(s[e], c2, HAS_MASK ? mv[e] : -m_run);
@@ -533,19 +589,8 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                         sum[g & 1] = (g < 2 ? 0.f : sum[g & 1]) + ((x[4 * g] + x[4 * g + 1]) + (x[4 * g + 2] + x[4 * g + 3]));
                         asm volatile("" : "+v"(sum[g & 1]));
                     }
-                }
-            };
-            mfma_region<2 * DB, NS>(
-                [&](auto fi, auto mi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value;
-                    oacc[f % DB] = mfma_split_step<decltype(mi)::value>(fr.template get<(f & 1)>(), pb[f / DB], oacc[f % DB]);
-                },
-                [&](auto fi, auto pi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value;
-                    if constexpr (f < 2 * DB) next_v(fi, pi, vt, f);
-                    else next_k(fi, pi, kn, 0);
-                },
-                r2_step);
+                });
+            if constexpr (TILE_SUMS && NC == 1) static_for<0, 4>([&](auto part) __attribute__((always_inline)) { add_block(last_db{}, part); });
             rs = sum[0] + sum[1];
 #pragma unroll
             for (int j = 0; j < PER_THREAD; ++j) next_tile(j, item_is_v(j) ? n + 3 : n + 5);
@@ -556,12 +601,16 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
         }
         if (mine > 0) {
             // the last tile of this wave: no S to look ahead for
+            if (TILE_SUMS && NC == 2) oacc[DB - 1] += c[NC - 1];
             static_for<0, 2 * SPLIT_STEPS>(split_p);
             const unsigned char *vt = v_ring + (n & 1) * Tile::BYTES;
 #pragma unroll
-            for (int f = 0; f < 2 * DB; ++f) {
-                const int o = (f % DB) * 2048 + (f / DB) * 1024;
-                oacc[f % DB] = mfma_split(Tile::get_col(vt, c_addr[0] + o, c_addr[1] + o), pb[f / DB], oacc[f % DB]);
+            for (int db = 0; db < DB; ++db) {
+                const int o = db * 2048;
+                f32x16_t t = mfma_split(Tile::get_col(vt, c_addr[0] + o, c_addr[1] + o), pb[0], TILE_SUMS ? zero : oacc[db]);
+                t = mfma_split(Tile::get_col(vt, c_addr[0] + o + 1024, c_addr[1] + o + 1024), pb[1], t);
+                if (TILE_SUMS) oacc[db] += t;
+                else oacc[db] = t;
             }
         }
         // under the causal mask a wave is done before others of its workgroup: it still stages tiles for them
@@ -570,7 +619,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
             for (int j = 0; j < PER_THREAD; ++j) {
                 float xi[8];
                 wait_vmem_le<2 * (PER_THREAD - 1)>();
-                read_raw(j, xi);
+                read_raw(j, 0, xi, std::integral_constant<int, 8>{});
                 Tile::put(put_tile(j, n), put_at[j], split_8(xi[0], xi[1], xi[2], xi[3], xi[4], xi[5], xi[6], xi[7]));
                 request(j);
                 next_tile(j, item_is_v(j) ? n + 3 : n + 5);
@@ -727,11 +776,11 @@ constexpr int flash_f32_waves_per_simd()
     return QW * KW == 8 ? 2 : (D == 64 ? 2 : (KW == 1 ? 2 : 1));
 }
 
-template <int D, int QW, int KW, bool CAUSAL, bool HAS_MASK = false>
+template <int D, int QW, int KW, bool CAUSAL, bool HAS_MASK = false, bool TILE_SUMS = false>
 __global__ void __launch_bounds__(QW * KW * 64, (flash_f32_waves_per_simd<D, QW, KW>())) flash_f32_kernel(const FlashF32Params p)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<D, QW, KW>()];
-    flash_f32_body<D, QW, KW, CAUSAL, HAS_MASK>(p, lds, (int)blockIdx.x);
+    flash_f32_body<D, QW, KW, CAUSAL, HAS_MASK, TILE_SUMS>(p, lds, (int)blockIdx.x);
 }
 
 }  // namespace arhip
