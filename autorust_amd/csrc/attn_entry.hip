@@ -228,6 +228,7 @@ __device__ __forceinline__ FlashBwdParams bwd_params(const float *Q, const float
     p.nt = (int)gridDim.x;
     p.total_q = p.total_kv = (int)(gridDim.x * gridDim.y);
     p.lpt_q = p.lpt_kv = (int)gridDim.y;  // causal: longest tile first over all heads
+    p.halves = p.total_q < 2 * 256;
     p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
     return p;
 }

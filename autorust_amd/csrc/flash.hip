@@ -552,6 +552,10 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     const int nt = (int)((N + rows_wg - 1) / rows_wg);
     p.nt = nt;
     // causal: longest tile first over all heads, so that no head's long tiles are left for the end
+    // Sums in two halves on grids of fewer than two workgroups per compute unit (as f32_tile_sums).  Relative error of dV and us, one
+    // sum / two halves (and log2(e) lse unrounded): B8 H6 N789 D64 6.2e-7 / 5.1e-7 and 214 / 218, B1 H16 N2048 D128 9.3e-7 / 7.7e-7
+    // and 588 / 582, B1 H4 N512 D128 6.1e-7 / 5.3e-7 and 82 / 85
+    p.halves = B * Hkv * ((N + 127) / 128) < 2 * (int64_t)dev->cus;
     p.total_q = (int)(nt * B * Hq);
     p.total_kv = (int)(nt * B * Hkv);
     p.lpt_q = causal ? (int)(B * Hq) : 0;

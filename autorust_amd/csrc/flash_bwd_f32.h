@@ -41,6 +41,7 @@ struct FlashBwdParams {
     int nt;  // tiles per head: query tiles (dQ kernel) or key tiles (dK/dV kernel)
     int total_q, total_kv;  // workgroups in the dQ grid (nt * B * Hq) and in the dK/dV grid (nt * B * Hkv)
     int lpt_q, lpt_kv;  // causal: B * Hq / B * Hkv, and the grids run longest tile first over all heads; else 0
+    int halves;  // 128 rows per workgroup: long sums are formed in two halves (bwd_first_half)
     float scale;
 };
 
@@ -147,6 +148,38 @@ __device__ __forceinline__ void mul_cols(const unsigned char *tile, const int (&
         for (int db = 0; db < D / 32; ++db) {
             const int o = db * 2048 + ks * 1024;
             acc[db] = mfma_split(SplitTile<D>::get_col(tile, c_addr[0] + o, c_addr[1] + o), b[ks], acc[db]);
+        }
+}
+
+// A long sum is rounded with every matrix instruction, by an amount that grows with it.  So the sums over the first half of the
+// tiles go to the place of the result they belong to, and are taken in again at the end, from 16 tiles on (causal, where most rows
+// have shorter sums: from 48).  A third span, read back and added between two tiles, cost 5 to 12 % at head size 128, where it leaves
+// values without a register.  row: the lane's row of the result.
+template <bool CAUSAL>
+__device__ __forceinline__ int bwd_first_half(int tiles, bool halves) { return halves && tiles >= (CAUSAL ? 48 : 16) ? tiles / 2 : 0; }
+template <int D>
+__device__ __forceinline__ void put_aside(float *row, int h, bool in_range, f32x16 (&acc)[D / 32])
+{
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            if (in_range)
+                *(float4 *)(row + db * 32 + 8 * g + 4 * h) =
+                    make_float4(acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+    }
+}
+template <int D>
+__device__ __forceinline__ void take_in(const float *row, int h, f32x16 (&acc)[D / 32])
+{
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const float4 x = *(const float4 *)(row + db * 32 + 8 * g + 4 * h);
+            acc[db][4 * g] += x.x; acc[db][4 * g + 1] += x.y; acc[db][4 * g + 2] += x.z; acc[db][4 * g + 3] += x.w;
         }
 }
 
@@ -339,8 +372,9 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         dor[s] = split_8(*(const float4 *)(p.dout + qoff + 16 * s), *(const float4 *)(p.dout + qoff + 16 * s + 4));
     }
     const bool beyond = beyond_split<KSTEPS>(qr) || beyond_split<KSTEPS>(dor);
-    // P = exp(x - lse) as v_exp_f32 (base 2) of x * log2(e) - lse * log2(e); a row that saw no key has P = 0
-    const float c2 = p.scale * BWD_LOG2E, lse2 = lse > BWD_LSE_FLOOR ? lse * BWD_LOG2E : __builtin_inff();
+    // P = exp(x - lse) as v_exp_f32 (base 2) of x * log2(e) - lse * log2(e), the second product unrounded (rounded, it would shift a
+    // whole row of P by half a unit in its last place); a row that saw no key has P = 0
+    const float c2 = p.scale * BWD_LOG2E, neg_lse = lse > BWD_LSE_FLOOR ? -lse : -__builtin_inff();
 
     f32x16_t acc[DB];
 #pragma unroll
@@ -365,7 +399,7 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         }
     };
     auto make_ds = [&](int r) __attribute__((always_inline)) {
-        ds[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cx, -lse2)) * (dp[r] - di);
+        ds[r] = __builtin_amdgcn_exp2f(fmaf(neg_lse, BWD_LOG2E, s[r] * cx)) * (dp[r] - di);
     };
     // the same in steps 0 .. 23: exponents and exponentials two at a time, then the differences and the products four at a time
     auto ds_step = [&](auto ic) __attribute__((always_inline)) {
@@ -373,7 +407,7 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         if constexpr (i < 16) {
             constexpr int e = (i >> 1) * 2;
 #pragma unroll
-            for (int r = e; r < e + 2; ++r) ds[r] = (i & 1) ? __builtin_amdgcn_exp2f(ds[r]) : fmaf(s[r], cx, -lse2);
+            for (int r = e; r < e + 2; ++r) ds[r] = (i & 1) ? __builtin_amdgcn_exp2f(ds[r]) : fmaf(neg_lse, BWD_LOG2E, s[r] * cx);
             pin(ds[e], ds[e + 1]);
         } else {
             constexpr int e = ((i - 16) >> 1) * 4;
@@ -438,66 +472,74 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         }
         __syncthreads();  // V(0) has been read: its slot is written next
         int k_cur = 0;  // ring slot of K(n)
+        const int half = bwd_first_half<CAUSAL>(my_tiles, p.halves != 0);
         auto slot = [](int k) __attribute__((always_inline)) { return k >= 3 ? k - 3 : k; };
         SplitFrag fr;
         int n = 0;
+        float *aside = p.dq + ((size_t)bh * N + rr) * D;
 #pragma clang loop unroll(disable)
-        for (; n < my_tiles - 1; ++n) {
-            const unsigned char *kt = k_ring + k_cur * Tile::BYTES, *kt1 = k_ring + slot(k_cur + 1) * Tile::BYTES,
-                                *vt1 = v_ring + ((n + 1) & 1) * Tile::BYTES;
-            unsigned char *kt2 = k_ring + slot(k_cur + 2) * Tile::BYTES, *vt2 = v_ring + (n & 1) * Tile::BYTES;
-            auto load_row = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
-                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
-                fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
-            };
-            auto load_col = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
-                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
-                const int o = (i % DB) * 2048 + (i / DB) * 1024;
-                fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
-            };
-            // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
-            static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, kt1, 0); });
-            static_for<0, 4>(split_ds);
-            ARHIP_FENCE();
+        for (int part = half > 0 ? 0 : 1; part < 2; ++part) {
+            const int end = part == 0 ? half : my_tiles - 1;
+#pragma clang loop unroll(disable)
+            for (; n < end; ++n) {
+                const unsigned char *kt = k_ring + k_cur * Tile::BYTES, *kt1 = k_ring + slot(k_cur + 1) * Tile::BYTES,
+                                    *vt1 = v_ring + ((n + 1) & 1) * Tile::BYTES;
+                unsigned char *kt2 = k_ring + slot(k_cur + 2) * Tile::BYTES, *vt2 = v_ring + (n & 1) * Tile::BYTES;
+                auto load_row = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                    fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
+                };
+                auto load_col = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                    const int o = (i % DB) * 2048 + (i / DB) * 1024;
+                    fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
+                };
+                // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
+                static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, kt1, 0); });
+                static_for<0, 4>(split_ds);
+                ARHIP_FENCE();
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-            mfma_region<2 * KSTEPS, 2 * SPLIT_STEPS - 4 + PairStage<D, NW * 64>::STEPS>(
-                [&](auto fi, auto mi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value, m = decltype(mi)::value;
-                    if constexpr (f < KSTEPS) s = mfma_split_step<m>(fr.template get<(f & 1)>(), qr[f], s);
-                    else dp = mfma_split_step<m>(fr.template get<(f & 1)>(), dor[f - KSTEPS], dp);
-                },
-                [&](auto fi, auto pi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value;
-                    if constexpr (f < KSTEPS) load_row(fi, pi, kt1, f);
-                    else if constexpr (f < 2 * KSTEPS) load_row(fi, pi, vt1, f - KSTEPS);
-                    else load_col(fi, pi, kt, 0);
-                },
-                [&](auto ic) __attribute__((always_inline)) {
-                    constexpr int i = decltype(ic)::value;
-                    if constexpr (i < 2 * SPLIT_STEPS - 4) split_ds(std::integral_constant<int, i + 4>{});
-                    else stage.template split_step<i - (2 * SPLIT_STEPS - 4)>(kt2, vt2, tid);
-                });
-            if (n + 3 < ntiles) stage.fetch(kp, vp, tid, (n + 3) * F32_BK, kend - 1);
-            add_mask((n + 1) * F32_BK);
-            // ---- R2 ----
-            mfma_region<2 * DB, 24>(
-                [&](auto fi, auto mi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value;
-                    acc[f % DB] = mfma_split_step<decltype(mi)::value>(fr.template get<(f & 1)>(), db_[f / DB], acc[f % DB]);
-                },
-                [&](auto fi, auto pi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value;
-                    if constexpr (f < 2 * DB) load_col(fi, pi, kt, f);
-                },
-                ds_step);
-            drop_dead((n + 1) * F32_BK);
-            k_cur = slot(k_cur + 1);
-            __syncthreads();
+                for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+                mfma_region<2 * KSTEPS, 2 * SPLIT_STEPS - 4 + PairStage<D, NW * 64>::STEPS>(
+                    [&](auto fi, auto mi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value, m = decltype(mi)::value;
+                        if constexpr (f < KSTEPS) s = mfma_split_step<m>(fr.template get<(f & 1)>(), qr[f], s);
+                        else dp = mfma_split_step<m>(fr.template get<(f & 1)>(), dor[f - KSTEPS], dp);
+                    },
+                    [&](auto fi, auto pi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value;
+                        if constexpr (f < KSTEPS) load_row(fi, pi, kt1, f);
+                        else if constexpr (f < 2 * KSTEPS) load_row(fi, pi, vt1, f - KSTEPS);
+                        else load_col(fi, pi, kt, 0);
+                    },
+                    [&](auto ic) __attribute__((always_inline)) {
+                        constexpr int i = decltype(ic)::value;
+                        if constexpr (i < 2 * SPLIT_STEPS - 4) split_ds(std::integral_constant<int, i + 4>{});
+                        else stage.template split_step<i - (2 * SPLIT_STEPS - 4)>(kt2, vt2, tid);
+                    });
+                if (n + 3 < ntiles) stage.fetch(kp, vp, tid, (n + 3) * F32_BK, kend - 1);
+                add_mask((n + 1) * F32_BK);
+                // ---- R2 ----
+                mfma_region<2 * DB, 24>(
+                    [&](auto fi, auto mi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value;
+                        acc[f % DB] = mfma_split_step<decltype(mi)::value>(fr.template get<(f & 1)>(), db_[f / DB], acc[f % DB]);
+                    },
+                    [&](auto fi, auto pi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value;
+                        if constexpr (f < 2 * DB) load_col(fi, pi, kt, f);
+                    },
+                    ds_step);
+                drop_dead((n + 1) * F32_BK);
+                k_cur = slot(k_cur + 1);
+                __syncthreads();
+            }
+            if (part == 0) put_aside<D>(aside, h, q_row < N, acc);
         }
         if (my_tiles > 0) {
             static_for<0, 2 * SPLIT_STEPS>(split_ds);
             mul_cols<D>(k_ring + k_cur * Tile::BYTES, c_addr, db_, acc);
+            if (half > 0) take_in<D>(aside, h, acc);
         }
         // under the causal mask a wave is done before others of its workgroup: it still stages tiles for them
         for (; n < ntiles - 1; ++n) {
@@ -633,7 +675,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
         const size_t off = step_head(st) * N * D;
         to.fetch(p.q + off, p.dout + off, stid, step_q0(st), N - 1);
     };
-    // base-2 units: P = 2^(x log2(e) - lse log2(e)); rows that saw no key (and rows past the end) have P = 0
+    // -lse; rows that saw no key (and rows past the end) have P = 0
     auto fetch_stats = [&](int st, int to = 0) __attribute__((always_inline)) {
         if (stid < F32_BK) {
             const size_t at = step_head(st) * N + min(step_q0(st) + stid, N - 1);
@@ -644,7 +686,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
     auto put_stats = [&](float *stat, int st, int from = 0) __attribute__((always_inline)) {
         if (stid < F32_BK) {
             const bool live = step_q0(st) + stid < N;
-            stat[stid] = live && st_l[from] > BWD_LSE_FLOOR ? st_l[from] * BWD_LOG2E : __builtin_inff();
+            stat[stid] = live && st_l[from] > BWD_LSE_FLOOR ? -st_l[from] : -__builtin_inff();
             stat[32 + stid] = live ? st_d[from] : 0.f;
         }
     };
@@ -695,7 +737,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
             s[r] = fmaf(p.mask[(size_t)qi * N + jj], BWD_LOG2E, s[r] * c2);
         }
     };
-    auto make_p = [&](int r) __attribute__((always_inline)) { pr[r] = __builtin_amdgcn_exp2f(fmaf(s[r], cx, -stat_of(r))); };
+    auto make_p = [&](int r) __attribute__((always_inline)) { pr[r] = __builtin_amdgcn_exp2f(fmaf(stat_of(r), BWD_LOG2E, s[r] * cx)); };
     auto make_ds = [&](int r) __attribute__((always_inline)) { ds[r] = pr[r] * (dp[r] - stat_of(r)); };
     // keys past the key length or below the diagonal have P = 0
     auto drop_dead = [&](int q0) __attribute__((always_inline)) {
@@ -772,95 +814,109 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
             make_all(step_q0(0), stats);
         }
         int cur = 0;  // ring slot of step n
+        const int half = bwd_first_half<CAUSAL>(mine, p.halves != 0);
+        float *k_aside = p.dk + ((size_t)kv_bh * N + jj) * D, *v_aside = p.dv + ((size_t)kv_bh * N + jj) * D;
         auto slot = [](int k) __attribute__((always_inline)) { return k >= 3 ? k - 3 : k; };
         SplitFrag fr;
         int n = 0;
 #pragma clang loop unroll(disable)
-        for (; n < mine - 1; ++n) {
-            const int s1 = slot(cur + 1), s2 = slot(cur + 2);
-            const unsigned char *qt = q_ring + cur * Tile::BYTES, *ot = o_ring + cur * Tile::BYTES;
-            const unsigned char *qt1 = q_ring + s1 * Tile::BYTES, *ot1 = o_ring + s1 * Tile::BYTES;
-            unsigned char *qt2 = q_ring + s2 * Tile::BYTES, *ot2 = o_ring + s2 * Tile::BYTES;
-            auto load_row = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
-                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
-                fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
-            };
-            auto load_col = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
-                constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
-                const int o = (i % DB) * 2048 + (i / DB) * 1024;
-                fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
-            };
-            // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
-            static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, qt1, 0); });
-            static_for<0, 4>(split_p);
-            ARHIP_FENCE();
+        for (int part = half > 0 ? 0 : 1; part < 2; ++part) {
+            const int end = part == 0 ? half : mine - 1;
+#pragma clang loop unroll(disable)
+            for (; n < end; ++n) {
+                const int s1 = slot(cur + 1), s2 = slot(cur + 2);
+                const unsigned char *qt = q_ring + cur * Tile::BYTES, *ot = o_ring + cur * Tile::BYTES;
+                const unsigned char *qt1 = q_ring + s1 * Tile::BYTES, *ot1 = o_ring + s1 * Tile::BYTES;
+                unsigned char *qt2 = q_ring + s2 * Tile::BYTES, *ot2 = o_ring + s2 * Tile::BYTES;
+                auto load_row = [&](auto fi, auto pi, const unsigned char *tile, int st) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                    fr.template set<(f & 1), P>(Tile::template get_row_part<P>(tile, r_addr[st & 1] + (st >> 1) * 2048));
+                };
+                auto load_col = [&](auto fi, auto pi, const unsigned char *tile, int i) __attribute__((always_inline)) {
+                    constexpr int f = decltype(fi)::value, P = decltype(pi)::value;
+                    const int o = (i % DB) * 2048 + (i / DB) * 1024;
+                    fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
+                };
+                // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
+                static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, qt1, 0); });
+                static_for<0, 4>(split_p);
+                ARHIP_FENCE();
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-            mfma_region<2 * KSTEPS, 4 * SPLIT_STEPS - 4>(
-                [&](auto fi, auto mi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value, m = decltype(mi)::value;
-                    if constexpr (f < KSTEPS) s = mfma_split_step<m>(fr.template get<(f & 1)>(), kr[f], s);
-                    else dp = mfma_split_step<m>(fr.template get<(f & 1)>(), vr[f - KSTEPS], dp);
-                },
-                [&](auto fi, auto pi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value;
-                    if constexpr (f < KSTEPS) load_row(fi, pi, qt1, f);
-                    else if constexpr (f < 2 * KSTEPS) load_row(fi, pi, ot1, f - KSTEPS);
-                    else load_col(fi, pi, ot, 0);
-                },
-                [&](auto ic) __attribute__((always_inline)) {
-                    constexpr int i = decltype(ic)::value;
-                    if constexpr (i < 2 * SPLIT_STEPS - 4) split_p(std::integral_constant<int, i + 4>{});
-                    else split_ds(std::integral_constant<int, i - (2 * SPLIT_STEPS - 4)>{});
-                });
-            add_mask(step_q0(n + 1));
-            read_stats(stats + s1 * 64);
-            // ---- R2 ----
-            constexpr int CONV = decltype(stage)::STEPS;
-            mfma_region<4 * DB, 24 + CONV>(
-                [&](auto fi, auto mi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value, m = decltype(mi)::value, g = f % (2 * DB);
-                    if constexpr (f < 2 * DB) dv[g % DB] = mfma_split_step<m>(fr.template get<(f & 1)>(), pb[g / DB], dv[g % DB]);
-                    else dk[g % DB] = mfma_split_step<m>(fr.template get<(f & 1)>(), db_[g / DB], dk[g % DB]);
-                },
-                [&](auto fi, auto pi) __attribute__((always_inline)) {
-                    constexpr int f = decltype(fi)::value;
-                    if constexpr (f < 2 * DB) load_col(fi, pi, ot, f);
-                    else if constexpr (f < 4 * DB) load_col(fi, pi, qt, f - 2 * DB);
-                },
-                [&](auto ic) __attribute__((always_inline)) {
-                    constexpr int i = decltype(ic)::value;
-                    if constexpr (i < 16) {
-                        constexpr int e = (i >> 1) * 2;
+                for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+                mfma_region<2 * KSTEPS, 4 * SPLIT_STEPS - 4>(
+                    [&](auto fi, auto mi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value, m = decltype(mi)::value;
+                        if constexpr (f < KSTEPS) s = mfma_split_step<m>(fr.template get<(f & 1)>(), kr[f], s);
+                        else dp = mfma_split_step<m>(fr.template get<(f & 1)>(), vr[f - KSTEPS], dp);
+                    },
+                    [&](auto fi, auto pi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value;
+                        if constexpr (f < KSTEPS) load_row(fi, pi, qt1, f);
+                        else if constexpr (f < 2 * KSTEPS) load_row(fi, pi, ot1, f - KSTEPS);
+                        else load_col(fi, pi, ot, 0);
+                    },
+                    [&](auto ic) __attribute__((always_inline)) {
+                        constexpr int i = decltype(ic)::value;
+                        if constexpr (i < 2 * SPLIT_STEPS - 4) split_p(std::integral_constant<int, i + 4>{});
+                        else split_ds(std::integral_constant<int, i - (2 * SPLIT_STEPS - 4)>{});
+                    });
+                add_mask(step_q0(n + 1));
+                read_stats(stats + s1 * 64);
+                // ---- R2 ----
+                constexpr int CONV = decltype(stage)::STEPS;
+                mfma_region<4 * DB, 24 + CONV>(
+                    [&](auto fi, auto mi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value, m = decltype(mi)::value, g = f % (2 * DB);
+                        if constexpr (f < 2 * DB) dv[g % DB] = mfma_split_step<m>(fr.template get<(f & 1)>(), pb[g / DB], dv[g % DB]);
+                        else dk[g % DB] = mfma_split_step<m>(fr.template get<(f & 1)>(), db_[g / DB], dk[g % DB]);
+                    },
+                    [&](auto fi, auto pi) __attribute__((always_inline)) {
+                        constexpr int f = decltype(fi)::value;
+                        if constexpr (f < 2 * DB) load_col(fi, pi, ot, f);
+                        else if constexpr (f < 4 * DB) load_col(fi, pi, qt, f - 2 * DB);
+                    },
+                    [&](auto ic) __attribute__((always_inline)) {
+                        constexpr int i = decltype(ic)::value;
+                        if constexpr (i < 16) {
+                            constexpr int e = (i >> 1) * 2;
 #pragma unroll
-                        for (int r = e; r < e + 2; ++r) pr[r] = (i & 1) ? __builtin_amdgcn_exp2f(pr[r]) : fmaf(s[r], cx, -stat_of(r));
-                        pin(pr[e], pr[e + 1]);
-                        if constexpr (i == 15) read_stats(stats + s1 * 64 + 32);
-                    } else if constexpr (i < 24) {
-                        constexpr int e = ((i - 16) >> 1) * 4;
+                            for (int r = e; r < e + 2; ++r) pr[r] = (i & 1) ? __builtin_amdgcn_exp2f(pr[r]) : fmaf(stat_of(r), BWD_LOG2E, s[r] * cx);
+                            pin(pr[e], pr[e + 1]);
+                            if constexpr (i == 15) read_stats(stats + s1 * 64 + 32);
+                        } else if constexpr (i < 24) {
+                            constexpr int e = ((i - 16) >> 1) * 4;
 #pragma unroll
-                        for (int r = e; r < e + 4; ++r) {
-                            ds[r] = (i & 1) ? pr[r] * ds[r] : dp[r] - stat_of(r);
-                            asm volatile("" : "+v"(ds[r]));
+                            for (int r = e; r < e + 4; ++r) {
+                                ds[r] = (i & 1) ? pr[r] * ds[r] : dp[r] - stat_of(r);
+                                asm volatile("" : "+v"(ds[r]));
+                            }
+                        } else {
+                            stage.template split_step<i - 24>(qt2, ot2, tid);
                         }
-                    } else {
-                        stage.template split_step<i - 24>(qt2, ot2, tid);
-                    }
-                });
-            if (n + 2 < steps) put_stats(stats + s2 * 64, n + 2);
-            if (n + 3 < steps) {
-                fetch_tiles(stage, n + 3);
-                fetch_stats(n + 3);
+                    });
+                if (n + 2 < steps) put_stats(stats + s2 * 64, n + 2);
+                if (n + 3 < steps) {
+                    fetch_tiles(stage, n + 3);
+                    fetch_stats(n + 3);
+                }
+                drop_dead(step_q0(n + 1));
+                cur = s1;
+                __syncthreads();
             }
-            drop_dead(step_q0(n + 1));
-            cur = s1;
-            __syncthreads();
+            if (part == 0) {
+                put_aside<D>(k_aside, h, key < N, dk);
+                put_aside<D>(v_aside, h, key < N, dv);
+            }
         }
         if (mine > 0) {
             static_for<0, 2 * SPLIT_STEPS>(split_p);
             mul_cols<D>(o_ring + cur * Tile::BYTES, c_addr, pb, dv);
             static_for<0, 2 * SPLIT_STEPS>(split_ds);
             mul_cols<D>(q_ring + cur * Tile::BYTES, c_addr, db_, dk);
+            if (half > 0) {
+                take_in<D>(k_aside, h, dk);
+                take_in<D>(v_aside, h, dv);
+            }
         }
         // a wave that is done before others of its workgroup still stages tiles for them
         for (; n < steps - 1; ++n) {
