@@ -94,12 +94,25 @@ __device__ __forceinline__ AttnParams dense_params(const void *q, const void *k,
 }  // namespace
 
 namespace {
+// the forms of a tiling: causal or not, with an additive mask or without
+template <int D, int QW, int KW, bool TILE_SUMS>
+__device__ __forceinline__ void flash_f32_forms(const FlashF32Params &p, unsigned char *lds, int wg, int causal)
+{
+    if (p.mask != nullptr) {
+        if (causal) flash_f32_body<D, QW, KW, true, true, TILE_SUMS>(p, lds, wg);
+        else flash_f32_body<D, QW, KW, false, true, TILE_SUMS>(p, lds, wg);
+    } else {
+        if (causal) flash_f32_body<D, QW, KW, true, false, TILE_SUMS>(p, lds, wg);
+        else flash_f32_body<D, QW, KW, false, false, TILE_SUMS>(p, lds, wg);
+    }
+}
+
 __device__ __forceinline__ void flash_f32_entry(unsigned char *lds, const float *Q, const float *K, const float *V, float *O,
-                                                const float *M, const int *L, int N, int head_dim, int causal, int has_mask,
+                                                float *LSE, const float *M, const int *L, int N, int head_dim, int causal, int has_mask,
                                                 int hq, int hkv)
 {
     FlashF32Params p = {};
-    p.q = Q; p.k = K; p.v = V; p.o = O;
+    p.q = Q; p.k = K; p.v = V; p.o = O; p.lse = LSE;
     p.mask = has_mask ? M : nullptr;
     p.kv_len = L;
     p.Hq = hq; p.Hkv = hkv; p.N = N;
@@ -111,13 +124,8 @@ __device__ __forceinline__ void flash_f32_entry(unsigned char *lds, const float 
     dense(p.os, hq, N, head_dim);
     p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
     const int wg = linear_wg();
-    if (head_dim == 64) {
-        if (causal) flash_f32_body<64, 4, 1, true, false, true>(p, lds, wg);
-        else flash_f32_body<64, 4, 1, false, false, true>(p, lds, wg);
-    } else if (head_dim == 128) {
-        if (causal) flash_f32_body<128, 4, 1, true>(p, lds, wg);
-        else flash_f32_body<128, 4, 1, false>(p, lds, wg);
-    }
+    if (head_dim == 64) flash_f32_forms<64, 4, 1, true>(p, lds, wg, causal);
+    else if (head_dim == 128) flash_f32_forms<128, 4, 1, false>(p, lds, wg, causal);
 }
 }  // namespace
 
@@ -127,7 +135,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_f32(const float *Q, c
                                                                 int has_mask, int hq, int hkv)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<128, 4, 1>()];
-    flash_f32_entry(lds, Q, K, V, O, M, nullptr, N, head_dim, causal, has_mask, hq, hkv);
+    flash_f32_entry(lds, Q, K, V, O, nullptr, M, nullptr, N, head_dim, causal, has_mask, hq, hkv);
 }
 
 extern "C" __global__ void __launch_bounds__(256) ar_flash_f32_lens(const float *Q, const float *K, const float *V, float *O,
@@ -135,7 +143,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_f32_lens(const float 
                                                                      int causal, int has_mask, int hq, int hkv)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<128, 4, 1>()];
-    flash_f32_entry(lds, Q, K, V, O, M, L, N, head_dim, causal, has_mask, hq, hkv);
+    flash_f32_entry(lds, Q, K, V, O, nullptr, M, L, N, head_dim, causal, has_mask, hq, hkv);
 }
 
 extern "C" __global__ void __launch_bounds__(256) ar_fl_fwd(const float *Q, const float *K, const float *V, float *O,
@@ -143,25 +151,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_fwd(const float *Q, cons
                                                              int has_mask, int hq, int hkv)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[flash_f32_lds_bytes<128, 4, 1>()];
-    FlashF32Params p = {};
-    p.q = Q; p.k = K; p.v = V; p.o = O; p.lse = LSE;
-    p.mask = has_mask ? M : nullptr;
-    p.Hq = hq; p.Hkv = hkv; p.N = N;
-    p.nq = (int)gridDim.x;
-    p.total = (int)(gridDim.x * gridDim.y);
-    p.lpt_heads = (int)gridDim.y;  // causal: longest query tile first over all heads
-    dense(p.qs, hq, N, head_dim);
-    dense(p.ks, hkv, N, head_dim);
-    dense(p.os, hq, N, head_dim);
-    p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
-    const int wg = linear_wg();
-    if (head_dim == 64) {
-        if (causal) flash_f32_body<64, 4, 1, true, false, true>(p, lds, wg);
-        else flash_f32_body<64, 4, 1, false, false, true>(p, lds, wg);
-    } else if (head_dim == 128) {
-        if (causal) flash_f32_body<128, 4, 1, true>(p, lds, wg);
-        else flash_f32_body<128, 4, 1, false>(p, lds, wg);
-    }
+    flash_f32_entry(lds, Q, K, V, O, LSE, M, nullptr, N, head_dim, causal, has_mask, hq, hkv);
 }
 
 #endif
@@ -184,8 +174,7 @@ __device__ __forceinline__ void flash_f32_short(const float *Q, const float *K, 
     dense(p.os, hq, N, 64);
     p.scale = 0.125f;
     const int wg = linear_wg();
-    if (causal) flash_f32_body<64, 1, 4, true>(p, lds, wg);
-    else flash_f32_body<64, 1, 4, false>(p, lds, wg);
+    flash_f32_forms<64, 1, 4, false>(p, lds, wg, causal);
 }
 }  // namespace
 

@@ -41,7 +41,7 @@ constexpr int F32_BK = 32;  // keys per tile
 struct FlashF32Params {
     const float *q, *k, *v;
     float *o;
-    const float *mask;      // additive [N,N] or null
+    const float *mask;      // additive [N,N], read by the forms with HAS_MASK
     const int32_t *kv_len;  // [B] or null
     float *lse;             // optional [B,Hq,N]: m + log(l), src/runtime/cuda_flash_train.rs:141
     int Hq, Hkv, N, nq;
@@ -149,8 +149,7 @@ __device__ __forceinline__ void flash_f32_plain(const FlashF32Params &p, const f
 // HAS_MASK: p.mask is not null, and the tiles that hide no key take it in stride: a lane's 16 values of a tile, four keys at a
 // time, are requested where the tile's S is begun and folded into the exponent's addend (log2(e) mask - m) behind the
 // split of P, in the same region.  (Waiting for them there also waits for the K / V tiles requested before, which the
-// next instructions want anyway.)  Without it p.mask is still honoured, every tile taking exact_softmax with 16 scattered
-// loads: B2 H12 N1024 D64 118 us, 45 us without a mask.
+// next instructions want anyway.) 
 //
 // TILE_SUMS (QW > 1): the products of a key tile are summed from zero and then added to O, which is rounded once per tile instead
 // of with each of its 12 matrix instructions.
@@ -268,7 +267,6 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
                 float xv = s[r] * c2;
                 if constexpr (HAS_MASK) xv = fmaf(mv[r], LOG2E, xv);
-                else if (p.mask != nullptr && key < N && q_row < N) xv = fmaf(p.mask[(size_t)q_row * N + key], LOG2E, xv);
                 if (key >= kend || (CAUSAL && key > q_row)) xv = -__builtin_inff();
                 x[r] = xv;
                 mx = fmaxf(mx, xv);
@@ -300,7 +298,7 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
         pb[1] = split_8(x[8], x[9], x[10], x[11], x[12], x[13], x[14], x[15]);
     };
     // (QW > 1 with HAS_MASK: the interleaved softmax scales by c2 whatever its sign and knows no maximum)
-    const bool always_generic = HAS_MASK ? QW == 1 : (p.mask != nullptr || !(c2 >= 0.f));
+    const bool always_generic = HAS_MASK ? QW == 1 : !(c2 >= 0.f);
     auto is_generic = [&](int k0) __attribute__((always_inline)) {
         return always_generic || k0 + F32_BK > kend || (CAUSAL && k0 + F32_BK - 1 > wq0);
     };
@@ -402,7 +400,6 @@ __device__ __forceinline__ void flash_f32_body(const FlashF32Params &p, unsigned
                 const int key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
                 float xv = s[r] * c2;
                 if constexpr (HAS_MASK) xv = fmaf(m_row[min(key, N - 1)], LOG2E, xv);
-                else if (p.mask != nullptr && key < N && q_row < N) xv = fmaf(p.mask[(size_t)q_row * N + key], LOG2E, xv);
                 if (key >= kend || (CAUSAL && key > q_row)) xv = -__builtin_inff();
                 x[r] = xv;
                 mx = fmaxf(mx, xv);

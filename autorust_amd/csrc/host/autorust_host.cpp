@@ -425,11 +425,22 @@ bool mid_variant(const std::shared_ptr<Device> &dev, int64_t b, int64_t h, int64
 
 }  // namespace
 
-// The fp32 kernels at head size 64: 128 queries (keys) per workgroup, or 32 whose tiles are dealt out between the waves where
+// The fp32 backward at head size 64: 128 queries (keys) per workgroup, or 32 whose tiles are dealt out between the waves where
 // 128 would leave half the chip idle (the rule of arhip_flash_bwd)
-static bool short_f32(const std::shared_ptr<Device> &dev, int64_t b, int64_t heads, int64_t n)
+static bool short_bwd(const std::shared_ptr<Device> &dev, int64_t b, int64_t heads, int64_t n)
 {
     return b * heads * ((n + 127) / 128) < (int64_t)dev->compute_units() / 2;
+}
+
+// The same for the forward entries, whose 128-query form has a compute unit to itself and, under the causal mask or with an additive
+// one, takes up to twice as long for a tile of its longest workgroup.  32 / 128 queries, us, at 128, 192, 256 workgroups of 128:
+// plain 27 / 33, 64 / 62, 148 / 122; causal 21 / 33, 43 / 57, 80 / 105; masked 29 / 42, 68 / 82, 154 / 156 (at 336: 85 / 122, at 512:
+// 290 / 292); causal and masked 23 / 48, 46 / 83, 88 / 151 (at 512: 155 / 171).
+static bool short_fwd(const std::shared_ptr<Device> &dev, int64_t b, int64_t heads, int64_t n, bool causal, bool mask)
+{
+    const int64_t wgs = b * heads * ((n + 127) / 128), cus = dev->compute_units();
+    if (mask) return causal ? wgs <= 2 * cus : wgs < 2 * cus;
+    return wgs <= (causal ? cus : cus / 2);
 }
 
 std::vector<HostCall> attention_host_calls(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor *attn_mask,
@@ -456,7 +467,7 @@ std::vector<HostCall> attention_host_calls(const Tensor &q, const Tensor &k, con
 
     if (kern == Kernel::FlashF32) {
         // few, short heads: 32 queries per workgroup instead of 128
-        if (d == 64 && short_f32(dev, b, h, n) && !key_lengths)
+        if (d == 64 && short_fwd(dev, b, h, n, is_causal, has_mask) && !key_lengths)
             calls.push_back(make_call(dev, "ar_flash_f32_short", {q, k, v, out, mslot}, {F, F, F, F, F},
                                       {(n + 31) / 32, b * h, 1}, {256, 1, 1}, vals));
         else
@@ -632,7 +643,7 @@ std::optional<TrainOut> fused_attention_train(const Tensor &q, const Tensor &k, 
     const DType F = DType::Float32;
     Tensor out = Tensor::empty(dev, {b, h, n, d}, F), lse = Tensor::empty(dev, {b * h, n}, F);
     const Tensor mslot = attn_mask ? *attn_mask : out;
-    const bool shrt = d == 64 && short_f32(dev, b, h, n);
+    const bool shrt = d == 64 && short_fwd(dev, b, h, n, is_causal, attn_mask != nullptr);
     const HostCall call = make_call(dev, shrt ? "ar_fl_fwd_short" : "ar_fl_fwd", {q, k, v, out, lse, mslot}, {F, F, F, F, F, F},
                                     {(n + (shrt ? 31 : 127)) / (shrt ? 32 : 128), b * h, 1}, {256, 1, 1},
                                     {n, d, (int64_t)is_causal, (int64_t)(attn_mask != nullptr), h, hk});
@@ -656,7 +667,7 @@ std::optional<Grads> fused_attention_backward(const Tensor &q, const Tensor &k, 
     const Tensor mslot = attn_mask ? *attn_mask : g.dq;   // the reference's dummy (cuda_flash_train.rs:442-449)
     const std::vector<int64_t> vals = {n, d, (int64_t)is_causal, (int64_t)(attn_mask != nullptr), h, hk};
     // few, short heads: 32 queries / keys per workgroup (the rule of arhip_flash_bwd)
-    const bool shrt = d == 64 && short_f32(dev, b, hk, n);
+    const bool shrt = d == 64 && short_bwd(dev, b, hk, n);
     const int64_t rows = shrt ? 32 : 128;
     const std::vector<HostCall> calls = {
         make_call(dev, "ar_fl_prep", {out, dout, delta}, {F, F, F}, {(n + 3) / 4, b * h, 1}, {256, 1, 1}, {n, d}),

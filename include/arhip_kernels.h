@@ -31,8 +31,8 @@
 /* fp32 exact mode: replaces `ar_flash_f32`, src/runtime/cuda_flash.rs:53-141.
  * (const float *Q, *K, *V, float *O, const float *M, 6 ints); general tiling. */
 #define ARHIP_KERNEL_FLASH_F32 "ar_flash_f32"
-/* the variant for few, short heads (B * hq * ceil(N/128) below half the compute units): same
- * arguments, head_dim 64 only; 32 queries per workgroup, block [256,1,1], grid [ceil(N/32), B*hq, 1]. */
+/* the variant for few, short heads (B * hq * ceil(N/128) up to half the compute units, all of them under the causal
+ * mask, twice as many with an additive one): same arguments, head_dim 64 only; 32 queries per workgroup, block [256,1,1], grid [ceil(N/32), B*hq, 1]. */
 #define ARHIP_KERNEL_FLASH_F32_SHORT "ar_flash_f32_short"
 
 /* Training kernels, f32: replace `ar_fl_fwd`, `ar_fl_prep`, `ar_fl_bwd_dq`, `ar_fl_bwd_dkv`,

@@ -169,16 +169,30 @@ fn mid_variant(dev: &str, b: i64, h: i64, n: i64, d: i64, causal: bool, has_lens
 }
 
 /// The fp32 kernels take 128 queries (keys) per workgroup, or 32 with the tiles of the other side dealt out
-/// between the waves where 128 would leave half the chip idle (`*_short`, `head_dim` 64).
-fn short_f32(dev: &str, b: i64, heads: i64, n: i64, d: i64) -> bool {
-    d == 64 && b * heads * ((n + 127) / 128) < crate::runtime::ops_hip::compute_units(dev) / 2
+/// between the waves (`*_short`, `head_dim` 64).  Forward: up to half a workgroup of 128 queries per compute
+/// unit, up to one under the causal mask, up to two with an additive mask (the rule of the C++ mirror).
+fn short_fwd(dev: &str, b: i64, h: i64, n: i64, d: i64, opts: Options) -> bool {
+    let (wgs, cus) = (b * h * ((n + 127) / 128), crate::runtime::ops_hip::compute_units(dev));
+    d == 64
+        && match (opts.has_mask, opts.causal) {
+            (true, true) => wgs <= 2 * cus,
+            (true, false) => wgs < 2 * cus,
+            (false, true) => wgs <= cus,
+            (false, false) => wgs <= cus / 2,
+        }
+}
+
+/// The same for dQ and dK/dV (the rule of `arhip_flash_bwd`).
+fn short_bwd(dev: &str, b: i64, n: i64, d: i64, opts: Options) -> bool {
+    let (wgs, cus) = (b * opts.h_kv * ((n + 127) / 128), crate::runtime::ops_hip::compute_units(dev));
+    d == 64 && 2 * wgs < cus
 }
 
 /// fp32 exact mode: `bufs = [q, k, v, o, mask-or-o]`, all f32 `[b, h, n, d]`; `lens`: int32 `[b]` key lengths.
 #[allow(clippy::too_many_arguments)]
 pub fn host_call_f32(dev: &str, bufs: Vec<Buffer>, lens: Option<Buffer>, b: i64, h: i64, n: i64, d: i64, opts: Options) -> HostCall {
     let f = dtype::FLOAT32;
-    if lens.is_none() && short_f32(dev, b, h, n, d) {
+    if lens.is_none() && short_fwd(dev, b, h, n, d, opts) {
         call("ar_flash_f32_short", bufs, &[f, f, f, f, f], [(n + 31) / 32, b * h, 1], [256, 1, 1], vals(n, d, h, opts), &[])
     } else {
         attn_call("ar_flash_f32", bufs, &[f, f, f, f, f], lens, [(n + 127) / 128, b * h, 1], [256, 1, 1], vals(n, d, h, opts))
@@ -345,7 +359,7 @@ pub fn host_calls_sage(
 /// Forward that also writes `lse [b*h, n]`: `bufs = [q, k, v, o, lse, mask-or-o]`.
 pub fn host_call_train_fwd(dev: &str, bufs: Vec<Buffer>, b: i64, h: i64, n: i64, d: i64, opts: Options) -> HostCall {
     let f = dtype::FLOAT32;
-    if short_f32(dev, b, h, n, d) {
+    if short_fwd(dev, b, h, n, d, opts) {
         call("ar_fl_fwd_short", bufs, &[f, f, f, f, f, f], [(n + 31) / 32, b * h, 1], [256, 1, 1], vals(n, d, h, opts), &[])
     } else {
         call("ar_fl_fwd", bufs, &[f, f, f, f, f, f], [(n + 127) / 128, b * h, 1], [256, 1, 1], vals(n, d, h, opts), &[])
@@ -361,7 +375,7 @@ pub fn host_calls_train_bwd(
     dq: Buffer, dk: Buffer, dv: Buffer, b: i64, h: i64, n: i64, d: i64, opts: Options,
 ) -> Vec<HostCall> {
     let f = dtype::FLOAT32;
-    let short = short_f32(dev, b, opts.h_kv, n, d);
+    let short = short_bwd(dev, b, n, d, opts);
     let tiles = if short { (n + 31) / 32 } else { (n + 127) / 128 };
     let (dq_name, dkv_name) = if short { ("ar_fl_bwd_dq_short", "ar_fl_bwd_dkv_short") } else { ("ar_fl_bwd_dq", "ar_fl_bwd_dkv") };
     vec![

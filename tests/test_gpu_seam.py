@@ -73,6 +73,24 @@ def test_ar_flash_f32_short_by_name(dev, kernels, case):
     assert np.abs(got - want).max() < 2e-5
 
 
+@pytest.mark.parametrize("entry,per_wg,d", [("ar_flash_f32", 128, 64), ("ar_flash_f32", 128, 128), ("ar_flash_f32_short", 32, 64)])
+@pytest.mark.parametrize("n", [1, 33, 97, 128, 129, 257])
+@pytest.mark.parametrize("causal", [False, True])
+def test_masked_f32_entries_at_the_edges_of_their_tiles(dev, kernels, entry, per_wg, d, n, causal):
+    b, hq, hkv = 1, 4, 2
+    q, k, v = (synth.normal(990 + 10 ** 6 * i, (b, h, n, d)) for i, h in enumerate((hq, hkv, hkv)))
+    mask = synth.normal(995, (n, n))
+    mask[np.triu_indices(n, 1)] *= 4.0
+    mask[n // 2, : n // 2] = -np.inf
+    with Bufs(dev) as bufs:
+        dq, dk, dv, dm = bufs.put(q), bufs.put(k), bufs.put(v), bufs.put(mask)
+        do = bufs.new(q.nbytes)
+        dev.launch(kernels, entry, _grid(n, per_wg, b, hq), (256, 1, 1), [dq, dk, dv, do, dm], [n, d, int(causal), 1, hq, hkv])
+        got = do.copyout(np.float32, q.shape)
+    want = oracle.sdpa_f64(q, k, v, mask=mask, causal=causal)
+    assert np.abs(got - want).max() < 5e-6
+
+
 @pytest.mark.parametrize("case", CASES, ids=str)
 def test_ar_flash_bf16_by_name(dev, kernels, case):
     b, hq, hkv, n, d, causal, has_mask = case

@@ -1,4 +1,4 @@
-"""What the C++ host layer waits for (csrc/host/): a launch is submitted without waiting only while everything that can see its
+"""What the C++ host layer submits and waits for (csrc/host/): a launch is submitted without waiting only while everything that can see its
 buffers goes to the same stream.  CPU tests: the host layer on a stand-in for libarhip that logs launches and waits.  GPU tests:
 results read through the address on another stream, and buffers shared between two handles."""
 import ctypes
@@ -41,15 +41,15 @@ class _Stub:
     def device(self):
         return ctypes.c_void_p(self.h.arh_device_open(0))
 
-    def tensor(self, dev, dtype=FLOAT32):
-        x = np.zeros((1, 2, 64, 64), np.float32)
-        shape = (ctypes.c_int64 * 4)(*x.shape)
-        return ctypes.c_void_p(self.h.arh_tensor_from_slice(dev, x.ctypes.data_as(ctypes.c_void_p), shape, 4, dtype))
+    def tensor(self, dev, dtype=FLOAT32, shape=(1, 2, 64, 64)):
+        x = np.zeros(shape, np.float32)
+        dims = (ctypes.c_int64 * len(shape))(*shape)
+        return ctypes.c_void_p(self.h.arh_tensor_from_slice(dev, x.ctypes.data_as(ctypes.c_void_p), dims, len(shape), dtype))
 
-    def attention(self, q, k, v, api=2):
+    def attention(self, q, k, v, api=2, mask=None, causal=False):
         """The new tensor and the log of the call."""
         self.h.stub_clear()
-        out = self.h.arh_attention(q, k, v, None, ctypes.c_double(0.0), 0, api, self.sess, None, None)
+        out = self.h.arh_attention(q, k, v, mask, ctypes.c_double(0.0), int(causal), api, self.sess, None, None)
         assert out
         return ctypes.c_void_p(out), self.h.stub_log().decode().split("\n")[:-1]
 
@@ -109,6 +109,22 @@ def test_buffers_of_another_handle_are_waited_for_on_both_sides(stub, api, dtype
         me = log[i].split()[1]
         (other,) = handles - {me}
         assert log[i - 1] == "sync " + other and log[i + 1] == "sync " + me, log
+
+
+# B, H, N (on 256 compute units), and whether the 32-query entry serves them: plain, causal, masked, causal and masked
+@pytest.mark.parametrize("shape,short", [((4, 8, 512), (1, 1, 1, 1)), ((2, 12, 1024), (0, 1, 1, 1)), ((8, 8, 512), (0, 1, 1, 1)),
+                                         ((8, 6, 789), (0, 0, 1, 1)), ((8, 16, 512), (0, 0, 0, 1)), ((8, 16, 640), (0, 0, 0, 0))])
+def test_entry_of_the_fp32_forward(stub, shape, short):
+    s = _Stub(stub)
+    d = s.device()
+    x = s.tensor(d, shape=shape + (64,))
+    m = s.tensor(d, shape=(shape[2], shape[2]))
+    for want, mask, causal in zip(short, (None, None, m, m), (False, True, False, True)):
+        out, log = s.attention(x, x, x, mask=mask, causal=causal)
+        assert [line.split()[2] for line in log] == ["ar_flash_f32_short" if want else "ar_flash_f32"], (causal, mask)
+        stub.arh_tensor_free(out)
+    for t in (x, m):
+        stub.arh_tensor_free(t)
 
 
 def _arrays(b=2, h=4, n=300, d=64):
