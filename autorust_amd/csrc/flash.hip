@@ -546,8 +546,11 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     const long rows = (long)(B * Hq * N);
     // 4 waves per workgroup: 128 queries / keys that share their tiles, or (head size 64, so few workgroups that half the chip would
     // idle behind them) the same 32 queries / keys with the tiles of the other side dealt out between the waves.  128 against 32
-    // rows per workgroup: B1 H12 N197 40 / 26 us, B4 H8 N512 (128 workgroups: the line) 73 / 77, B8 H12 N197 46 / 70
-    const bool split = D == 64 && B * Hkv * ((N + 127) / 128) < dev->cus / 2;
+    // rows per workgroup: B1 H12 N197 40 / 26 us, B4 H8 N512 (128 workgroups: the line) 73 / 77, causal 74 / 61, B8 H12 N197 46 / 70.
+    // Head size 128 has 128 rows only: B1 H4 N512 85 us, B1 H8 N1024 155 us, B1 H4 N4096 causal 564 us, where 32 rows on the fp32
+    // instruction took 90, 169 and 623.
+    const int64_t wgs = B * Hkv * ((N + 127) / 128);
+    const bool split = D == 64 && (causal ? 2 * wgs <= dev->cus : 2 * wgs < dev->cus);
     const int rows_wg = split ? 32 : 128;
     const int nt = (int)((N + rows_wg - 1) / rows_wg);
     p.nt = nt;
@@ -555,7 +558,7 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     // Sums in two halves on grids of fewer than two workgroups per compute unit (as f32_tile_sums).  Relative error of dV and us, one
     // sum / two halves (and log2(e) lse unrounded): B8 H6 N789 D64 6.2e-7 / 5.1e-7 and 214 / 218, B1 H16 N2048 D128 9.3e-7 / 7.7e-7
     // and 588 / 582, B1 H4 N512 D128 6.1e-7 / 5.3e-7 and 82 / 85
-    p.halves = B * Hkv * ((N + 127) / 128) < 2 * (int64_t)dev->cus;
+    p.halves = wgs < 2 * (int64_t)dev->cus;
     p.total_q = (int)(nt * B * Hq);
     p.total_kv = (int)(nt * B * Hkv);
     p.lpt_q = causal ? (int)(B * Hq) : 0;

@@ -427,9 +427,10 @@ bool mid_variant(const std::shared_ptr<Device> &dev, int64_t b, int64_t h, int64
 
 // The fp32 backward at head size 64: 128 queries (keys) per workgroup, or 32 whose tiles are dealt out between the waves where
 // 128 would leave half the chip idle (the rule of arhip_flash_bwd)
-static bool short_bwd(const std::shared_ptr<Device> &dev, int64_t b, int64_t heads, int64_t n)
+static bool short_bwd(const std::shared_ptr<Device> &dev, int64_t b, int64_t heads, int64_t n, bool causal)
 {
-    return b * heads * ((n + 127) / 128) < (int64_t)dev->compute_units() / 2;
+    const int64_t wgs = b * heads * ((n + 127) / 128), cus = dev->compute_units();
+    return causal ? 2 * wgs <= cus : 2 * wgs < cus;
 }
 
 // The same for the forward entries, whose 128-query form has a compute unit to itself and, under the causal mask or with an additive
@@ -667,7 +668,7 @@ std::optional<Grads> fused_attention_backward(const Tensor &q, const Tensor &k, 
     const Tensor mslot = attn_mask ? *attn_mask : g.dq;   // the reference's dummy (cuda_flash_train.rs:442-449)
     const std::vector<int64_t> vals = {n, d, (int64_t)is_causal, (int64_t)(attn_mask != nullptr), h, hk};
     // few, short heads: 32 queries / keys per workgroup (the rule of arhip_flash_bwd)
-    const bool shrt = d == 64 && short_bwd(dev, b, hk, n);
+    const bool shrt = d == 64 && short_bwd(dev, b, hk, n, is_causal);
     const int64_t rows = shrt ? 32 : 128;
     const std::vector<HostCall> calls = {
         make_call(dev, "ar_fl_prep", {out, dout, delta}, {F, F, F}, {(n + 3) / 4, b * h, 1}, {256, 1, 1}, {n, d}),

@@ -47,7 +47,7 @@
 #define ARHIP_KERNEL_FL_PREP "ar_fl_prep"
 #define ARHIP_KERNEL_FL_BWD_DQ "ar_fl_bwd_dq"
 #define ARHIP_KERNEL_FL_BWD_DKV "ar_fl_bwd_dkv"
-/* the variants for few, short heads (B * hkv * ceil(N/128) below half the compute units): the same
+/* the variants for few, short heads (the backward: B * hkv * ceil(N/128) below half the compute units, causal: up to half): the same
  * arguments, head_dim 64 only; 32 queries (keys for dK/dV) per workgroup, block [256,1,1], grid.x =
  * ceil(N/32); `ar_fl_prep` is shared. */
 #define ARHIP_KERNEL_FL_FWD_SHORT "ar_fl_fwd_short"

@@ -185,7 +185,7 @@ fn short_fwd(dev: &str, b: i64, h: i64, n: i64, d: i64, opts: Options) -> bool {
 /// The same for dQ and dK/dV (the rule of `arhip_flash_bwd`).
 fn short_bwd(dev: &str, b: i64, n: i64, d: i64, opts: Options) -> bool {
     let (wgs, cus) = (b * opts.h_kv * ((n + 127) / 128), crate::runtime::ops_hip::compute_units(dev));
-    d == 64 && 2 * wgs < cus
+    d == 64 && if opts.causal { 2 * wgs <= cus } else { 2 * wgs < cus }
 }
 
 /// fp32 exact mode: `bufs = [q, k, v, o, mask-or-o]`, all f32 `[b, h, n, d]`; `lens`: int32 `[b]` key lengths.

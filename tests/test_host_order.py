@@ -127,6 +127,21 @@ def test_entry_of_the_fp32_forward(stub, shape, short):
         stub.arh_tensor_free(t)
 
 
+@pytest.mark.parametrize("shape,causal,short", [((1, 12, 1024), False, True), ((4, 8, 512), False, False), ((4, 8, 512), True, True),
+                                                ((1, 8, 2048), True, True), ((2, 12, 700), True, False)])
+def test_entries_of_the_fp32_backward(stub, shape, causal, short):
+    s = _Stub(stub)
+    d = s.device()
+    x, lse = s.tensor(d, shape=shape + (64,)), s.tensor(d, shape=(shape[0] * shape[1], shape[2]))
+    grads = [ctypes.c_void_p() for _ in range(3)]
+    stub.stub_clear()
+    assert stub.arh_fused_attention_backward(x, x, x, x, lse, x, None, int(causal), s.sess, *(ctypes.byref(g) for g in grads)) == 1
+    names = [line.split()[2] for line in stub.stub_log().decode().split("\n")[:-1]]
+    assert names == ["ar_fl_prep"] + [n + "_short" * short for n in ("ar_fl_bwd_dq", "ar_fl_bwd_dkv")]
+    for t in [x, lse] + grads:
+        stub.arh_tensor_free(t)
+
+
 def _arrays(b=2, h=4, n=300, d=64):
     return [synth.normal(s, (b, h, n, d)) for s in (1, 2, 3)]
 
