@@ -21,7 +21,7 @@ HOST_LIB = os.path.join(HERE, "libautorust_host.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # the pipelined kernel's variants compile in translation units of their own (pipe_launch.h), side by side
-SOURCES = ["device.hip", "flash.hip", "sage_quant.hip", "f32_mask.hip", "pipe_bf16.hip", "pipe_bf16_mask.hip", "pipe_i8.hip", "pipe_i8_keys.hip", "pipe_i8_qf.hip",
+SOURCES = ["device.hip", "flash.hip", "sage_quant.hip", "f32_mask.hip", "f32_bwd_mask.hip", "pipe_bf16.hip", "pipe_bf16_mask.hip", "pipe_i8.hip", "pipe_i8_keys.hip", "pipe_i8_qf.hip",
            "pipe_i8_keys_qf.hip", "pipe_fp8.hip", "pipe_fp8_qf.hip", "pipe_fp8_keys.hip"]
 HEADERS = ["arhip_internal.h", "attn_fwd.h", "attn_pipe.h", "pipe_launch.h", "pipe_tu.h", "lane_max.h", "f32_split.h", "flash_f32.h", "f32_launch.h", "flash_bwd_f32.h",
            "sage_quant_kernels.h", os.path.join("..", "..", "include", "arhip.h")]

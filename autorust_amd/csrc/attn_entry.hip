@@ -138,6 +138,8 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_f32(const float *Q, c
     flash_f32_entry(lds, Q, K, V, O, nullptr, M, nullptr, N, head_dim, causal, has_mask, hq, hkv);
 }
 
+#endif
+#if ARHIP_PART(2)
 extern "C" __global__ void __launch_bounds__(256) ar_flash_f32_lens(const float *Q, const float *K, const float *V, float *O,
                                                                      const float *M, const int *L, int N, int head_dim,
                                                                      int causal, int has_mask, int hq, int hkv)
@@ -146,6 +148,8 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_f32_lens(const float 
     flash_f32_entry(lds, Q, K, V, O, nullptr, M, L, N, head_dim, causal, has_mask, hq, hkv);
 }
 
+#endif
+#if ARHIP_PART(1)
 extern "C" __global__ void __launch_bounds__(256) ar_fl_fwd(const float *Q, const float *K, const float *V, float *O,
                                                              float *LSE, const float *M, int N, int head_dim, int causal,
                                                              int has_mask, int hq, int hkv)
@@ -221,9 +225,33 @@ __device__ __forceinline__ FlashBwdParams bwd_params(const float *Q, const float
     p.scale = 1.0f / __builtin_sqrtf((float)head_dim);
     return p;
 }
+
+// the forms of a kernel: causal or not, with an additive mask or without
+template <int D, bool SPLIT>
+__device__ __forceinline__ void bwd_dq_forms(const FlashBwdParams &p, unsigned char *lds, int wg, int causal)
+{
+    if (p.mask != nullptr) {
+        if (causal) bwd_dq_body<D, true, SPLIT, true>(p, lds, wg);
+        else bwd_dq_body<D, false, SPLIT, true>(p, lds, wg);
+    } else {
+        if (causal) bwd_dq_body<D, true, SPLIT, false>(p, lds, wg);
+        else bwd_dq_body<D, false, SPLIT, false>(p, lds, wg);
+    }
+}
+template <int D, bool SPLIT>
+__device__ __forceinline__ void bwd_dkv_forms(const FlashBwdParams &p, unsigned char *lds, int wg, int causal)
+{
+    if (p.mask != nullptr) {
+        if (causal) bwd_dkv_body<D, true, SPLIT, true>(p, lds, wg);
+        else bwd_dkv_body<D, false, SPLIT, true>(p, lds, wg);
+    } else {
+        if (causal) bwd_dkv_body<D, true, SPLIT, false>(p, lds, wg);
+        else bwd_dkv_body<D, false, SPLIT, false>(p, lds, wg);
+    }
+}
 }  // namespace
 
-#if ARHIP_PART(1)
+#if ARHIP_PART(4)
 extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dq(const float *Q, const float *K, const float *V,
                                                                 const float *dO, const float *LSE, const float *D,
                                                                 const float *M, float *dQ, int N, int head_dim, int causal,
@@ -233,15 +261,12 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dq(const float *Q, c
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dq = dQ;
     const int wg = linear_wg();
-    if (head_dim == 64) {
-        if (causal) bwd_dq_body<64, true, false>(p, lds, wg);
-        else bwd_dq_body<64, false, false>(p, lds, wg);
-    } else if (head_dim == 128) {
-        if (causal) bwd_dq_body<128, true, false>(p, lds, wg);
-        else bwd_dq_body<128, false, false>(p, lds, wg);
-    }
+    if (head_dim == 64) bwd_dq_forms<64, false>(p, lds, wg, causal);
+    else if (head_dim == 128) bwd_dq_forms<128, false>(p, lds, wg, causal);
 }
 
+#endif
+#if ARHIP_PART(5)
 extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv(const float *Q, const float *K, const float *V,
                                                                  const float *dO, const float *LSE, const float *D,
                                                                  const float *M, float *dK, float *dV, int N, int head_dim,
@@ -251,19 +276,14 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv(const float *Q, 
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dk = dK; p.dv = dV;
     const int wg = linear_wg();
-    if (head_dim == 64) {
-        if (causal) bwd_dkv_body<64, true, false>(p, lds, wg);
-        else bwd_dkv_body<64, false, false>(p, lds, wg);
-    } else if (head_dim == 128) {
-        if (causal) bwd_dkv_body<128, true, false>(p, lds, wg);
-        else bwd_dkv_body<128, false, false>(p, lds, wg);
-    }
+    if (head_dim == 64) bwd_dkv_forms<64, false>(p, lds, wg, causal);
+    else if (head_dim == 128) bwd_dkv_forms<128, false>(p, lds, wg, causal);
 }
 
 #endif
 // The same for short shapes: 32 queries (dQ) / 32 keys (dK, dV) per workgroup, grid [ceil(N/32), B*hq, 1] /
 // [ceil(N/32), B*hkv, 1], the tiles of the other side dealt out between the four waves.  head_dim 64 only.
-#if ARHIP_PART(1)
+#if ARHIP_PART(3)
 extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dq_short(const float *Q, const float *K, const float *V,
                                                                          const float *dO, const float *LSE, const float *D,
                                                                          const float *M, float *dQ, int N, int head_dim,
@@ -274,8 +294,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dq_short(const float
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dq = dQ;
     const int wg = linear_wg();
-    if (causal) bwd_dq_body<64, true, true>(p, lds, wg);
-    else bwd_dq_body<64, false, true>(p, lds, wg);
+    bwd_dq_forms<64, true>(p, lds, wg, causal);
 }
 
 extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv_short(const float *Q, const float *K, const float *V,
@@ -288,8 +307,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_fl_bwd_dkv_short(const floa
     FlashBwdParams p = bwd_params(Q, K, V, dO, LSE, D, M, N, head_dim, has_mask, hq, hkv);
     p.dk = dK; p.dv = dV;
     const int wg = linear_wg();
-    if (causal) bwd_dkv_body<64, true, true>(p, lds, wg);
-    else bwd_dkv_body<64, false, true>(p, lds, wg);
+    bwd_dkv_forms<64, true>(p, lds, wg, causal);
 }
 
 #endif

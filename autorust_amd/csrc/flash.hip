@@ -563,21 +563,12 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     p.total_kv = (int)(nt * B * Hkv);
     p.lpt_q = causal ? (int)(B * Hq) : 0;
     p.lpt_kv = causal ? (int)(B * Hkv) : 0;
-    const dim3 block(256);
-    auto go = [&](auto d, auto c) {
-        constexpr int DD = decltype(d)::value;
-        constexpr bool C = decltype(c)::value;
-        constexpr int PR = bwd_prep_rows<DD>();
-        hipLaunchKernelGGL((bwd_prep_kernel<DD>), dim3((unsigned)((rows + PR - 1) / PR)), block, 0, dev->stream, o, dout, delta, rows);
-        if (DD == 128 || split) {
-            hipLaunchKernelGGL((bwd_kernel<DD, C, DD == 64>), dim3((unsigned)(p.total_kv + p.total_q)), block, 0, dev->stream, p);
-        } else {
-            hipLaunchKernelGGL((bwd_dq_kernel<C>), dim3((unsigned)p.total_q), block, 0, dev->stream, p);
-            hipLaunchKernelGGL((bwd_dkv_kernel<C>), dim3((unsigned)p.total_kv), block, 0, dev->stream, p);
-        }
-    };
-    auto by_mask = [&](auto d) { causal ? go(d, std::true_type{}) : go(d, std::false_type{}); };
-    D == 64 ? by_mask(std::integral_constant<int, 64>{}) : by_mask(std::integral_constant<int, 128>{});
+    const int prep_rows = D == 64 ? bwd_prep_rows<64>() : bwd_prep_rows<128>();
+    const dim3 prep_grid((unsigned)((rows + prep_rows - 1) / prep_rows)), block(256);
+    if (D == 64) hipLaunchKernelGGL((bwd_prep_kernel<64>), prep_grid, block, 0, dev->stream, o, dout, delta, rows);
+    else hipLaunchKernelGGL((bwd_prep_kernel<128>), prep_grid, block, 0, dev->stream, o, dout, delta, rows);
+    if (mask != nullptr) launch_f32_bwd_mask(dev->stream, p, (int)D, causal != 0, split);
+    else launch_bwd<false>(dev->stream, p, (int)D, causal != 0, split);
     arhip_note_selected(ARHIP_K_FLASH_BWD);
     return t.end();
 }

@@ -313,7 +313,10 @@ __device__ __forceinline__ void bwd_dkv_plain(const FlashBwdParams &p, int b, in
 // matrix instructions and most of the chip idle): the waves share the same 32 queries and deal the
 // key tiles out between them (wave w takes tiles w, w + 4, ...), each staging its tiles in its own
 // LDS slab with no workgroup barrier; the partial dQ of the waves are added through LDS in wave order.
-template <int D, bool CAUSAL, bool SPLIT>
+// HAS_MASK: p.mask is not null.  The 16 mask values of a lane are requested where the logits they belong to are begun: asked for where
+// they are added, their way from memory was waited for in every tile (whole backward, B1 H2 N1024 D128 253 -> 149 us, B2 H6
+// N1500 D64 causal 300 -> 252, B2 H12 N1024 D64 318 -> 197).
+template <int D, bool CAUSAL, bool SPLIT, bool HAS_MASK>
 __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned char *lds, int wg_linear)
 {
     constexpr int NW = 4;
@@ -389,14 +392,28 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
     float ds[16], t4[4];  // dS / scale; scratch of ds_step
     split8 db_[2];
     // what the logits are multiplied by in the exponent: c2, or 1 where the mask has been added (add_mask)
-    const float cx = p.mask != nullptr ? 1.f : c2;
-    auto add_mask = [&](int k0) __attribute__((always_inline)) {
-        if (p.mask == nullptr) return;
+    const float cx = HAS_MASK ? 1.f : c2;
+    float mv[16];
+    const float *m_row = HAS_MASK ? p.mask + (size_t)rr * N : nullptr;
+    auto fetch_mask = [&](int k0) __attribute__((always_inline)) {
+        typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_u;  // rows of any N: 4-byte aligned
+        if constexpr (!HAS_MASK) return;
+        if (k0 + F32_BK <= N) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int key = min(k0 + 8 * (r >> 2) + 4 * h + (r & 3), N - 1);
-            s[r] = fmaf(p.mask[(size_t)rr * N + key], BWD_LOG2E, s[r] * c2);
+            for (int g = 0; g < 4; ++g) {
+                const f32x4_u v = *(const f32x4_u *)(m_row + k0 + 8 * g + 4 * h);
+                mv[4 * g] = v[0]; mv[4 * g + 1] = v[1]; mv[4 * g + 2] = v[2]; mv[4 * g + 3] = v[3];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mv[r] = m_row[min(k0 + 8 * (r >> 2) + 4 * h + (r & 3), N - 1)];
         }
+        ARHIP_FENCE();
+    };
+    auto add_mask = [&]() __attribute__((always_inline)) {
+        if constexpr (!HAS_MASK) return;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = fmaf(mv[r], BWD_LOG2E, s[r] * c2);
     };
     auto make_ds = [&](int r) __attribute__((always_inline)) {
         ds[r] = __builtin_amdgcn_exp2f(fmaf(neg_lse, BWD_LOG2E, s[r] * cx)) * (dp[r] - di);
@@ -439,10 +456,11 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         for (int it = wave; it < ntiles; it += NW) {
             const int k0 = it * F32_BK;
             stage.put(kt, vt, lane);
+            fetch_mask(k0);
             if (it + NW < ntiles) stage.fetch(kp, vp, lane, k0 + NW * F32_BK, kend - 1);
             s = mul_rows<D>(kt, r_addr, qr);
             dp = mul_rows<D>(vt, r_addr, dor);
-            add_mask(k0);
+            add_mask();
 #pragma unroll
             for (int r = 0; r < 16; ++r) make_ds(r);
             drop_dead(k0);
@@ -463,9 +481,10 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
         }
         __syncthreads();
         if (my_tiles > 0) {
+            fetch_mask(0);
             s = mul_rows<D>(k_ring, r_addr, qr);
             dp = mul_rows<D>(v_ring, r_addr, dor);
-            add_mask(0);
+            add_mask();
 #pragma unroll
             for (int r = 0; r < 16; ++r) make_ds(r);
             drop_dead(0);
@@ -494,6 +513,7 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
                     const int o = (i % DB) * 2048 + (i / DB) * 1024;
                     fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
                 };
+                fetch_mask((n + 1) * F32_BK);
                 // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
                 static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, kt1, 0); });
                 static_for<0, 4>(split_ds);
@@ -518,7 +538,7 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
                         else stage.template split_step<i - (2 * SPLIT_STEPS - 4)>(kt2, vt2, tid);
                     });
                 if (n + 3 < ntiles) stage.fetch(kp, vp, tid, (n + 3) * F32_BK, kend - 1);
-                add_mask((n + 1) * F32_BK);
+                add_mask();
                 // ---- R2 ----
                 mfma_region<2 * DB, 24>(
                     [&](auto fi, auto mi) __attribute__((always_inline)) {
@@ -618,7 +638,7 @@ __device__ __forceinline__ void bwd_dq_body(const FlashBwdParams &p, unsigned ch
 // dK and dV.  Workgroup wg_linear in [0, nt * B * Hkv), four waves: 128 keys of one K/V head.  SPLIT: the waves
 // share the same 32 keys and deal the (head of the group, query tile) steps out between them, each in
 // its own LDS slab; the partial dK and dV of the waves are added through LDS in wave order.
-template <int D, bool CAUSAL, bool SPLIT>
+template <int D, bool CAUSAL, bool SPLIT, bool HAS_MASK>
 __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned char *lds, int wg_linear)
 {
     constexpr int NW = 4;
@@ -728,14 +748,18 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
         return (r & 3) == 0 ? v.x : (r & 3) == 1 ? v.y : (r & 3) == 2 ? v.z : v.w;
     };
     // what the logits are multiplied by in the exponent: c2, or 1 where the mask has been added (add_mask)
-    const float cx = p.mask != nullptr ? 1.f : c2;
-    auto add_mask = [&](int q0) __attribute__((always_inline)) {
-        if (p.mask == nullptr) return;
+    const float cx = HAS_MASK ? 1.f : c2;
+    float mv[16];
+    auto fetch_mask = [&](int q0) __attribute__((always_inline)) {
+        if constexpr (!HAS_MASK) return;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int qi = min(q0 + 8 * (r >> 2) + 4 * h + (r & 3), N - 1);
-            s[r] = fmaf(p.mask[(size_t)qi * N + jj], BWD_LOG2E, s[r] * c2);
-        }
+        for (int r = 0; r < 16; ++r) mv[r] = p.mask[(size_t)min(q0 + 8 * (r >> 2) + 4 * h + (r & 3), N - 1) * N + jj];
+        ARHIP_FENCE();
+    };
+    auto add_mask = [&]() __attribute__((always_inline)) {
+        if constexpr (!HAS_MASK) return;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = fmaf(mv[r], BWD_LOG2E, s[r] * c2);
     };
     auto make_p = [&](int r) __attribute__((always_inline)) { pr[r] = __builtin_amdgcn_exp2f(fmaf(stat_of(r), BWD_LOG2E, s[r] * cx)); };
     auto make_ds = [&](int r) __attribute__((always_inline)) { ds[r] = pr[r] * (dp[r] - stat_of(r)); };
@@ -748,7 +772,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
             if (!key_live || (CAUSAL && kq > 8 * (r >> 2) + (r & 3))) pr[r] = ds[r] = 0.f;
     };
     auto make_all = [&](int q0, const float *stat) __attribute__((always_inline)) {
-        add_mask(q0);
+        add_mask();
         read_stats(stat);
 #pragma unroll
         for (int r = 0; r < 16; ++r) make_p(r);
@@ -777,6 +801,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
                 fetch_tiles(stage, st + NW);
                 fetch_stats(st + NW);
             }
+            fetch_mask(step_q0(st));
             s = mul_rows<D>(qs, r_addr, kr);
             dp = mul_rows<D>(dos, r_addr, vr);
             make_all(step_q0(st), stat);
@@ -809,6 +834,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
         }
         __syncthreads();
         if (mine > 0) {
+            fetch_mask(step_q0(0));
             s = mul_rows<D>(q_ring, r_addr, kr);
             dp = mul_rows<D>(o_ring, r_addr, vr);
             make_all(step_q0(0), stats);
@@ -837,6 +863,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
                     const int o = (i % DB) * 2048 + (i / DB) * 1024;
                     fr.template set<(f & 1), P>(Tile::template get_col_part<P>(tile, c_addr[0] + o, c_addr[1] + o));
                 };
+                fetch_mask(step_q0(n + 1));
                 // ---- R1 ----  (a few vector steps first: the first fragment has just become visible)
                 static_for<0, 3>([&](auto pi) __attribute__((always_inline)) { load_row(std::integral_constant<int, 0>{}, pi, qt1, 0); });
                 static_for<0, 4>(split_p);
@@ -860,7 +887,7 @@ __device__ __forceinline__ void bwd_dkv_body(const FlashBwdParams &p, unsigned c
                         if constexpr (i < 2 * SPLIT_STEPS - 4) split_p(std::integral_constant<int, i + 4>{});
                         else split_ds(std::integral_constant<int, i - (2 * SPLIT_STEPS - 4)>{});
                     });
-                add_mask(step_q0(n + 1));
+                add_mask();
                 read_stats(stats + s1 * 64);
                 // ---- R2 ----
                 constexpr int CONV = decltype(stage)::STEPS;
@@ -1028,30 +1055,49 @@ __global__ void __launch_bounds__(256) bwd_prep_kernel(const float *o, const flo
 // do with each other, so where either grid alone leaves compute units idle (few or short heads, the end of any grid) the other's
 // workgroups run there; and it is a launch fewer.  Forward and backward, us: B1 H12 N197 D64 26 -> 24, B2 H16 N2048 D128 causal
 // 817 -> 800.
-template <int D, bool CAUSAL, bool SPLIT>
+template <int D, bool CAUSAL, bool SPLIT, bool HAS_MASK>
 __global__ void __launch_bounds__(256, 1) bwd_kernel(const FlashBwdParams p)
 {
     constexpr int LQ = bwd_dq_lds_bytes<D, SPLIT>(), LKV = bwd_dkv_lds_bytes<D, SPLIT>();
     __shared__ __attribute__((aligned(16))) unsigned char lds[LQ > LKV ? LQ : LKV];
     const int wg = (int)blockIdx.x;
-    if (wg < p.total_kv) bwd_dkv_body<D, CAUSAL, SPLIT>(p, lds, wg);
-    else bwd_dq_body<D, CAUSAL, SPLIT>(p, lds, wg - p.total_kv);
+    if (wg < p.total_kv) bwd_dkv_body<D, CAUSAL, SPLIT, HAS_MASK>(p, lds, wg);
+    else bwd_dq_body<D, CAUSAL, SPLIT, HAS_MASK>(p, lds, wg - p.total_kv);
 }
 
 // Head size 64, 128 rows per workgroup: dQ fits 256 registers, so that a SIMD holds two of its waves, and dK/dV does not.  In one
 // kernel either dQ would lose its second wave or dK/dV spill 73 registers (B8 H12 N197: 41 us together, 16 + 23 one after the other).
-template <bool CAUSAL>
+template <bool CAUSAL, bool HAS_MASK>
 __global__ void __launch_bounds__(256, 2) bwd_dq_kernel(const FlashBwdParams p)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dq_lds_bytes<64, false>()];
-    bwd_dq_body<64, CAUSAL, false>(p, lds, (int)blockIdx.x);
+    bwd_dq_body<64, CAUSAL, false, HAS_MASK>(p, lds, (int)blockIdx.x);
 }
 
-template <bool CAUSAL>
+template <bool CAUSAL, bool HAS_MASK>
 __global__ void __launch_bounds__(256, 1) bwd_dkv_kernel(const FlashBwdParams p)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[bwd_dkv_lds_bytes<64, false>()];
-    bwd_dkv_body<64, CAUSAL, false>(p, lds, (int)blockIdx.x);
+    bwd_dkv_body<64, CAUSAL, false, HAS_MASK>(p, lds, (int)blockIdx.x);
+}
+
+// The kernels of a backward pass behind the row scalar
+template <bool HAS_MASK>
+void launch_bwd(hipStream_t stream, const FlashBwdParams &p, int D, bool causal, bool split)
+{
+    auto go = [&](auto d, auto c) {
+        constexpr int DD = decltype(d)::value;
+        constexpr bool C = decltype(c)::value;
+        const dim3 block(256), q_grid((unsigned)p.total_q), kv_grid((unsigned)p.total_kv), both((unsigned)(p.total_kv + p.total_q));
+        if (DD == 128 || split) {
+            hipLaunchKernelGGL((bwd_kernel<DD, C, DD == 64, HAS_MASK>), both, block, 0, stream, p);
+        } else {
+            hipLaunchKernelGGL((bwd_dq_kernel<C, HAS_MASK>), q_grid, block, 0, stream, p);
+            hipLaunchKernelGGL((bwd_dkv_kernel<C, HAS_MASK>), kv_grid, block, 0, stream, p);
+        }
+    };
+    auto by_mask = [&](auto d) { causal ? go(d, std::true_type{}) : go(d, std::false_type{}); };
+    D == 64 ? by_mask(std::integral_constant<int, 64>{}) : by_mask(std::integral_constant<int, 128>{});
 }
 
 }  // namespace arhip

@@ -51,3 +51,25 @@ def test_f32_backward_tilings(dev, shape, mode):
         for name, x, w in zip(("o", "lse", "dq", "dk", "dv"), got, want):
             x = x[b:b + 1, hs] if name in ("o", "lse", "dq") else x[b:b + 1, h:h + 1]
             assert np.abs(x - w).max() <= 1e-5 * max(1.0, np.abs(w).max()), (name, b, h)
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 2, 1, 64), (1, 4, 2, 65, 64), (16, 8, 8, 33, 64), (16, 8, 8, 129, 64), (8, 32, 16, 97, 64),
+                                   (16, 8, 8, 1, 128), (16, 8, 8, 65, 128), (8, 8, 8, 257, 128)], ids=str)
+def test_f32_backward_tilings_causal_with_a_mask(dev, shape):
+    """A causal launch with an additive mask that hides some keys: the mask of a tile is asked for ahead, in whole vectors except at
+    the end of a row."""
+    B, Hq, Hkv, N, D = shape
+    q, do = (synth.normal(920 + 10 ** 6 * i, (B, Hq, N, D)) for i in range(2))
+    k, v = (synth.normal(930 + 10 ** 6 * i, (B, Hkv, N, D)) for i in range(2))
+    mask = synth.normal(940, (N, N))
+    mask[:, N // 3] = -np.inf
+    mask[N // 2, : N // 4] = -np.inf
+    np.fill_diagonal(mask, 0.25)
+    got = run_fwd_bwd(dev, q, k, v, do, mask=mask, causal=True)
+    g = Hq // Hkv
+    for b, h in ((0, 0), (B - 1, Hkv - 1)):
+        hs = slice(h * g, (h + 1) * g)
+        want = oracle.attention_backward_f64(q[b:b + 1, hs], k[b:b + 1, h:h + 1], v[b:b + 1, h:h + 1], do[b:b + 1, hs], mask=mask, causal=True)
+        for name, x, w in zip(("o", "lse", "dq", "dk", "dv"), got, want):
+            x = x[b:b + 1, hs] if name in ("o", "lse", "dq") else x[b:b + 1, h:h + 1]
+            assert np.abs(x - w).max() <= 1e-5 * max(1.0, np.abs(w).max()), (name, b, h)
