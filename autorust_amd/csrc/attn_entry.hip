@@ -321,11 +321,11 @@ __device__ __forceinline__ void flash_bf16_entry(unsigned char *lds, const uint1
 #define AR_BF16(DD)                                                                                       \
     do {                                                                                                  \
         if (has_mask) {                                                                                   \
-            if (causal) attn_fwd_body<DD, 4, true, true, MODE_BF16, false, false, false>(p, lds, wg);     \
-            else attn_fwd_body<DD, 4, false, true, MODE_BF16, false, false, false>(p, lds, wg);           \
+            if (causal) attn_fwd_body<DD, true, true, MODE_BF16, false, false, false>(p, lds, wg);     \
+            else attn_fwd_body<DD, false, true, MODE_BF16, false, false, false>(p, lds, wg);           \
         } else {                                                                                          \
-            if (causal) attn_fwd_body<DD, 4, true, false, MODE_BF16, false, false, false>(p, lds, wg);    \
-            else attn_fwd_body<DD, 4, false, false, MODE_BF16, false, false, false>(p, lds, wg);          \
+            if (causal) attn_fwd_body<DD, true, false, MODE_BF16, false, false, false>(p, lds, wg);    \
+            else attn_fwd_body<DD, false, false, MODE_BF16, false, false, false>(p, lds, wg);          \
         }                                                                                                 \
     } while (0)
     if (head_dim == 64) AR_BF16(64);
@@ -339,7 +339,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_bf16(const uint16_t *
                                                                  uint16_t *O, const float *M, int N, int head_dim, int causal,
                                                                  int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, 4, MODE_BF16, false>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, MODE_BF16, false>()];
     flash_bf16_entry(lds, Q, K, V, O, M, nullptr, N, head_dim, causal, has_mask, hq, hkv);
 }
 
@@ -347,7 +347,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_bf16_lens(const uint1
                                                                       uint16_t *O, const float *M, const int *L, int N,
                                                                       int head_dim, int causal, int has_mask, int hq, int hkv)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, 4, MODE_BF16, false>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, MODE_BF16, false>()];
     flash_bf16_entry(lds, Q, K, V, O, M, L, N, head_dim, causal, has_mask, hq, hkv);
 }
 
@@ -428,11 +428,11 @@ __device__ __forceinline__ void flash_sage_entry(unsigned char *lds, const void 
 #define AR_SAGE(DD, PK)                                                                                 \
     do {                                                                                                \
         if (has_mask) {                                                                                 \
-            if (causal) attn_fwd_body<DD, 4, true, true, QMODE, PK, true, false>(p, lds, wg);           \
-            else attn_fwd_body<DD, 4, false, true, QMODE, PK, true, false>(p, lds, wg);                 \
+            if (causal) attn_fwd_body<DD, true, true, QMODE, PK, true, false>(p, lds, wg);           \
+            else attn_fwd_body<DD, false, true, QMODE, PK, true, false>(p, lds, wg);                 \
         } else {                                                                                        \
-            if (causal) attn_fwd_body<DD, 4, true, false, QMODE, PK, true, false>(p, lds, wg);          \
-            else attn_fwd_body<DD, 4, false, false, QMODE, PK, true, false>(p, lds, wg);                \
+            if (causal) attn_fwd_body<DD, true, false, QMODE, PK, true, false>(p, lds, wg);          \
+            else attn_fwd_body<DD, false, false, QMODE, PK, true, false>(p, lds, wg);                \
         }                                                                                               \
     } while (0)
     if (head_dim == 64) {
@@ -452,7 +452,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_sage(const int8_t *Q8
                                                                  int head_dim, int causal, int has_mask, int hq, int hkv,
                                                                  int bq, int bk)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, 4, MODE_I8, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, MODE_I8, true>()];
     flash_sage_entry<MODE_I8>(lds, Q8, K8, V, O, M, nullptr, SQ, SK, N, head_dim, causal, has_mask, hq, hkv, bq, bk);
 }
 
@@ -461,7 +461,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_sage_lens(const int8_
                                                                       int N, int head_dim, int causal, int has_mask, int hq, int hkv,
                                                                       int bq, int bk)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, 4, MODE_I8, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, MODE_I8, true>()];
     flash_sage_entry<MODE_I8>(lds, Q8, K8, V, O, M, L, SQ, SK, N, head_dim, causal, has_mask, hq, hkv, bq, bk);
 }
 
@@ -474,7 +474,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_sage_fp8(const uint8_
                                                                      int N, int head_dim, int causal, int has_mask, int hq,
                                                                      int hkv, int bq, int bk)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, 4, MODE_FP8, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, MODE_FP8, true>()];
     flash_sage_entry<MODE_FP8>(lds, Q8, K8, V, O, M, nullptr, SQ, SK, N, head_dim, causal, has_mask, hq, hkv, bq, bk);
 }
 
@@ -483,7 +483,7 @@ extern "C" __global__ void __launch_bounds__(256) ar_flash_sage_fp8_lens(const u
                                                                           const float *SK, int N, int head_dim, int causal,
                                                                           int has_mask, int hq, int hkv, int bq, int bk)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, 4, MODE_FP8, true>()];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<128, MODE_FP8, true>()];
     flash_sage_entry<MODE_FP8>(lds, Q8, K8, V, O, M, L, SQ, SK, N, head_dim, causal, has_mask, hq, hkv, bq, bk);
 }
 

@@ -2,7 +2,7 @@
 // FlashAttention path and the int8 (SageAttention-style) path.
 //
 // Work decomposition
-//   grid  : one workgroup per (batch*head, tile of BQ = 32*NW queries)
+//   grid  : one workgroup per (batch*head, tile of 128 queries)
 //   wave  : 32 queries.  The wave computes S^T = K . Q^T, so that in the MFMA
 //           result layout every lane owns ONE query (column lane%32) and 16 of
 //           the 32 keys of a block.  Row max / row sum are per-lane reductions
@@ -158,7 +158,7 @@ __device__ __forceinline__ uint2 lds_read_tr16(const unsigned char *p)
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // LDS bytes attn_fwd_body needs for a tiling variant
-template <int D, int NW, int MODE, bool PER_KEY>
+template <int D, int MODE, bool PER_KEY>
 constexpr int attn_fwd_lds_bytes()
 {
     constexpr int QKB = (MODE != MODE_BF16) ? 1 : 2;
@@ -168,13 +168,13 @@ constexpr int attn_fwd_lds_bytes()
 // The kernel body.  lds: attn_fwd_lds_bytes<...>() bytes of workgroup memory, 16-byte aligned;
 // wg_linear: this workgroup's index in [0, p.total) (the entry points below and the named entry
 // points of the loadable code object derive it from their grids).
-template <int D, int NW, bool CAUSAL, bool HAS_MASK, int MODE, bool PER_KEY, bool OUT_F32, bool DBG>
+template <int D, bool CAUSAL, bool HAS_MASK, int MODE, bool PER_KEY, bool OUT_F32, bool DBG>
 __device__ __forceinline__ void attn_fwd_body(const AttnParams &p, unsigned char *lds, int wg_linear)
 {
-    constexpr int QW = NW;      // waves of a workgroup, each with 32 queries of its own
+    constexpr int QW = 4;       // waves of a workgroup, each with 32 queries of its own
     constexpr int NSTAGE = 2;
     constexpr int NSLOT = 1;    // register sets for tiles in flight
-    constexpr int T = NW * 64;
+    constexpr int T = QW * 64;
     constexpr int BQ = QW * 32;
     constexpr int QK_BYTES = (MODE != MODE_BF16) ? 1 : 2;        // bytes per q/k element
     constexpr int KROW = D * QK_BYTES + 16;                    // padded K row in LDS
@@ -196,7 +196,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnParams &p, unsigned char
     static_assert(!PER_KEY || MODE != MODE_BF16, "per-key scales belong to the 8-bit paths");
     static_assert(!DBG || MODE == MODE_I8, "the logits export is int32");
 
-    static_assert(NSTAGE * STAGE == attn_fwd_lds_bytes<D, NW, MODE, PER_KEY>(), "LDS size bookkeeping");
+    static_assert(NSTAGE * STAGE == attn_fwd_lds_bytes<D, MODE, PER_KEY>(), "LDS size bookkeeping");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -628,11 +628,11 @@ __device__ __forceinline__ void attn_fwd_body(const AttnParams &p, unsigned char
     }
 }
 
-template <int D, int NW, bool CAUSAL, bool HAS_MASK, int MODE, bool PER_KEY, bool OUT_F32, bool DBG>
-__global__ void __launch_bounds__(NW * 64, (NW == 4 ? 2 : 1)) attn_fwd_kernel(const AttnParams p)
+template <int D, bool CAUSAL, bool HAS_MASK, int MODE, bool PER_KEY, bool OUT_F32, bool DBG>
+__global__ void __launch_bounds__(256, 2) attn_fwd_kernel(const AttnParams p)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<D, NW, MODE, PER_KEY>()];
-    attn_fwd_body<D, NW, CAUSAL, HAS_MASK, MODE, PER_KEY, OUT_F32, DBG>(p, lds, (int)blockIdx.x);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[attn_fwd_lds_bytes<D, MODE, PER_KEY>()];
+    attn_fwd_body<D, CAUSAL, HAS_MASK, MODE, PER_KEY, OUT_F32, DBG>(p, lds, (int)blockIdx.x);
 }
 
 }  // namespace arhip

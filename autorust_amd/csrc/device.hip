@@ -118,7 +118,11 @@ extern "C" int arhip_open(int ordinal, arhip_device **out)
     d->ordinal = ordinal;
     d->arch = arch;
     d->cus = prop.multiProcessorCount;
-    if (const char *e = getenv("ARHIP_ATTN_WAVES")) d->attn_waves = atoi(e);
+    if (const char *e = getenv("ARHIP_ATTN_WAVES")) {
+        const int w = atoi(e);
+        if (w == 4 || w == 8 || w == 40) d->attn_waves = w;
+        else fprintf(stderr, "arhip_open: ARHIP_ATTN_WAVES=%s is ignored (4, 8 or 40)\n", e);
+    }
     hipError_t e = hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&d->ev0);
     if (e == hipSuccess) e = hipEventCreate(&d->ev1);

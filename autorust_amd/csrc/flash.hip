@@ -45,24 +45,24 @@ static int check_common(const char *fn, arhip_device *dev, const void *q, const 
     return ARHIP_OK;
 }
 
-// CAUSAL / HAS_MASK dispatch for one tiling variant.
-template <int D, int NW, int MODE, bool PER_KEY, bool OUT_F32, bool DBG, bool MASKS>
+// CAUSAL / HAS_MASK dispatch of the general kernel.
+template <int D, int MODE, bool PER_KEY, bool OUT_F32, bool DBG, bool MASKS>
 static void launch_attn(hipStream_t stream, const AttnParams &p, bool causal, bool has_mask)
 {
-    const dim3 grid((unsigned)p.total), block(NW * 64);
+    const dim3 grid((unsigned)p.total), block(256);
     if constexpr (MASKS) {
         if (has_mask) {
             if (causal)
-                hipLaunchKernelGGL((attn_fwd_kernel<D, NW, true, true, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
+                hipLaunchKernelGGL((attn_fwd_kernel<D, true, true, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
             else
-                hipLaunchKernelGGL((attn_fwd_kernel<D, NW, false, true, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
+                hipLaunchKernelGGL((attn_fwd_kernel<D, false, true, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
             return;
         }
     }
     if (causal)
-        hipLaunchKernelGGL((attn_fwd_kernel<D, NW, true, false, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((attn_fwd_kernel<D, true, false, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
     else
-        hipLaunchKernelGGL((attn_fwd_kernel<D, NW, false, false, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((attn_fwd_kernel<D, false, false, MODE, PER_KEY, OUT_F32, DBG>), grid, block, 0, stream, p);
 }
 
 // The software-pipelined kernel (no additive mask): 8 waves per workgroup, or 4 (two workgroups per compute
@@ -263,9 +263,9 @@ extern "C" int arhip_flash_fwd_lse(arhip_device *dev, const void *q, const void 
         if (hm) launch_pipe_bf16_mask(dev->stream, p, (int)D, c, nw);
         else launch_pipe_bf16(dev->stream, p, (int)D, c, nw);
     } else if (D == 64) {
-        launch_attn<64, 4, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
+        launch_attn<64, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
     } else {
-        launch_attn<128, 4, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
+        launch_attn<128, MODE_BF16, false, false, false, true>(dev->stream, p, c, hm);
     }
     arhip_note_selected(ARHIP_K_FLASH_BF16);
     return t.end();
@@ -354,25 +354,25 @@ static int sage_fwd_impl(arhip_device *dev, const int8_t *q8, const int8_t *k8,
     arhip_call_timer t{dev, wait, secs};
     t.kernel = ARHIP_K_SAGE;
     if (int rc = t.begin()) return rc;
-#define SAGE_V(DD, NWW, PK, DB_, MK)                                                                   \
+#define SAGE_V(DD, PK, DB_, MK)                                                                   \
     do {                                                                                               \
-        if (f32o) launch_attn<DD, NWW, MODE_I8, PK, true, DB_, MK>(dev->stream, p, c, hm);             \
-        else launch_attn<DD, NWW, MODE_I8, PK, false, DB_, MK>(dev->stream, p, c, hm);                 \
+        if (f32o) launch_attn<DD, MODE_I8, PK, true, DB_, MK>(dev->stream, p, c, hm);             \
+        else launch_attn<DD, MODE_I8, PK, false, DB_, MK>(dev->stream, p, c, hm);                 \
     } while (0)
 #define SAGE_D(DD)                                                                                     \
     do {                                                                                               \
         if (dbg) {                                                                                     \
-            if (per_key) SAGE_V(DD, 4, true, true, false);                                             \
-            else SAGE_V(DD, 4, false, true, false);                                                    \
+            if (per_key) SAGE_V(DD, true, true, false);                                             \
+            else SAGE_V(DD, false, true, false);                                                    \
         } else if (pipe && pipe_keys) launch_pipe_i8_keys(dev->stream, p, DD, c, nw);                  \
-        else if (per_key) SAGE_V(DD, 4, true, false, true);                                            \
+        else if (per_key) SAGE_V(DD, true, false, true);                                            \
         else if (pipe) launch_pipe_i8(dev->stream, p, DD, c, nw);                                      \
-        else SAGE_V(DD, 4, false, false, true);                                                        \
+        else SAGE_V(DD, false, false, true);                                                        \
     } while (0)
 #define SAGE_F(DD, PK)                                                                                 \
     do {                                                                                               \
-        if (f32o) launch_attn<DD, 4, MODE_FP8, PK, true, false, true>(dev->stream, p, c, hm);          \
-        else launch_attn<DD, 4, MODE_FP8, PK, false, false, true>(dev->stream, p, c, hm);              \
+        if (f32o) launch_attn<DD, MODE_FP8, PK, true, false, true>(dev->stream, p, c, hm);          \
+        else launch_attn<DD, MODE_FP8, PK, false, false, true>(dev->stream, p, c, hm);              \
     } while (0)
     if (fp8 && pipe) {
         if (pipe_keys) launch_pipe_fp8_keys(dev->stream, p, (int)D, c, nw);

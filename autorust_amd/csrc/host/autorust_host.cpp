@@ -332,7 +332,7 @@ uint64_t selections(Kernel k) { return k == Kernel::None ? 0 : g_selected[(int)k
 static void note_selected(Kernel k)
 {
     static std::once_flag once[3];
-    static const char *what[3] = {"[attention] flash: fp32 exact, fp32 MFMA (gfx950)",
+    static const char *what[3] = {"[attention] flash: fp32 exact, operands in three parts on the bf16 MFMA (gfx950)",
                                   "[attention] flash: bf16 MFMA, software-pipelined for long sequences (gfx950)",
                                   "[attention] sage: int8 MFMA for q.k^T, bf16 MFMA for p.v, K smoothing + block scales (gfx950)"};
     g_selected[(int)k].fetch_add(1, std::memory_order_relaxed);

@@ -94,7 +94,7 @@ pub fn note_selected(kind: usize) {
             eprintln!(
                 "{}",
                 [
-                    "[attention] flash: fp32 exact, fp32 MFMA (gfx950)",
+                    "[attention] flash: fp32 exact, operands in three parts on the bf16 MFMA (gfx950)",
                     "[attention] flash: bf16 MFMA, software-pipelined for long sequences (gfx950)",
                     "[attention] sage: int8 MFMA for q.k^T, bf16 MFMA for p.v, K smoothing + block scales (gfx950)",
                 ][kind]

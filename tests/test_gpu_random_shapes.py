@@ -1,7 +1,7 @@
 """Seeded random sweep over shapes, head groupings, masks and tiling variants: every case is
 compared with the float64 oracle.  The tiling variant does not change the function, so the
-same case is also run with the tiling forced (the general kernel with 1 and 4 waves, the pipelined one with
-8 and, "40", 4 waves): ARHIP_ATTN_WAVES is read
+same case is also run with the tiling forced ("4": the general kernel, "8" and "40": the pipelined one with 8 and 4
+waves; any other value is ignored): ARHIP_ATTN_WAVES is read
 when a device is opened, so those runs open a device handle of their own."""
 import contextlib
 
