@@ -28,7 +28,7 @@ from autorust_amd import _lib, synth  # noqa: E402
 from autorust_amd.device import BF16, F32, Device  # noqa: E402
 
 PEAK_BF16 = 2500.0   # TFLOP/s, MI355X dense bf16 MFMA
-PEAK_F32 = 157.3     # TFLOP/s, MI355X dense fp32 MFMA
+PEAK_F32 = PEAK_BF16 / 6   # TFLOP/s of the fp32 kernels: an fp32 product is six products of bf16 parts on the bf16 MFMA
 PEAK_INT8 = 5000.0   # TOP/s, MI355X dense int8 MFMA (dense fp8 MFMA: the same 5000 TFLOP/s)
 PEAK_HBM = 8000.0    # GB/s, MI355X HBM3E
 
@@ -185,7 +185,7 @@ class FlashWorkload:
                            kv_len=self.kv, causal=self.causal, wait=False)
 
     def roofline(self, secs):
-        # the bound is the larger of ops / matrix peak and bytes / HBM rate (fp32 tensors: fp32 MFMA peak)
+        # the bound is the larger of ops / matrix peak and bytes / HBM rate (fp32 tensors: a sixth of the bf16 MFMA peak)
         ai = self.ops / self.kernel_bytes
         peak = PEAK_BF16 if self.dt == BF16 else PEAK_F32
         if ai > peak * 1e12 / (PEAK_HBM * 1e9):
@@ -193,7 +193,7 @@ class FlashWorkload:
             kern = "flash_f32_kernel" if self.dt != BF16 else "attn_pipe_kernel<bf16>"
             return {"bound": "mfma", "achieved": ach, "peak": peak, "unit": "TFLOP/s", "frac": ach / peak,
                     "traffic": None, "kernel": kern, "launch_ms": secs * 1e3, "ops_per_launch": self.ops,
-                    "peak_note": "dense %s MFMA" % self.dtype}
+                    "peak_note": "dense bf16 MFMA" + ("" if self.dt == BF16 else ", six products per fp32 product")}
         ach = self.kernel_bytes / secs / 1e9
         return {"bound": "hbm", "achieved": ach, "peak": PEAK_HBM, "unit": "GB/s", "frac": ach / PEAK_HBM,
                 "traffic": None, "kernel": "attn_pipe_kernel<bf16>" if self.dt == BF16 else "flash_f32_kernel",
@@ -236,7 +236,7 @@ class TrainWorkload:
         ach = bwd_ops / secs / 1e12
         return {"bound": "mfma", "achieved": ach, "peak": PEAK_F32, "unit": "TFLOP/s", "frac": ach / PEAK_F32,
                 "traffic": None, "kernel": "bwd_prep + bwd_dq + bwd_dkv (f32)", "launch_ms": secs * 1e3,
-                "ops_per_launch": bwd_ops, "peak_note": "dense fp32 MFMA"}
+                "ops_per_launch": bwd_ops, "peak_note": "dense bf16 MFMA, six products per fp32 product"}
 
     def free(self):
         for b in (self.dq, self.dk, self.dv, self.ddo, self.o, self.gq, self.gk, self.gv, self.lse, self.delta):
