@@ -17,8 +17,8 @@
 //   blocks: inside a tile the online softmax advances 32 keys at a time and the
 //           wave alternates between the matrix pipe and the vector ALU; every
 //           LDS fragment is requested one phase before the MFMAs that use it.
-//           With 8 waves per workgroup each SIMD holds two waves, and one of
-//           them can exponentiate while the other multiplies.
+//           With two workgroups on a compute unit each SIMD holds two waves,
+//           and one of them can exponentiate while the other multiplies.
 //   lazy  : the exponent reference only moves (and the accumulators are only
 //           rescaled) when a row maximum outgrows it by 2^60; softmax does not
 //           depend on the reference, so the result is the same function.

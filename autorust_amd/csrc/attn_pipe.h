@@ -1,6 +1,5 @@
-// Fused attention forward on gfx950: the software-pipelined kernel, which serves every launch without an
-// additive mask or the logits export (attn_fwd_kernel, attn_fwd.h, keeps those), bf16, int8 and FP8 E4M3
-// operands, K scales over whole 64-key tiles or per key (PER_KEY), the Q quantiser of the int8 path inside its
+// Fused attention forward on gfx950: the software-pipelined kernel: bf16 operands, with an additive mask too (HAS_MASK),
+// int8 and FP8 E4M3 operands without one (attn_fwd_kernel, attn_fwd.h, keeps those and the logits export), K scales over whole 64-key tiles or per key (PER_KEY), the Q quantiser of the int8 path inside its
 // prologue on request (QFUSE).  Same arithmetic and MFMA decomposition as attn_fwd_kernel (S^T = K . Q^T, one
 // query per lane, O^T += V^T . P^T), different plumbing:
 //

@@ -20,10 +20,14 @@
 // A staged tile is split once and read twice, by rows for the first products and by columns (transposing reads) for the second.
 // The factor `scale` of dS is applied to the sums at the end.
 //
-// Bound: the matrix pipe (seven products of 2 N^2 D per head for the five of the mathematics: S and dP are formed in both
-// kernels).  Against the same kernels on v_mfma_f32_32x32x2_f32, whole backward: B2 H16 N2048 D128 2026 -> 1131 us, causal
-// 1119 -> 610 us, D64 992 -> 579 us, B8 H6 N789 D64 causal 201 -> 120 us, B8 H12 N197 D64 78 -> 46 us, B1 H12 N197 D64 30 -> 26 us;
-// relative error of dQ (2-norm, against float64) 1.07e-6 -> 9.4e-7 at N = 2048, 4.8e-7 -> 4.7e-7 at N = 197.
+// Bound: long sequences, the matrix pipe (seven products of 2 N^2 D per head for the five of the mathematics: S and dP are formed
+// in both kernels): B2 H16 N2048 D128 busy in 70 % of the SIMD cycles, 4.2 vector instructions per matrix instruction.  At B8 H6 N789
+// D64 33 % (dK/dV, one wave per SIMD) and 41 % (dQ): splitting, and few tiles per wave.
+// Against the same kernels on v_mfma_f32_32x32x2_f32, whole backward, microseconds on one card: B2 H16 N2048 D128 2038 -> 1096,
+// causal 1122 -> 594, D64 996 -> 570, causal D64 778 -> 332, B8 H6 N789 D64 347 -> 213, B8 H12 N197 D64 85 -> 51, B1 H12 N197 D64
+// 34 -> 21, B1 H4 N4096 D128 causal 623 -> 487, with a mask B2 H12 N1024 D64 399 -> 195.  Relative error (2-norm, against float64)
+// of dQ, dK, dV: N789 5.8, 5.7, 5.5e-7 -> 5.3, 5.2, 5.1e-7; B1 H16 N2048 D128 8.0, 8.0, 7.7e-7 -> 7.8, 7.8, 7.7e-7; of dQ at
+// B2 H16 N2048 D128 1.08e-6 -> 9.2e-7.
 #pragma once
 
 #include <hip/hip_runtime.h>

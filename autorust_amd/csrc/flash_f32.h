@@ -13,12 +13,16 @@
 //   result C[32 x 32]: lane holds column lane%32, rows 8*(r/4) + 4*(lane/32) + r%4
 // P is split in registers, in the order the S^T result left it there; Q is split once, K and V while they are staged.
 //
-// Bound: the matrix pipe, at a clock that its power draw sets.  Against the same kernel on v_mfma_f32_32x32x2_f32 (which
-// never runs beside a vector instruction): B2 H16 N2048 D128 639 -> 299 us (107 -> 230 TFLOP/s of attention, 1380 TFLOP/s of
-// bf16 products; a loop of nothing but such products on random data holds 1740 ... 1840), D64 290 -> 159 us, causal D128 352 ->
-// 187 us, B8 H6 N789 D64 87 -> 55 us, B8 H12 N197 D64 23.3 -> 16.5 us, B1 H12 N197 D64 9.9 -> 9.0 us.  Relative error (2-norm,
-// against float64) on the same inputs: 9.1e-7 -> 7.7e-7, 8.7e-7 -> 7.4e-7, 4.5e-7 -> 3.8e-7, 3.9e-7 -> 4.9e-7, 3.3e-7 -> 3.0e-7,
-// 3.1e-7 -> 2.4e-7.
+// Bound: long sequences, the matrix pipe at a clock that its power draw sets (B2 H16 N2048 D128: busy in 78 % of the SIMD cycles at
+// 1.6 GHz, 3.8 vector instructions per matrix instruction, no LDS bank conflicts; 220 TFLOP/s of attention are 1320 TFLOP/s of bf16
+// products, and a loop of nothing but such products on random data holds 1740 ... 1840).  Short ones, instruction issue and waiting:
+// B8 H6 N789 D64 41 % busy, 7.0 vector instructions per matrix instruction (splitting three tiles before the first product, TILE_SUMS,
+// the last tile's key tests), waves waiting in 34 % of their cycles.
+// Against the same kernel on v_mfma_f32_32x32x2_f32 (which never runs beside a vector instruction), microseconds on one card:
+// B2 H16 N2048 D128 647 -> 312, D64 295 -> 167, causal D128 354 -> 193, causal D64 217 -> 114, B1 H16 N2048 D128 386 -> 203, B8 H6
+// N789 D64 98 -> 64, B8 H12 N197 D64 27 -> 20, B1 H12 N197 D64 12.5 -> 11.6, with a mask B2 H12 N1024 D64 116 -> 76.  Relative error
+// (2-norm, against float64) on the same inputs: B2 H16 N2048 D128 9.1e-7 -> 7.8e-7, D64 8.7e-7 -> 7.4e-7, causal D128 4.5e-7 ->
+// 3.8e-7, B1 H16 N2048 D128 5.8e-7 -> 3.8e-7, N789 3.9e-7 -> 2.6e-7, N197 3.3e-7 -> 2.3e-7 (B8), 3.1e-7 -> 2.4e-7 (B1).
 // Tried on B2 H16 N2048 (D64 / D128): the same loop with the phases one after the other, as the compiler schedules them
 // 184 / 402 us; interleaved by hand but with the compiler free to sink vector work past the matrix instructions 178 / 331 us;
 // values pinned where they are computed 168 / 336 us; tiles through registers instead of straight to LDS 168 / 325 us; a row
