@@ -675,13 +675,13 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     // 206 / 212, B8 H16 N1024 771 / 811; four heads to a K/V head, B8 H24 N197 60.7 / 60.9, B3 H8 N1000 causal 183 / 193.
     // (O may lie where a result or the row scalar goes: then it has to be read before they are written)
     const uintptr_t q_bytes = (uintptr_t)rows * D * 4, kv_bytes = (uintptr_t)(B * Hkv * N) * D * 4;
-    auto apart = [&](const void *x, uintptr_t bytes) {
-        const uintptr_t a = (uintptr_t)o, b = (uintptr_t)x;
-        return a + q_bytes <= b || b + bytes <= a;
+    auto apart = [](const void *x, uintptr_t x_bytes, const void *y, uintptr_t y_bytes) {
+        const uintptr_t a = (uintptr_t)x, b = (uintptr_t)y;
+        return a + x_bytes <= b || b + y_bytes <= a;
     };
     // (Head size 128 on 32 rows per workgroup has no registers for a third tensor.)
-    const bool own_d = mask == nullptr && !(D == 128 && split) && Hq / Hkv * N <= 512 && apart(dq, q_bytes) && apart(dk, kv_bytes) && apart(dv, kv_bytes) &&
-                       apart(delta, (uintptr_t)rows * 4);
+    const bool own_d = mask == nullptr && !(D == 128 && split) && Hq / Hkv * N <= 512 && apart(o, q_bytes, dq, q_bytes) && apart(o, q_bytes, dk, kv_bytes) &&
+                       apart(o, q_bytes, dv, kv_bytes) && apart(o, q_bytes, delta, (uintptr_t)rows * 4);
     if (own_d) {
         p.o = o;
         p.delta_out = delta;
@@ -691,9 +691,25 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
         if (D == 64) hipLaunchKernelGGL((bwd_prep_kernel<64>), prep_grid, block, 0, dev->stream, o, dout, delta, rows);
         else hipLaunchKernelGGL((bwd_prep_kernel<128>), prep_grid, block, 0, dev->stream, o, dout, delta, rows);
     }
-    if (mask != nullptr) launch_f32_bwd_mask(dev->stream, p, (int)D, causal != 0, split);
-    else if (D == 64) launch_f32_bwd_64(dev->stream, p, causal != 0, split);
-    else launch_f32_bwd_128(dev->stream, p, causal != 0, split);
+    auto launch = [&]() {
+        if (mask != nullptr) launch_f32_bwd_mask(dev->stream, p, (int)D, causal != 0, split);
+        else if (D == 64) launch_f32_bwd_64(dev->stream, p, causal != 0, split);
+        else launch_f32_bwd_128(dev->stream, p, causal != 0, split);
+    };
+    // dK and dV may lie where K and V do, of which a dK/dV workgroup reads the rows that it writes; those of dQ read all of them, first
+    bool kv_kept = true;
+    for (const float *out : {dk, dv})
+        for (const float *in : {k, v}) kv_kept &= apart(out, kv_bytes, in, kv_bytes);
+    if (kv_kept) {
+        launch();
+    } else {
+        const int total_kv = p.total_kv;
+        p.total_kv = 0;
+        launch();
+        p.total_kv = total_kv;
+        p.total_q = 0;
+        launch();
+    }
     arhip_note_selected(ARHIP_K_FLASH_BWD);
     return t.end();
 }

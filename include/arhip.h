@@ -174,7 +174,8 @@ int arhip_flash_fwd_lse(arhip_device *dev, const void *q, const void *k, const v
  *   arhip_flash_fwd_lse(dtype = ARHIP_F32) produced for the same q, k, v, mask, kv_len, causal and
  *   scale.  dq [B,Hq,N,D], dk and dv [B,Hkv,N,D] are written in full (no zero-fill needed: the
  *   sum over a GQA group happens inside the kernel, in a fixed order, without atomics).  delta is a
- *   caller-provided scratch of B*Hq*N floats.  D is 64 or 128 (the reference: 64). */
+ *   caller-provided scratch of B*Hq*N floats.  dk and dv may be k and v, and dq may be o.  D is 64 or 128 (the
+ *   reference: 64). */
 int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k, const float *v, const float *o,
                     const float *lse, const float *dout, float *dq, float *dk, float *dv, float *delta,
                     const float *mask, const int32_t *kv_len,
