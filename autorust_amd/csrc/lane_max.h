@@ -1,4 +1,4 @@
-// Maxima over groups of lanes without LDS: a __shfl_xor is an LDS round trip of some 100 cycles, and a reduction is a chain of
+// Maxima and sums over groups of lanes without LDS: a __shfl_xor is an LDS round trip of some 100 cycles, and a reduction is a chain of
 // them; the vector ALU's own lane exchanges take a few cycles each.
 #pragma once
 
@@ -37,6 +37,24 @@ __device__ __forceinline__ float lane_group_max(float x)
         x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
     }
     return x;
+}
+
+// x, the same in every lane, as a scalar
+__device__ __forceinline__ float wave_value(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
+
+// sum of x over the 64 lanes, in every lane
+__device__ __forceinline__ float lane_sum(float x)
+{
+    x += dpp_read<0xB1>(x);
+    x += dpp_read<0x4E>(x);
+    x += dpp_read<0x141>(x);
+    x += dpp_read<0x140>(x);
+    uint32_t u = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    u = __float_as_uint(x);
+    const auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __uint_as_float(t[0]) + __uint_as_float(t[1]);
 }
 
 }  // namespace arhip
