@@ -11,6 +11,7 @@ import oracle
 from autorust_amd import synth
 from autorust_amd.device import F32
 from gpu_util import run_flash
+from test_gpu_bwd import run_fwd_bwd
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +70,44 @@ def test_forward_zero_channels(dev, shape):
     got = run_flash(dev, q, k, v, F32)
     close(got, oracle.sdpa_f64(*heads(q, k, v)), TOL)
     assert (got[..., 41:] == 0).all()
+
+
+def difference_terms(q, k, v, do, mask=None, causal=False):
+    """What dQ and dK are sums of before dP and D cancel: P (|dO| . |V| + |D|) scale times |K| and |Q|."""
+    q, k, v, do = heads(q, k, v, do)
+    s = q @ k.swapaxes(-1, -2) / np.sqrt(q.shape[-1]) + (0 if mask is None else mask.astype(np.float64))
+    if causal:
+        s = np.where(np.tri(q.shape[2], dtype=bool), s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    d = np.abs((p @ v * do).sum(-1, keepdims=True))
+    t = p * (np.abs(do) @ np.abs(v).swapaxes(-1, -2) + d) / np.sqrt(q.shape[-1])
+    return t @ np.abs(k), t.swapaxes(-1, -2) @ np.abs(q), np.zeros_like(v)
+
+
+def check_backward(dev, q, k, v, do, tol=TOL, mask=None, causal=False, rows=slice(None), only=("dq", "dk", "dv")):
+    """Rows and channels of dq, dk, dv (of the rows `rows`) by their own norms, and four roundings of 2^-24 of the terms that cancel in them."""
+    got = run_fwd_bwd(dev, q, k, v, do, mask=mask, causal=causal)
+    want = oracle.attention_backward_f64(*heads(q, k, v, do), mask=mask, causal=causal)
+    terms = difference_terms(q, k, v, do, mask=mask, causal=causal)
+    for name, g, w, t in zip(("dq", "dk", "dv"), got[2:], want[2:], terms):
+        if name not in only:
+            continue
+        g, w, t = g[:1, :2, rows].astype(np.float64), np.asarray(w, np.float64)[:, :, rows], t[:, :, rows]
+        assert np.isfinite(g).all(), name
+        for axis in (-1, -2):
+            err, ref, cancel = (np.linalg.norm(x, axis=axis) for x in (g - w, w, t))
+            bound = tol * ref + 2.0 ** -22 * cancel
+            assert (err <= bound).all(), (name, axis, (err[bound > 0] / bound[bound > 0]).max() * tol)
+
+
+@pytest.mark.parametrize("which", ["q", "dout"])
+@pytest.mark.parametrize("e", [20, 30, 38])
+@pytest.mark.parametrize("N, causal", [(9, False), (16, False), (32, False), (129, True), (160, True), (257, True)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_backward_a_single_tile_of_queries(dev, D, N, causal, e, which):
+    """Key blocks that see no second tile of queries (all of N <= 32, the last one of a causal head): channels 8 .. 15 of Q, or of dO, 2^-e of the
+    others come out in dK and dV as they should."""
+    q, k, v, do = (synth.normal(985 + i, (8, 16, N, D)) for i in range(4))
+    (q if which == "q" else do)[..., 8:16] *= F(2.0 ** -e)
+    check_backward(dev, q, k, v, do, causal=causal, rows=slice(N - 1 - (N - 1) % 128, None), only=("dk", "dv"))
