@@ -111,3 +111,32 @@ def test_backward_a_single_tile_of_queries(dev, D, N, causal, e, which):
     q, k, v, do = (synth.normal(985 + i, (8, 16, N, D)) for i in range(4))
     (q if which == "q" else do)[..., 8:16] *= F(2.0 ** -e)
     check_backward(dev, q, k, v, do, causal=causal, rows=slice(N - 1 - (N - 1) % 128, None), only=("dk", "dv"))
+
+
+@pytest.mark.parametrize("how", ["key", "mask", "one key"])
+@pytest.mark.parametrize("gap, causal", [(8, False), (14, False), (20, False), (28, False), (20, True)])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_backward_keys_that_few_attend_to(dev, shape, gap, causal, how):
+    """Every other key, or a single one, `gap` below the others in the logits, by K or by an additive mask: its rows of dK and dV are made of small probabilities alone."""
+    N = shape[2]
+    q, k, v, do = (synth.normal(990 + i, shape) for i in range(4))
+    mask = None
+    if how == "mask":
+        mask = np.zeros((N, N), F)
+        mask[:, ::2] = -gap
+    else:
+        q[..., 0], k[..., 0] = 4, 0
+        k[..., slice(0, None, 2) if how == "key" else N // 2, 0] = -gap / 4 * np.sqrt(shape[3])
+    # (causal: query 0 sees key 0 alone, which all later ones avoid; its difference of dP and D is nothing but roundings)
+    check_backward(dev, q, k, v, do, TOL + gap * 2.0 ** -19, mask=mask, causal=causal, rows=slice(1 if causal else 0, None), only=("dk", "dv"))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("e", [14, 20, 28])
+@pytest.mark.parametrize("which", ["q", "dout"])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_backward_small_rows(dev, shape, which, e, causal):
+    """The later half of the rows of Q, or of dO, 2^-e of the earlier: under the causal mask late keys see no others."""
+    q, k, v, do = (synth.normal(995 + i, shape) for i in range(4))
+    (q if which == "q" else do)[..., shape[2] // 2:, :] *= F(2.0 ** -e)
+    check_backward(dev, q, k, v, do, causal=causal)
