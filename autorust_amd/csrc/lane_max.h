@@ -43,6 +43,12 @@ __device__ __forceinline__ float lane_group_max(float x)
 __device__ __forceinline__ float wave_value(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 
 // sum of x over the 64 lanes, in every lane
+__device__ __forceinline__ float xrow_max(float x)  // of lane and lane ^ 16
+{
+    const uint32_t u = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 __device__ __forceinline__ float lane_sum(float x)
 {
     x += dpp_read<0xB1>(x);

@@ -140,3 +140,27 @@ def test_backward_small_rows(dev, shape, which, e, causal):
     q, k, v, do = (synth.normal(995 + i, shape) for i in range(4))
     (q if which == "q" else do)[..., shape[2] // 2:, :] *= F(2.0 ** -e)
     check_backward(dev, q, k, v, do, causal=causal)
+
+
+@pytest.mark.parametrize("e", [10, 14, 20, 30])
+@pytest.mark.parametrize("shape, causal", [(s, False) for s in SHAPES] + [(s, True) for s in SHAPES + [(8, 16, 129, 64), (8, 16, 129, 128)]], ids=str)
+def test_backward_wide_channels(dev, shape, causal, e):
+    """Every eighth channel of an operand 2^e times the rest, with its counterpart in a product the other way or not: the other channels of the results."""
+    q, k, v, do = (synth.normal(1000 + i, shape) for i in range(4))
+    up = np.where(np.arange(shape[3]) % 8 == 0, F(2.0 ** e), F(1))
+    for x in ((q / up, k * up, v, do), (q * up, k / up, v, do), (q, k, v * up, do), (q, k, v, do * up), (q, k, v / up, do * up), (q, k, v * up, do / up)):
+        # (causal: query 0 sees one key, its difference of dP and D is nothing but roundings)
+        check_backward(dev, *x, causal=causal, rows=slice(1 if causal else 0, None))
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v", "dout", "all"])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_backward_zero_channels(dev, shape, which):
+    """Padding: channels that are zero, in all operands or in one; and one row that has them, 2^-30 of the others."""
+    x = dict(zip(("q", "k", "v", "dout"), (synth.normal(1010 + i, shape) for i in range(4))))
+    for name in x if which == "all" else [which]:
+        x[name][..., 41:] = 0
+    check_backward(dev, *x.values())
+    if which != "all" and shape[2] <= 257:
+        x[which][..., 3, 41:] = F(2.0 ** -30)
+        check_backward(dev, *x.values())
