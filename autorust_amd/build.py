@@ -6,6 +6,7 @@
 hipcc cross-compiles without a GPU.  The library lands in-tree
 (autorust_amd/libarhip.so) so that it travels with the source tree.
 """
+import hashlib
 import os
 import struct
 import subprocess
@@ -55,12 +56,21 @@ def _run(cmd):
         sys.stderr.write(out + "\n")
 
 
+def _entries_id(files):
+    """Of the sources that the named entry points are built from: a symbol of this name in their code objects tells libarhip.so that they are its own."""
+    h = hashlib.sha256()
+    for f in files:
+        h.update(open(f, "rb").read())
+    return "arhip_entries_" + h.hexdigest()[:16]
+
+
 def build(force=False, verbose=False):
     noise = "is not a recognized feature for this target"
     srcs = [os.path.join(CSRC, s) for s in SOURCES]
     headers = [os.path.join(CSRC, h) for h in HEADERS]
-    deps = srcs + headers + [os.path.abspath(__file__)]
     entry_src = os.path.join(CSRC, "attn_entry.hip")
+    deps = srcs + headers + [entry_src, os.path.abspath(__file__)]
+    mark = "-DARHIP_ENTRIES_ID=" + _entries_id([entry_src] + headers)
     probe_src = os.path.join(CSRC, "probes.hip")
     # every hipcc job that is due is queued (the objects of libarhip.so, the parts of the entry-point code object, the
     # probes) and MAX_JOBS of them run at a time, in the order queued
@@ -74,12 +84,12 @@ def build(force=False, verbose=False):
         for s in srcs:
             o = s[:-4] + ".o"
             objs.append(o)
-            start([HIPCC] + FLAGS + ["-c", s, "-o", o])
+            start([HIPCC] + FLAGS + [mark, "-c", s, "-o", o])
     parts = []
     if force or _newer(KERNELS, [entry_src] + headers):
         for k in range(1, ENTRY_PARTS + 1):
             parts.append(os.path.join(CSRC, "attn_entry.part%d.co" % k))
-            start([HIPCC] + FLAGS + ["-DARHIP_ENTRY_PART=%d" % k, "--genco", entry_src, "-o", parts[-1]])
+            start([HIPCC] + FLAGS + [mark, "-DARHIP_ENTRY_PART=%d" % k, "--genco", entry_src, "-o", parts[-1]])
     if os.path.exists(probe_src) and (force or _newer(PROBES, [probe_src])):
         start([HIPCC] + FLAGS + ["--genco", probe_src, "-o", PROBES])
     failed = False

@@ -21,6 +21,7 @@ struct arhip_module_entry {
     struct kernel {
         hipFunction_t fn;
         const void *entry;  // what a launch of this name must look like (device.hip), or null
+        bool own;           // of a code object that was built with this library
     };
     std::map<std::string, kernel, std::less<>> fns;  // (found by std::string_view)
 };

@@ -40,7 +40,7 @@
 //     ar_flash_sage_fp8_long_lens, ar_flash_sage_fp8_mid_lens                 (Q8, K8, V, O, M, L, SQ, SK,  ints as above)
 // (The reference's fused kernels take a dense [n, n] mask only, src/models/flash_attention.rs:389-396; its
 // Tensor API reaches key-padding masks through the general path, src/tensor/mod.rs:2405-2447.)
-// arhip_launch checks a launch by one of these names and, where the typed entries would take a form that no kernel of this file has (fp32: 32, 128
+// arhip_launch checks a launch by one of these names and, for the code objects of its own build and where the typed entries would take a form that no kernel of this file has (fp32: 32, 128
 // or 256 queries per workgroup with the registers of one head size; two groups of waves), launches that form on the same arguments.
 // head_dim must be 64 or 128; any other value makes the kernel return without writing.
 // The *_long entries address K and V with 32-bit byte offsets: (N + 320) * head_dim * 2 < 2^31.
@@ -58,6 +58,10 @@
 #define ARHIP_ENTRY_PART 0
 #endif
 #define ARHIP_PART(k) (ARHIP_ENTRY_PART == 0 || ARHIP_ENTRY_PART == (k))
+// of the same sources as the library, which looks for a symbol of this name before it launches a form of its own (arhip_launch)
+#ifdef ARHIP_ENTRIES_ID
+extern "C" __device__ __attribute__((used)) const int ARHIP_ENTRIES_ID = 1;
+#endif
 
 using namespace arhip;
 

@@ -508,6 +508,22 @@ const named_entry *find_named_entry(const char *name)
     return nullptr;
 }
 
+// Whether a code object is of the same sources as this library: only then is one of its kernels as good as another (a caller's own kernel of
+// the same name, or an older build's, is what is to run).
+bool built_with_library(hipModule_t mod)
+{
+#ifdef ARHIP_ENTRIES_ID
+#define ARHIP_TEXT_(x) #x
+#define ARHIP_TEXT(x) ARHIP_TEXT_(x)
+    hipDeviceptr_t at = nullptr;
+    size_t size = 0;
+    return hipModuleGetGlobal(&at, &size, mod, ARHIP_TEXT(ARHIP_ENTRIES_ID)) == hipSuccess;
+#else
+    (void)mod;
+    return false;
+#endif
+}
+
 int check_named_entry(const named_entry *e, const char *name, const unsigned grid[3], const unsigned block[3], int nbufs,
                       const int64_t *vals, int nvals)
 {
@@ -566,15 +582,18 @@ extern "C" int arhip_launch(arhip_device *dev, void *module, const char *name,
     auto it = m->fns.find(std::string_view(name));
     if (it == m->fns.end()) {
         hipError_t err = hipErrorNotFound;
+        bool own = false;
         for (hipModule_t mod : m->mods) {
             err = hipModuleGetFunction(&fn, mod, name);
-            if (err == hipSuccess) break;
+            if (err != hipSuccess) continue;
+            own = built_with_library(mod);
+            break;
         }
         (void)hipGetLastError();  // a miss in an earlier part of a container is not an error of this launch
         if (err != hipSuccess) {
             return arhip_fail(ARHIP_EHIP, "arhip_launch: no kernel named %s in the module: %s", name, hipGetErrorString(err));
         }
-        it = m->fns.emplace(name, arhip_module_entry::kernel{fn, find_named_entry(name)}).first;
+        it = m->fns.emplace(name, arhip_module_entry::kernel{fn, find_named_entry(name), own}).first;
     } else {
         fn = it->second.fn;
     }
@@ -609,7 +628,7 @@ extern "C" int arhip_launch(arhip_device *dev, void *module, const char *name,
     arhip_call_timer t{dev, wait, secs};
     if (int rc = t.begin()) return rc;
     const named_entry *e = (const named_entry *)it->second.entry;
-    if (e && e->family != ARHIP_NAMED_PLAIN &&
+    if (e && it->second.own && e->family != ARHIP_NAMED_PLAIN &&
         arhip_named_form(dev, e->family, e->rows, strstr(name, "_lens") != nullptr, grid, bufs, vals))
         return t.end();
     ARHIP_HIP(hipModuleLaunchKernel(fn, grid[0], grid[1], grid[2], block[0], block[1], block[2], 0,

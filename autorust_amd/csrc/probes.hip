@@ -84,6 +84,15 @@ extern "C" __global__ void probe_axpb(const float *x, float *y, int n)
 
 // Plain streaming copy of n 16-byte words: the calibration kernel for the HBM traffic
 // counters (its traffic is known: n*16 bytes read, n*16 bytes written).
+// A kernel of a host's own by the name of an attention entry: every row of O becomes its number
+extern "C" __global__ void ar_flash_f32(const float *, const float *, const float *, float *O, const float *, int n, int head_dim, int, int, int, int)
+{
+    for (int i = (int)threadIdx.x; i < 128 * head_dim; i += (int)blockDim.x) {
+        const int row = (int)blockIdx.x * 128 + i / head_dim;
+        if (row < n) O[((size_t)blockIdx.y * n + row) * head_dim + i % head_dim] = (float)row;
+    }
+}
+
 extern "C" __global__ void probe_copy(const uint4 *src, uint4 *dst, long n)
 {
     const long stride = (long)gridDim.x * blockDim.x;

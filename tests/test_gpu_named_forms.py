@@ -42,6 +42,18 @@ def test_f32(dev, kernels, case):
             assert lse.copyout(np.float32, q.shape[:3]).tobytes() == lse2.copyout(np.float32, q.shape[:3]).tobytes()
 
 
+@pytest.mark.parametrize("case", [c for c in F32_CASES if c[0] == "ar_flash_f32" and not c[7]], ids=str)
+def test_a_module_of_the_callers(dev, case):
+    """A kernel of one of these names in another module is the one that runs, also where the library's entry would take another form."""
+    probes = dev.module_load(open(_lib.PROBES_PATH, "rb").read())
+    name, B, Hq, Hkv, N, D = case[:6]
+    with Bufs(dev) as bufs:
+        o = bufs.new(B * Hq * N * D * 4)
+        dev.launch(probes, name, ((N + 127) // 128, B * Hq, 1), (256, 1, 1), [o, o, o, o, o], [N, D, 0, 0, Hq, Hkv])
+        got = o.copyout(np.float32, (B * Hq, N, D))
+        assert (got == np.arange(N, dtype=np.float32)[:, None]).all()
+
+
 # two groups of waves: 2 + 2 on 64 queries, 4 + 4 on 128
 PIPE_CASES = [(1, 8, 2, 1000, 64, False, None), (2, 4, 4, 513, 128, True, [513, 70]), (1, 16, 16, 2048, 64, False, None), (1, 16, 16, 2047, 128, True, None)]
 
