@@ -1,5 +1,6 @@
 """The fp32 kernels on operands whose values are far apart: fp32 operands are taken as two fp16 values each, scaled by the largest value
 of a row or of a stream of tiles, so these are the inputs on which a scale can be wrong.  Every tiling, against the float64 oracle.
+(Values that lose bits with nothing larger beside them, in single channels and rows: test_gpu_f32_lost_bits.py.)
 
 Bounds: a product of such operands is off by at most 2^-22 of itself and a sum of them by a few roundings of 2^-24, as long as the
 values that matter are within the window of the scale; outside of it the kernels take the fp32 matrix instruction.  Either way errors
@@ -12,6 +13,7 @@ from autorust_amd import synth
 from autorust_amd.device import F32
 from gpu_util import run_flash
 from test_gpu_bwd import run_fwd_bwd
+from test_gpu_f32_lost_bits import close_backward
 
 pytestmark = pytest.mark.gpu
 
@@ -28,7 +30,7 @@ def _inputs(shape, kind):
         for x in (k, v, do):
             x[..., 8:16] *= f(-20)
         q[..., 8:16] *= f(-18)
-    elif kind == "channels against each other":   # as much of every logit comes from either half of the channels
+    elif kind == "channels against each other":   # as much of every logit comes from either half of the channels; within the window
         q[..., : shape[3] // 2] *= f(9)
         k[..., : shape[3] // 2] *= f(-9)
     elif kind == "growing":                  # later rows 2^10 times the first tile's
@@ -78,12 +80,15 @@ def test_backward(dev, shape, kind, causal):
         ref = np.linalg.norm(w.astype(np.float64), axis=-2)
         # (a channel that cancels almost to nothing is held to the others)
         assert (err <= TOL * np.maximum(ref, 2.0 ** -21 * ref.max(axis=-1, keepdims=True))).all(), (name, (err / ref).max())
+    # and by rows.  (Causal: query 0 sees one key, its difference of dP and D is nothing but roundings.)
+    close_backward(got[2:], q, k, v, do, causal=causal, rows=slice(1 if causal else 0, None), axes=(-1,))
 
 
 @pytest.mark.parametrize("shape", [(8, 12, 63, 64), (1, 2, 300, 64), (8, 16, 512, 64), (8, 12, 63, 128), (1, 2, 512, 128), (8, 16, 300, 128)],
                          ids=str)
 def test_rows_of_dv_whose_keys_few_attend_to(dev, shape):
-    """Every other key has logits 8 below the rest: its row of dV is made of probabilities of 2^-20 alone.  Held to itself: a logit of 8 is
+    """Every other key has logits 8 below the rest: its row of dV is made of probabilities of 2^-20 alone, which two halves still hold (further
+    below, and dK: test_gpu_f32_lost_bits.py).  Held to itself: a logit of 8 is
     off by 2^-21 at most, its exponential by as much, and the probabilities' two halves end at 2^-39."""
     q, k, v, do = (synth.normal(77 + 10 ** 6 * i, shape) for i in range(4))
     q[..., 0] = 4

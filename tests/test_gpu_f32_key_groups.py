@@ -24,8 +24,10 @@ def test_forward(dev, case, wide):
     B, Hq, Hkv, N, causal, has_mask, lens = case
     D = 64
     q, k, v = (synth.normal(s, (B, H, N, D)) for s, H in ((31, Hq), (32, Hkv), (33, Hkv)))
-    if wide:  # rows that no common scale fits: the workgroups redo them in fp32
-        v = v * np.float32(2.0) ** np.random.default_rng(5).integers(-30, 31, (B, Hkv, N, 1)).astype(np.float32)
+    if wide:  # rows and channels that no common scale fits: the workgroups redo them in fp32
+        rng = np.random.default_rng(5)
+        v = v * np.float32(2.0) ** rng.integers(-30, 31, (B, Hkv, N, 1)).astype(np.float32)
+        v = v * np.float32(2.0) ** rng.integers(-15, 16, (B, Hkv, 1, D)).astype(np.float32)
     mask = synth.normal(34, (N, N)) if has_mask else None
     kv_len = np.array(lens, np.int32) if lens else None
     with Bufs(dev) as bufs:
@@ -41,6 +43,10 @@ def test_forward(dev, case, wide):
     want_lse = oracle.lse_f64(q, k, mask=mask, kv_len=kv_len, causal=causal)
     # |P error| is some 2^-20 of P (a logit of up to 8 carries 2^-21 of itself and the exponential a unit): 2^-19 of the largest |V| of the head
     bound = 2.0 ** -19 * np.abs(v).max(axis=(2, 3)).repeat(Hq // Hkv, axis=1)[:, :, None, None]
+    if wide:  # ... and of what the row sees in the channel
+        bound = 2.0 ** -19 * oracle.sdpa_f64(q, k, np.abs(v), mask=mask, kv_len=kv_len, causal=causal)
+        if lens:
+            bound[kv_len == 0] = 0.0
     assert (np.abs(got - want) <= bound).all()
     seen = np.isfinite(want_lse) & (want_lse > -1e29)
     assert np.abs(got_lse - want_lse)[seen].max() <= 4e-6 and (got_lse[~seen] < -1e29).all()

@@ -86,16 +86,19 @@ def difference_terms(q, k, v, do, mask=None, causal=False):
 
 
 def check_backward(dev, q, k, v, do, tol=TOL, mask=None, causal=False, rows=slice(None), only=("dq", "dk", "dv")):
+    close_backward(run_fwd_bwd(dev, q, k, v, do, mask=mask, causal=causal)[2:], q, k, v, do, tol, mask, causal, rows, only)
+
+
+def close_backward(got, q, k, v, do, tol=TOL, mask=None, causal=False, rows=slice(None), only=("dq", "dk", "dv"), axes=(-1, -2)):
     """Rows and channels of dq, dk, dv (of the rows `rows`) by their own norms, and four roundings of 2^-24 of the terms that cancel in them."""
-    got = run_fwd_bwd(dev, q, k, v, do, mask=mask, causal=causal)
     want = oracle.attention_backward_f64(*heads(q, k, v, do), mask=mask, causal=causal)
     terms = difference_terms(q, k, v, do, mask=mask, causal=causal)
-    for name, g, w, t in zip(("dq", "dk", "dv"), got[2:], want[2:], terms):
+    for name, g, w, t in zip(("dq", "dk", "dv"), got, want[2:], terms):
         if name not in only:
             continue
         g, w, t = g[:1, :2, rows].astype(np.float64), np.asarray(w, np.float64)[:, :, rows], t[:, :, rows]
         assert np.isfinite(g).all(), name
-        for axis in (-1, -2):
+        for axis in axes:
             err, ref, cancel = (np.linalg.norm(x, axis=axis) for x in (g - w, w, t))
             bound = tol * ref + 2.0 ** -22 * cancel
             assert (err <= bound).all(), (name, axis, (err[bound > 0] / bound[bound > 0]).max() * tol)
