@@ -137,8 +137,10 @@ static bool mask_wants_4_waves(arhip_device *dev, int64_t heads, int64_t N, int6
 // serve them: B8 H12 N197 D64 7.8 -> 7.0 us, B4 H16 N256 D128 11.8 -> 9.0 us, B32 H12 N64 D64 9.1 -> 5.6 us, B8 H12 N400 D64
 // 27.8 -> 12.9 us).  special: 8-bit launches with an additive mask, K scales over a number of keys that is no power of two or
 // the logits export take the general kernel with 4 waves of 32 queries, as do K/V too large for 32-bit offsets.
-// (ARHIP_ATTN_WAVES, read once when the device is opened, is a tuning aid; results do not depend on it.  4: the general
-// kernel; 8, 40: the pipelined kernel with 8 / 4 waves; 42, 22: with two groups of 4 / 2 waves.)
+// (ARHIP_ATTN_WAVES, read once when the device is opened, is a tuning aid.  4: the general
+// kernel; 8, 40: the pipelined kernel with 8 / 4 waves, the same bits; 42, 22: with two groups of 4 / 2 waves, whose sums have exponent references of
+// their own: bf16 and 8-bit results differ by the rounding of P to bf16, 2^-8 of the largest |V| at most, and so they do with the size of the grid, by
+// which pipe_form chooses.)
 static bool use_pipe(arhip_device *dev, bool special, int64_t N, int64_t kv_token_stride)
 {
     return !special && dev->attn_waves != 4 && pipe_addressable(N, kv_token_stride, 2);
