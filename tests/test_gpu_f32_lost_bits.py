@@ -167,3 +167,31 @@ def test_backward_zero_channels(dev, shape, which):
     if which != "all" and shape[2] <= 257:
         x[which][..., 3, 41:] = F(2.0 ** -30)
         check_backward(dev, *x.values())
+
+
+@pytest.mark.parametrize("gap", [8, 14, 20, 28])
+@pytest.mark.parametrize("shape", [(1, 2, 32, 64), (1, 4, 300, 64), (16, 16, 100, 64), (1, 16, 800, 64), (8, 16, 260, 64), (1, 4, 300, 128), (4, 12, 200, 128)], ids=str)
+def test_backward_channels_that_few_have(dev, shape, gap):
+    """A channel of K, of Q and of dO that is zero wherever keys and queries attend to each other: what dQ, dK and dV have of it is made of probabilities
+    `gap` below the others alone."""
+    N, half = shape[2], shape[2] // 2
+    last = -(-half // 128) * 128  # whole blocks of the later half of the keys
+    q, k, v, do = (synth.normal(1020 + i, shape) for i in range(4))
+    q[..., 0], k[..., 0] = 4, 0
+    k[..., ::2, 0] = -gap / 4 * np.sqrt(shape[3])
+    check_backward(dev, q, k, v, do, TOL + gap * 2.0 ** -19, only=("dq",))
+    q, k, v, do = (synth.normal(1030 + i, shape) for i in range(4))
+    mask = np.zeros((N, N), F)
+    mask[:half, half:] = -gap
+    q[..., half:, 9] = do[..., half:, 9] = 0
+    if last < N:
+        check_backward(dev, q, k, v, do, TOL + gap * 2.0 ** -19, mask=mask, rows=slice(last, None), only=("dk", "dv"))
+
+
+@pytest.mark.parametrize("e", [14, 20, 28])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_backward_small_rows_of_v(dev, shape, e):
+    """The earlier half of the rows of V 2^-e of the later: under the causal mask early queries see no others, dP is small, and dQ with it."""
+    q, k, v, do = (synth.normal(1040 + i, shape) for i in range(4))
+    v[..., : shape[2] // 2, :] *= F(2.0 ** -e)
+    check_backward(dev, q, k, v, do, causal=True, rows=slice(1, None))
