@@ -89,9 +89,14 @@ static int sage_quant_impl(arhip_device *dev, const void *x, const int64_t x_str
     // workgroup's reading of its whole head stays below 32 MB over all of them (a few us of L2 bandwidth), two where a head's partial
     // sums are no more than a workgroup's own 64 rows.
     const bool one = smooth && block > 1 && nchunk * D <= SMOOTH_LDS_FLOATS && rows * D * (dtype == ARHIP_F32 ? 4 : 2) * nblk <= (32 << 20);
-    const bool two = smooth && block > 1 && !one && nchunk <= 32;
+    // bf16 in blocks of 64 tokens (smooth_quant_64_kernel): two launches while the workgroups' reading of the partial sums stays below 40 MB and
+    // does not slow down a grid that fills the chip several times.  us, two / three launches: B3 H4 N4096 D128 10.3 / 11.6, H16
+    // N3000 12.2 / 13.5, H24 N1400 D64 11.8 / 13.6, B2 H16 N3000 D128 19.0 / 19.4, B4 H24 N1030 (1632 workgroups) 16.5 / 16.3, H64 N2048 (2048)
+    // 18.5 / 18.3, B8 H40 N400 (2240) 22.5 / 20.8, B2 H8 N6150 (76 MB) 18.3 / 17.3, B2 H32 N4096 (134 MB) 33.7 / 31.2.
+    const bool by64 = smooth && !one && block == MEAN_CHUNK && dtype == ARHIP_BF16;
+    const int64_t wgs64 = B * H * ((nchunk * D + 127) / 128);
+    const bool two = smooth && block > 1 && !one && (by64 ? wgs64 <= 6 * (int64_t)dev->cus && wgs64 * nchunk * D * 4 <= (40 << 20) : nchunk <= 32);
     if (smooth && !one) {
-        // (two channels per thread while that leaves every SIMD less than two waves of it)
         auto partial = [&](auto t, auto ch) {
             using T = decltype(t);
             constexpr int C = decltype(ch)::value;
@@ -99,13 +104,24 @@ static int sage_quant_impl(arhip_device *dev, const void *x, const int64_t x_str
             hipLaunchKernelGGL((k_mean_partial_kernel<T, C>), dim3((unsigned)((nchunk + cpb - 1) / cpb), (unsigned)(B * H)), dim3(256), 0,
                                dev->stream, (const T *)x, (float *)workspace, (int)N, (int)D, nchunk, lay);
         };
-        auto typ = [&](auto ch) { dtype == ARHIP_F32 ? partial(0.f, ch) : partial((uint16_t)0, ch); };
-        if (B * H * nchunk * (D / 2) <= 2 * 4 * 64 * (int64_t)dev->cus) typ(std::integral_constant<int, 2>{});
-        else typ(std::integral_constant<int, 8>{});
+        // (f32: two channels per thread while that leaves every SIMD less than two waves of it)
+        if (dtype == ARHIP_BF16) partial((uint16_t)0, std::integral_constant<int, 2>{});
+        else if (B * H * nchunk * (D / 2) <= 2 * 4 * 64 * (int64_t)dev->cus) partial(0.f, std::integral_constant<int, 2>{});
+        else partial(0.f, std::integral_constant<int, 8>{});
         if (!two) hipLaunchKernelGGL(k_mean_final_kernel, dim3((unsigned)(B * H)), dim3((unsigned)D), 0, dev->stream,
                            (const float *)workspace, mean, (int)N, (int)D, nchunk);
     }
-    if (one || two) {
+    if (by64) {
+        auto go = [&](auto d, auto f8, auto pt) {
+            constexpr int DD = decltype(d)::value;
+            hipLaunchKernelGGL((smooth_quant_64_kernel<DD, decltype(f8)::value, decltype(pt)::value>),
+                               dim3((unsigned)(wgs64 / (B * H)), (unsigned)(B * H)), dim3(256), 0, dev->stream, (const uint16_t *)x, x8, scales,
+                               (const float *)workspace, mean, (int)N, nchunk, lay);
+        };
+        auto part = [&](auto d, auto f8) { two ? go(d, f8, std::true_type{}) : go(d, f8, std::false_type{}); };
+        auto fmt = [&](auto d) { fp8 ? part(d, std::true_type{}) : part(d, std::false_type{}); };
+        D == 64 ? fmt(std::integral_constant<int, 64>{}) : fmt(std::integral_constant<int, 128>{});
+    } else if (one || two) {
         auto go = [&](auto t, auto f8, auto single) {
             using T = decltype(t);
             hipLaunchKernelGGL((smooth_quant_blocks_kernel<T, decltype(f8)::value, decltype(single)::value>),

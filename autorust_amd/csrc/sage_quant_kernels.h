@@ -100,7 +100,7 @@ template <typename T, int C>
 __device__ __forceinline__ void k_mean_chunk(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, int bh, int c, int g)
 {
     float s[C];
-    sum_rows<(C == 8 ? 16 : 32), C>(x, lay.head(bh) + g * C, lay.st, c * MEAN_CHUNK, min(N, (c + 1) * MEAN_CHUNK), s);
+    sum_rows<(C == 8 ? 16 : sizeof(T) == 2 ? 64 : 32), C>(x, lay.head(bh) + g * C, lay.st, c * MEAN_CHUNK, min(N, (c + 1) * MEAN_CHUNK), s);
     float *o = part + ((size_t)bh * nchunk + c) * D + g * C;
     if constexpr (C == 8) {
         *(float4 *)o = make_float4(s[0], s[1], s[2], s[3]);
@@ -111,8 +111,9 @@ __device__ __forceinline__ void k_mean_chunk(const T *x, float *part, int N, int
 }
 
 // One thread owns C adjacent channels of one 64-token chunk: D/C threads read a whole row
-// (coalesced), 256/(D/C) chunks per workgroup.  C = 8 for the memory's rate, 2 where the tensor is small and a
-// wave's own instructions are the time (B2 Hkv8 N2016 D64: 6.0 -> 4.5 us).
+// (coalesced), 256/(D/C) chunks per workgroup.  bf16: C = 2, a whole chunk's rows in flight and four times the waves of C = 8
+// (B4 H32 N8192 D128 55 -> 48 us, 5.6 TB/s, B2 H32 N4096 15.4 -> 11.7, H32 N2048 6.7 -> 4.2).  f32: C = 8 for the memory's rate, 2 where the tensor
+// is small and a wave's own instructions are the time (B2 Hkv8 N2016 D64: 6.0 -> 4.5 us).
 template <typename T, int C>
 __device__ __forceinline__ void k_mean_partial_body(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, const dim3 bid)
 {
@@ -327,6 +328,102 @@ __global__ void __launch_bounds__(smooth_threads<ONE>()) smooth_quant_blocks_ker
     }
     __syncthreads();
     quant_block<T, true, FP8, NT>(x, x8, scales, mu, N, D, blk, nblk, lay, blockIdx);
+}
+
+// The codes of 8 values that share a scale of ordinary size: quantise8 without what only matters elsewhere.  |v inv| is at most 127 (448) and
+// a rounding or two, so int8 needs no clamp, and the sum with 1.5 * 2^23 is rounded to a whole number as rintf rounds, whose last byte is the
+// code; a NaN's is 0, as the conversion's is, where its last bits are (every NaN that comes of bf16 values).  (v_med3_f32 takes the
+// smallest of its operands where one is NaN: -448, as fmaxf does.)
+template <bool FP8>
+__device__ __forceinline__ uint2 quantise8_usual(const float (&v)[8], float inv)
+{
+    uint32_t w[2];
+    if constexpr (FP8) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float c[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_fmed3f(v[4 * j + i] * inv, -448.0f, 448.0f);
+            int r = 0;
+            r = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], r, false);
+            r = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], r, true);
+            w[j] = (uint32_t)r;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32_t b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[i] = __float_as_uint(v[4 * j + i] * inv + 12582912.0f);
+            const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+            w[j] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+        }
+    }
+    return make_uint2(w[0], w[1]);
+}
+
+// quant_blocks<uint16_t, true, FP8> for blocks of 64 tokens, the same results: 16 bytes of 4 rows per thread, so that a workgroup has one block at
+// D = 128 and two at D = 64.  PART: the mean comes from the partial sums, which are read and added behind the requests of the rows (a
+// launch less); else it is there.
+// Bound: memory.  B4 H32 N8192 D128 (402 MB) 78 -> 66 us, B2 H32 N4096 D128 20 -> 16, B2 H32 N11403 D64 32 -> 25, against quant_blocks, which
+// issues twice as many instructions per value (8 to unpack, quantise and clamp one) and at D = 64 fills its threads half.
+template <int D, bool FP8, bool PART>
+__global__ void __launch_bounds__(256) smooth_quant_64_kernel(const uint16_t *x, int8_t *x8, float *scales, const float *part, float *mean,
+                                                              int N, int nchunk, const XLayout lay)
+{
+    constexpr int GPR = D / 8, TPB = 16 * GPR, BLOCKS = 256 / TPB;  // threads per row and per block, blocks per workgroup
+    __shared__ float red[4], mu_of[PART ? D : 1];
+    const int tid = threadIdx.x, g = tid % GPR * 8;
+    // from the end: the rows that the sums were formed of last are those that a cache may still hold (B4 H32 N8192 D128 126 -> 122 us
+    // for the whole pre-pass)
+    const int bh = gridDim.y - 1 - blockIdx.y, c = (gridDim.x - 1 - blockIdx.x) * BLOCKS + tid / TPB;
+    const int r0 = c * 64 + tid % TPB / GPR;  // the thread's first row; the others are 16 apart
+    const uint16_t *src = x + lay.head(bh) + g;
+
+    uint4 raw[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) raw[i] = *(const uint4 *)(src + (size_t)min(r0 + 16 * i, N - 1) * lay.st);
+    float mu[8];
+    if constexpr (PART) {
+        if (tid < D) {
+            mu_of[tid] = mean_of_chunks(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
+            if (blockIdx.x == 0) mean[(size_t)bh * D + tid] = mu_of[tid];
+        }
+        __syncthreads();
+    }
+    const float *m = PART ? mu_of + g : mean + (size_t)bh * D + g;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mu[i] = m[i];
+    float v[4][8], mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t w[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[i][2 * j] = __uint_as_float(w[j] << 16) - mu[2 * j];
+            v[i][2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u) - mu[2 * j + 1];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(v[i][j]));
+    }
+    // (rows past the end repeat the last one, which is of the same block where the block has a row at all)
+    mx = lane_group_max<64>(mx);
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    const int w0 = tid / TPB * (TPB / 64);
+    mx = fmaxf(red[w0], red[w0 + 1]);
+    if constexpr (TPB == 256) mx = fmaxf(mx, fmaxf(red[2], red[3]));
+    const float scale = (mx > 0.f) ? mx / QFormat<FP8>::QMAX : 1.f;
+    const float inv = 1.f / scale;
+    if (c < nchunk && tid % TPB == 0) scales[(size_t)bh * nchunk + c] = scale;
+    const bool usual = scale > 0x1p-100f && scale < 0x1p100f;
+    int8_t *dst = x8 + (size_t)bh * N * D + g;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = r0 + 16 * i;
+        const uint2 q = usual ? quantise8_usual<FP8>(v[i], inv) : quantise8<FP8>(v[i], inv);
+        if (r < N) *(uint2 *)(dst + (size_t)r * D) = q;
+    }
 }
 
 template <typename T, bool SMOOTH, bool FP8 = false>

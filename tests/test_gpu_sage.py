@@ -338,3 +338,39 @@ def test_smoothing_quantiser_by_sequence_length(dev, D, B, H, N):
                 assert np.array_equal(mean.copyout(np.float32, mu.shape), mu)
                 assert np.array_equal(sc.copyout(np.float32, wants.shape), wants)
                 assert np.array_equal(x8.copyout(want8.dtype, want8.shape), want8), (dtype, fp8)
+
+
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("B,H,N,D", [(1, 2, 1025, 64), (2, 3, 2111, 128), (6, 30, 1100, 64), (8, 40, 400, 128)])
+def test_smoothing_quantiser_of_bf16_blocks_of_64(dev, B, H, N, D, strided):
+    """bf16 rows in blocks of 64 tokens (two launches, and three) against the same values as f32 rows, which take the general quantiser: the
+    same bits, also where a block's scale is infinite, tiny or of nothing, and where values are infinite or NaN."""
+    x = synth.normal(971, (B, H, N, D)) + np.float32(3.0) * synth.normal(972, (1, H, 1, D))
+    x[0, 1, 64:128] *= np.float32(2.0 ** -118)         # (its mean is the head's: the blocks behind it differ by it only)
+    x[B - 1, 0] *= np.float32(2.0 ** -121)             # scales of a whole head near the smallest normal number
+    x[B - 1, 0, :64] = np.float32(1e-40)
+    x[0, H - 1, 5, 3] = np.inf
+    x[0, H - 1, N - 1, 7] = np.nan
+    x[B - 1, H - 1, 70, 1], x[B - 1, H - 1, 71, 1] = np.float32(3e38), np.float32(-3e38)
+    x[B - 1, 1] = 0.0
+    bits = synth.to_bf16_bits(x)
+    got = {}
+    for dtype in (F32, BF16):
+        src = bits if dtype == BF16 else (bits.astype(np.uint32) << 16).view(np.float32)
+        if strided:
+            src = np.ascontiguousarray(src.transpose(0, 2, 1, 3))
+        for fp8 in (False, True):
+            with Bufs(dev) as bufs:
+                dx = bufs.put(src)
+                x8, sc, mean = bufs.new(x.size), bufs.new(B * H * ((N + 63) // 64) * 4), bufs.new(B * H * D * 4)
+                ws = bufs.new(dev.sage_quant_workspace(B, H, N, D))
+                if strided:
+                    if fp8:
+                        continue
+                    dev.sage_quant(dx, x8, sc, B, H, N, D, 64, dtype, mean=mean, workspace=ws, smooth=True, x_strides=(N * H * D, D, H * D))
+                else:
+                    (dev.sage_quant_fp8 if fp8 else dev.sage_quant)(dx, x8, sc, B, H, N, D, 64, dtype, mean=mean, workspace=ws, smooth=True)
+                got[dtype, fp8] = (mean.copyout(np.uint32, (B, H, D)), sc.copyout(np.uint32, (B, H, (N + 63) // 64)), x8.copyout(np.uint8, x.shape))
+    for fp8 in (False,) if strided else (False, True):
+        for a, b in zip(got[F32, fp8], got[BF16, fp8]):
+            assert np.array_equal(a, b), fp8
