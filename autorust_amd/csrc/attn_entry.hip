@@ -224,7 +224,7 @@ __device__ __forceinline__ FlashBwdParams bwd_params(const float *Q, const float
     p.q = Q; p.k = K; p.v = V; p.dout = dO; p.lse = LSE; p.delta = D;
     p.mask = has_mask ? M : nullptr;
     p.Hq = hq; p.Hkv = hkv; p.N = N;
-    p.nt = (int)gridDim.x;
+    p.nt_q = p.nt_kv = (int)gridDim.x;
     p.total_q = p.total_kv = (int)(gridDim.x * gridDim.y);
     p.lpt_q = p.lpt_kv = (int)gridDim.y;  // causal: longest tile first over all heads
     p.halves = p.total_q < 2 * 256;

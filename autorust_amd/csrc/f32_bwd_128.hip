@@ -3,6 +3,6 @@
 
 namespace arhip {
 
-void launch_f32_bwd_128(hipStream_t stream, const FlashBwdParams &p, bool causal, bool split) { launch_bwd<128, false>(stream, p, causal, split); }
+void launch_f32_bwd_128(hipStream_t stream, const FlashBwdParams &p, bool causal, BwdForm form) { launch_bwd<128, false>(stream, p, causal, form); }
 
 }  // namespace arhip

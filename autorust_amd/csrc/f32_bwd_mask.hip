@@ -3,10 +3,10 @@
 
 namespace arhip {
 
-void launch_f32_bwd_mask(hipStream_t stream, const FlashBwdParams &p, int D, bool causal, bool split)
+void launch_f32_bwd_mask(hipStream_t stream, const FlashBwdParams &p, int D, bool causal, BwdForm form)
 {
-    if (D == 64) launch_bwd<64, true>(stream, p, causal, split);
-    else launch_bwd<128, true>(stream, p, causal, split);
+    if (D == 64) launch_bwd<64, true>(stream, p, causal, form);
+    else launch_bwd<128, true>(stream, p, causal, form);
 }
 
 }  // namespace arhip

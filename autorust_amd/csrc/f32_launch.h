@@ -27,8 +27,8 @@ void launch_f32_forms(hipStream_t stream, const FlashF32Params &p, bool causal, 
 void launch_f32_64(hipStream_t stream, const FlashF32Params &p, bool causal, int form);
 void launch_f32_128(hipStream_t stream, const FlashF32Params &p, bool causal, int form, bool tile_sums);
 void launch_f32_mask(hipStream_t stream, const FlashF32Params &p, int D, bool causal, int form, bool tile_sums);
-void launch_f32_bwd_64(hipStream_t stream, const FlashBwdParams &p, bool causal, bool split);
-void launch_f32_bwd_128(hipStream_t stream, const FlashBwdParams &p, bool causal, bool split);
-void launch_f32_bwd_mask(hipStream_t stream, const FlashBwdParams &p, int D, bool causal, bool split);
+void launch_f32_bwd_64(hipStream_t stream, const FlashBwdParams &p, bool causal, BwdForm form);
+void launch_f32_bwd_128(hipStream_t stream, const FlashBwdParams &p, bool causal, BwdForm form);
+void launch_f32_bwd_mask(hipStream_t stream, const FlashBwdParams &p, int D, bool causal, BwdForm form);
 
 }  // namespace arhip

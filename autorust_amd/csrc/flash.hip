@@ -625,6 +625,29 @@ extern "C" int arhip_sage_fwd_fp8(arhip_device *dev, const uint8_t *q8, const ui
                          N, D, bq, bk, causal, out_dtype, scale, nullptr, nullptr, wait, secs, true);
 }
 
+// Rows per workgroup of the backward where several query heads share a K/V head.  A dK/dV workgroup has the tiles of all of them to go
+// through, and there are fewer such workgroups, so with 128 keys each long chains are left on a few compute units; 32 keys, with the
+// tiles dealt out between four waves, have a chain of a quarter and four times the workgroups, at 1.6 times the time per tile.  dQ keeps 128 rows.  In
+// us: what the longest chain takes, and what all workgroups take on all compute units (32 keys: one at a time, and the last ones
+// alone where there is not work for two rounds).
+// Whole backward, 128 keys / 32: D64 B5 H4/1 N1930 478 / 305, causal 447 / 183, B2 H16/4 N1024 231 / 134, causal 216 / 88, B1 H32/8 N512 113 / 50, B2
+// H32/8 N200 58 / 28, B4 H24/6 N70 25 / 18, B12 H16/4 N86 27 / 23, B2 H64/8 N610 causal 283 / 139, B3 H20/10 N188 27 / 32, B2 H40/10 N2048
+// 863 / 1190; D128 B2 H16/4 N1024 299 / 233, causal 295 / 155, B1 H32/8 N512 152 / 89, B8 H8/2 N512 163 / 133, B2 H8/2 N1200 331 / 187, B3 H24/6
+// N700 231 / 276, causal 219 / 177, B12 H32/8 N170 136 / 169.  (150 shapes with 2, 4 and 8 heads to a K/V head: 17 % less in the mean.)
+static BwdForm bwd_shared_form(int64_t kv_heads, int64_t group, int64_t N, int64_t D, bool causal, int cus)
+{
+    const int64_t t32 = (N + 31) / 32, t128 = (N + 127) / 128, wgs128 = kv_heads * (1 + group) * t128;
+    const int64_t kv32 = kv_heads * t32, q128 = kv_heads * group * t128;
+    const double steps = (double)(group * t32), most = causal ? 0.5 + 0.5 / t32 : 1.0, most128 = causal ? 0.5 + 0.5 / t128 : 1.0;
+    const double pairs = (double)(kv_heads * group) * (double)(t32 * t32) * most128;
+    const bool d64 = D == 64;
+    const double by128 = std::max((d64 ? 8 : 12) + (d64 ? 1.7 : 2.15) * (wgs128 > cus ? 1.1 : 1.0) * steps, d64 ? 2.6e-3 * pairs + 10 : 5.6e-3 * pairs + 15);
+    const double chain = d64 ? 8.5 + 0.55 * steps : 14 + 1.1 * steps, kv = d64 ? 8.5 + 0.55 * steps * most : 14 + 1.1 * steps * most;
+    const double q = d64 ? 6 + 1.7 * t32 * most128 : 6 + 2.6 * t32 * most128, full = (double)(kv32 + q128) / cus;
+    const double by32 = std::max(chain, (kv32 * kv + q128 * q) / cus + (full > 1 ? std::max(0.0, 2 - full) * q : 0.0));
+    return steps > 2 && by32 < by128 ? BWD_128_32 : BWD_128;
+}
+
 extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k, const float *v, const float *o,
                                const float *lse, const float *dout, float *dq, float *dk, float *dv, float *delta,
                                const float *mask, const int32_t *kv_len,
@@ -661,14 +684,15 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     const bool split = D == 128 ? N > 96 && wgs32 * 2 <= cus * (causal ? (N >= 2048 ? 4 : N >= 512 ? 3 : 2) : N >= 1200 ? 3 : 2)
                        : causal ? N > 32 && (wgs32 <= cus || (N >= 256 && wgs32 * (tiles32 + 1) * 5 <= cus * tiles32 * 12))
                                 : N > 32 && wgs32 <= cus * (N >= 512 ? 2 : 1);
-    const int rows_wg = split ? 32 : 128;
-    const int nt = (int)((N + rows_wg - 1) / rows_wg);
-    p.nt = nt;
+    const BwdForm form = split ? BWD_32 : Hq == Hkv ? BWD_128 : bwd_shared_form(B * Hkv, Hq / Hkv, N, D, causal != 0, dev->cus);
+    auto tiles = [&](int rows_wg) { return (int)((N + rows_wg - 1) / rows_wg); };
+    p.nt_q = tiles(form == BWD_32 ? 32 : 128);
+    p.nt_kv = tiles(form == BWD_128 ? 128 : 32);
     // causal: longest tile first over all heads, so that no head's long tiles are left for the end
     // Sums of dK and dV in two halves on grids of fewer than two workgroups per compute unit (as f32_tile_sums).
     p.halves = wgs < 2 * (int64_t)dev->cus;
-    p.total_q = (int)(nt * B * Hq);
-    p.total_kv = (int)(nt * B * Hkv);
+    p.total_q = (int)(p.nt_q * B * Hq);
+    p.total_kv = (int)(p.nt_kv * B * Hkv);
     p.lpt_q = causal ? (int)(B * Hq) : 0;
     p.lpt_kv = causal ? (int)(B * Hkv) : 0;
     // The row scalar: formed by the same launch on short heads, by one before it else.  The rule goes by the queries whose tiles a key
@@ -682,7 +706,7 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
         return a + x_bytes <= b || b + y_bytes <= a;
     };
     // (Head size 128 on 32 rows per workgroup has no registers for a third tensor.)
-    const bool own_d = mask == nullptr && !(D == 128 && split) && Hq / Hkv * N <= 512 && apart(o, q_bytes, dq, q_bytes) && apart(o, q_bytes, dk, kv_bytes) &&
+    const bool own_d = mask == nullptr && !(D == 128 && form != BWD_128) && Hq / Hkv * N <= 512 && apart(o, q_bytes, dq, q_bytes) && apart(o, q_bytes, dk, kv_bytes) &&
                        apart(o, q_bytes, dv, kv_bytes) && apart(o, q_bytes, delta, (uintptr_t)rows * 4);
     if (own_d) {
         p.o = o;
@@ -694,9 +718,9 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
         else hipLaunchKernelGGL((bwd_prep_kernel<128>), prep_grid, block, 0, dev->stream, o, dout, delta, rows);
     }
     auto launch = [&]() {
-        if (mask != nullptr) launch_f32_bwd_mask(dev->stream, p, (int)D, causal != 0, split);
-        else if (D == 64) launch_f32_bwd_64(dev->stream, p, causal != 0, split);
-        else launch_f32_bwd_128(dev->stream, p, causal != 0, split);
+        if (mask != nullptr) launch_f32_bwd_mask(dev->stream, p, (int)D, causal != 0, form);
+        else if (D == 64) launch_f32_bwd_64(dev->stream, p, causal != 0, form);
+        else launch_f32_bwd_128(dev->stream, p, causal != 0, form);
     };
     // dK and dV may lie where K and V do, of which a dK/dV workgroup reads the rows that it writes; those of dQ read all of them, first
     bool kv_kept = true;
