@@ -6,7 +6,9 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <atomic>
 #include <map>
+#include <mutex>
 #include <string>
 #include <string_view>
 #include <unordered_map>
@@ -41,7 +43,18 @@ struct arhip_device {
     std::vector<hipEvent_t> prof_pool;
     bool capturing = false;  // between arhip_graph_begin and arhip_graph_end
     int attn_waves = 0;      // ARHIP_ATTN_WAVES at open (0: choose by shape)
+    // What has been put on the stream, counted when it is there, and how much of that is known to be done; arhip_sync (device.hip)
+    std::atomic<uint64_t> issued{0}, finished{0};
+    std::atomic<bool> stream_shared{false};  // a caller has the stream, and may put work on it that is not counted
+    uint32_t *done = nullptr;                // pinned host memory: the last number that the stream has written there
+    uint32_t *done_at = nullptr;             // the device's address of it
+    hipEvent_t done_event = nullptr;
+    uint32_t done_number = 0;                // given out and put on the stream in order, under done_mutex
+    std::mutex done_mutex;
 };
+
+// Waits for all of the handle's work.
+int arhip_drain(arhip_device *dev);
 
 // Records a message for arhip_last_error() and returns `code`.
 int arhip_fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));

@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 
@@ -64,8 +65,24 @@ int arhip_call_timer::begin()
     return ARHIP_OK;
 }
 
+static void now_finished(arhip_device *dev, uint64_t upto)
+{
+    uint64_t was = dev->finished.load();
+    while (was < upto && !dev->finished.compare_exchange_weak(was, upto)) {
+    }
+}
+
+int arhip_drain(arhip_device *dev)
+{
+    const uint64_t upto = dev->issued.load();
+    ARHIP_HIP(hipStreamSynchronize(dev->stream));
+    now_finished(dev, upto);
+    return ARHIP_OK;
+}
+
 int arhip_call_timer::end()
 {
+    if (!dev->capturing) ++dev->issued;
     ARHIP_HIP(hipGetLastError());
     if (dev->capturing) return ARHIP_OK;
     if (p0) {
@@ -73,8 +90,10 @@ int arhip_call_timer::end()
         dev->prof_log.push_back({kernel, p0, p1});
     }
     if (wait) {
+        const uint64_t upto = dev->issued.load();
         ARHIP_HIP(hipEventRecord(dev->ev1, dev->stream));
         ARHIP_HIP(hipEventSynchronize(dev->ev1));
+        now_finished(dev, upto);
         float ms = 0.f;
         ARHIP_HIP(hipEventElapsedTime(&ms, dev->ev0, dev->ev1));
         if (secs) *secs = (double)ms * 1e-3;
@@ -132,6 +151,16 @@ extern "C" int arhip_open(int ordinal, arhip_device **out)
         delete d;
         return arhip_fail(ARHIP_EHIP, "arhip_open: stream/event creation failed: %s", hipGetErrorString(e));
     }
+    // (without it arhip_sync waits as the other calls do)
+    if (hipHostMalloc((void **)&d->done, sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&d->done_at, d->done, 0) != hipSuccess ||
+        hipEventCreateWithFlags(&d->done_event, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        if (d->done) (void)hipHostFree(d->done);
+        d->done = nullptr;
+    } else {
+        *d->done = 0;
+    }
     if (int rc = arhip_static_scratch_setup(ordinal)) {
         (void)arhip_close(d);
         return rc;
@@ -158,14 +187,21 @@ extern "C" int arhip_close(arhip_device *dev)
     (void)hipEventDestroy(dev->ev1);
     (void)hipEventDestroy(dev->tm0);
     (void)hipEventDestroy(dev->tm1);
+    if (dev->done_event) (void)hipEventDestroy(dev->done_event);
     (void)hipStreamDestroy(dev->stream);
+    if (dev->done) (void)hipHostFree(dev->done);
     delete dev;
     return ARHIP_OK;
 }
 
 extern "C" const char *arhip_arch(arhip_device *dev) { return dev ? dev->arch.c_str() : ""; }
 extern "C" int arhip_compute_units(arhip_device *dev) { return dev ? dev->cus : 0; }
-extern "C" void *arhip_stream(arhip_device *dev) { return dev ? (void *)dev->stream : nullptr; }
+extern "C" void *arhip_stream(arhip_device *dev)
+{
+    if (!dev) return nullptr;
+    dev->stream_shared = true;
+    return (void *)dev->stream;
+}
 
 #define ARHIP_DEV(dev)                                              \
     do {                                                            \
@@ -187,7 +223,7 @@ extern "C" int arhip_free(arhip_device *dev, void *dptr)
 {
     ARHIP_DEV(dev);
     if (!dptr) return ARHIP_OK;
-    ARHIP_HIP(hipStreamSynchronize(dev->stream));
+    if (int rc = arhip_drain(dev)) return rc;
     ARHIP_HIP(hipFree(dptr));
     return ARHIP_OK;
 }
@@ -198,8 +234,8 @@ extern "C" int arhip_copyin(arhip_device *dev, void *dst, const void *host, size
     if (bytes == 0) return ARHIP_OK;
     ARHIP_REQUIRE(dst && host, "arhip_copyin: null pointer");
     ARHIP_HIP(hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, dev->stream));
-    ARHIP_HIP(hipStreamSynchronize(dev->stream));  // the host buffer may be reused on return
-    return ARHIP_OK;
+    ++dev->issued;
+    return arhip_drain(dev);  // the host buffer may be reused on return
 }
 
 extern "C" int arhip_copyout(arhip_device *dev, void *host, const void *src, size_t bytes)
@@ -208,8 +244,8 @@ extern "C" int arhip_copyout(arhip_device *dev, void *host, const void *src, siz
     if (bytes == 0) return ARHIP_OK;
     ARHIP_REQUIRE(host && src, "arhip_copyout: null pointer");
     ARHIP_HIP(hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, dev->stream));
-    ARHIP_HIP(hipStreamSynchronize(dev->stream));
-    return ARHIP_OK;
+    ++dev->issued;
+    return arhip_drain(dev);
 }
 
 extern "C" int arhip_copy_d2d(arhip_device *dev, void *dst, const void *src, size_t bytes)
@@ -218,6 +254,7 @@ extern "C" int arhip_copy_d2d(arhip_device *dev, void *dst, const void *src, siz
     if (bytes == 0) return ARHIP_OK;
     ARHIP_REQUIRE(dst && src, "arhip_copy_d2d: null pointer");
     ARHIP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, dev->stream));
+    ++dev->issued;
     return ARHIP_OK;
 }
 
@@ -240,6 +277,7 @@ extern "C" int arhip_fill_zero(arhip_device *dev, void *dst, size_t bytes)
     if (blocks == 0) blocks = 1;
     hipLaunchKernelGGL(arhip_fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, dev->stream,
                        (uint32_t *)dst, words, (uint8_t *)dst + words * 4, tail);
+    ++dev->issued;
     ARHIP_HIP(hipGetLastError());
     return ARHIP_OK;
 }
@@ -254,11 +292,49 @@ extern "C" int arhip_mem_info(arhip_device *dev, size_t *free_bytes, size_t *tot
     return ARHIP_OK;
 }
 
+__global__ void arhip_done_kernel(uint32_t *at, uint32_t number)
+{
+    __hip_atomic_store(at, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A stream synchronisation sends a marker behind the kernels and waits for its signal, which takes 3 us more than a kernel of one thread that
+// writes a number to host memory, for which the host looks (a kernel of 18 us launched and waited for 28.1 -> 24.9 us, of 49 us 60.1 -> 56.9; by
+// an event 60, by a stream's value write 57.3, by polling the stream 60).  The marker goes behind that kernel, where nobody waits for it:
+// without one a device-wide synchronisation that follows would have to send its own (33 us for both instead of 30, 28 with stream
+// synchronisations, 30 against 33 where the host does 5 us of other work in between).  The end of every kernel writes back what it stored, so work that
+// begins later anywhere finds it.  Work that takes longer than the look is waited for as before, and so is a stream that others may use (or that
+// has failed); where nothing has been issued since the last wait there is nothing to do.
 extern "C" int arhip_sync(arhip_device *dev)
 {
     ARHIP_DEV(dev);
-    ARHIP_HIP(hipStreamSynchronize(dev->stream));
-    return ARHIP_OK;
+    if (dev->done == nullptr || dev->stream_shared || dev->capturing) return arhip_drain(dev);
+    const uint64_t upto = dev->issued.load();
+    if (dev->finished.load() >= upto) return ARHIP_OK;
+    uint32_t number;
+    hipError_t e;
+    {
+        std::lock_guard<std::mutex> lock(dev->done_mutex);
+        number = ++dev->done_number;
+        void *args[] = {&dev->done_at, &number};
+        e = hipLaunchKernel((const void *)arhip_done_kernel, dim3(1), dim3(1), args, 0, dev->stream);
+        if (e == hipSuccess) e = hipEventRecord(dev->done_event, dev->stream);
+    }
+    if (e == hipSuccess) {
+        constexpr auto LOOK = std::chrono::microseconds(300);
+        const auto until = std::chrono::steady_clock::now() + LOOK;
+        do {
+            for (int i = 0; i < 32; ++i) {
+                if ((int32_t)(__atomic_load_n(dev->done, __ATOMIC_ACQUIRE) - number) >= 0) {
+                    now_finished(dev, upto);
+                    return ARHIP_OK;
+                }
+                __builtin_ia32_pause();
+            }
+        } while (std::chrono::steady_clock::now() < until);
+    } else {
+        (void)hipGetLastError();
+    }
+    return arhip_drain(dev);
 }
 
 extern "C" int arhip_timer_start(arhip_device *dev)
@@ -298,7 +374,7 @@ extern "C" int arhip_kprof_collect_stats(arhip_device *dev, int kernel, double *
                                          double *min_secs, double *median_secs)
 {
     ARHIP_DEV(dev);
-    ARHIP_HIP(hipStreamSynchronize(dev->stream));
+    if (int rc = arhip_drain(dev)) return rc;
     double tot = 0.0;
     uint64_t n = 0;
     std::vector<double> each;
@@ -334,7 +410,7 @@ extern "C" int arhip_graph_begin(arhip_device *dev)
 {
     ARHIP_DEV(dev);
     ARHIP_REQUIRE(!dev->capturing, "arhip_graph_begin: a capture is already open");
-    ARHIP_HIP(hipStreamSynchronize(dev->stream));
+    if (int rc = arhip_drain(dev)) return rc;
     ARHIP_HIP(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
     dev->capturing = true;
     return ARHIP_OK;
@@ -372,7 +448,7 @@ extern "C" int arhip_graph_destroy(arhip_device *dev, void *graph_exec)
 {
     ARHIP_DEV(dev);
     if (!graph_exec) return ARHIP_OK;
-    ARHIP_HIP(hipStreamSynchronize(dev->stream));
+    if (int rc = arhip_drain(dev)) return rc;
     ARHIP_HIP(hipGraphExecDestroy((hipGraphExec_t)graph_exec));
     return ARHIP_OK;
 }
