@@ -90,12 +90,12 @@ static int sage_quant_impl(arhip_device *dev, const void *x, const int64_t x_str
     // sums are no more than a workgroup's own 64 rows.
     const bool one = smooth && block > 1 && nchunk * D <= SMOOTH_LDS_FLOATS && rows * D * (dtype == ARHIP_F32 ? 4 : 2) * nblk <= (32 << 20);
     // bf16 in blocks of 64 tokens (smooth_quant_64_kernel): two launches while the workgroups' reading of the partial sums stays below 40 MB and
-    // does not slow down a grid that fills the chip several times.  us, two / three launches: B3 H4 N4096 D128 10.3 / 11.6, H16
-    // N3000 12.2 / 13.5, H24 N1400 D64 11.8 / 13.6, B2 H16 N3000 D128 19.0 / 19.4, B4 H24 N1030 (1632 workgroups) 16.5 / 16.3, H64 N2048 (2048)
-    // 18.5 / 18.3, B8 H40 N400 (2240) 22.5 / 20.8, B2 H8 N6150 (76 MB) 18.3 / 17.3, B2 H32 N4096 (134 MB) 33.7 / 31.2.
+    // does not slow down a grid that fills the chip several times.  us, two / three launches: B3 H4 N4096 D128 10.9 / 11.7, H16 N3000 (752
+    // workgroups) 10.4 / 11.4, H24 N1400 D64 8.7 / 10.1, B4 H20 N1000 D128 (1280) 14.1 / 13.9, B2 H16 N3000 (1504) 17.4 / 16.1, B4 H24 N1030 (1632)
+    // 16.1 / 15.5, H64 N2048 (2048) 18.2 / 17.6, B2 H8 N6150 (76 MB) 20.5 / 17.8, B2 H32 N4096 (134 MB) 34.2 / 30.2.
     const bool by64 = smooth && !one && block == MEAN_CHUNK && dtype == ARHIP_BF16;
     const int64_t wgs64 = B * H * ((nchunk * D + 127) / 128);
-    const bool two = smooth && block > 1 && !one && (by64 ? wgs64 <= 6 * (int64_t)dev->cus && wgs64 * nchunk * D * 4 <= (40 << 20) : nchunk <= 32);
+    const bool two = smooth && block > 1 && !one && (by64 ? wgs64 <= 4 * (int64_t)dev->cus && wgs64 * nchunk * D * 4 <= (40 << 20) : nchunk <= 32);
     if (smooth && !one) {
         auto partial = [&](auto t, auto ch) {
             using T = decltype(t);

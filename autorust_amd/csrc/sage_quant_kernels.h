@@ -100,7 +100,7 @@ template <typename T, int C>
 __device__ __forceinline__ void k_mean_chunk(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, int bh, int c, int g)
 {
     float s[C];
-    sum_rows<(C == 8 ? 16 : sizeof(T) == 2 ? 64 : 32), C>(x, lay.head(bh) + g * C, lay.st, c * MEAN_CHUNK, min(N, (c + 1) * MEAN_CHUNK), s);
+    sum_rows<(C == 8 ? 16 : 32), C>(x, lay.head(bh) + g * C, lay.st, c * MEAN_CHUNK, min(N, (c + 1) * MEAN_CHUNK), s);
     float *o = part + ((size_t)bh * nchunk + c) * D + g * C;
     if constexpr (C == 8) {
         *(float4 *)o = make_float4(s[0], s[1], s[2], s[3]);
@@ -111,8 +111,9 @@ __device__ __forceinline__ void k_mean_chunk(const T *x, float *part, int N, int
 }
 
 // One thread owns C adjacent channels of one 64-token chunk: D/C threads read a whole row
-// (coalesced), 256/(D/C) chunks per workgroup.  bf16: C = 2, a whole chunk's rows in flight and four times the waves of C = 8
-// (B4 H32 N8192 D128 55 -> 48 us, 5.6 TB/s, B2 H32 N4096 15.4 -> 11.7, H32 N2048 6.7 -> 4.2).  f32: C = 8 for the memory's rate, 2 where the tensor
+// (coalesced), 256/(D/C) chunks per workgroup.  bf16: C = 2, four times the waves of C = 8
+// (B4 H32 N8192 D128 55.8 -> 54.0 us, 5.0 TB/s, B2 H32 N4096 15.9 -> 12.9, B2 H32 N11403 D64 19.4 -> 17.9; with the 64 rows of a chunk in flight
+// 52.5, 13.9 and 19.5, and B2 H40 N2020 D128 10.0 in place of 8.7).  f32: C = 8 for the memory's rate, 2 where the tensor
 // is small and a wave's own instructions are the time (B2 Hkv8 N2016 D64: 6.0 -> 4.5 us).
 template <typename T, int C>
 __device__ __forceinline__ void k_mean_partial_body(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, const dim3 bid)
@@ -139,34 +140,29 @@ __global__ void __launch_bounds__(256) k_mean_partial_kernel(const T *x, float *
     k_mean_partial_body<T, C>(x, part, N, D, nchunk, lay, blockIdx);
 }
 
-// (p[0] + p[D] + ...) / N: the mean of one channel from its nchunk partial sums, in chunk order (loads batched, adds in order)
+// (p[0] + p[D] + ...) / N: the mean of one channel from its nchunk partial sums, in chunk order (U loads batched, adds in order).
+// Its time is the number of load round trips, of a kernel of few waves or at the head of a workgroup's work; the last sum stands in for those past
+// the end and is not added (22 sums took 2 + 6 trips with batches of 32 and 8 and single ones: pre-pass of B2 H24 N1400 D128 13.8 -> 12.7 us, H16
+// N3000 11.1 -> 9.4).
+template <int U>
 __device__ __forceinline__ float mean_of_chunks(const float *p, int N, int D, int nchunk)
 {
     float tot = 0.f;
-    int c = 0;
-    // few waves run this kernel (one per 64 channels of a head), so its time is the number of load round trips
-    for (; c + 32 <= nchunk; c += 32) {
-        float v[32];
+    for (int c = 0; c < nchunk; c += U) {
+        float v[U];
 #pragma unroll
-        for (int i = 0; i < 32; ++i) v[i] = p[(size_t)(c + i) * D];
+        for (int i = 0; i < U; ++i) v[i] = p[(size_t)min(c + i, nchunk - 1) * D];
 #pragma unroll
-        for (int i = 0; i < 32; ++i) tot += v[i];
+        for (int i = 0; i < U; ++i)
+            if (c + i < nchunk) tot += v[i];
     }
-    for (; c + 8 <= nchunk; c += 8) {
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = p[(size_t)(c + i) * D];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) tot += v[i];
-    }
-    for (; c < nchunk; ++c) tot += p[(size_t)c * D];
     return tot / (float)N;
 }
 
 __device__ __forceinline__ void k_mean_final_body(const float *part, float *mean, int N, int D, int nchunk, const dim3 bid)
 {
     const int bh = bid.x, d = threadIdx.x;
-    mean[(size_t)bh * D + d] = mean_of_chunks(part + (size_t)bh * nchunk * D + d, N, D, nchunk);
+    mean[(size_t)bh * D + d] = mean_of_chunks<32>(part + (size_t)bh * nchunk * D + d, N, D, nchunk);
 }
 
 __global__ void k_mean_final_kernel(const float *part, float *mean, int N, int D, int nchunk)
@@ -323,7 +319,7 @@ __global__ void __launch_bounds__(smooth_threads<ONE>()) smooth_quant_blocks_ker
         __syncthreads();
     }
     if (tid < D) {
-        mu[tid] = ONE ? mean_of_chunks(sums + tid, N, D, nchunk) : mean_of_chunks(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
+        mu[tid] = ONE ? mean_of_chunks<8>(sums + tid, N, D, nchunk) : mean_of_chunks<32>(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
         if (blockIdx.x == 0) mean[(size_t)bh * D + tid] = mu[tid];
     }
     __syncthreads();
@@ -386,7 +382,7 @@ __global__ void __launch_bounds__(256) smooth_quant_64_kernel(const uint16_t *x,
     float mu[8];
     if constexpr (PART) {
         if (tid < D) {
-            mu_of[tid] = mean_of_chunks(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
+            mu_of[tid] = mean_of_chunks<32>(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
             if (blockIdx.x == 0) mean[(size_t)bh * D + tid] = mu_of[tid];
         }
         __syncthreads();
