@@ -693,6 +693,12 @@ extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k
     p.halves = wgs < 2 * (int64_t)dev->cus;
     p.total_q = (int)(p.nt_q * B * Hq);
     p.total_kv = (int)(p.nt_kv * B * Hkv);
+    // Head size 64, 128 rows: two workgroups fit a compute unit, and where there are more of them than that, but no more than three, the last dQ ones
+    // begin where the first ones end, alone with a dK/dV one that has as long to go: the sooner the first ones are done the better.  us,
+    // without / with priority: B8 H6 N789 (672 workgroups) 110 / 99, N700 (576) 92 / 86, B7 H12 N400 (672) 58 / 54, B8 H8 N700 (768) 112 / 103; B6 H10
+    // N789 (840) 128 / 133, B12 H12 N300 (864) 57 / 61, B4 H16 N512 (512) 55 / 59, causal B8 H6 N789 (longest first) 60 / 65.
+    const int64_t all = p.total_q + p.total_kv;
+    p.dq_ahead = D == 64 && form == BWD_128 && !causal && all > 2 * cus && all <= 3 * cus;
     p.lpt_q = causal ? (int)(B * Hq) : 0;
     p.lpt_kv = causal ? (int)(B * Hkv) : 0;
     // The row scalar: formed by the same launch on short heads, by one before it else.  The rule goes by the queries whose tiles a key

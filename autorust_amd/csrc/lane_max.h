@@ -49,12 +49,16 @@ __device__ __forceinline__ float xrow_max(float x)  // of lane and lane ^ 16
     const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-__device__ __forceinline__ float lane_sum(float x)
+__device__ __forceinline__ float lane_sum_16(float x)  // of each aligned group of 16, in every lane of it
 {
     x += dpp_read<0xB1>(x);
     x += dpp_read<0x4E>(x);
     x += dpp_read<0x141>(x);
-    x += dpp_read<0x140>(x);
+    return x + dpp_read<0x140>(x);
+}
+__device__ __forceinline__ float lane_sum(float x)
+{
+    x = lane_sum_16(x);
     uint32_t u = __float_as_uint(x);
     const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
     x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
