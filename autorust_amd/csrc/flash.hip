@@ -628,24 +628,39 @@ extern "C" int arhip_sage_fwd_fp8(arhip_device *dev, const uint8_t *q8, const ui
 // Rows per workgroup of the backward where several query heads share a K/V head.  A dK/dV workgroup has the tiles of all of them to go
 // through, and there are fewer such workgroups, so with 128 keys each long chains are left on a few compute units; 32 keys, with the
 // tiles dealt out between four waves, have a chain of a quarter and four times the workgroups, at 1.6 times the time per tile.  dQ keeps 128 rows.  In
-// us: what the longest chain takes, and what all workgroups take on all compute units (32 keys: one at a time, and the last ones
-// alone where there is not work for two rounds).
+// us: what the longest chain takes, and what all workgroups take on all compute units (one at a time, and the last ones alone where
+// there is not work for two rounds); 32 keys are taken where they are ahead by more than the estimate is wrong by.
 // Whole backward, 128 keys / 32: D64 B5 H4/1 N1930 478 / 305, causal 447 / 183, B2 H16/4 N1024 231 / 134, causal 216 / 88, B1 H32/8 N512 113 / 50, B2
 // H32/8 N200 58 / 28, B4 H24/6 N70 25 / 18, B12 H16/4 N86 27 / 23, B2 H64/8 N610 causal 283 / 139, B3 H20/10 N188 27 / 32, B2 H40/10 N2048
 // 863 / 1190; D128 B2 H16/4 N1024 299 / 233, causal 295 / 155, B1 H32/8 N512 152 / 89, B8 H8/2 N512 163 / 133, B2 H8/2 N1200 331 / 187, B3 H24/6
-// N700 231 / 276, causal 219 / 177, B12 H32/8 N170 136 / 169.  (150 shapes with 2, 4 and 8 heads to a K/V head: 17 % less in the mean.)
+// N700 231 / 276, causal 219 / 177, B12 H32/8 N170 136 / 169.
+// Short heads, 32 keys beside 128: D128 B7 H40/10 N64 causal 64 / 57, B12 H24/6 N16 22 / 21.  (600 shapes with 2, 4 and 8 heads to a K/V head, D64
+// and 128: 17 % less in the mean, and none that loses more than 2 %; without the factor 18 % and seven that lose up to 24 %.)
 static BwdForm bwd_shared_form(int64_t kv_heads, int64_t group, int64_t N, int64_t D, bool causal, int cus)
 {
-    const int64_t t32 = (N + 31) / 32, t128 = (N + 127) / 128, wgs128 = kv_heads * (1 + group) * t128;
-    const int64_t kv32 = kv_heads * t32, q128 = kv_heads * group * t128;
-    const double steps = (double)(group * t32), most = causal ? 0.5 + 0.5 / t32 : 1.0, most128 = causal ? 0.5 + 0.5 / t128 : 1.0;
-    const double pairs = (double)(kv_heads * group) * (double)(t32 * t32) * most128;
-    const bool d64 = D == 64;
-    const double by128 = std::max((d64 ? 8 : 12) + (d64 ? 1.7 : 2.15) * (wgs128 > cus ? 1.1 : 1.0) * steps, d64 ? 2.6e-3 * pairs + 10 : 5.6e-3 * pairs + 15);
-    const double chain = d64 ? 8.5 + 0.55 * steps : 14 + 1.1 * steps, kv = d64 ? 8.5 + 0.55 * steps * most : 14 + 1.1 * steps * most;
-    const double q = d64 ? 6 + 1.7 * t32 * most128 : 6 + 2.6 * t32 * most128, full = (double)(kv32 + q128) / cus;
-    const double by32 = std::max(chain, (kv32 * kv + q128 * q) / cus + (full > 1 ? std::max(0.0, 2 - full) * q : 0.0));
-    return steps > 2 && by32 < by128 ? BWD_128_32 : BWD_128;
+    const int64_t t32 = (N + 31) / 32, t128 = (N + 127) / 128, q128 = kv_heads * group * t128, kv128 = kv_heads * t128, kv32 = kv_heads * t32;
+    const double steps = (double)(group * t32);
+    if (steps <= 2) return BWD_128;
+    // of the tiles that a workgroup goes through without the causal mask
+    const double of32 = causal ? 0.5 + 0.5 / t32 : 1.0, of128 = causal ? 0.5 + 0.5 / t128 : 1.0;
+    // workgroups of dK/dV that take kv each in the mean, `chain` the longest, and of dQ, one on a compute unit
+    auto alone = [&](int64_t n_kv, double kv, double chain, double q) {
+        const double full = (double)(n_kv + q128) / cus;
+        return std::max(chain, full > 1 ? ((double)n_kv * kv + (double)q128 * q) / cus + std::max(0.0, 2 - full) * q : q);
+    };
+    double by128, by32;
+    if (D == 64) {
+        const double pairs = (double)(kv_heads * group) * (double)(t32 * t32) * of128;
+        by128 = std::max(8 + 1.7 * (kv128 + q128 > cus ? 1.1 : 1.0) * steps, 2.6e-3 * pairs + 10);
+        by32 = alone(kv32, 8.5 + 0.55 * steps * of32, 8.5 + 0.55 * steps, 6 + 1.7 * t32 * of128);
+    } else {
+        // (the row scalar: a third tensor for 128 keys on short heads, a launch of 5 us else)
+        const bool own_d = group * N <= 512;
+        const double step = own_d ? 2.7 : 2.15;
+        by128 = alone(kv128, 13 + step * steps * of128, 13 + step * steps, (own_d ? 15 : 13) + 2.2 * t32 * of128) + (own_d ? 0 : 5);
+        by32 = alone(kv32, 14 + 1.1 * steps * of32, 14 + 1.1 * steps, 11 + 2.4 * t32 * of128) + 5;
+    }
+    return by32 < 0.88 * by128 ? BWD_128_32 : BWD_128;
 }
 
 extern "C" int arhip_flash_bwd(arhip_device *dev, const float *q, const float *k, const float *v, const float *o,
