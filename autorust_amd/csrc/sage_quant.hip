@@ -108,8 +108,12 @@ static int sage_quant_impl(arhip_device *dev, const void *x, const int64_t x_str
         if (dtype == ARHIP_BF16) partial((uint16_t)0, std::integral_constant<int, 2>{});
         else if (B * H * nchunk * (D / 2) <= 2 * 4 * 64 * (int64_t)dev->cus) partial(0.f, std::integral_constant<int, 2>{});
         else partial(0.f, std::integral_constant<int, 8>{});
-        if (!two) hipLaunchKernelGGL(k_mean_final_kernel, dim3((unsigned)(B * H)), dim3((unsigned)D), 0, dev->stream,
-                           (const float *)workspace, mean, (int)N, (int)D, nchunk);
+        auto final = [&](auto d) {
+            constexpr int DD = decltype(d)::value;
+            hipLaunchKernelGGL((k_mean_final_kernel<DD>), dim3((unsigned)(B * H)), dim3(DD), 0, dev->stream, (const float *)workspace, mean,
+                               (int)N, nchunk);
+        };
+        if (!two) D == 64 ? final(std::integral_constant<int, 64>{}) : final(std::integral_constant<int, 128>{});
     }
     if (by64) {
         auto go = [&](auto d, auto f8, auto pt) {

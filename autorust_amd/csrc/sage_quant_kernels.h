@@ -145,10 +145,9 @@ __global__ void __launch_bounds__(256) k_mean_partial_kernel(const T *x, float *
 // the end and is not added (22 sums took 2 + 6 trips with batches of 32 and 8 and single ones: pre-pass of B2 H24 N1400 D128 13.8 -> 12.7 us, H16
 // N3000 11.1 -> 9.4).
 template <int U>
-__device__ __forceinline__ float mean_of_chunks(const float *p, int N, int D, int nchunk)
+__device__ __forceinline__ float mean_of_chunks(const float *p, int N, int D, int nchunk, float tot = 0.f, int c = 0)
 {
-    float tot = 0.f;
-    for (int c = 0; c < nchunk; c += U) {
+    for (; c < nchunk; c += U) {
         float v[U];
 #pragma unroll
         for (int i = 0; i < U; ++i) v[i] = p[(size_t)min(c + i, nchunk - 1) * D];
@@ -165,9 +164,28 @@ __device__ __forceinline__ void k_mean_final_body(const float *part, float *mean
     mean[(size_t)bh * D + d] = mean_of_chunks<32>(part + (size_t)bh * nchunk * D + d, N, D, nchunk);
 }
 
-__global__ void k_mean_final_kernel(const float *part, float *mean, int N, int D, int nchunk)
+// One wave or two per head: bound by the round trips to the partial sums, 1.1 us each, so 128 and 64 of them go together where there are as
+// many (D by the template: their offsets are immediates; from D = 128 at run time they spill 428 scalar registers).  B1 H64 N32768 D128 (512 sums) in
+// batches of 32 17.5 us, so 8.0; B4 H32 N8192 4.9 -> 4.7.
+template <int D>
+__global__ void __launch_bounds__(D) k_mean_final_kernel(const float *part, float *mean, int N, int nchunk)
 {
-    k_mean_final_body(part, mean, N, D, nchunk, blockIdx);
+    const int bh = blockIdx.x, d = threadIdx.x;
+    const float *p = part + (size_t)bh * nchunk * D + d;
+    float tot = 0.f;
+    int c = 0;
+    auto full = [&](auto u) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value;
+        float v[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) v[i] = p[(size_t)c * D + i * D];
+#pragma unroll
+        for (int i = 0; i < U; ++i) tot += v[i];
+        c += U;
+    };
+    while (nchunk - c >= 128) full(std::integral_constant<int, 128>{});
+    if (nchunk - c >= 64) full(std::integral_constant<int, 64>{});
+    mean[(size_t)bh * D + d] = mean_of_chunks<32>(p, N, D, nchunk, tot, c);
 }
 
 // FP8 E4M3 (OCP "FN" flavour: bias 7, no infinities, largest finite 448) of the reference's AR_FP8

@@ -374,3 +374,21 @@ def test_smoothing_quantiser_of_bf16_blocks_of_64(dev, B, H, N, D, strided):
     for fp8 in (False,) if strided else (False, True):
         for a, b in zip(got[F32, fp8], got[BF16, fp8]):
             assert np.array_equal(a, b), fp8
+
+
+@pytest.mark.parametrize("chunks", [33, 64, 65, 96, 128, 129, 161, 193, 257])
+def test_mean_of_a_head_over_many_chunks(dev, chunks):
+    """The mean from 33 partial sums of 64 tokens to several batches of them: the sums of the chunks added in order, the same bits."""
+    B, H, N, D = 1, 4, 64 * chunks - 31, 64
+    x = synth.normal(973, (B, H, N, D)) + np.float32(2.0)
+    with Bufs(dev) as bufs:
+        x8, sc, mean = bufs.new(x.size), bufs.new(B * H * chunks * 4), bufs.new(B * H * D * 4)
+        ws = bufs.new(dev.sage_quant_workspace(B, H, N, D))
+        dev.sage_quant(bufs.put(x), x8, sc, B, H, N, D, 64, F32, mean=mean, workspace=ws, smooth=True)
+        tot = np.zeros((B, H, D), np.float32)
+        for c in range(chunks):
+            part = np.zeros((B, H, D), np.float32)
+            for r in range(64 * c, min(64 * c + 64, N)):
+                part = part + x[:, :, r]
+            tot = tot + part
+        assert np.array_equal(mean.copyout(np.float32, tot.shape), tot / np.float32(N))
