@@ -140,28 +140,63 @@ __global__ void __launch_bounds__(256) k_mean_partial_kernel(const T *x, float *
     k_mean_partial_body<T, C>(x, part, N, D, nchunk, lay, blockIdx);
 }
 
-// (p[0] + p[D] + ...) / N: the mean of one channel from its nchunk partial sums, in chunk order (U loads batched, adds in order).
-// Its time is the number of load round trips, of a kernel of few waves or at the head of a workgroup's work; the last sum stands in for those past
-// the end and is not added (22 sums took 2 + 6 trips with batches of 32 and 8 and single ones: pre-pass of B2 H24 N1400 D128 13.8 -> 12.7 us, H16
-// N3000 11.1 -> 9.4).
-template <int U>
+// (p[0] + p[D] + ...) / N: the mean of one channel from its nchunk partial sums in memory, in chunk order, on top of tot, the first c of them.
+// Its time is the number of load round trips, of a kernel of few waves or at the head of a workgroup's work, and behind that the number of loads: up
+// to 32 at a time, the last sum stands in for those past the end and is not added, in the smallest of four sizes that holds what is left.
+// Pre-pass of f32 rows, us, with exact batches of 32, 8 and 1 / batches of 32 only / now: blocks of 64, B2 H24 N1400 D64 (22 sums) 13.7 / 12.9 / 12.5, B1
+// H8 N789 D128 (13) 9.6 / 8.8 / 8.3, B3 H12 N508 D128 (8) 9.9 / 10.9 / 9.9, B2 H4 N2169 D128 (34) 10.5 / 11.0 / 10.4; rows, B2 H4 N96 D128 (2) 7.2 / 7.5 / 7.2.
 __device__ __forceinline__ float mean_of_chunks(const float *p, int N, int D, int nchunk, float tot = 0.f, int c = 0)
 {
-    for (; c < nchunk; c += U) {
+    auto trip = [&](auto u) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value;
         float v[U];
 #pragma unroll
         for (int i = 0; i < U; ++i) v[i] = p[(size_t)min(c + i, nchunk - 1) * D];
 #pragma unroll
         for (int i = 0; i < U; ++i)
             if (c + i < nchunk) tot += v[i];
+        c += U;
+    };
+    while (nchunk - c > 16) trip(std::integral_constant<int, 32>{});
+    if (nchunk - c > 8) trip(std::integral_constant<int, 16>{});
+    else if (nchunk - c > 4) trip(std::integral_constant<int, 8>{});
+    else if (nchunk - c > 0) trip(std::integral_constant<int, 4>{});
+    return tot / (float)N;
+}
+
+// The same from all sums, in LDS: no trip to save there, and a read or a condition more is time that every workgroup waits, so exactly as many as
+// there are.  Pre-pass, us, in batches of 8 of which the last one is not full / now: bf16, B1 H8 N513 D64 5.0 / 4.9, B2 H6 N577 6.4 / 6.3, B2 H4 N700
+// D128 7.9 / 7.8, f32 to fp8, B4 H16 N60 D128 5.8 / 5.6.  FINE: batches of 4 and 2 in between (bf16, B1 H12 N960 D64 6.2 / 6.1, B1 H6 N300 4.7 / 4.6;
+// f32 to fp8, B4 H16 N60 D128 5.6 / 5.8).
+template <bool FINE>
+__device__ __forceinline__ float mean_of_lds_chunks(const float *p, int N, int D, int nchunk)
+{
+    float tot = 0.f;
+    int c = 0;
+    auto batches = [&](auto u) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value;
+        for (; c + U <= nchunk; c += U) {
+            float v[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i) v[i] = p[(c + i) * D];
+#pragma unroll
+            for (int i = 0; i < U; ++i) tot += v[i];
+        }
+    };
+    batches(std::integral_constant<int, 32>{});
+    batches(std::integral_constant<int, 8>{});
+    if constexpr (FINE) {
+        batches(std::integral_constant<int, 4>{});
+        batches(std::integral_constant<int, 2>{});
     }
+    batches(std::integral_constant<int, 1>{});
     return tot / (float)N;
 }
 
 __device__ __forceinline__ void k_mean_final_body(const float *part, float *mean, int N, int D, int nchunk, const dim3 bid)
 {
     const int bh = bid.x, d = threadIdx.x;
-    mean[(size_t)bh * D + d] = mean_of_chunks<32>(part + (size_t)bh * nchunk * D + d, N, D, nchunk);
+    mean[(size_t)bh * D + d] = mean_of_chunks(part + (size_t)bh * nchunk * D + d, N, D, nchunk);
 }
 
 // One wave or two per head: bound by the round trips to the partial sums, 1.1 us each, so 128 and 64 of them go together where there are as
@@ -185,7 +220,7 @@ __global__ void __launch_bounds__(D) k_mean_final_kernel(const float *part, floa
     };
     while (nchunk - c >= 128) full(std::integral_constant<int, 128>{});
     if (nchunk - c >= 64) full(std::integral_constant<int, 64>{});
-    mean[(size_t)bh * D + d] = mean_of_chunks<32>(p, N, D, nchunk, tot, c);
+    mean[(size_t)bh * D + d] = mean_of_chunks(p, N, D, nchunk, tot, c);
 }
 
 // FP8 E4M3 (OCP "FN" flavour: bias 7, no infinities, largest finite 448) of the reference's AR_FP8
@@ -337,7 +372,7 @@ __global__ void __launch_bounds__(smooth_threads<ONE>()) smooth_quant_blocks_ker
         __syncthreads();
     }
     if (tid < D) {
-        mu[tid] = ONE ? mean_of_chunks<8>(sums + tid, N, D, nchunk) : mean_of_chunks<32>(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
+        mu[tid] = ONE ? mean_of_lds_chunks<!(FP8 && sizeof(T) == 4)>(sums + tid, N, D, nchunk) : mean_of_chunks(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
         if (blockIdx.x == 0) mean[(size_t)bh * D + tid] = mu[tid];
     }
     __syncthreads();
@@ -400,7 +435,7 @@ __global__ void __launch_bounds__(256) smooth_quant_64_kernel(const uint16_t *x,
     float mu[8];
     if constexpr (PART) {
         if (tid < D) {
-            mu_of[tid] = mean_of_chunks<32>(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
+            mu_of[tid] = mean_of_chunks(part + (size_t)bh * nchunk * D + tid, N, D, nchunk);
             if (blockIdx.x == 0) mean[(size_t)bh * D + tid] = mu_of[tid];
         }
         __syncthreads();
