@@ -14,6 +14,15 @@ from gpu_util import Bufs
 
 pytestmark = pytest.mark.gpu
 WORDS = 64
+LOOKERS = 5  # handles that look, in turn: streams share the four hardware queues, and one on the queue of the work always comes behind it
+
+
+@pytest.fixture
+def lookers():
+    got = [Device(0) for _ in range(LOOKERS)]
+    yield got
+    for d in got:
+        d.close()
 
 
 class _Queue:
@@ -46,22 +55,19 @@ class _Queue:
 
 # (the look takes 300 us)
 @pytest.mark.parametrize("H,N,passes,least,most", [(8, 4096, 1, 5e-5, 2.9e-4), (24, 8192, 3, 1.5e-3, 1.0)], ids=["within the look", "beyond the look"])
-def test_the_last_of_a_queue_is_there(dev, H, N, passes, least, most):
-    other = Device(0)
-    try:
-        with Bufs(dev) as bufs:
-            queue = _Queue(dev, bufs, H, N, passes)
-            assert least < queue.seconds() < most
-            early = 0
-            for i in range(1, 40):
-                queue.submit(i)
-                if i % 2:
-                    early += (queue.seen_by(other) == np.float32(i)).all()
-                dev.sync()
-                assert (queue.seen_by(other) == np.float32(i + 1)).all(), i
-            assert early >= 1
-    finally:
-        other.close()
+def test_the_last_of_a_queue_is_there(dev, lookers, H, N, passes, least, most):
+    with Bufs(dev) as bufs:
+        queue = _Queue(dev, bufs, H, N, passes)
+        assert least < queue.seconds() < most
+        early = 0
+        for i in range(1, 41):
+            other = lookers[i % LOOKERS]
+            queue.submit(i)
+            if i % 2:
+                early += (queue.seen_by(other) == np.float32(i)).all()
+            dev.sync()
+            assert (queue.seen_by(other) == np.float32(i + 1)).all(), i
+        assert early >= 1
 
 
 def test_threads_with_queues_on_a_handle(dev):
@@ -86,10 +92,10 @@ def test_threads_with_queues_on_a_handle(dev):
     assert not wrong
 
 
-def test_copies_that_a_caller_put_on_the_stream():
+def test_copies_that_a_caller_put_on_the_stream(lookers):
     hip = ctypes.CDLL("libamdhip64.so")
     hip.hipMemcpyAsync.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_void_p]
-    dev, other = Device(0), Device(0)
+    dev = Device(0)
     try:
         with Bufs(dev) as bufs:
             n = 256 << 20
@@ -97,7 +103,8 @@ def test_copies_that_a_caller_put_on_the_stream():
             queue.submit(0)
             dev.sync()
             stream, early = dev.lib.arhip_stream(dev.handle), 0
-            for i in range(1, 9):
+            for i in range(1, 21):
+                other = lookers[i % LOOKERS]
                 for _ in range(20):
                     assert hip.hipMemcpyAsync(b.ptr, a.ptr, n, 3, stream) == 0  # device to device
                 assert hip.hipMemcpyAsync(queue.out.ptr, queue.table.ptr + i * WORDS * 4, WORDS * 4, 3, stream) == 0
@@ -108,4 +115,3 @@ def test_copies_that_a_caller_put_on_the_stream():
             assert early >= 1
     finally:
         dev.close()
-        other.close()
