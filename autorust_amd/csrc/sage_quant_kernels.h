@@ -112,8 +112,8 @@ __device__ __forceinline__ void k_mean_chunk(const T *x, float *part, int N, int
 
 // One thread owns C adjacent channels of one 64-token chunk: D/C threads read a whole row
 // (coalesced), 256/(D/C) chunks per workgroup.  bf16: C = 2, four times the waves of C = 8
-// (B4 H32 N8192 D128 55.8 -> 54.0 us, 5.0 TB/s, B2 H32 N4096 15.9 -> 12.9, B2 H32 N11403 D64 19.4 -> 17.9; with the 64 rows of a chunk in flight
-// 52.5, 13.9 and 19.5, and B2 H40 N2020 D128 10.0 in place of 8.7).  f32: C = 8 for the memory's rate, 2 where the tensor
+// (by kernel trace, B4 H32 N8192 D128 56 -> 48 us, 5.6 TB/s, B2 H32 N4096 14.6 -> 11.9, B2 H32 N11403 D64 15.8 -> 15.4; with the 64 rows of a chunk
+// in flight 3 % less, 8 and 9 % more, and B2 H40 N2020 D128 10.0 in place of 8.7).  f32: C = 8 for the memory's rate, 2 where the tensor
 // is small and a wave's own instructions are the time (B2 Hkv8 N2016 D64: 6.0 -> 4.5 us).
 template <typename T, int C>
 __device__ __forceinline__ void k_mean_partial_body(const T *x, float *part, int N, int D, int nchunk, const XLayout lay, const dim3 bid)
@@ -414,8 +414,8 @@ __device__ __forceinline__ uint2 quantise8_usual(const float (&v)[8], float inv)
 // quant_blocks<uint16_t, true, FP8> for blocks of 64 tokens, the same results: 16 bytes of 4 rows per thread, so that a workgroup has one block at
 // D = 128 and two at D = 64.  PART: the mean comes from the partial sums, which are read and added behind the requests of the rows (a
 // launch less); else it is there.
-// Bound: memory.  B4 H32 N8192 D128 (402 MB) 78 -> 66 us, B2 H32 N4096 D128 20 -> 16, B2 H32 N11403 D64 32 -> 25, against quant_blocks, which
-// issues twice as many instructions per value (8 to unpack, quantise and clamp one) and at D = 64 fills its threads half.
+// Bound: memory.  By kernel trace, B4 H32 N8192 D128 (402 MB, a part of which a cache holds) 84 -> 59 us, B2 H32 N4096 D128 21 -> 16, B2 H32 N11403
+// D64 28 -> 21, against quant_blocks, which issues twice as many instructions per value (8 to unpack, quantise and clamp one) and at D = 64 fills its threads half.
 template <int D, bool FP8, bool PART>
 __global__ void __launch_bounds__(256) smooth_quant_64_kernel(const uint16_t *x, int8_t *x8, float *scales, const float *part, float *mean,
                                                               int N, int nchunk, const XLayout lay)

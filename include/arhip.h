@@ -73,7 +73,9 @@ int arhip_copy_d2d(arhip_device *dev, void *dst, const void *src, size_t bytes);
 int arhip_fill_zero(arhip_device *dev, void *dst, size_t bytes);      /* fill kernel, async */
 int arhip_mem_info(arhip_device *dev, size_t *free_bytes, size_t *total_bytes);  /* memory_info */
 int arhip_sync(arhip_device *dev);                                    /* Prog::flush */
-/* the handle's stream as a hipStream_t, for callers that order their own work on it */
+/* the handle's stream as a hipStream_t, for callers that order their own work on it.  The caller may put work there that this library does not
+ * know of, so from the first call on, for the rest of the handle's life, arhip_sync waits by a stream synchronisation every time (some 3 us more
+ * behind short work than looking for the number that it otherwise has the stream write): do not ask for the stream only to keep it. */
 void *arhip_stream(arhip_device *dev);
 
 /* ---- timing on the handle's stream (HIP events) ---- */
